@@ -234,10 +234,11 @@ int oph_pc_huygens(oph_ctx* ctx, int nx, int ny, double pitch, double lambda, do
  * point amplitude, initial phase and plane carrier:
  *   U[i][j] = sum_n a_n exp(i (k z_n + phi_n)) exp(i k ((X_j - x_n)^2 + (Y_i - y_n)^2)/(2 z_n)),
  *   X_j = (j - nx/2) pitch, Y_i = (i - ny/2) pitch (row index i is y).
- * method OPH_FRESNEL_VALU sums it directly (FP64 phase reduction, FP32
- * accumulation); the MFMA methods evaluate the same field as the separable
- * complex contraction (pixels x points)(points x pixels) with chirp factors
- * rounded to BF16 or FP16 (optionally split hi + lo) and FP32 accumulation.
+ * The field is evaluated as the separable complex contraction (pixels x
+ * points)(points x pixels).  Method OPH_FRESNEL_VALU keeps the chirp factors in
+ * FP32 (phases reduced in FP64, FP32 sums of 256 points added in FP64); the
+ * MFMA methods round them to BF16 or FP16 (optionally split hi + lo) and
+ * accumulate in FP32.
  * When the points lie on few depth planes (at most 4096 distinct z, >= 256
  * points per plane on average) the contraction runs plane by plane with the
  * plane's chirp exp(i k (X^2 + Y^2)/(2 z_p)) applied once per plane (same

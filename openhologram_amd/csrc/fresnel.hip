@@ -1,5 +1,5 @@
-// fresnel.hip -- Fresnel point-cloud hologram on gfx950: a plain FP32 VALU
-// kernel and the separable form as an MFMA complex contraction.
+// fresnel.hip -- Fresnel point-cloud hologram on gfx950: the separable form of
+// the sum as an MFMA complex contraction in FP32, FP16 or BF16.
 //
 // Field (the direct Fresnel sum of CWO/cwoPLS.cpp:370-422, with the point
 // amplitude, its initial phase and the plane carrier exp(i k z_n)):
@@ -76,98 +76,140 @@ __global__ void fresnel_prep(const double* x, const double* y, const double* z, 
 }
 
 // ---------------------------------------------------------------------------
-// plain kernel: a 64x64 pixel tile per workgroup, 4x4 pixels per thread,
-// points staged in LDS; per (point, thread) the phase at the block centre in
-// FP64, per pixel the exact quadratic offset c (2 ex dx0 + ex^2 + 2 ey dy0 + ey^2)
-// in FP32 (a few turns at most).  Each staged batch of PT points is summed
-// in FP32 and the batch sums in FP64, so a pixel's rounding error does not
-// grow with the point count (1e6 points in one sum: ~2e-5 relative in FP32).
+// FP32 contraction (OPH_FRESNEL_VALU): the separable form U = A B^T with the
+// chirp factors in FP32 (phases reduced in FP64) on v_mfma_f32_32x32x2_f32.
+// A workgroup of 4 waves owns a 64 x 128 pixel tile; each wave contracts 32
+// rows x 64 columns.  The points come in chunks of F32_PTS: while a chunk is
+// contracted from one LDS buffer the next one's factors are generated into
+// the other (a lane owns one row or column, each wave a quarter of the
+// points, whose records are wave-uniform), one barrier per chunk.  A factor
+// costs one FP64 phase and one sin/cos for every row and column of the tile
+// instead of one per pixel: 192 per point and 8,192 pixels.  Sums run in FP32
+// over F32_BATCH points and in FP64 across batches, so a pixel's rounding
+// error does not grow with the point count.
+//
+// Bound by the matrix cores (128 cycles per point and 32 x 32 pixels) and, as
+// vector and matrix instructions do not overlap on a SIMD here, by the
+// generation in turn with them: 1280 x 720 with 20,000 points 1.30 ms = 113
+// TFLOP/s of the 152 a large FP32 product reaches; without generation 1.15 ms
+// (interleaving the two instruction by instruction changed nothing).  A sum
+// per pixel on the vector unit, with its sin and cos, took 4.95 ms.
 
-constexpr int PT = 256;
+constexpr int F32_PTS = 16, F32_BATCH = 256;
+constexpr int F32_R = 64, F32_C = 128;
 
-struct ValuArgs {
+struct F32Args {
     const FrPoint* pts;
-    int64_t n, chunk;
+    int64_t npad, chunk;   // multiples of KC
     int nx, ny;
     double p;
-    float2* partial;
+    float2* out;           // [chunks][ny][nx]
 };
 
-__global__ __launch_bounds__(256) void fresnel_valu(ValuArgs a) {
-    __shared__ double s_x[PT], s_y[PT], s_c[PT];
-    __shared__ float s_f0[PT], s_a[PT];
-    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 16 + tx;
-    const int c0 = blockIdx.x * 64 + tx * 4, r0 = blockIdx.y * 64 + ty * 4;
-    const double X0 = (c0 + 1.5 - a.nx / 2) * a.p, Y0 = (r0 + 1.5 - a.ny / 2) * a.p;
-    float ex[4], ey[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        ex[k] = (float)((k - 1.5) * a.p);
-        ey[k] = (float)((k - 1.5) * a.p);
-    }
-    double sre[4][4], sim[4][4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) sre[r][c] = sim[r][c] = 0.0;
+struct F32Lds {
+    float2 A[F32_PTS][F32_R];
+    float2 B[F32_PTS][F32_C];
+};
+
+__global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
+    __shared__ F32Lds lds[2];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = blockIdx.y * F32_R, col0 = blockIdx.x * F32_C;
+    const double Y = (row0 + lane - a.ny / 2) * a.p;
+    const double X0 = (col0 + lane - a.nx / 2) * a.p, X1 = (col0 + 64 + lane - a.nx / 2) * a.p;
     const int64_t pb = (int64_t)blockIdx.z * a.chunk;
-    const int64_t pe = min(a.n, pb + a.chunk);
-    for (int64_t base = pb; base < pe; base += PT) {
-        __syncthreads();
-        const int64_t j = base + tid;
-        if (j < pe) {
-            const FrPoint q = a.pts[j];
-            s_x[tid] = q.x;
-            s_y[tid] = q.y;
-            s_c[tid] = q.c;
-            s_f0[tid] = q.f0;
-            s_a[tid] = q.a;
+    const int nch = (int)((min(a.npad, pb + a.chunk) - pb) / F32_PTS);
+
+    // this wave's quarter of chunk c: the records (wave-uniform, by scalar
+    // loads), then one point's factors (k) into L
+    constexpr int PW = F32_PTS / 4;
+    typedef const __attribute__((address_space(4))) FrPoint* PtsPtr;
+    struct { double x, y, c; float f0, a; } q[PW];
+    auto records = [&](int c) {
+        PtsPtr p = (PtsPtr)(uintptr_t)(a.pts + pb + (int64_t)c * F32_PTS + wave * PW);
+#pragma unroll
+        for (int k = 0; k < PW; ++k) {
+            q[k].x = p[k].x;
+            q[k].y = p[k].y;
+            q[k].c = p[k].c;
+            q[k].f0 = p[k].f0;
+            q[k].a = p[k].a;
         }
-        __syncthreads();
-        const int cnt = (int)min((int64_t)PT, pe - base);
-        float re[4][4], im[4][4];
+    };
+    auto generate = [&](F32Lds& L) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) re[r][c] = im[r][c] = 0.f;
-        for (int k = 0; k < cnt; ++k) {
-            const double dx0 = X0 - s_x[k], dy0 = Y0 - s_y[k];
-            const double cc = s_c[k];
-            double t = fma(cc, fma(dx0, dx0, dy0 * dy0), (double)s_f0[k]);
-            const float f0 = (float)(t - rint(t));
-            const float cf = (float)cc, am = s_a[k];
-            const float dxf = (float)dx0, dyf = (float)dy0;
-            float A[4], B[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) A[c] = cf * fmaf(2.f * ex[c], dxf, ex[c] * ex[c]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) B[r] = cf * fmaf(2.f * ey[r], dyf, ey[r] * ey[r]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float ph = f0 + (A[c] + B[r]);
-                    re[r][c] = fmaf(am, cos_turns(ph), re[r][c]);
-                    im[r][c] = fmaf(am, sin_turns(ph), im[r][c]);
-                }
+        for (int k = 0; k < PW; ++k) {
+            const int pt = wave * PW + k;
+            const double dy = Y - q[k].y, d0 = X0 - q[k].x, d1 = X1 - q[k].x;
+            const float ty = (float)frac_turns(fma(q[k].c, dy * dy, (double)q[k].f0));
+            const float t0 = (float)frac_turns(q[k].c * (d0 * d0)), t1 = (float)frac_turns(q[k].c * (d1 * d1));
+            L.A[pt][lane] = make_float2(q[k].a * cos_turns(ty), q[k].a * sin_turns(ty));
+            L.B[pt][lane] = make_float2(cos_turns(t0), sin_turns(t0));
+            L.B[pt][64 + lane] = make_float2(cos_turns(t1), sin_turns(t1));
         }
+    };
+
+    f32x16 re[2], im[2];
+    double sre[2][16], sim[2][16];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+    for (int b = 0; b < 2; ++b) {
+        re[b] = im[b] = (f32x16)0.f;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                sre[r][c] += (double)re[r][c];
-                sim[r][c] += (double)im[r][c];
-            }
+        for (int v = 0; v < 16; ++v) sre[b][v] = sim[b][v] = 0.0;
     }
-    float2* dst = a.partial + (size_t)blockIdx.z * a.nx * a.ny;
+    const int wr = 32 * (wave & 1), wc = 64 * (wave >> 1);
+    if (nch > 0) {
+        records(0);
+        generate(lds[0]);
+    }
+    for (int c = 0; c < nch; ++c) {
+        // (the last chunk generates itself once more, into the idle buffer)
+        records(min(c + 1, nch - 1));
+        __syncthreads();   // chunk c is complete; the other buffer's readers are done
+        const F32Lds& L = lds[c & 1];
+        F32Lds& N = lds[(c + 1) & 1];
+        generate(N);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = r0 + r;
-        if (row >= a.ny) continue;
+        for (int k = 0; k < F32_PTS; k += 2) {
+            const int pt = k + (lane >> 5);
+            const float2 A = L.A[pt][wr + (lane & 31)];
+            float2 B[2];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int col = c0 + c;
-            if (col < a.nx) dst[(size_t)row * a.nx + col] = make_float2((float)sre[r][c], (float)sim[r][c]);
+            for (int b = 0; b < 2; ++b) B[b] = L.B[pt][wc + 32 * b + (lane & 31)];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                re[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, B[b].x, re[b], 0, 0, 0);
+                im[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, B[b].y, im[b], 0, 0, 0);
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                re[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(-A.y, B[b].y, re[b], 0, 0, 0);
+                im[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.y, B[b].x, im[b], 0, 0, 0);
+            }
+        }
+        if ((c + 1) % (F32_BATCH / F32_PTS) == 0 || c + 1 == nch) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    sre[b][v] += (double)re[b][v];
+                    sim[b][v] += (double)im[b][v];
+                }
+                re[b] = im[b] = (f32x16)0.f;
+            }
+        }
+    }
+    // register v of a lane: row 8 (v/4) + 4 (lane/32) + v%4, column lane%32
+    float2* dst = a.out + (size_t)blockIdx.z * a.nx * a.ny;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const int col = col0 + wc + 32 * b + (lane & 31);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int row = row0 + wr + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+            if (row < a.ny && col < a.nx)
+                dst[(size_t)row * a.nx + col] = make_float2((float)sre[b][v], (float)sim[b][v]);
         }
     }
 }
@@ -973,24 +1015,37 @@ extern "C" int oph_pc_fresnel(oph_ctx* ctx, int nx, int ny, double pitch, double
         OPH_LAUNCH(ctx, "fresnel_prep", fresnel_prep, dim3((unsigned)((npad + 255) / 256)), dim3(256), 0, dx, dy,
                    dz, da, dp, n, npad, lambda, fp, skip);
     if (method == OPH_FRESNEL_VALU) {
-        const int gx = (nx + 63) / 64, gy = (ny + 63) / 64;
-        int64_t chunks = (4LL * ctx->cu_count + (int64_t)gx * gy - 1) / ((int64_t)gx * gy);
-        const int64_t maxc = (n + 1023) / 1024;
-        if (chunks > maxc) chunks = maxc;
-        if (chunks > 16) chunks = 16;
-        if (chunks < 1) chunks = 1;
-        ValuArgs v{};
+        const int gx = (nx + F32_C - 1) / F32_C, gy = (ny + F32_R - 1) / F32_R;
+        // points split over grid.z so that the resident workgroups (two per
+        // CU) are filled: the split with the fewest point chunks per slot,
+        // at least 1024 points each (1280 x 720, 20,000 points: 120 tiles in
+        // 17 parts fill 3.98 of 4 rounds, 1.35 ms against 1.43 in 4 parts,
+        // 0.94 of a round) and at most 256 MiB of partial fields
+        const int64_t tiles_f = (int64_t)gx * gy, slots = 2LL * std::max(ctx->cu_count, 1);
+        int64_t chunks = 1;
+        double best = 1e300;
+        for (int64_t k = 1; k <= std::min<int64_t>(32, std::max<int64_t>(1, n / 1024)); ++k) {
+            if (k > 1 && (size_t)k * npix > ((size_t)1 << 25)) break;
+            const double cost = (double)((tiles_f * k + slots - 1) / slots) / (double)k;
+            if (cost < best * 0.98) {
+                best = cost;
+                chunks = k;
+            }
+        }
+        F32Args v{};
         v.pts = fp;
-        v.n = n;
-        v.chunk = n > 0 ? (n + chunks - 1) / chunks : 1;
+        v.npad = npad;
+        v.chunk = std::max<int64_t>(KC, (npad / KC + chunks - 1) / chunks * KC);
+        chunks = std::max<int64_t>(1, (npad + v.chunk - 1) / v.chunk);
         v.nx = nx;
         v.ny = ny;
         v.p = pitch;
-        v.partial = static_cast<float2*>(oph_scratch(ctx, SLOT_WORK0, chunks * npix * sizeof(float2)));
-        if (!v.partial) return OPH_ENOMEM;
-        OPH_LAUNCH(ctx, "fresnel_valu", fresnel_valu, dim3(gx, gy, (unsigned)chunks), dim3(16, 16), 0, v);
-        OPH_LAUNCH(ctx, "fresnel_sum_chunks", fresnel_sum_chunks, dim3((unsigned)((npix + 255) / 256)), dim3(256),
-                   0, v.partial, (int)chunks, (int64_t)npix, o);
+        v.out = chunks == 1 ? o : static_cast<float2*>(oph_scratch(ctx, SLOT_WORK0, chunks * npix * sizeof(float2)));
+        if (!v.out) return OPH_ENOMEM;
+        OPH_LAUNCH(ctx, "fresnel_valu", fresnel_f32, dim3(gx, gy, (unsigned)chunks), dim3(256), 0, v);
+        if (chunks > 1)
+            OPH_LAUNCH(ctx, "fresnel_sum_chunks", fresnel_sum_chunks, dim3((unsigned)((npix + 255) / 256)), dim3(256),
+                       0, v.out, (int)chunks, (int64_t)npix, o);
     } else {
         MfmaArgs m{};
         m.pts = fp;

@@ -126,3 +126,18 @@ def test_fresnel_1e6pts_4096sq_sampled(ctx):
             assert err < FR1E6_GENERAL_BOUND[m]
     finally:
         del os.environ["OPH_FRESNEL_PLANES"]
+
+
+@pytest.mark.parametrize("nx,ny,n", [(1, 1, 1), (128, 64, 16), (129, 65, 33), (97, 200, 257), (300, 70, 5003)])
+def test_fresnel_f32_contraction_edges(ctx, nx, ny, n):
+    """FP32 contraction at the edges of its 64 x 128 tiles, 16-point chunks,
+    256-point batches and point splits.  Bound: each term carries the rounding
+    of two reduced phases (2^-25 turns each, 4e-7 rad together at most), three
+    FP32 products and an FP32 sum of 256 terms (well under 1e-6 together for
+    terms of random phase): 2e-6 relative in the 2-norm."""
+    print(f"case: fresnel f32 {nx}x{ny} P={n}", flush=True)
+    x, y, p, z, a, ph = scenes.fresnel_points(n, planes=5, seed=n, half=0.6e-3)
+    U = ctx.fresnel(nx, ny, 8e-6, 532e-9, x, y, z, a, ph, method="valu")
+    err = rel_l2(U, O.fresnel(nx, ny, 8e-6, 532e-9, x, y, z, a, ph))
+    print("rel-L2", err)
+    assert err < 2e-6

@@ -3,10 +3,12 @@
 // Replaces the KETI generator loop (K/ophgen_pointcloud/ophgen_pointcloud.cpp:
 // 195-249) and its CUDA kernel (K/ophgen_pointcloud_gpu/ophgen_pointcloud_gpu.cpp:
 // 391-415).  Same field, different machine mapping:
-//   * a workgroup owns a 64x64 pixel tile, each thread a 4x4 pixel block, and
-//     accumulates the complex field in registers (the reference does one
-//     global read-modify-write per point per pixel);
-//   * points are staged 256 at a time in LDS and read by broadcast;
+//   * a workgroup owns a 64x64 pixel tile and accumulates the complex field in
+//     registers (the reference does one global read-modify-write per point
+//     per pixel); tiles far enough from the points sum them as a separable
+//     contraction on the FP32 matrix cores (below), the others directly:
+//   * each thread owns a 4x4 pixel block, points are staged 256 at a time in
+//     LDS and read by broadcast;
 //   * the phase k r needs ~1e6 rad of range at 1e-6 rad resolution, beyond
 //     FP32: per (point, thread) the distance r0 to the block centre is formed
 //     in FP64 and reduced to a fraction of a turn in FP64; per pixel the
@@ -27,6 +29,9 @@
 //   X_j = (j - nx/2) p, Y_i = (i - ny/2) p, r = |(X_j - x_n, Y_i - y_n, z_n + z)|;
 // there 1/r = (1/r0)(1 + q/r0^2)^(-1/2) ~ (1/r0)(1 - q/(2 r0^2)) per pixel
 // (relative error 3/8 (q/r0^2)^2 < 1e-8 wherever the phase expansion holds).
+#include <algorithm>
+#include <cmath>
+
 #include "oph_internal.h"
 
 namespace {
@@ -35,6 +40,7 @@ constexpr int TPB_X = 16, TPB_Y = 16;     // threads per workgroup
 constexpr int BX = 4, BY = 4;             // pixels per thread
 constexpr int TILE_X = TPB_X * BX, TILE_Y = TPB_Y * BY;
 constexpr int PBATCH = TPB_X * TPB_Y;     // points staged per batch
+constexpr int RS_MINPTS = 256;            // points per grid.z chunk, at least
 
 struct RsArgs {
     const double* x;
@@ -54,13 +60,19 @@ struct RsArgs {
     float2* partial;        // [chunks][ny][nx]
 };
 
-template <bool HUYGENS>
-__global__ __launch_bounds__(256) void rs_accumulate(RsArgs a) {
-    __shared__ double s_x[PBATCH], s_y[PBATCH], s_zz[PBATCH], s_ph[PBATCH];
-    __shared__ float s_a[PBATCH];
+struct RsStage {
+    double x[PBATCH], y[PBATCH], zz[PBATCH], ph[PBATCH];
+    float a[PBATCH];
+};
 
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int tid = ty * TPB_X + tx;
+// A sin and cos per pixel and point, for tiles too close to the points for
+// the contraction below.
+template <bool HUYGENS>
+__device__ __forceinline__ void rs_tile_direct(const RsArgs& a, RsStage& S) {
+    double *s_x = S.x, *s_y = S.y, *s_zz = S.zz, *s_ph = S.ph;
+    float* s_a = S.a;
+    const int tid = threadIdx.x;
+    const int tx = tid % TPB_X, ty = tid / TPB_X;
     const int c0 = blockIdx.x * TILE_X + tx * BX;
     const int r0 = blockIdx.y * TILE_Y + ty * BY;
     // block centre (KETI: X = (col + 1/2) px - Lx/2, Y = Ly/2 - (row + 1/2) py)
@@ -178,6 +190,250 @@ __global__ __launch_bounds__(256) void rs_accumulate(RsArgs a) {
             if (col < a.nx) dst[(size_t)row * a.nx + col] = make_float2(re[r][c], im[r][c]);
         }
     }
+}
+
+// ---- separable contraction ------------------------------------------------
+// Over a 32 x 32 pixel block the phase about the block centre is, with
+// A = ex (2 dx + ex), B = ey (2 dy + ey) and q = A + B,
+//   (r - r0)/lambda = c1 q - c2 q^2 + c3 q^3 - ...,
+// c1 = 1/(2 r0 lambda), c2 = c1/(4 r0^2), c3 = c2/(2 r0^2): a part in A, a
+// part in B, and the cross term -2 c2 A' B' with A' = A (1 - eta A),
+// eta = 3/(4 r0^2) (third order included).  So
+//   exp(i 2 pi r/lambda) = F(row) E(col) sum_k (i delta A' B')^k / k!,  delta = -4 pi c2,
+// and the sum over points is a complex contraction of K = (points x terms) on
+// v_mfma_f32_32x32x2_f32: per point and block 32 row and 32 column factors
+// (a sin and cos each) instead of 1,024, one to five terms by the size of
+// the cross term (one below 6e-7 rad; two up to 1.5e-3 rad cover a 100 mm
+// distance at 8 um for most points).  The factors' phases are polynomials of
+// the pixel offset j = -15.5 .. 15.5, FP32 with the linear coefficient,
+// reduced modulo 2 in FP64 (2 j is odd, so j 2 is a whole turn), split so
+// that its high part times j is exact.
+//
+// A wave owns a block.  It takes 64 points at a time: each lane forms one
+// point's record for the block in FP64, then the wave contracts them in
+// pairs (lanes 0-31 the factors of the even point, 32-63 of the odd one).
+// Points out of the expansion's range (RsRange) take the FP64 phase per
+// pixel; a tile with more than 1/8 such points runs rs_tile_direct.
+//
+// The complex product takes three real ones instead of four, which costs the
+// sums a factor 1.4 in rounding; they are formed over 64 points at a time and
+// added per batch, which more than makes up for it (1000 points at 1024^2:
+// 3.6e-7 from FP64, 7.1e-7 with one sum per pixel of 1000 products).
+// Bound by matrix and vector instructions in turn (they do not overlap on a
+// SIMD here).  1024^2 with 1000 points at 100 mm: 161 us, of which 20 us are
+// the factors; 4096 x 2160 with 1453 points at 0.462 um: 1.71 ms.  A sin and
+// cos per pixel and point took 457 us and 4.40 ms.  Records in the order of
+// their terms are worth 8% (a pair takes the larger count of its two).
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int RS_TERMS = 5;
+
+struct RsRec {
+    float4 x, y;   // high and low linear, quadratic, cubic coefficient along x and y
+    float4 c;      // phase at the block centre, amplitude, quartic coefficients
+    float4 m;      // 2 dx, 2 dy, delta, eta
+};
+
+// Terms the contraction needs for one point and block (0: out of range).
+// ax, ay: largest A and B over the block; hm: largest half extent.  The
+// thresholds keep the first dropped term, (delta A' B')^k / k! of root mean
+// square 1/(2 k + 1) over the block, and the dropped phase terms (fourth
+// order in q, fifth in the offset) below 3e-7 rad.
+__device__ __forceinline__ int rs_terms(float r0, float yr, float c2, float ax, float ay, float dm, float hm,
+                                        float inv_l, bool huygens) {
+    const float u = (ax + ay) * yr * yr;
+    const float c3 = 0.5f * c2 * yr * yr;
+    const float e4 = r0 * inv_l * (5.f / 128.f) * (u * u) * (u * u);
+    const float e5 = 8.f * c3 * dm * (hm * hm) * (hm * hm) * hm;
+    if (!(e4 + e5 <= 5e-8f) || (huygens && !(u <= 1.5e-3f))) return 0;
+    const float d = 12.5663706f * c2 * ax * ay;
+    return d <= 6e-7f ? 1 : d <= 2e-3f ? 2 : d <= 2.5e-2f ? 3 : d <= 9e-2f ? 4 : d <= 0.2f ? 5 : 0;
+}
+
+template <bool HUYGENS>
+__device__ __forceinline__ void rs_block_mfma(const RsArgs& a, RsRec* rec, int c0, int r0) {
+    const int lane = threadIdx.x & 63;
+    const double spy = a.ydir * a.py;
+    const double X0 = (c0 + 15.5) * a.px + a.x_off, Y0 = (r0 + 15.5) * spy + a.y_off;
+    const float hx = (float)(15.5 * a.px), hy = (float)(15.5 * a.py), hm = fmaxf(hx, hy);
+    const float inv_l = (float)a.inv_lambda;
+    // this lane's row and column offset (the same index of the block on both axes)
+    const float j = (float)(lane & 31) - 15.5f;
+    const float ex = j * (float)a.px, ey = j * (float)spy;
+    f32x16 re = (f32x16)0.f, im = (f32x16)0.f;
+    const int64_t p_begin = (int64_t)blockIdx.z * a.chunk;
+    const int64_t p_end = min(a.n, p_begin + a.chunk);
+    for (int64_t base = p_begin; base < p_end; base += 64) {
+        int terms = 0;
+        int first[RS_TERMS + 2];   // first record with at least k terms
+        {
+            const int64_t n = base + lane;
+            RsRec q = {};
+            if (n < p_end) {
+                const double dx = X0 - a.x[n] * a.sx, dy = Y0 - a.y[n] * a.sy;
+                const double zs = a.z[n] * a.sz + a.oz;
+                const double s0 = fma(dx, dx, fma(dy, dy, zs * zs));
+                const double yr = rsqrt_f64(s0), rr = s0 * yr;
+                const double t0 = fma(rr, a.inv_lambda, (a.phase ? a.phase[n] * 0.15915494309189535 : 0.0) + a.ph0);
+                const double c1 = 0.5 * a.inv_lambda * yr;
+                const float yrf = (float)yr, y2 = yrf * yrf, c1f = (float)c1;
+                const float c2 = 0.25f * c1f * y2, c3 = 0.5f * c2 * y2;
+                const float dxf = (float)dx, dyf = (float)dy, pxf = (float)a.px, pyf = (float)spy;
+                float am = a.amp ? (float)a.amp[n] : 1.f;
+                if (HUYGENS) am *= yrf;
+                auto axis = [&](double d, double p, float df, float pf, float& quartic) {
+                    double s = 2.0 * c1 * d * p;
+                    s -= 2.0 * rint(0.5 * s);
+                    const double hi = rint(s * 131072.0) * (1.0 / 131072.0);
+                    const float d2 = df * df, p2 = pf * pf;
+                    quartic = fmaf(12.f * c3, d2, -c2) * p2 * p2;
+                    return make_float4((float)hi, (float)(s - hi), fmaf(-4.f * c2, d2, c1f) * p2,
+                                       df * fmaf(8.f * c3, d2, -4.f * c2) * p2 * pf);
+                };
+                float qx, qy;
+                q.x = axis(dx, a.px, dxf, pxf, qx);
+                q.y = axis(dy, spy, dyf, pyf, qy);
+                q.c = make_float4((float)(t0 - rint(t0)), am, qx, qy);
+                q.m = make_float4(2.f * dxf, 2.f * dyf, -12.5663706f * c2, 0.75f * y2);
+                terms = rs_terms((float)rr, yrf, c2, hx * fmaf(2.f, fabsf(dxf), hx), hy * fmaf(2.f, fabsf(dyf), hy),
+                                 fmaxf(fabsf(dxf), fabsf(dyf)), hm, inv_l, HUYGENS);
+                if (terms == 0) q = {};   // summed per pixel below
+            }
+            // records in order of their number of terms, so that the two points
+            // of a pair mostly need the same; those of none (out of range, past
+            // the end) last, with amplitude 0
+            int at = 0, below = 0;
+#pragma unroll
+            for (int k = 1; k <= RS_TERMS + 1; ++k) {
+                const uint64_t m = __ballot(terms == k % (RS_TERMS + 1));
+                if (terms == k % (RS_TERMS + 1)) at = below + __popcll(m & ((1ull << lane) - 1));
+                below += __popcll(m);
+                if (k <= RS_TERMS) first[k + 1] = below;
+            }
+            rec[at] = q;
+        }
+        // (one wave's LDS accesses complete in order: only the compiler must
+        // not move them)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int cnt = first[RS_TERMS + 1];
+        // a complex product from three real ones: sums of fr er, fi ei and
+        // (fr + fi)(er + ei), over these 64 points
+        f32x16 s1 = (f32x16)0.f, s2 = (f32x16)0.f, s3 = (f32x16)0.f;
+        for (int p = 0; p < cnt; p += 2) {
+            const RsRec q = rec[p + (lane >> 5)];
+            float mx = j * q.x.x, my = j * q.y.x;
+            mx -= rintf(mx);
+            my -= rintf(my);
+            const float tx = fmaf(fmaf(fmaf(fmaf(q.c.z, j, q.x.w), j, q.x.z), j, q.x.y), j, mx);
+            const float ty = fmaf(fmaf(fmaf(fmaf(q.c.w, j, q.y.w), j, q.y.z), j, q.y.y), j, my + q.c.x);
+            float er = cos_turns(tx), ei = sin_turns(tx);
+            float fr = q.c.y * cos_turns(ty), fi = q.c.y * sin_turns(ty);
+            if (HUYGENS) {
+                // 1/r = (1/r0)(1 - q/(2 r0^2) + 3/8 (q/r0^2)^2), per axis
+                const float ua = ex * (q.m.x + ex) * q.m.w, ub = ey * (q.m.y + ey) * q.m.w;   // 3/4 A/r0^2
+                const float ga = fmaf(ua, fmaf(ua, 2.f / 3.f, -2.f / 3.f), 1.f);
+                const float gb = fmaf(ub, fmaf(ub, 2.f / 3.f, -2.f / 3.f), 1.f);
+                er *= ga;
+                ei *= ga;
+                fr *= gb;
+                fi *= gb;
+            }
+            auto contract = [&]() {
+                s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(fr, er, s1, 0, 0, 0);
+                s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(fi, ei, s2, 0, 0, 0);
+                s3 = __builtin_amdgcn_mfma_f32_32x32x2f32(fr + fi, er + ei, s3, 0, 0, 0);
+            };
+            contract();
+            if (p + 1 >= first[2]) {
+                const float A = ex * (q.m.x + ex), B = ey * (q.m.y + ey);
+                const float g = q.m.z * A * fmaf(-q.m.w, A, 1.f), b = B * fmaf(-q.m.w, B, 1.f);
+                auto next = [&](float w) {   // E *= i g w, F *= b
+                    const float gw = g * w, t = er;
+                    er = -ei * gw;
+                    ei = t * gw;
+                    fr *= b;
+                    fi *= b;
+                    contract();
+                };
+                next(1.f);
+                if (p + 1 >= first[3]) {
+                    next(0.5f);
+                    if (p + 1 >= first[4]) {
+                        next(1.f / 3.f);
+                        if (p + 1 >= first[5]) next(0.25f);
+                    }
+                }
+            }
+        }
+        // points out of range: FP64 phase per pixel (register v of a lane is
+        // row 8 (v/4) + 4 (lane/32) + v%4, column lane%32)
+        re += s1 - s2;
+        im += s3 - (s1 + s2);
+        uint64_t far = __ballot(terms == 0 && base + lane < p_end);
+        while (far) {
+            const int k = __ffsll((long long)far) - 1;
+            far &= far - 1;
+            const int64_t n = base + k;
+            const double dx = (c0 + (lane & 31)) * a.px + a.x_off - a.x[n] * a.sx;
+            const double zs = a.z[n] * a.sz + a.oz, ys = a.y[n] * a.sy;
+            const double dxz = fma(dx, dx, zs * zs);
+            const double ph = (a.phase ? a.phase[n] * 0.15915494309189535 : 0.0) + a.ph0;
+            const float am = a.amp ? (float)a.amp[n] : 1.f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int row = r0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                const double dy = row * spy + a.y_off - ys;
+                const double s = fma(dy, dy, dxz), yr = rsqrt_f64(s);
+                const double t = fma(s * yr, a.inv_lambda, ph);
+                const float f = (float)(t - rint(t));
+                const float ap = HUYGENS ? (float)(am * yr) : am;
+                re[v] = fmaf(ap, cos_turns(f), re[v]);
+                im[v] = fmaf(ap, sin_turns(f), im[v]);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    float2* dst = a.partial + (size_t)blockIdx.z * a.nx * a.ny;
+    const int col = c0 + (lane & 31);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int row = r0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+        if (row < a.ny && col < a.nx) dst[(size_t)row * a.nx + col] = make_float2(re[v], im[v]);
+    }
+}
+
+// A 64 x 64 tile and one chunk of the points.  The form is chosen per
+// workgroup from a sample of up to 256 of its points, spread over the chunk.
+template <bool HUYGENS>
+__global__ __launch_bounds__(256, 3) void rs_accumulate(RsArgs a) {
+    __shared__ union {
+        RsStage stage;
+        RsRec rec[4][64];
+    } sm;
+    const int tile_x = blockIdx.x * TILE_X, tile_y = blockIdx.y * TILE_Y;
+    const int64_t p_begin = (int64_t)blockIdx.z * a.chunk;
+    const int64_t cnt = min(a.n, p_begin + a.chunk) - p_begin;
+    bool out = false;
+    const int64_t samples = min((int64_t)256, cnt);
+    if ((int)threadIdx.x < samples) {
+        const int64_t n = p_begin + cnt * threadIdx.x / samples;
+        const float dx = (float)((tile_x + 31.5) * a.px + a.x_off - a.x[n] * a.sx);
+        const float dy = (float)(a.ydir * (tile_y + 31.5) * a.py + a.y_off - a.y[n] * a.sy);
+        const float zs = (float)(a.z[n] * a.sz + a.oz);
+        const float s0 = fmaf(dx, dx, fmaf(dy, dy, zs * zs)), yr = rsqrtf(s0);
+        const float hx = (float)(15.5 * a.px), hy = (float)(15.5 * a.py), inv_l = (float)a.inv_lambda;
+        out = rs_terms(s0 * yr, yr, 0.125f * inv_l * yr * yr * yr, hx * fmaf(2.f, fabsf(dx), hx),
+                       hy * fmaf(2.f, fabsf(dy), hy), fmaxf(fabsf(dx), fabsf(dy)), fmaxf(hx, hy), inv_l, HUYGENS) == 0;
+    }
+    const int n_out = __syncthreads_count(out);
+    if (8 * (int64_t)n_out > samples) {
+        rs_tile_direct<HUYGENS>(a, sm.stage);
+        return;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c0 = tile_x + 32 * (wave & 1), r0 = tile_y + 32 * (wave >> 1);
+    if (c0 < a.nx && r0 < a.ny) rs_block_mfma<HUYGENS>(a, sm.rec[wave], c0, r0);
 }
 
 struct FinArgs {
@@ -304,9 +560,11 @@ int rs_run(oph_ctx* ctx, const RsJob& J, const oph_points* pts, void* out, int f
     const int gx = (nx + TILE_X - 1) / TILE_X, gy = (ny + TILE_Y - 1) / TILE_Y;
     const int64_t tiles = (int64_t)gx * gy;
     // split points so that the grid holds >= 4 workgroups per CU, keeping
-    // >= 1024 points per chunk
+    // >= RS_MINPTS points per chunk (1024^2, 1000 points: 4 chunks of 250;
+    // 128 or 256 points at least and 2, 4 or 8 workgroups per CU measured the
+    // same to 2%)
     int64_t chunks = (4LL * ctx->cu_count + tiles - 1) / tiles;
-    const int64_t max_by_pts = (n + 1023) / 1024;
+    const int64_t max_by_pts = (n + RS_MINPTS - 1) / RS_MINPTS;
     if (chunks > max_by_pts) chunks = max_by_pts;
     if (chunks > 16) chunks = 16;
     if (chunks < 1) chunks = 1;
@@ -317,10 +575,10 @@ int rs_run(oph_ctx* ctx, const RsJob& J, const oph_points* pts, void* out, int f
 
     if (J.huygens)
         OPH_LAUNCH(ctx, "huygens_accumulate", rs_accumulate<true>, dim3(gx, gy, (unsigned)chunks),
-                   dim3(TPB_X, TPB_Y), 0, a);
+                   dim3(256), 0, a);
     else
         OPH_LAUNCH(ctx, "rs_accumulate", rs_accumulate<false>, dim3(gx, gy, (unsigned)chunks),
-                   dim3(TPB_X, TPB_Y), 0, a);
+                   dim3(256), 0, a);
 
     const size_t obytes = npix * (fmt == OPH_OUT_C128 ? 16 : fmt == OPH_OUT_C64 ? 8 : 4);
     void* dout = out;

@@ -117,3 +117,35 @@ def test_huygens_vs_oracle(ctx, nx, ny, z):
     V = ctx.huygens(nx, ny, 8e-6, 532e-9, z, x, y, zz, a, ph, ph=0.25, fmt=oph.OUT_C64, out=U.astype(np.complex64),
                     accumulate=True)
     assert rel_l2(V, 2 * ref) < 1e-5
+
+
+@pytest.mark.parametrize("nx,ny,n,zlo,zhi,near", [
+    (70, 45, 1, 0.1, 0.1, 0),        # one point, partial blocks
+    (33, 97, 63, 0.09, 0.11, 0),     # one short batch of the contraction
+    (128, 64, 65, 0.2, 0.3, 0),      # one point past a batch, whole tiles
+    (200, 130, 1100, 0.04, 0.06, 0),  # two to five terms, split over chunks
+    (96, 100, 130, 0.1, 0.12, 7),    # some points out of the expansion's range
+    (100, 70, 300, 2e-3, 4e-3, 0),   # tiles too close: a sin and cos per pixel
+])
+@pytest.mark.parametrize("huygens", [False, True])
+def test_rs_contraction_edges(ctx, nx, ny, n, zlo, zhi, near, huygens):
+    """Separable contraction at its edges (partial blocks, batches of 64
+    points, one to five terms, points out of range summed per pixel) and the
+    direct form.  Bound per term: reduced phases 2 x 2^-25 turns and the centre
+    phase 2^-25 (5e-7 rad), dropped terms 3e-7 rad, FP32 products and sums of
+    at most 64 terms (under 5e-7): 2e-6 in the 2-norm."""
+    print(f"case: rs contraction {nx}x{ny} P={n} z {zlo}..{zhi} near {near} huygens {huygens}", flush=True)
+    g = scenes.SplitMix64(100 + n)
+    x, y, z = g.uniform(n, -5e-3, 5e-3), g.uniform(n, -5e-3, 5e-3), g.uniform(n, zlo, zhi)
+    z[:near] = 3e-3
+    a, ph = g.uniform(n, 0.1, 1.0), g.uniform(n, 0.0, 2 * np.pi)
+    if huygens:
+        U = ctx.huygens(nx, ny, 8e-6, 532e-9, 0.0, x, y, z, a, ph)
+        ref = O.huygens(nx, ny, 8e-6, 532e-9, 0.0, x, y, z, a, ph)
+    else:
+        spec = dict(nx=nx, ny=ny, pitch=(8e-6, 6e-6), lambda_=532e-9)
+        U = ctx.pc_rs(spec, x, y, z, a, ph)
+        ref = O.rs(_s64(spec), x, y, z, a, ph)
+    err = rel_l2(U, ref)
+    print("rel-L2", err)
+    assert err < 2e-6

@@ -88,12 +88,16 @@ __global__ void fresnel_prep(const double* x, const double* y, const double* z, 
 // over F32_BATCH points and in FP64 across batches, so a pixel's rounding
 // error does not grow with the point count.
 //
-// Bound by the matrix cores (128 cycles per point and 32 x 32 pixels) and, as
+// The complex product takes three real ones (sums of A.x B.x, A.y B.y and
+// (A.x + A.y)(B.x + B.y)): a quarter fewer matrix instructions; the sums'
+// rounding grows by 1.4, the error against FP64 from 4.1e-7 to 4.2e-7.
+//
+// Bound by the matrix cores (96 cycles per point and 32 x 32 pixels) and, as
 // vector and matrix instructions do not overlap on a SIMD here, by the
-// generation in turn with them: 1280 x 720 with 20,000 points 1.30 ms = 113
-// TFLOP/s of the 152 a large FP32 product reaches; without generation 1.15 ms
-// (interleaving the two instruction by instruction changed nothing).  A sum
-// per pixel on the vector unit, with its sin and cos, took 4.95 ms.
+// generation in turn with them: 1280 x 720 with 20,000 points 1.08 ms (1.30
+// with four products, of which the generation is 0.16; interleaving the two
+// instruction by instruction changed nothing).  A sum per pixel on the vector
+// unit, with its sin and cos, took 4.95 ms.
 
 constexpr int F32_PTS = 16, F32_BATCH = 256;
 constexpr int F32_R = 64, F32_C = 128;
@@ -150,11 +154,11 @@ __global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
         }
     };
 
-    f32x16 re[2], im[2];
+    f32x16 s1[2], s2[2], s3[2];   // sums of A.x B.x, A.y B.y, (A.x + A.y)(B.x + B.y)
     double sre[2][16], sim[2][16];
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-        re[b] = im[b] = (f32x16)0.f;
+        s1[b] = s2[b] = s3[b] = (f32x16)0.f;
 #pragma unroll
         for (int v = 0; v < 16; ++v) sre[b][v] = sim[b][v] = 0.0;
     }
@@ -179,13 +183,9 @@ __global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
             for (int b = 0; b < 2; ++b) B[b] = L.B[pt][wc + 32 * b + (lane & 31)];
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
-                re[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, B[b].x, re[b], 0, 0, 0);
-                im[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, B[b].y, im[b], 0, 0, 0);
-            }
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                re[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(-A.y, B[b].y, re[b], 0, 0, 0);
-                im[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.y, B[b].x, im[b], 0, 0, 0);
+                s1[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x, B[b].x, s1[b], 0, 0, 0);
+                s2[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.y, B[b].y, s2[b], 0, 0, 0);
+                s3[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A.x + A.y, B[b].x + B[b].y, s3[b], 0, 0, 0);
             }
         }
         if ((c + 1) % (F32_BATCH / F32_PTS) == 0 || c + 1 == nch) {
@@ -193,10 +193,10 @@ __global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
             for (int b = 0; b < 2; ++b) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
-                    sre[b][v] += (double)re[b][v];
-                    sim[b][v] += (double)im[b][v];
+                    sre[b][v] += (double)(s1[b][v] - s2[b][v]);
+                    sim[b][v] += (double)(s3[b][v] - (s1[b][v] + s2[b][v]));
                 }
-                re[b] = im[b] = (f32x16)0.f;
+                s1[b] = s2[b] = s3[b] = (f32x16)0.f;
             }
         }
     }
@@ -1020,7 +1020,7 @@ extern "C" int oph_pc_fresnel(oph_ctx* ctx, int nx, int ny, double pitch, double
         // CU) are filled: the split with the fewest point chunks per slot,
         // at least 1024 points each (1280 x 720, 20,000 points: 120 tiles in
         // 17 parts fill 3.98 of 4 rounds, 1.35 ms against 1.43 in 4 parts,
-        // 0.94 of a round) and at most 256 MiB of partial fields
+        // 0.94 of a round; four-product form) and at most 256 MiB of partial fields
         const int64_t tiles_f = (int64_t)gx * gy, slots = 2LL * std::max(ctx->cu_count, 1);
         int64_t chunks = 1;
         double best = 1e300;

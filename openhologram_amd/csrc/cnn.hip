@@ -333,119 +333,198 @@ __global__ void relu_mask(float* g, const float* act, int64_t n) {
 }
 
 // ---- weight gradient -------------------------------------------------------------
-// dW[n][k] = sum_p dY[p][n] X[p + off(tap k)][c k], db[n] = sum_p dY[p][n].
-// GEMM M = COUT (padded to 32), N = 9 CIN + 1 (bias column), K = pixels.
-// Pixels are taken in 8-row x 32-column tiles of one image.  A workgroup
-// stages a tile in LDS as BF16: dY transposed ([channel][pixel], so the 8
-// pixels of an A fragment are 16 contiguous bytes) and X as three copies of
-// its channel planes shifted by dx = -1, 0, +1 (so the 8 pixels of a B
-// fragment at any tap are 16 aligned bytes).  Five waves take two of the ten
-// 32-column N tiles each.  Workgroup g accumulates tiles g, g + G, ... in
-// registers (a fixed order) and writes part[g][32][NCOL]; dw_reduce sums the
-// partials in workgroup order (deterministic).
+// dW[n][tap][c] = sum_p dY[p][n] X[p + off(tap)][c], db[n] = sum_p dY[p][n].
+// As a GEMM over pixels (K) with M = COUT, N = CIN per tap: with q = p + off,
+// the B operand (X at q) is the same for all taps and the A operand is dY
+// shifted, so a wave keeps one X fragment for the taps of its column and
+// reuses each dY row for three of them.  Pixels are taken in 8 x 32 tiles of
+// X; dY is staged with a one-pixel halo.  Both stay pixel-major in LDS as they
+// come from HBM (BF16, 64 bytes per pixel): ds_read_b64_tr_b16 hands each lane
+// four pixels of its channel, at any pixel offset and without bank conflicts
+// (a row of 16 lanes reads four whole pixels).
+//
+// Six waves: wave (d, h) takes the taps of column d (three rows of taps) over
+// rows 4h .. 4h + 3 of the tile; wave d = 1 also the bias (the centre tap's dY
+// against ones).  The two row halves are added in LDS at the end.  Workgroup g
+// accumulates tiles g, g + G, ... in registers (a fixed order), the next
+// tile's pixels loaded while the current one is contracted, and writes
+// part[g][COUT][9 CIN + 1]; dw_reduce sums the partials in workgroup order
+// (deterministic).
+//
+// Bound by the latency of the few tiles a workgroup has: 8 x 128^2 pixels (two
+// tiles each) 12.0 us = 3.3 TB/s of dY (with halo) and X.  512 workgroups of
+// one tile 17 us; 168 registers for three workgroups per CU spill, 16 us.
+// (Operands transposed on the way into LDS by 2-byte stores, with three
+// shifted copies of X, took 71 us in bank conflicts.)
 
-constexpr int DW_WAVES = 5;
+constexpr int DW_WAVES = 6, DW_THREADS = 64 * DW_WAVES;
 constexpr int DW_MAX_GROUPS = 256;
 
 struct DwArgs {
     const float* dy;   // [npix][COUT]
     const float* x;    // [npix][CIN]
-    float* part;       // [groups][32][ncol]
+    float* part;       // [groups][COUT][ncol]
     int B, H, W;
     int tiles_x, tiles_y;
 };
 
+// Pixels of a ROWS x COLS window whose first is (y0, x0), C channels (32 or 2)
+// of an NHWC image: loaded to registers (zeros outside the image, without a
+// branch per load), then stored to LDS as BF16, 32 channels per pixel (the
+// channels from C on are not written).
+template <int ROWS, int COLS, int C>
+struct DwStage {
+    static constexpr int Q = C / 4 > 0 ? C / 4 : 1;   // pieces per pixel
+    static constexpr int N = (ROWS * COLS * Q + DW_THREADS - 1) / DW_THREADS;
+    typedef typename std::conditional<C == 2, float2, float4>::type V;
+    V v[N];
+    __device__ __forceinline__ void load(const float* img, int y0, int x0, int H, int W) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int i = threadIdx.x + DW_THREADS * k, px = i / Q;
+            const int y = y0 + px / COLS, x = x0 + px % COLS;
+            const bool ok = px < ROWS * COLS && y >= 0 && y < H && x >= 0 && x < W;
+            const V t = reinterpret_cast<const V*>(img)[ok ? ((size_t)y * W + x) * Q + i % Q : 0];
+            v[k] = ok ? t : V{};
+        }
+    }
+    __device__ __forceinline__ void store(__bf16* lds) const {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int i = threadIdx.x + DW_THREADS * k;
+            if (i >= ROWS * COLS * Q) break;
+            __bf16* d = lds + (i / Q) * 32 + 4 * (i % Q);
+            if constexpr (C == 2)
+                *reinterpret_cast<bf16x2*>(d) = bf16x2{(__bf16)v[k].x, (__bf16)v[k].y};
+            else
+                *reinterpret_cast<bf16x4*>(d) =
+                    bf16x4{(__bf16)v[k].x, (__bf16)v[k].y, (__bf16)v[k].z, (__bf16)v[k].w};
+        }
+    }
+};
+
+// MFMA operand from pixel-major LDS: lane l gets channel l % 32 of pixels
+// 8 (l / 32) .. + 7 after `px` (a pixel's 32 channels at px, 64 bytes apart)
+__device__ __forceinline__ bf16x8 dw_fragment(const __bf16* px, int lane) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* P;
+    // a group of 16 lanes reads 4 pixels x 16 channels, lane i of it 4
+    // channels of pixel i / 4, and lane i receives channel i of the four
+    const int g = lane >> 4, i = lane & 15;
+    const __bf16* s = px + (8 * (g >> 1) + (i >> 2)) * 32 + 16 * (g & 1) + 4 * (i & 3);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(s));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(s + 4 * 32));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 template <int CIN, int COUT>
-__global__ __launch_bounds__(64 * DW_WAVES) void conv3x3_dw(DwArgs a) {
+__global__ __launch_bounds__(DW_THREADS, 2) void conv3x3_dw(DwArgs a) {
     constexpr int NCOL = 9 * CIN + 1;
-    constexpr int NT = (NCOL + 31) / 32;
-    constexpr int TPW = (NT + DW_WAVES - 1) / DW_WAVES;  // N tiles per wave
-    constexpr int TP = CT_H * CT_W;                      // pixels per tile
-    constexpr int XR = CT_H + 2;                         // X rows incl. halo
-    __shared__ __attribute__((aligned(16))) __bf16 sdy[32 * TP];
-    __shared__ __attribute__((aligned(16))) __bf16 sx[3 * CIN * XR * CT_W];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = lane & 31, kh = 8 * (lane >> 5);
-    f32x16 acc[TPW];
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) acc[t] = (f32x16)0.f;
+    constexpr int DR = CT_H + 2, DC = CT_W + 2;   // dY with its halo
+    constexpr int NDY = DR * DC * 32, NX = CT_H * CT_W * 32;
+    // the tiles, and at the end the row-half sums
+    constexpr int SUMS = 3 * 4 * 16 * 64 * sizeof(float) / sizeof(__bf16);
+    __shared__ __attribute__((aligned(16))) __bf16 lds[NDY + NX > SUMS ? NDY + NX : SUMS];
+    __bf16 *sdy = lds, *sx = lds + NDY;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int d = wave % 3, half = wave / 3;
     const int ntiles = a.tiles_x * a.tiles_y * a.B;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    if (COUT < 32 || CIN < 32)   // the channels no tile writes
+        for (int i = threadIdx.x; i < (NDY + NX) / 8; i += DW_THREADS)
+            reinterpret_cast<bf16x8*>(lds)[i] = (bf16x8)(__bf16)0.f;
+    f32x16 acc[3] = {(f32x16)0.f, (f32x16)0.f, (f32x16)0.f}, accb = (f32x16)0.f;
+    const bf16x8 ones = (bf16x8)(__bf16)1.f;
+    DwStage<DR, DC, COUT> ry;
+    DwStage<CT_H, CT_W, CIN> rx;
+    auto fetch = [&](int tile) {
         const int tx = tile % a.tiles_x, ty = (tile / a.tiles_x) % a.tiles_y, b = tile / (a.tiles_x * a.tiles_y);
-        const int x0 = tx * CT_W, y0 = ty * CT_H;
         const size_t img = (size_t)b * a.H * a.W;
-        __syncthreads();  // the previous tile's reads are done
-        for (int i = threadIdx.x; i < TP * 32; i += 64 * DW_WAVES) {
-            const int px = i / 32, n = i % 32;
-            const int yy = y0 + px / CT_W, xx = x0 + px % CT_W;
-            float v = 0.f;
-            if (n < COUT && yy < a.H && xx < a.W) v = a.dy[(img + (size_t)yy * a.W + xx) * COUT + n];
-            sdy[n * TP + px] = (__bf16)v;
-        }
-        for (int i = threadIdx.x; i < XR * (CT_W + 2) * CIN; i += 64 * DW_WAVES) {
-            const int px = i / CIN, c = i % CIN;
-            const int r = px / (CT_W + 2), j = px % (CT_W + 2);   // j = 0..33 <-> x0 - 1 + j
-            const int yy = y0 + r - 1, xx = x0 + j - 1;
-            float v = 0.f;
-            if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) v = a.x[(img + (size_t)yy * a.W + xx) * CIN + c];
-            const __bf16 bv = (__bf16)v;
-            // shifted copy d (dx = d - 1) holds column jj = j - d at [d][c][r][jj]
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const int jj = j - d;
-                if (jj >= 0 && jj < CT_W) sx[((d * CIN + c) * XR + r) * CT_W + jj] = bv;
-            }
-        }
+        ry.load(a.dy + img * COUT, ty * CT_H - 1, tx * CT_W - 1, a.H, a.W);
+        rx.load(a.x + img * CIN, ty * CT_H, tx * CT_W, a.H, a.W);
+    };
+    fetch(blockIdx.x);
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        __syncthreads();  // the previous tile's reads (or the clearing) are done
+        ry.store(sdy);
+        rx.store(sx);
         __syncthreads();
+        if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
 #pragma unroll
-        for (int tt = 0; tt < TPW; ++tt) {
-            const int t = wave + DW_WAVES * tt;
-            if (t >= NT) break;
-            const int col = 32 * t + row;   // B column of this lane: (tap, c) or the bias column
-            const int tap = col / CIN, c = col % CIN;
-            const bool is_w = col < NCOL - 1, is_b = col == NCOL - 1;
-            const int dyo = tap / 3, dxo = tap % 3;  // row offset into the halo rows, shifted copy
-#pragma unroll 4
-            for (int s = 0; s < TP / 16; ++s) {
-                const int p0 = 16 * s + kh;               // 8 pixels of one tile row
-                const int pr = p0 / CT_W, pc = p0 % CT_W;
-                const bf16x8 A = *reinterpret_cast<const bf16x8*>(sdy + row * TP + p0);
-                bf16x8 Bv;
-                if (is_w)
-                    Bv = *reinterpret_cast<const bf16x8*>(sx + ((dxo * CIN + c) * XR + pr + dyo) * CT_W + pc);
-                else
-                    Bv = (bf16x8)(__bf16)(is_b ? 1.f : 0.f);
-                acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, acc[tt], 0, 0, 0);
+        for (int s = 0; s < CT_W / 16; ++s) {
+            // X row r meets dY halo rows r .. r + 2 (tap rows 2, 1, 0), from
+            // halo column 2 - d
+            const __bf16* py = sdy + (4 * half * DC + 16 * s + 2 - d) * 32;
+            const __bf16* px = sx + (4 * half * CT_W + 16 * s) * 32;
+            bf16x8 A[6];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) A[r] = dw_fragment(py + r * DC * 32, lane);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                A[r + 2] = dw_fragment(py + (r + 2) * DC * 32, lane);
+                const bf16x8 X = dw_fragment(px + r * CT_W * 32, lane);
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[r + 2 - t], X, acc[t], 0, 0, 0);
+                if (d == 1) accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[r + 1], ones, accb, 0, 0, 0);
             }
         }
     }
-    float* dst = a.part + (size_t)blockIdx.x * 32 * NCOL;
-#pragma unroll
-    for (int tt = 0; tt < TPW; ++tt) {
-        const int t = wave + DW_WAVES * tt;
-        if (t >= NT) break;
+    // add the row halves: [d][register][lane]
+    __syncthreads();
+    float* sum = reinterpret_cast<float*>(lds) + d * 4 * 16 * 64 + lane;
+    if (half == 1) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const int r = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);  // output channel
-            const int col = 32 * t + (lane & 31);
-            if (col < NCOL) dst[(size_t)r * NCOL + col] = acc[tt][v];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) sum[(16 * t + v) * 64] = acc[t][v];
+            sum[(48 + v) * 64] = accb[v];
         }
+    }
+    __syncthreads();
+    if (half == 1) return;
+    float* dst = a.part + (size_t)blockIdx.x * COUT * NCOL;
+    const int c = lane & 31;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int n = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);  // output channel
+        if (n >= COUT) continue;
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            if (c < CIN) dst[(size_t)n * NCOL + (3 * t + d) * CIN + c] = acc[t][v] + sum[(16 * t + v) * 64];
+        if (d == 1 && c == 0) dst[(size_t)n * NCOL + NCOL - 1] = accb[v] + sum[(48 + v) * 64];
     }
 }
 
-// Sum of the workgroup partials into the gradient (W and b): one wave per
-// element; lane j adds partials j, j + 64, ... in order, then the lanes are
-// combined by a fixed butterfly (the same order on every run).
-__global__ __launch_bounds__(256) void dw_reduce(const float* part, int groups, int cout, int ncol, float* gw,
-                                                 float* gb) {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= cout * ncol) return;
-    const int r = i / ncol, col = i % ncol;
+// Sum of the workgroup partials into the gradient (W and b).  A workgroup
+// takes 32 neighbouring elements (128-byte reads); its eight rows of threads
+// add the partials of an eighth of the groups each, in order, and the eight
+// sums are added in order (the same on every run).  9.5 MB in 4.6 us (one wave
+// per element, its lanes reading 37 KB apart, took 13).
+__global__ __launch_bounds__(256) void dw_reduce(const float* __restrict__ part, int groups, int cout, int ncol,
+                                                 float* gw, float* gb) {
+    __shared__ double sums[8][32];
+    const int e = threadIdx.x & 31, k = threadIdx.x >> 5;
+    const int i = blockIdx.x * 32 + e, n = cout * ncol;
+    const int per = (groups + 7) / 8, lo = k * per, hi = min(groups, lo + per);
     double s = 0.0;
-    for (int g = lane; g < groups; g += 64) s += part[((size_t)g * 32 + r) * ncol + col];
+    if (i < n) {
+        int g = lo;
+        for (; g + 8 <= hi; g += 8) {
+            float v[8];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane != 0) return;
+            for (int j = 0; j < 8; ++j) v[j] = part[(size_t)(g + j) * n + i];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s += v[j];
+        }
+        for (; g < hi; ++g) s += part[(size_t)g * n + i];
+    }
+    sums[k][e] = s;
+    __syncthreads();
+    if (k != 0 || i >= n) return;
+#pragma unroll
+    for (int j = 1; j < 8; ++j) s += sums[j][e];
+    const int r = i / ncol, col = i % ncol;
     if (col == ncol - 1)
         gb[r] = (float)s;
     else
@@ -473,12 +552,20 @@ __global__ void mse_grad(const float* y, const float* t, float* dy, int64_t n, d
     if (threadIdx.x == 0) part[blockIdx.x] = s[0];
 }
 
-__global__ void sum_partials(double* part, int n) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int i = 0; i < n; ++i) s += part[i];
-        part[n] = s;
+// One workgroup: each thread adds every 1024th partial in order, then a tree
+// in LDS (the same order on every run).  (One thread adding them all waited
+// for 1,024 loads in turn: 59 us.)
+__global__ __launch_bounds__(1024) void sum_partials(double* part, int n) {
+    __shared__ double s[1024];
+    double t = 0.0;
+    for (int i = threadIdx.x; i < n; i += 1024) t += part[i];
+    s[threadIdx.x] = t;
+    __syncthreads();
+    for (int off = 512; off > 0; off >>= 1) {
+        if ((int)threadIdx.x < off) s[threadIdx.x] += s[threadIdx.x + off];
+        __syncthreads();
     }
+    if (threadIdx.x == 0) part[n] = s[0];
 }
 
 __global__ void adam_step(float* p, const float* g, float* m, float* v, int64_t n, float lr, float b1, float b2,
@@ -1281,11 +1368,11 @@ int conv_dw(oph_ctx* ctx, oph_cnn* net, const float* dy, const float* x, int B, 
     DwArgs a{dy, x, net->part, B, H, W, (W + CT_W - 1) / CT_W, (H + CT_H - 1) / CT_H};
     const int64_t ntiles = (int64_t)a.tiles_x * a.tiles_y * B;
     const int groups = (int)std::min<int64_t>(ntiles, DW_MAX_GROUPS);
-    const size_t need = (size_t)groups * 32 * NCOL * sizeof(float);
+    const size_t need = (size_t)groups * COUT * NCOL * sizeof(float);
     if (need > net->part_bytes) return oph_fail(ctx, OPH_ENOMEM, "weight-gradient workspace too small");
     if (ntiles > INT32_MAX) return oph_fail(ctx, OPH_EINVAL, "too many pixels");
-    OPH_LAUNCH(ctx, "conv3x3_dw", (conv3x3_dw<CIN, COUT>), dim3((unsigned)groups), dim3(64 * DW_WAVES), 0, a);
-    OPH_LAUNCH(ctx, "dw_reduce", dw_reduce, dim3((COUT * NCOL + 3) / 4), dim3(256), 0, net->part, groups, COUT,
+    OPH_LAUNCH(ctx, "conv3x3_dw", (conv3x3_dw<CIN, COUT>), dim3((unsigned)groups), dim3(DW_THREADS), 0, a);
+    OPH_LAUNCH(ctx, "dw_reduce", dw_reduce, dim3((COUT * NCOL + 31) / 32), dim3(256), 0, net->part, groups, COUT,
                NCOL, gw, gb);
     return OPH_OK;
 }
@@ -1457,7 +1544,7 @@ int backward(oph_ctx* ctx, oph_cnn* net, const float* x, const float* t, int B, 
     const unsigned nb = (unsigned)((n2 + 255) / 256);
     float* dy = A.g2;  // 2-channel output gradient (fits in a C-channel buffer)
     OPH_LAUNCH(ctx, "mse_grad", mse_grad, dim3(nb), dim3(256), 0, A.y, t, dy, n2, net->red);
-    OPH_LAUNCH(ctx, "sum_partials", sum_partials, dim3(1), dim3(64), 0, net->red, (int)nb);
+    OPH_LAUNCH(ctx, "sum_partials", sum_partials, dim3(1), dim3(1024), 0, net->red, (int)nb);
     const Frags F{net->blocks};
     const bf16x8* WB = net->wb;
     int rc;

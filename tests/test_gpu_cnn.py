@@ -187,3 +187,29 @@ def test_learned_correction_1024_configuration(ctx):
         assert info["fallback"] and np.array_equal(u, full)
     else:
         assert not info["fallback"]
+
+
+@pytest.mark.parametrize("B,h,w", [(1, 1, 1), (1, 8, 32), (2, 9, 33), (3, 17, 70), (1, 130, 160)])
+def test_cnn_gradients_tile_edges(ctx, B, h, w):
+    """Gradients at the edges of the weight gradient's 8 x 32 pixel tiles (one
+    pixel, one whole tile, one row and column more, several workgroups) against
+    the FP64 oracle, and the same on a second call.  Bound: BF16 operands
+    (2^-9 relative) through five layers each way, as in the full test."""
+    print(f"case: cnn gradients {B}x{h}x{w}", flush=True)
+    rng = np.random.default_rng(31)
+    net = oph.lib.Cnn(ctx, blocks=1, channels=32, seed=5)
+    p = rng.normal(0, 0.05, net.n).astype(np.float32)
+    net.set_params(p)
+    x = rng.normal(0, 1, (B, h, w, 2)).astype(np.float32)
+    t = rng.normal(0, 1, (B, h, w, 2)).astype(np.float32)
+    loss, g = net.gradients(x, t)
+    loss2, g2 = net.gradients(x, t)
+    assert loss == loss2 and np.array_equal(g, g2)
+    lr_, gr = R.loss_and_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), 32, 1)
+    print("loss", loss, lr_, "grad rel", _rel(g, gr))
+    assert abs(loss - lr_) / lr_ < 1e-2
+    assert _rel(g, gr) < 3e-2
+    shapes, _ = R.layout(32, 1)
+    for name, o, s in shapes:
+        n = int(np.prod(s))
+        assert _rel(g[o:o + n], gr[o:o + n]) < 0.1, name

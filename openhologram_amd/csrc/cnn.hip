@@ -12,11 +12,12 @@
 // MFMA: M = pixels, N = output channels, K = 9 taps x input channels; each
 // wave produces 32 pixels x 32 channels with v_mfma_f32_32x32x16_bf16,
 // operands rounded to BF16 (weights and activations), FP32 accumulation;
-// bias, ReLU and the residual add are fused into the epilogue.  The input
-// gradient is the same convolution with flipped taps and transposed
-// channels; the weight gradient is a GEMM over pixels (M = output channels,
-// N = 9 x input channels + 1 bias column) split into pixel chunks whose
-// partial sums are reduced in a fixed order (deterministic).
+// bias, ReLU and the residual add are fused into the epilogue, and a block's
+// two convolutions into one kernel.  The input gradient is the same
+// convolution with flipped taps and transposed channels; the weight gradient
+// is a GEMM over pixels (M = output channels, N = input channels per tap, and
+// a bias column) split into pixel chunks whose partial sums are reduced in a
+// fixed order (deterministic).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -93,38 +94,6 @@ struct ConvArgsT {
     int B, H, W;
     int relu;
 };
-typedef ConvArgsT<float, float> ConvArgs;
-
-// A operand for lane (pixel p, k0..k0+7): taps/channels of the input patch
-template <int CIN>
-__device__ __forceinline__ bf16x8 load_patch(const ConvArgs& a, int b, int y, int x, int k0) {
-    bf16x8 v;
-    if constexpr (CIN % 8 == 0) {
-        const int tap = k0 / CIN, c = k0 % CIN;
-        const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-        if (tap < 9 && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
-            const float4* s =
-                reinterpret_cast<const float4*>(a.in + (((size_t)b * a.H + yy) * a.W + xx) * CIN + c);
-            const float4 p0 = s[0], p1 = s[1];
-            v[0] = (__bf16)p0.x; v[1] = (__bf16)p0.y; v[2] = (__bf16)p0.z; v[3] = (__bf16)p0.w;
-            v[4] = (__bf16)p1.x; v[5] = (__bf16)p1.y; v[6] = (__bf16)p1.z; v[7] = (__bf16)p1.w;
-        } else {
-            v = (bf16x8)(__bf16)0.f;
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int k = k0 + e;
-            const int tap = k / CIN, c = k % CIN;
-            const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-            float f = 0.f;
-            if (tap < 9 && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
-                f = a.in[(((size_t)b * a.H + yy) * a.W + xx) * CIN + c];
-            v[e] = (__bf16)f;
-        }
-    }
-    return v;
-}
 
 // Tiled forward convolution.  A workgroup of 8 waves owns an 8-row x 32-
 // column pixel tile of one image: it stages the tile and its one-pixel halo
@@ -151,57 +120,66 @@ __global__ __launch_bounds__(64 * CT_WAVES) void conv3x3_fwd(ConvArgsT<TI, TO> a
     constexpr int PS = tile_stride<CIN>();
     constexpr int TWH = CT_W + 2;
     __shared__ __attribute__((aligned(16))) __bf16 tile[(CT_H + 2) * TWH * PS];
+    __shared__ bf16x8 wf[KSTEPS * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int x0 = blockIdx.x * CT_W, y0 = blockIdx.y * CT_H, b = blockIdx.z;
     const size_t img = (size_t)b * a.H * a.W;
 
-    // stage the tile (+ halo) as BF16; outside the image is zero padding
-    if constexpr (std::is_same<TI, __bf16>::value && CIN % 8 == 0) {
-        constexpr int Q = CIN / 8;  // 16-byte vectors per pixel
-        for (int i = threadIdx.x; i < (CT_H + 2) * TWH * Q; i += 64 * CT_WAVES) {
-            const int pix = i / Q, q = i % Q;
-            const int yy = y0 + pix / TWH - 1, xx = x0 + pix % TWH - 1;
-            bf16x8 v = (bf16x8)(__bf16)0.f;
-            if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
-                v = reinterpret_cast<const bf16x8*>(a.in + (img + (size_t)yy * a.W + xx) * CIN)[q];
-            *reinterpret_cast<bf16x8*>(tile + pix * PS + 8 * q) = v;
-        }
-    } else if constexpr (CIN % 4 == 0 && std::is_same<TI, float>::value) {
-        constexpr int Q = CIN / 4;  // float4 per pixel
-        for (int i = threadIdx.x; i < (CT_H + 2) * TWH * Q; i += 64 * CT_WAVES) {
-            const int pix = i / Q, q = i % Q;
-            const int yy = y0 + pix / TWH - 1, xx = x0 + pix % TWH - 1;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
-                v = reinterpret_cast<const float4*>(a.in + (img + (size_t)yy * a.W + xx) * CIN)[q];
-            bf16x4 w4;
-            w4[0] = (__bf16)v.x;
-            w4[1] = (__bf16)v.y;
-            w4[2] = (__bf16)v.z;
-            w4[3] = (__bf16)v.w;
-            *reinterpret_cast<bf16x4*>(tile + pix * PS + 4 * q) = w4;
-        }
-    } else {
-        for (int i = threadIdx.x; i < (CT_H + 2) * TWH * CIN; i += 64 * CT_WAVES) {
-            const int pix = i / CIN, c = i % CIN;
-            const int yy = y0 + pix / TWH - 1, xx = x0 + pix % TWH - 1;
-            float v = 0.f;
-            if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) v = (float)a.in[(img + (size_t)yy * a.W + xx) * CIN + c];
-            tile[pix * PS + c] = (__bf16)v;
-        }
-    }
-    // weights -> registers (one 16-byte fragment per k step)
-    const int n = lane & 31, kh = lane >> 5;
-    bf16x8 Bf[KSTEPS];
+    const int kh = lane >> 5, col = lane & 31;
+    // stage the tile (+ halo) as BF16; outside the image is zero padding.
+    // Every piece of the thread is requested before any is stored: a load
+    // always happens (the image's first piece outside it) and is dropped.
+    constexpr int VC = CIN % 4 == 0 ? 4 : CIN;   // channels per piece
+    constexpr int Q = CIN / VC, NP = ((CT_H + 2) * TWH * Q + 64 * CT_WAVES - 1) / (64 * CT_WAVES);
+    typedef TI VecI __attribute__((ext_vector_type(VC)));
+    typedef __bf16 VecB __attribute__((ext_vector_type(VC)));
+    VecI pre[NP];
 #pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) Bf[s] = a.wf[s * 64 + lane];
+    for (int k = 0; k < NP; ++k) {
+        const int i = threadIdx.x + 64 * CT_WAVES * k, pix = i / Q;
+        const int yy = y0 + pix / TWH - 1, xx = x0 + pix % TWH - 1;
+        const bool ok = pix < (CT_H + 2) * TWH && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
+        const VecI t = reinterpret_cast<const VecI*>(a.in)[ok ? (img + (size_t)yy * a.W + xx) * Q + i % Q : 0];
+        pre[k] = ok ? t : (VecI)(TI)0.f;
+    }
+    // the weight fragments, once per workgroup
+    constexpr int NW = (KSTEPS * 64 + 64 * CT_WAVES - 1) / (64 * CT_WAVES);
+    bf16x8 wp[NW];
+#pragma unroll
+    for (int k = 0; k < NW; ++k) wp[k] = a.wf[min((int)threadIdx.x + 64 * CT_WAVES * k, KSTEPS * 64 - 1)];
+    // residual of this lane's outputs, in flight with the tile
+    constexpr int NV = COUT < 4 ? COUT : 4;  // channels per run (COUT is 2 or a multiple of 4)
+    static_assert(COUT < 4 || COUT % 4 == 0, "output channels");
+    constexpr int NQ = COUT < 32 ? 1 : 4;
+    float rv[2][NQ][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int ch0 = 8 * q + 4 * kh, y = y0 + 2 * wave + h, x = x0 + col;
+            const bool ok = a.res && y < a.H && x < a.W && ch0 < COUT;
+            const TO* r = (ok ? a.res : a.out) + (ok ? (img + (size_t)y * a.W + x) * COUT + ch0 : 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rv[h][q][i] = ok && i < NV ? (float)r[i < NV ? i : 0] : 0.f;
+        }
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const int i = threadIdx.x + 64 * CT_WAVES * k;
+        if (i >= (CT_H + 2) * TWH * Q) break;
+        VecB w;
+#pragma unroll
+        for (int e = 0; e < VC; ++e) w[e] = (__bf16)pre[k][e];
+        *reinterpret_cast<VecB*>(tile + (i / Q) * PS + VC * (i % Q)) = w;
+    }
+#pragma unroll
+    for (int k = 0; k < NW; ++k) wf[min((int)threadIdx.x + 64 * CT_WAVES * k, KSTEPS * 64 - 1)] = wp[k];
     __syncthreads();
 
-    const int col = lane & 31;
     f32x16 acc[2] = {(f32x16)0.f, (f32x16)0.f};
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
         const int k0 = 16 * s + 8 * kh;
+        const bf16x8 Wf = wf[s * 64 + lane];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int r = 2 * wave + h;
@@ -227,35 +205,17 @@ __global__ __launch_bounds__(64 * CT_WAVES) void conv3x3_fwd(ConvArgsT<TI, TO> a
                     A[e] = tap < 9 ? tile[((r + tap / 3) * TWH + col + tap % 3) * PS + c] : (__bf16)0.f;
                 }
             }
-            acc[h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(Bf[s], A, acc[h], 0, 0, 0);
+            acc[h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(Wf, A, acc[h], 0, 0, 0);
         }
     }
     // epilogue: the weights are the MFMA A operand, so register v of lane
     // (col, kh) is output channel 8 (v/4) + 4 kh + v%4 of pixel col: four
     // runs of four consecutive channels per lane (vector stores, one bounds
     // check per pixel)
-    constexpr int NV = COUT < 4 ? COUT : 4;  // channels per run (COUT is 2 or a multiple of 4)
-    static_assert(COUT < 4 || COUT % 4 == 0, "output channels");
     const int x = x0 + col;
     if (x >= a.W) return;
-    // residuals first, all in flight together (out may not be assumed
-    // distinct from res by the compiler, which would otherwise serialise
-    // each load behind the previous store)
-    float rv[2][4][4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int ch0 = 8 * q + 4 * kh, y = y0 + 2 * wave + h;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) rv[h][q][i] = 0.f;
-            if (!a.res || y >= a.H || ch0 >= COUT) continue;
-            const TO* r = a.res + (img + (size_t)y * a.W + x) * COUT + ch0;
-#pragma unroll
-            for (int i = 0; i < NV; ++i) rv[h][q][i] = (float)r[i];
-        }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < NQ; ++q) {
         const int ch0 = 8 * q + 4 * kh;
         if (ch0 >= COUT) continue;
         float bias[4] = {0.f, 0.f, 0.f, 0.f};
@@ -326,62 +286,20 @@ __global__ void pack_weights(const float* __restrict__ P, bf16x8* __restrict__ o
     out[L.foff + f] = v;
 }
 
-// relu'(pre) from the post-activation: g *= [act > 0]
-__global__ void relu_mask(float* g, const float* act, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !(act[i] > 0.f)) g[i] = 0.f;
-}
-
-// ---- weight gradient -------------------------------------------------------------
-// dW[n][tap][c] = sum_p dY[p][n] X[p + off(tap)][c], db[n] = sum_p dY[p][n].
-// As a GEMM over pixels (K) with M = COUT, N = CIN per tap: with q = p + off,
-// the B operand (X at q) is the same for all taps and the A operand is dY
-// shifted, so a wave keeps one X fragment for the taps of its column and
-// reuses each dY row for three of them.  Pixels are taken in 8 x 32 tiles of
-// X; dY is staged with a one-pixel halo.  Both stay pixel-major in LDS as they
-// come from HBM (BF16, 64 bytes per pixel): ds_read_b64_tr_b16 hands each lane
-// four pixels of its channel, at any pixel offset and without bank conflicts
-// (a row of 16 lanes reads four whole pixels).
-//
-// Six waves: wave (d, h) takes the taps of column d (three rows of taps) over
-// rows 4h .. 4h + 3 of the tile; wave d = 1 also the bias (the centre tap's dY
-// against ones).  The two row halves are added in LDS at the end.  Workgroup g
-// accumulates tiles g, g + G, ... in registers (a fixed order), the next
-// tile's pixels loaded while the current one is contracted, and writes
-// part[g][COUT][9 CIN + 1]; dw_reduce sums the partials in workgroup order
-// (deterministic).
-//
-// Bound by the latency of the few tiles a workgroup has: 8 x 128^2 pixels (two
-// tiles each) 12.0 us = 3.3 TB/s of dY (with halo) and X.  512 workgroups of
-// one tile 17 us; 168 registers for three workgroups per CU spill, 16 us.
-// (Operands transposed on the way into LDS by 2-byte stores, with three
-// shifted copies of X, took 71 us in bank conflicts.)
-
-constexpr int DW_WAVES = 6, DW_THREADS = 64 * DW_WAVES;
-constexpr int DW_MAX_GROUPS = 256;
-
-struct DwArgs {
-    const float* dy;   // [npix][COUT]
-    const float* x;    // [npix][CIN]
-    float* part;       // [groups][COUT][ncol]
-    int B, H, W;
-    int tiles_x, tiles_y;
-};
-
 // Pixels of a ROWS x COLS window whose first is (y0, x0), C channels (32 or 2)
-// of an NHWC image: loaded to registers (zeros outside the image, without a
-// branch per load), then stored to LDS as BF16, 32 channels per pixel (the
-// channels from C on are not written).
-template <int ROWS, int COLS, int C>
-struct DwStage {
+// of an NHWC image: loaded to registers by NT threads (zeros outside the image;
+// a load always happens, without a branch), then stored to LDS as BF16, PS
+// elements per pixel (the channels from C on are not written).
+template <int ROWS, int COLS, int C, int NT, int PS>
+struct Window {
     static constexpr int Q = C / 4 > 0 ? C / 4 : 1;   // pieces per pixel
-    static constexpr int N = (ROWS * COLS * Q + DW_THREADS - 1) / DW_THREADS;
+    static constexpr int N = (ROWS * COLS * Q + NT - 1) / NT;
     typedef typename std::conditional<C == 2, float2, float4>::type V;
     V v[N];
     __device__ __forceinline__ void load(const float* img, int y0, int x0, int H, int W) {
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            const int i = threadIdx.x + DW_THREADS * k, px = i / Q;
+            const int i = threadIdx.x + NT * k, px = i / Q;
             const int y = y0 + px / COLS, x = x0 + px % COLS;
             const bool ok = px < ROWS * COLS && y >= 0 && y < H && x >= 0 && x < W;
             const V t = reinterpret_cast<const V*>(img)[ok ? ((size_t)y * W + x) * Q + i % Q : 0];
@@ -391,9 +309,9 @@ struct DwStage {
     __device__ __forceinline__ void store(__bf16* lds) const {
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            const int i = threadIdx.x + DW_THREADS * k;
+            const int i = threadIdx.x + NT * k;
             if (i >= ROWS * COLS * Q) break;
-            __bf16* d = lds + (i / Q) * 32 + 4 * (i % Q);
+            __bf16* d = lds + (i / Q) * PS + 4 * (i % Q);
             if constexpr (C == 2)
                 *reinterpret_cast<bf16x2*>(d) = bf16x2{(__bf16)v[k].x, (__bf16)v[k].y};
             else
@@ -404,18 +322,282 @@ struct DwStage {
 };
 
 // MFMA operand from pixel-major LDS: lane l gets channel l % 32 of pixels
-// 8 (l / 32) .. + 7 after `px` (a pixel's 32 channels at px, 64 bytes apart)
+// 8 (l / 32) .. + 7 from `px` on (PS elements apart)
+template <int PS>
 __device__ __forceinline__ bf16x8 dw_fragment(const __bf16* px, int lane) {
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) s16x4* P;
     // a group of 16 lanes reads 4 pixels x 16 channels, lane i of it 4
     // channels of pixel i / 4, and lane i receives channel i of the four
     const int g = lane >> 4, i = lane & 15;
-    const __bf16* s = px + (8 * (g >> 1) + (i >> 2)) * 32 + 16 * (g & 1) + 4 * (i & 3);
+    const __bf16* s = px + (8 * (g >> 1) + (i >> 2)) * PS + 16 * (g & 1) + 4 * (i & 3);
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(s));
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(s + 4 * 32));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(s + 4 * PS));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
+
+// One wave's part of a weight gradient over an 8 x 32 tile of X: the taps of
+// column d over NR rows of the tile from row r0 (py: dY at the tile's first
+// pixel, its row PW pixels long and stored with a halo of at least one; px: X,
+// 32 pixels a row).  X row r meets dY rows r + 1, r, r - 1 (tap rows 0, 1, 2),
+// each shifted by 1 - d columns: a dY fragment serves three taps, an X
+// fragment the three taps of the column.
+template <int PS, int PW, int NR>
+__device__ __forceinline__ void dw_tile(f32x16 (&acc)[3], const __bf16* py, const __bf16* px, int r0, int d, int lane) {
+    py += ((r0 - 1) * PW + 1 - d) * PS;
+    px += r0 * CT_W * PS;
+#pragma unroll
+    for (int s = 0; s < CT_W / 16; ++s) {
+        bf16x8 A[NR + 2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) A[r] = dw_fragment<PS>(py + (r * PW + 16 * s) * PS, lane);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            A[r + 2] = dw_fragment<PS>(py + ((r + 2) * PW + 16 * s) * PS, lane);
+            const bf16x8 X = dw_fragment<PS>(px + (r * CT_W + 16 * s) * PS, lane);
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[r + 2 - t], X, acc[t], 0, 0, 0);
+        }
+    }
+}
+
+// the bias gradient over the same rows: dY against ones (every column of the
+// result is the sum)
+template <int PS, int PW, int NR>
+__device__ __forceinline__ void db_tile(f32x16& acc, const __bf16* py, int r0, int lane) {
+    const bf16x8 ones = (bf16x8)(__bf16)1.f;
+#pragma unroll
+    for (int s = 0; s < CT_W / 16; ++s)
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dw_fragment<PS>(py + ((r0 + r) * PW + 16 * s) * PS, lane),
+                                                          ones, acc, 0, 0, 0);
+}
+
+// ---- residual block, FP32 activations (training) ------------------------------------
+// Forward: a = relu(conv1(h) + b1), h' = h + conv2(a) + b2.  Backward: da =
+// [a > 0] conv2^T(dh), dh' = dh + conv1^T(da) (the flipped, transposed
+// weights).  Both are: mid = f(conv(in)), out = in + conv(mid), with in, mid and
+// out in FP32 in HBM and the convolutions' operands rounded to BF16, as
+// conv3x3_fwd rounds them (same fragments and order of accumulation).
+//
+// One kernel instead of two: in is read once with a two-pixel halo; forward
+// stores a for the backward pass, backward also takes both weight gradients
+// (dW2 from dh and a, dW1 from da and h) from the tiles it has in LDS, so da
+// never goes to HBM.  A persistent workgroup of 8 waves per CU (both weight
+// sets in LDS) walks 8 x 32 tiles: it stages in on 12 x 36 pixels, computes mid
+// on 10 x 34 (ten rows of 32 pixels and a 10 x 2 strip, eleven units over the
+// waves) into LDS, then one output row per wave; backward, waves 0-5 add a tap
+// column of one of the two weight gradients each and waves 6 and 7 the bias
+// gradients (waves w and w + 4 share a SIMD: 154 to 172 matrix instructions
+// each per tile).  The next tile is loaded while the current one is computed.
+// Bound by the tiles' memory traffic (in with its halo 28 MB, mid or mask and
+// out 17 MB each, h 17 MB per 8 x 128^2 pixels): forward 18-19 us = 4.2 TB/s
+// where the two convolutions took 29; backward 30 us = 3.5 TB/s where two
+// convolutions, the ReLU mask and two weight gradients of one kernel each took
+// 67 (12 us a weight gradient, 3.3 TB/s).  FP32 forward of the 8-block network
+// at 1024^2: 1.68 -> 0.96 ms.
+constexpr int DW_MAX_GROUPS = 256;                    // partial weight gradients, at most
+constexpr int R32_IH = CT_H + 4, R32_IW = CT_W + 4;   // staged input
+constexpr int R32_MH = CT_H + 2, R32_MW = CT_W + 2;   // mid
+constexpr int R32_PS = 40;                            // LDS pixel stride (bf16)
+constexpr int R32_WAVES = 8, R32_THREADS = 64 * R32_WAVES;
+constexpr int R32_KS = 18;                            // k steps of a 32-channel convolution
+
+struct Rb32Args {
+    const float* in;      // [B][H][W][32]
+    const float* mask;    // backward: the post-activation a
+    float* mid;           // forward: a, for the backward pass (or null: not stored)
+    float* out;           // distinct from in
+    const float* h;       // backward: the block's input, and the partial weight
+    float* part;          // gradients [conv2, conv1][groups][32][289] (dw_reduce)
+    const bf16x8* w1;     // fragments of the first and second convolution (pack_weights)
+    const bf16x8* w2;
+    const float* b1;      // biases (forward)
+    const float* b2;
+    int B, H, W;
+};
+
+template <bool BWD>
+constexpr size_t R32_LDS = (size_t)(R32_IH * R32_IW + R32_MH * R32_MW + (BWD ? 2 * CT_H * CT_W : 0)) * R32_PS * 2 +
+                           2 * R32_KS * 64 * 16 + 256;
+
+// 32 pixels x 32 channels: operands from pixel-major LDS (src: this lane's
+// pixel at tap 0, its half of the channels), weights from LDS
+template <int IW>
+__device__ __forceinline__ f32x16 r32_conv(const __bf16* src, const bf16x8* w) {
+    f32x16 acc = (f32x16)0.f;
+#pragma unroll
+    for (int s = 0; s < R32_KS; ++s) {
+        const int tap = s / 2;
+        const bf16x8 X =
+            *reinterpret_cast<const bf16x8*>(src + ((tap / 3) * IW + tap % 3) * R32_PS + 16 * (s & 1));
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s * 64], X, acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+template <bool BWD>
+__global__ __launch_bounds__(R32_THREADS, 2) void resblock_f32(Rb32Args a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __bf16* in_t = reinterpret_cast<__bf16*>(smem);
+    __bf16* mid_t = in_t + R32_IH * R32_IW * R32_PS;
+    bf16x8* w_s = reinterpret_cast<bf16x8*>(mid_t + R32_MH * R32_MW * R32_PS);
+    float4* bias_s = reinterpret_cast<float4*>(w_s + 2 * R32_KS * 64);   // b1, b2
+    __bf16* a_t = reinterpret_cast<__bf16*>(bias_s + 16);                 // backward: a and h on the tile
+    __bf16* h_t = a_t + CT_H * CT_W * R32_PS;
+    const int lane = threadIdx.x & 63, px = lane & 31, kh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = threadIdx.x; i < 2 * R32_KS * 64; i += R32_THREADS)
+        w_s[i] = i < R32_KS * 64 ? a.w1[i] : a.w2[i - R32_KS * 64];
+    if (threadIdx.x < 64)
+        reinterpret_cast<float*>(bias_s)[threadIdx.x] =
+            BWD ? 0.f : threadIdx.x < 32 ? a.b1[threadIdx.x] : a.b2[threadIdx.x - 32];
+    const int tiles_x = (a.W + CT_W - 1) / CT_W, tiles_y = (a.H + CT_H - 1) / CT_H;
+    const int ntiles = tiles_x * tiles_y * a.B;
+    Window<R32_IH, R32_IW, 32, R32_THREADS, R32_PS> win;
+    Window<CT_H, CT_W, 32, R32_THREADS, R32_PS> hwin;
+    auto fetch = [&](int tile) {
+        const int tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, b = tile / (tiles_x * tiles_y);
+        win.load(a.in + (size_t)b * a.H * a.W * 32, ty * CT_H - 2, tx * CT_W - 2, a.H, a.W);
+        if constexpr (BWD) hwin.load(a.h + (size_t)b * a.H * a.W * 32, ty * CT_H, tx * CT_W, a.H, a.W);
+    };
+    // weight gradients: wave w < 6 tap column w % 3 of conv2 (w < 3) or conv1,
+    // wave 6 and 7 their biases (wacc[0])
+    const bool first = wave < 3 || wave == 6;   // conv2's, whose dY is dh
+    f32x16 wacc[3] = {(f32x16)0.f, (f32x16)0.f, (f32x16)0.f};
+    fetch(blockIdx.x);
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int x0 = tile % tiles_x * CT_W, y0 = (tile / tiles_x) % tiles_y * CT_H;
+        const size_t img = (size_t)(tile / (tiles_x * tiles_y)) * a.H * a.W;
+        __syncthreads();   // the previous tile's reads are done
+        win.store(in_t);
+        if constexpr (BWD) hwin.store(h_t);
+        __syncthreads();
+        // this wave's output row: residual, requested ahead of the next tile
+        const int oy = y0 + wave, ox = x0 + px;
+        const bool out_ok = oy < a.H && ox < a.W;
+        const size_t opx = out_ok ? img + (size_t)oy * a.W + ox : 0;
+        float4 rv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) rv[q] = reinterpret_cast<const float4*>(a.in + opx * 32)[2 * q + kh];
+        // mid units: u < 10: row u, columns 0..31; u = 10: the 20 pixels of
+        // columns 32 and 33
+        auto unit = [&](int u) {
+            const bool strip = u == R32_MH;
+            const int f = px < 2 * R32_MH ? px : 2 * R32_MH - 1;
+            const int mr = strip ? f >> 1 : u, mc = strip ? CT_W + (f & 1) : px;
+            const int yy = y0 - 1 + mr, xx = x0 - 1 + mc;
+            const bool inside = yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
+            const size_t p = inside ? img + (size_t)yy * a.W + xx : 0;
+            float4 mk[4];
+            if constexpr (BWD)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) mk[q] = reinterpret_cast<const float4*>(a.mask + p * 32)[2 * q + kh];
+            const f32x16 acc = r32_conv<R32_IW>(in_t + (mr * R32_IW + mc) * R32_PS + 8 * kh, w_s + lane);
+            if (strip && px >= 2 * R32_MH) return;
+            // (mid and a of a pixel belong to the tile it is in)
+            const bool own = mr >= 1 && mr <= CT_H && mc >= 1 && mc <= CT_W;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 bq = bias_s[2 * q + kh];
+                float4 v = make_float4(acc[4 * q] + bq.x, acc[4 * q + 1] + bq.y, acc[4 * q + 2] + bq.z,
+                                       acc[4 * q + 3] + bq.w);
+                if constexpr (BWD) {
+                    if (own) {
+                        const bf16x4 m = {(__bf16)mk[q].x, (__bf16)mk[q].y, (__bf16)mk[q].z, (__bf16)mk[q].w};
+                        *reinterpret_cast<bf16x4*>(a_t + ((mr - 1) * CT_W + mc - 1) * R32_PS + 8 * q + 4 * kh) =
+                            inside ? m : (bf16x4)(__bf16)0.f;
+                    }
+                    v.x = mk[q].x > 0.f ? v.x : 0.f;
+                    v.y = mk[q].y > 0.f ? v.y : 0.f;
+                    v.z = mk[q].z > 0.f ? v.z : 0.f;
+                    v.w = mk[q].w > 0.f ? v.w : 0.f;
+                } else {
+                    v = make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f));
+                }
+                if (!BWD && own && inside && a.mid) reinterpret_cast<float4*>(a.mid + p * 32)[2 * q + kh] = v;
+                // outside the image: the second convolution's zero padding
+                const bf16x4 o = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+                *reinterpret_cast<bf16x4*>(mid_t + (mr * R32_MW + mc) * R32_PS + 8 * q + 4 * kh) =
+                    inside ? o : (bf16x4)(__bf16)0.f;
+            }
+        };
+        if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
+        unit(wave);
+        if (wave >= 6) unit(wave + 2);   // rows 8 and 9
+        if (wave == 2) unit(R32_MH);     // the strip
+        __syncthreads();
+        if constexpr (BWD) {
+            const __bf16* py = first ? in_t + (2 * R32_IW + 2) * R32_PS : mid_t + (R32_MW + 1) * R32_PS;
+            const __bf16* px_t = first ? a_t : h_t;
+            if (first) {
+                if (wave < 6) dw_tile<R32_PS, R32_IW, CT_H>(wacc, py, px_t, 0, wave % 3, lane);
+                else db_tile<R32_PS, R32_IW, CT_H>(wacc[0], py, 0, lane);
+            } else {
+                if (wave < 6) dw_tile<R32_PS, R32_MW, CT_H>(wacc, py, px_t, 0, wave % 3, lane);
+                else db_tile<R32_PS, R32_MW, CT_H>(wacc[0], py, 0, lane);
+            }
+        }
+        const f32x16 acc = r32_conv<R32_MW>(mid_t + (wave * R32_MW + px) * R32_PS + 8 * kh,
+                                            w_s + R32_KS * 64 + lane);
+        if (out_ok) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 bq = bias_s[8 + 2 * q + kh];
+                reinterpret_cast<float4*>(a.out + opx * 32)[2 * q + kh] =
+                    make_float4(acc[4 * q] + bq.x + rv[q].x, acc[4 * q + 1] + bq.y + rv[q].y,
+                                acc[4 * q + 2] + bq.z + rv[q].z, acc[4 * q + 3] + bq.w + rv[q].w);
+            }
+        }
+    }
+    if constexpr (BWD) {
+        constexpr int NCOL = 9 * 32 + 1;
+        float* dst = a.part + ((size_t)(first ? 0 : gridDim.x) + blockIdx.x) * 32 * NCOL;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int n = 8 * (v >> 2) + 4 * kh + (v & 3);   // output channel
+            if (wave < 6) {
+#pragma unroll
+                for (int t = 0; t < 3; ++t) dst[(size_t)n * NCOL + (3 * t + wave % 3) * 32 + px] = wacc[t][v];
+            } else if (px == 0) {
+                dst[(size_t)n * NCOL + NCOL - 1] = wacc[0][v];
+            }
+        }
+    }
+}
+
+// ---- weight gradient -------------------------------------------------------------
+// dW[n][tap][c] = sum_p dY[p][n] X[p + off(tap)][c], db[n] = sum_p dY[p][n], for
+// the head and tail (the blocks' are taken in resblock_f32<true>).  As a GEMM
+// over pixels (K) with M = COUT, N = CIN per tap: with q = p + off, the B
+// operand (X at q) is the same for all taps and the A operand is dY shifted
+// (dw_tile).  Pixels are taken in 8 x 32 tiles of X; dY is staged with a
+// one-pixel halo.  Both stay pixel-major in LDS as they come from HBM (BF16, 64
+// bytes per pixel, channels beyond CIN or COUT zero): ds_read_b64_tr_b16 hands
+// each lane four pixels of its channel, at any pixel offset.
+//
+// Six waves: wave (d, h) takes the taps of column d (three rows of taps) over
+// rows 4h .. 4h + 3 of the tile; wave d = 1 also the bias.  The two row halves
+// are added in LDS at the end.  Workgroup g accumulates tiles g, g + G, ... in
+// registers (a fixed order), the next tile's pixels loaded while the current
+// one is contracted, and writes part[g][COUT][9 CIN + 1]; dw_reduce sums the
+// partials in workgroup order (deterministic).
+//
+// Bound by latency (two tiles a workgroup): 8 x 128^2 pixels 9.4 us head, 7.3
+// us tail.  (Operands transposed on the way into LDS by 2-byte stores, with
+// three shifted copies of X: 27 and 60 us, in bank conflicts.)
+
+constexpr int DW_WAVES = 6, DW_THREADS = 64 * DW_WAVES;
+
+struct DwArgs {
+    const float* dy;   // [npix][COUT]
+    const float* x;    // [npix][CIN]
+    float* part;       // [groups][COUT][ncol]
+    int B, H, W;
+    int tiles_x, tiles_y;
+};
 
 template <int CIN, int COUT>
 __global__ __launch_bounds__(DW_THREADS, 2) void conv3x3_dw(DwArgs a) {
@@ -434,9 +616,8 @@ __global__ __launch_bounds__(DW_THREADS, 2) void conv3x3_dw(DwArgs a) {
         for (int i = threadIdx.x; i < (NDY + NX) / 8; i += DW_THREADS)
             reinterpret_cast<bf16x8*>(lds)[i] = (bf16x8)(__bf16)0.f;
     f32x16 acc[3] = {(f32x16)0.f, (f32x16)0.f, (f32x16)0.f}, accb = (f32x16)0.f;
-    const bf16x8 ones = (bf16x8)(__bf16)1.f;
-    DwStage<DR, DC, COUT> ry;
-    DwStage<CT_H, CT_W, CIN> rx;
+    Window<DR, DC, COUT, DW_THREADS, 32> ry;
+    Window<CT_H, CT_W, CIN, DW_THREADS, 32> rx;
     auto fetch = [&](int tile) {
         const int tx = tile % a.tiles_x, ty = (tile / a.tiles_x) % a.tiles_y, b = tile / (a.tiles_x * a.tiles_y);
         const size_t img = (size_t)b * a.H * a.W;
@@ -450,25 +631,9 @@ __global__ __launch_bounds__(DW_THREADS, 2) void conv3x3_dw(DwArgs a) {
         rx.store(sx);
         __syncthreads();
         if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
-#pragma unroll
-        for (int s = 0; s < CT_W / 16; ++s) {
-            // X row r meets dY halo rows r .. r + 2 (tap rows 2, 1, 0), from
-            // halo column 2 - d
-            const __bf16* py = sdy + (4 * half * DC + 16 * s + 2 - d) * 32;
-            const __bf16* px = sx + (4 * half * CT_W + 16 * s) * 32;
-            bf16x8 A[6];
-#pragma unroll
-            for (int r = 0; r < 2; ++r) A[r] = dw_fragment(py + r * DC * 32, lane);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                A[r + 2] = dw_fragment(py + (r + 2) * DC * 32, lane);
-                const bf16x8 X = dw_fragment(px + r * CT_W * 32, lane);
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[r + 2 - t], X, acc[t], 0, 0, 0);
-                if (d == 1) accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[r + 1], ones, accb, 0, 0, 0);
-            }
-        }
+        const __bf16* py = sdy + (DC + 1) * 32;   // the tile's first pixel
+        dw_tile<32, DC, 4>(acc, py, sx, 4 * half, d, lane);
+        if (d == 1) db_tile<32, DC, 4>(accb, py, 4 * half, lane);
     }
     // add the row halves: [d][register][lane]
     __syncthreads();
@@ -499,10 +664,15 @@ __global__ __launch_bounds__(DW_THREADS, 2) void conv3x3_dw(DwArgs a) {
 // Sum of the workgroup partials into the gradient (W and b).  A workgroup
 // takes 32 neighbouring elements (128-byte reads); its eight rows of threads
 // add the partials of an eighth of the groups each, in order, and the eight
-// sums are added in order (the same on every run).  9.5 MB in 4.6 us (one wave
-// per element, its lanes reading 37 KB apart, took 13).
+// sums are added in order (the same on every run).  A block's two gradients, 19
+// MB, in 5.4 us (one wave per element, its lanes reading 37 KB apart: 26).
 __global__ __launch_bounds__(256) void dw_reduce(const float* __restrict__ part, int groups, int cout, int ncol,
-                                                 float* gw, float* gb) {
+                                                 float* gw, float* gb, float* gw_1, float* gb_1) {
+    if (blockIdx.y) {   // a second gradient, its partials after the first's
+        part += (size_t)groups * cout * ncol;
+        gw = gw_1;
+        gb = gb_1;
+    }
     __shared__ double sums[8][32];
     const int e = threadIdx.x & 31, k = threadIdx.x >> 5;
     const int i = blockIdx.x * 32 + e, n = cout * ncol;
@@ -578,11 +748,6 @@ __global__ void adam_step(float* p, const float* g, float* m, float* v, int64_t 
     m[i] = mi;
     v[i] = vi;
     p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-__global__ void add_inplace(float* a, const float* b, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] += b[i];
 }
 
 // ---- fused residual block (inference, BF16 activations) ----------------------
@@ -1373,14 +1538,41 @@ int conv_dw(oph_ctx* ctx, oph_cnn* net, const float* dy, const float* x, int B, 
     if (ntiles > INT32_MAX) return oph_fail(ctx, OPH_EINVAL, "too many pixels");
     OPH_LAUNCH(ctx, "conv3x3_dw", (conv3x3_dw<CIN, COUT>), dim3((unsigned)groups), dim3(DW_THREADS), 0, a);
     OPH_LAUNCH(ctx, "dw_reduce", dw_reduce, dim3((COUT * NCOL + 31) / 32), dim3(256), 0, net->part, groups, COUT,
-               NCOL, gw, gb);
+               NCOL, gw, gb, nullptr, nullptr);
+    return OPH_OK;
+}
+
+// One residual block with FP32 activations, forward, or (mask set) backward
+// with the weight gradients into gw2, gb2, gw1, gb1
+int resblock_f32_run(oph_ctx* ctx, const Rb32Args& a, float* gw2 = nullptr, float* gb2 = nullptr, float* gw1 = nullptr,
+                     float* gb1 = nullptr) {
+    static bool attr = false;
+    if (!attr) {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&resblock_f32<false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)R32_LDS<false>);
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&resblock_f32<true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)R32_LDS<true>);
+        hipGetLastError();
+        attr = true;
+    }
+    const int64_t ntiles = (int64_t)((a.W + CT_W - 1) / CT_W) * ((a.H + CT_H - 1) / CT_H) * a.B;
+    if (ntiles > INT32_MAX) return oph_fail(ctx, OPH_EINVAL, "too many pixels");
+    // one workgroup per CU (LDS), at most as many as there is room for partials
+    const int groups = (int)std::min<int64_t>(ntiles, std::min(std::max(ctx->cu_count, 1), DW_MAX_GROUPS));
+    if (!a.mask) {
+        OPH_LAUNCH(ctx, "resblock_f32", resblock_f32<false>, dim3(groups), dim3(R32_THREADS), R32_LDS<false>, a);
+        return OPH_OK;
+    }
+    OPH_LAUNCH(ctx, "resblock_f32_bwd", resblock_f32<true>, dim3(groups), dim3(R32_THREADS), R32_LDS<true>, a);
+    OPH_LAUNCH(ctx, "dw_reduce", dw_reduce, dim3((32 * (9 * 32 + 1) + 31) / 32, 2), dim3(256), 0, a.part, groups, 32,
+               9 * 32 + 1, gw2, gb2, gw1, gb1);
     return OPH_OK;
 }
 
 // dX = conv(dY, flipped/transposed W): input channels COUT, output CIN
 template <int CIN, int COUT>
-int conv_dx(oph_ctx* ctx, const float* dy, const bf16x8* wfrag, float* dx, const float* res, int B, int H, int W) {
-    return conv_fwd<COUT, CIN>(ctx, dy, wfrag, nullptr, res, dx, B, H, W, 0);
+int conv_dx(oph_ctx* ctx, const float* dy, const bf16x8* wfrag, float* dx, int B, int H, int W) {
+    return conv_fwd<COUT, CIN>(ctx, dy, wfrag, nullptr, nullptr, dx, B, H, W, 0);
 }
 
 constexpr int ksteps(int cin) { return (9 * cin + 15) / 16; }
@@ -1433,19 +1625,18 @@ uint64_t splitmix(uint64_t& s) {
 }
 
 // activation workspace: x copy handled by caller; h_0..h_NB and a_1..a_NB,
-// gradients dh, da, and the output
+// gradients dh (two), and the output
 struct Acts {
     float* h[CMAX + 1];
     float* a[CMAX + 1];
     float* y;
     float* g0;
-    float* g1;
     float* g2;
 };
 
 int ensure_workspace(oph_ctx* ctx, oph_cnn* net, int64_t npix, Acts& A) {
     const size_t per = (size_t)npix * net->ch * sizeof(float);
-    const size_t need = per * (2 * net->blocks + 1 + 3) + (size_t)npix * 2 * sizeof(float);
+    const size_t need = per * (2 * net->blocks + 1 + 2) + (size_t)npix * 2 * sizeof(float);
     if (need > net->act_bytes) {
         if (net->act) hipFree(net->act);
         net->act = nullptr;
@@ -1460,10 +1651,9 @@ int ensure_workspace(oph_ctx* ctx, oph_cnn* net, int64_t npix, Acts& A) {
     for (int b = 0; b <= net->blocks; ++b) { A.h[b] = reinterpret_cast<float*>(p); p += per; }
     for (int b = 1; b <= net->blocks; ++b) { A.a[b] = reinterpret_cast<float*>(p); p += per; }
     A.g0 = reinterpret_cast<float*>(p); p += per;
-    A.g1 = reinterpret_cast<float*>(p); p += per;
     A.g2 = reinterpret_cast<float*>(p); p += per;
     A.y = reinterpret_cast<float*>(p);
-    const size_t pneed = (size_t)DW_MAX_GROUPS * 32 * (9 * 32 + 1) * sizeof(float);
+    const size_t pneed = 2 * (size_t)DW_MAX_GROUPS * 32 * (9 * 32 + 1) * sizeof(float);
     if (pneed > net->part_bytes) {
         if (net->part) hipFree(net->part);
         net->part = nullptr;
@@ -1477,7 +1667,8 @@ int ensure_workspace(oph_ctx* ctx, oph_cnn* net, int64_t npix, Acts& A) {
     return OPH_OK;
 }
 
-int forward(oph_ctx* ctx, oph_cnn* net, const float* x, int B, int H, int W, Acts& A) {
+// keep: store the activations the backward pass needs
+int forward(oph_ctx* ctx, oph_cnn* net, const float* x, int B, int H, int W, Acts& A, bool keep) {
     const Layout L{net->ch, net->blocks};
     const float* P = net->params;
     const Frags F{net->blocks};
@@ -1486,9 +1677,8 @@ int forward(oph_ctx* ctx, oph_cnn* net, const float* x, int B, int H, int W, Act
     if (net->wf_rev != net->params_rev && (rc = pack(ctx, net, false))) return rc;
     if ((rc = conv_fwd<2, 32>(ctx, x, WF + F.head(), P + L.head_b(), nullptr, A.h[0], B, H, W, 0))) return rc;
     for (int b = 0; b < net->blocks; ++b) {
-        if ((rc = conv_fwd<32, 32>(ctx, A.h[b], WF + F.conv1(b), P + L.b1(b), nullptr, A.a[b + 1], B, H, W, 1)))
-            return rc;
-        if ((rc = conv_fwd<32, 32>(ctx, A.a[b + 1], WF + F.conv2(b), P + L.b2(b), A.h[b], A.h[b + 1], B, H, W, 0)))
+        if ((rc = resblock_f32_run(ctx, {A.h[b], nullptr, keep ? A.a[b + 1] : nullptr, A.h[b + 1], nullptr, nullptr,
+                                         WF + F.conv1(b), WF + F.conv2(b), P + L.b1(b), P + L.b2(b), B, H, W})))
             return rc;
     }
     return conv_fwd<32, 2>(ctx, A.h[net->blocks], WF + F.tail(), P + L.tail_b(), x, A.y, B, H, W, 0);
@@ -1540,7 +1730,7 @@ int backward(oph_ctx* ctx, oph_cnn* net, const float* x, const float* t, int B, 
     const float* P = net->params;
     float* G = net->grads;
     const int64_t npix = (int64_t)B * H * W;
-    const int64_t n2 = npix * 2, nc = npix * net->ch;
+    const int64_t n2 = npix * 2;
     const unsigned nb = (unsigned)((n2 + 255) / 256);
     float* dy = A.g2;  // 2-channel output gradient (fits in a C-channel buffer)
     OPH_LAUNCH(ctx, "mse_grad", mse_grad, dim3(nb), dim3(256), 0, A.y, t, dy, n2, net->red);
@@ -1552,16 +1742,14 @@ int backward(oph_ctx* ctx, oph_cnn* net, const float* x, const float* t, int B, 
     // tail: y = x + conv(h_NB)
     if ((rc = conv_dw<32, 2>(ctx, net, dy, A.h[net->blocks], B, H, W, G + L.tail_w(), G + L.tail_b()))) return rc;
     float* dh = A.g0;
-    if ((rc = conv_dx<32, 2>(ctx, dy, WB + F.tail_t(), dh, nullptr, B, H, W))) return rc;
+    if ((rc = conv_dx<32, 2>(ctx, dy, WB + F.tail_t(), dh, B, H, W))) return rc;
     for (int b = net->blocks - 1; b >= 0; --b) {
         // h_{b+1} = h_b + conv2(a); a = relu(conv1(h_b))
-        float* da = A.g1;
-        if ((rc = conv_dw<32, 32>(ctx, net, dh, A.a[b + 1], B, H, W, G + L.w2(b), G + L.b2(b)))) return rc;
-        if ((rc = conv_dx<32, 32>(ctx, dh, WB + F.conv2_t(b), da, nullptr, B, H, W))) return rc;
-        OPH_LAUNCH(ctx, "relu_mask", relu_mask, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, da, A.a[b + 1], nc);
-        if ((rc = conv_dw<32, 32>(ctx, net, da, A.h[b], B, H, W, G + L.w1(b), G + L.b1(b)))) return rc;
-        // dh_b = dh_{b+1} + conv1^T(da)
-        if ((rc = conv_dx<32, 32>(ctx, da, WB + F.conv1_t(b), A.g2, dh, B, H, W))) return rc;
+        // dh_b = dh_{b+1} + conv1^T(da), da = relu'(conv2^T(dh_{b+1}))
+        if ((rc = resblock_f32_run(ctx, {dh, A.a[b + 1], nullptr, A.g2, A.h[b], net->part, WB + F.conv2_t(b),
+                                         WB + F.conv1_t(b), nullptr, nullptr, B, H, W},
+                                   G + L.w2(b), G + L.b2(b), G + L.w1(b), G + L.b1(b))))
+            return rc;
         float* tmp = dh;
         dh = A.g2;
         A.g2 = tmp;
@@ -1685,7 +1873,7 @@ int oph_cnn_forward(oph_ctx* ctx, oph_cnn* n, const float* x, float* y, int B, i
     if (flags & OPH_CNN_BF16_ACTS) {
         if ((rc = forward_bf16(ctx, n, dx, dyv, B, H, W, A))) return rc;
     } else {
-        if ((rc = forward(ctx, n, dx, B, H, W, A))) return rc;
+        if ((rc = forward(ctx, n, dx, B, H, W, A, false))) return rc;
         OPH_HIP_CHECK(ctx, hipMemcpyAsync(dyv, A.y, bytes, hipMemcpyDeviceToDevice, ctx->stream));
     }
     if (!(flags & OPH_DEVICE_PTR))
@@ -1713,7 +1901,7 @@ static int train_or_grad(oph_ctx* ctx, oph_cnn* n, const float* x, const float* 
         dx = s;
         dt = s + npix * 2;
     }
-    if ((rc = forward(ctx, n, dx, B, H, W, A))) return rc;
+    if ((rc = forward(ctx, n, dx, B, H, W, A, true))) return rc;
     if ((rc = backward(ctx, n, dx, dt, B, H, W, A, loss))) return rc;
     if (update) {
         n->params_rev += 1;

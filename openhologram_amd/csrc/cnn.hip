@@ -95,11 +95,11 @@ struct ConvArgsT {
     int relu;
 };
 
-// Tiled forward convolution.  A workgroup of 8 waves owns an 8-row x 32-
+// Tiled forward convolution.  A workgroup of 4 waves owns an 8-row x 32-
 // column pixel tile of one image: it stages the tile and its one-pixel halo
 // in LDS once, as BF16 (pixel stride padded by 16 bytes so that the 16-byte
-// A-fragment reads of a half-wave fall on distinct banks), and each wave
-// keeps its B fragments (the weights, BF16) in registers for the whole tile.
+// A-fragment reads of a half-wave fall on distinct banks), and the weight
+// fragments (BF16) beside them.
 // Wave w computes tile rows 2w and 2w + 1: 32 pixels x 32 output channels
 // each, K = 9 CIN in steps of 16 on v_mfma_f32_32x32x16_bf16 (one weight
 // fragment feeds two MFMAs).  Lane l: pixel l%32, k half l/32;

@@ -22,116 +22,181 @@
 // N-1), 'right' zeroes -N/2 .. -1 (indices N/2 .. N-1); 'top'/'bottom' the
 // same on rows.
 //
-// Reductions (max |U|^2, min/max of a float array) are exact in any order;
-// every pass is one HBM sweep.
+// The mask depends on one axis only, and the other axis's transform and its
+// inverse cancel: 'left' and 'right' are a one-dimensional filter of every
+// row, 'top' and 'bottom' of every column, one pass over the field (forward
+// transform, mask and inverse transform of a line without leaving the
+// workgroup) instead of four transforms and the masking.
+//
+// Reductions (max |U|^2, min/max of a float array) are exact in any order: a
+// pass that needs one leaves a (min, max) pair per workgroup and the next pass
+// starts by combining them, so every pass is one HBM sweep and one launch.
+#include <algorithm>
 #include <cfloat>
+#include <cmath>
+#include <type_traits>
 
+#include "fft_engine.h"
 #include "fft_kernels.h"
 #include "oph_internal.h"
 
 namespace {
 
-constexpr int RT = 256;      // threads per reduction workgroup
-constexpr int RB = 1024;     // reduction workgroups (at most)
+constexpr int RT = 256;      // threads per workgroup
+constexpr int RB = 1024;     // workgroups of a reducing pass (and partial pairs), at most
+constexpr int MB = 8192;     // workgroups of the other passes, at most
 
-// part[2b] = min, part[2b+1] = max of f(i) over this workgroup's stride
-template <typename F>
-__device__ void reduce_minmax(F f, int64_t n, float* part) {
-    __shared__ float smin[RT], smax[RT];
-    float mn = FLT_MAX, mx = -FLT_MAX;
-    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) {
-        const float v = f(i);
-        mn = fminf(mn, v);
-        mx = fmaxf(mx, v);
+// (min, max) over the workgroup of each thread's (mn, mx); every thread of
+// the workgroup calls it and gets the result.  NT threads, a multiple of 64
+// (or fewer than 64).
+template <int NT>
+__device__ __forceinline__ float2 block_minmax(float mn, float mx) {
+    __shared__ float2 w[(NT + 63) / 64];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        mn = fminf(mn, __shfl_xor(mn, o, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     }
-    smin[threadIdx.x] = mn;
-    smax[threadIdx.x] = mx;
     __syncthreads();
-    for (int s = RT / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            smin[threadIdx.x] = fminf(smin[threadIdx.x], smin[threadIdx.x + s]);
-            smax[threadIdx.x] = fmaxf(smax[threadIdx.x], smax[threadIdx.x + s]);
-        }
-        __syncthreads();
+    if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = make_float2(mn, mx);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < (NT + 63) / 64; ++k) {
+        mn = fminf(mn, w[k].x);
+        mx = fmaxf(mx, w[k].y);
     }
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = smin[0];
-        part[2 * blockIdx.x + 1] = smax[0];
-    }
+    return make_float2(mn, mx);
 }
 
-__global__ __launch_bounds__(RT) void abs2_minmax_partial(const float2* __restrict__ u, int64_t n, float* part) {
-    reduce_minmax([=](int64_t i) { const float2 v = u[i]; return fmaf(v.x, v.x, v.y * v.y); }, n, part);
-}
-
-__global__ __launch_bounds__(RT) void minmax_partial_f(const float* __restrict__ s, int64_t n, float* part) {
-    reduce_minmax([=](int64_t i) { return s[i]; }, n, part);
-}
-
-// part[0] = min, part[1] = max over the nb partials (pairs)
-__global__ __launch_bounds__(RT) void minmax_combine(float* part, int nb) {
-    __shared__ float smin[RT], smax[RT];
+// (min, max) of the nb pairs an earlier pass left (RT threads)
+__device__ __forceinline__ float2 combine(const float2* __restrict__ part, int nb) {
     float mn = FLT_MAX, mx = -FLT_MAX;
     for (int i = threadIdx.x; i < nb; i += RT) {
-        mn = fminf(mn, part[2 * i]);
-        mx = fmaxf(mx, part[2 * i + 1]);
+        const float2 p = part[i];
+        mn = fminf(mn, p.x);
+        mx = fmaxf(mx, p.y);
     }
-    smin[threadIdx.x] = mn;
-    smax[threadIdx.x] = mx;
-    __syncthreads();
-    for (int s = RT / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            smin[threadIdx.x] = fminf(smin[threadIdx.x], smin[threadIdx.x + s]);
-            smax[threadIdx.x] = fmaxf(smax[threadIdx.x], smax[threadIdx.x + s]);
+    return block_minmax<RT>(mn, mx);
+}
+
+__global__ __launch_bounds__(RT) void abs2_minmax_partial(const float2* __restrict__ u, int64_t n, float2* part) {
+    float mn = FLT_MAX, mx = -FLT_MAX;
+    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) {
+        const float2 v = u[i];
+        const float a = fmaf(v.x, v.x, v.y * v.y);
+        mn = fminf(mn, a);
+        mx = fmaxf(mx, a);
+    }
+    const float2 m = block_minmax<RT>(mn, mx);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+// One-dimensional single-sideband filter of the lines of a field: columns
+// (COLS; B neighbouring ones per workgroup, thread T of line T % B) or rows
+// (B per workgroup, threads of a line side by side); the real part and each
+// workgroup's (min, max).  A line that is not finite spoils the whole field,
+// as it does in a two-dimensional transform: its (NaN, NaN) partial, which
+// ssb_scale looks for, carries that over.
+// Bound by HBM (8 bytes in, 4 out per pixel) and the transforms' LDS passes:
+// 2048^2 rows 19 us; with ssb_scale 28 us a call, where four transforms, two
+// copies, the masking, two reductions and the scaling took 115.
+template <int L>
+constexpr int ssb_lines(bool cols) { return cols ? fftk::col_lines(L) : fftk::row_lines(L); }
+
+template <int L, bool COLS>
+__global__ __launch_bounds__(ssb_lines<L>(COLS) * (L / 16)) void ssb_filter(const float2* __restrict__ u,
+                                                                           float* __restrict__ out, int lines,
+                                                                           int upper, float scale,
+                                                                           const float2* __restrict__ tw,
+                                                                           float2* part) {
+    constexpr int TPL = L / 16, B = ssb_lines<L>(COLS), NT = B * TPL;
+    // (columns: 4 more elements a line, so that the lanes of a wave, which hold
+    // neighbouring columns, fall on different banks)
+    constexpr int PL = fft::padded_len(L) + (COLS ? 4 : 0);
+    extern __shared__ float2 ssb_lds[];
+    const int b = COLS ? threadIdx.x % B : threadIdx.x / TPL;
+    const int t = COLS ? threadIdx.x / B : threadIdx.x % TPL;
+    float2* buf = ssb_lds + b * PL;
+    // (rows keep the twiddles in registers; a column workgroup is up to 1024
+    // threads of 128 registers and reads them from the table at each stage)
+    fft::Twiddles<COLS ? 16 : L> T;
+    if constexpr (!COLS) T.load(tw, t);
+    // element i of line l at l ls + i es
+    const size_t ls = COLS ? 1 : L, es = COLS ? (size_t)lines : 1;
+    float mn = FLT_MAX, mx = -FLT_MAX;
+    bool nan = false;
+    const int groups = (lines + B - 1) / B;
+    for (int g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
+        const int l = (COLS ? xcd_remap(g0, groups) : g0) * B + b;
+        const bool ok = l < lines;
+        const size_t at = (size_t)(ok ? l : 0) * ls;
+        float2 v[16];
+#pragma unroll
+        for (int m = 0; m < 16; ++m) v[m] = u[at + (size_t)(t + m * TPL) * es];
+        // (a zero the compiler cannot see through: it would hoist the table
+        // reads out of the loop into registers)
+        int tz = t;
+        if constexpr (COLS) asm volatile("" : "+v"(tz));
+        auto line = [&](auto sign) {
+            if constexpr (COLS) fft::line_regs_tw<L, sign>(v, buf, tw, tz);
+            else fft::line_regs<L, sign>(v, buf, T, t);
+        };
+        __syncthreads();   // the previous line's last-stage reads are done
+        line(std::integral_constant<int, -1>{});
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const int k = t + m * TPL;
+            const bool stop = upper ? k >= L / 2 : k < L / 2 || k == L - 1;
+            if (stop) v[m] = make_float2(0.f, 0.f);
         }
         __syncthreads();
+        line(std::integral_constant<int, +1>{});
+        if (!ok) continue;
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const float x = v[m].x * scale;
+            out[at + (size_t)(t + m * TPL) * es] = x;
+            mn = fminf(mn, x);
+            mx = fmaxf(mx, x);
+            nan |= !(fabsf(x) <= FLT_MAX);
+        }
     }
-    if (threadIdx.x == 0) {
-        part[0] = smin[0];
-        part[1] = smax[0];
-    }
-}
-
-// zero the stop band of a spectrum in FFT order
-__global__ void ssb_mask(float2* a, int nx, int ny, int passband) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)nx * ny) return;
-    const int c = (int)(i % nx), r = (int)(i / nx);
-    bool stop;
-    switch (passband) {
-        case OPH_PASS_LEFT: stop = c < nx / 2 || c == nx - 1; break;
-        case OPH_PASS_RIGHT: stop = c >= nx / 2; break;
-        case OPH_PASS_TOP: stop = r < ny / 2 || r == ny - 1; break;
-        default: stop = r >= ny / 2; break;
-    }
-    if (stop) a[i] = make_float2(0.f, 0.f);
-}
-
-__global__ void real_part(const float2* __restrict__ a, float* __restrict__ out, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = a[i].x;
+    const float2 p = block_minmax<NT>(mn, mx);
+    const bool bad = __syncthreads_or(nan);
+    if (threadIdx.x == 0) part[blockIdx.x] = bad ? make_float2(NAN, NAN) : p;
 }
 
 // out = (v - min)/(max - min)  (SSB: realPositive / max(realPositive))
-__global__ void shift_scale(float* out, int64_t n, const float* __restrict__ mm) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (out[i] - mm[0]) / (mm[1] - mm[0]);
+__global__ __launch_bounds__(RT) void ssb_scale(float* out, int64_t n, const float2* __restrict__ part, int nb) {
+    bool nan = false;
+    for (int i = threadIdx.x; i < nb; i += RT) nan |= part[i].x != part[i].x;
+    const bool bad = __syncthreads_or(nan);
+    const float2 m = combine(part, nb);
+    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT)
+        out[i] = bad ? NAN : (out[i] - m.x) / (m.y - m.x);
 }
 
-// NI first pass: |U + max|U||^2 (mm2[1] = max |U|^2)
-__global__ void ni_map(const float2* __restrict__ u, float* __restrict__ out, int64_t n, const float* __restrict__ mm2) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float ref = sqrtf(mm2[1]);
-    const float2 v = u[i];
-    const float re = v.x + ref;
-    out[i] = fmaf(re, re, v.y * v.y);
+// NI first pass: |U + max|U||^2, and its (min, max) per workgroup
+__global__ __launch_bounds__(RT) void ni_map(const float2* __restrict__ u, float* __restrict__ out, int64_t n,
+                                             const float2* __restrict__ part2, int nb, float2* part) {
+    const float ref = sqrtf(combine(part2, nb).y);
+    float mn = FLT_MAX, mx = -FLT_MAX;
+    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) {
+        const float2 v = u[i];
+        const float re = v.x + ref;
+        const float o = fmaf(re, re, v.y * v.y);
+        out[i] = o;
+        mn = fminf(mn, o);
+        mx = fmaxf(mx, o);
+    }
+    const float2 m = block_minmax<RT>(mn, mx);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
 // out /= max(out)
-__global__ void div_max(float* out, int64_t n, const float* __restrict__ mm) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = out[i] / mm[1];
+__global__ __launch_bounds__(RT) void div_max(float* out, int64_t n, const float2* __restrict__ part, int nb) {
+    const float mx = combine(part, nb).y;
+    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) out[i] = out[i] / mx;
 }
 
 __global__ void p2a_real_map(const float2* __restrict__ u, float* __restrict__ out, int64_t n, int p2a) {
@@ -142,62 +207,79 @@ __global__ void p2a_real_map(const float2* __restrict__ u, float* __restrict__ o
 }
 
 // Burckhardt (fn_encoding.m:60-83) and two-phase (:85-98), one pixel per
-// thread; mm2[1] = max |U|^2.  angle(U/m) = angle(U) for m > 0.
-__global__ void burckhardt_map(const float2* __restrict__ u, float* __restrict__ out, int nx, int64_t n,
-                               const float* __restrict__ mm2) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float m = sqrtf(mm2[1]);
-    const float2 v = u[i];
-    const float re = v.x / m, im = v.y / m;
-    const float am = sqrtf(fmaf(re, re, im * im));
-    const float ph = atan2f(im, re) + 3.14159265358979323846f;
-    constexpr float third = 2.09439510239319549f, two_third = 4.18879020478639098f, two_pi = 6.28318530717958648f;
-    constexpr float inv_s3 = 0.57735026918962576f;
-    float a1 = 0.f, a2 = 0.f, a3 = 0.f;
-    if (ph >= 0.f && ph < third) {
-        a1 = am * (cosf(ph) + sinf(ph) * inv_s3);
-        a2 = 2.f * sinf(ph) * inv_s3;
-    } else if (ph >= third && ph < two_third) {
-        const float q = ph - third;
-        a2 = am * (cosf(q) + sinf(q) * inv_s3);
-        a3 = 2.f * sinf(q) * inv_s3;
-    } else if (ph >= two_third && ph < two_pi) {
-        const float q = ph - two_third;
-        a3 = am * (cosf(q) + sinf(q) * inv_s3);
-        a1 = 2.f * sinf(q) * inv_s3;
+// thread and step (pixel i's components are out[3 i ..] and out[2 i ..]);
+// the pairs hold max |U|^2.  angle(U/m) = angle(U) for m > 0.
+__global__ __launch_bounds__(RT) void burckhardt_map(const float2* __restrict__ u, float* __restrict__ out, int64_t n,
+                                                     const float2* __restrict__ part2, int nb) {
+    const float m = sqrtf(combine(part2, nb).y);
+    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) {
+        const float2 v = u[i];
+        const float re = v.x / m, im = v.y / m;
+        const float am = sqrtf(fmaf(re, re, im * im));
+        const float ph = atan2f(im, re) + 3.14159265358979323846f;
+        constexpr float third = 2.09439510239319549f, two_third = 4.18879020478639098f, two_pi = 6.28318530717958648f;
+        constexpr float inv_s3 = 0.57735026918962576f;
+        float a1 = 0.f, a2 = 0.f, a3 = 0.f;
+        if (ph >= 0.f && ph < third) {
+            a1 = am * (cosf(ph) + sinf(ph) * inv_s3);
+            a2 = 2.f * sinf(ph) * inv_s3;
+        } else if (ph >= third && ph < two_third) {
+            const float q = ph - third;
+            a2 = am * (cosf(q) + sinf(q) * inv_s3);
+            a3 = 2.f * sinf(q) * inv_s3;
+        } else if (ph >= two_third && ph < two_pi) {
+            const float q = ph - two_third;
+            a3 = am * (cosf(q) + sinf(q) * inv_s3);
+            a1 = 2.f * sinf(q) * inv_s3;
+        }
+        out[3 * i] = a1;
+        out[3 * i + 1] = a2;
+        out[3 * i + 2] = a3;
     }
-    const int64_t r = i / nx, c = i % nx;
-    float* o = out + r * 3 * nx + 3 * c;
-    o[0] = a1;
-    o[1] = a2;
-    o[2] = a3;
 }
 
-__global__ void two_phase_map(const float2* __restrict__ u, float* __restrict__ out, int nx, int64_t n,
-                              const float* __restrict__ mm2) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float m = sqrtf(mm2[1]);
-    const float2 v = u[i];
-    const float re = v.x / m, im = v.y / m;
-    const float am = fminf(sqrtf(fmaf(re, re, im * im)), 1.f);
-    const float ph = atan2f(im, re) + 3.14159265358979323846f;
-    const float d = acosf(am);
-    const int64_t r = i / nx, c = i % nx;
-    float* o = out + r * 2 * nx + 2 * c;
-    o[0] = ph + d;
-    o[1] = ph - d;
+__global__ __launch_bounds__(RT) void two_phase_map(const float2* __restrict__ u, float* __restrict__ out, int64_t n,
+                                                    const float2* __restrict__ part2, int nb) {
+    const float m = sqrtf(combine(part2, nb).y);
+    for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) {
+        const float2 v = u[i];
+        const float re = v.x / m, im = v.y / m;
+        const float am = fminf(sqrtf(fmaf(re, re, im * im)), 1.f);
+        const float ph = atan2f(im, re) + 3.14159265358979323846f;
+        const float d = acosf(am);
+        out[2 * i] = ph + d;
+        out[2 * i + 1] = ph - d;
+    }
 }
 
-int reduce(oph_ctx* ctx, const char* name, int which, const void* src, int64_t n, float* part) {
-    const int nb = (int)std::min<int64_t>(RB, (n + RT - 1) / RT);
-    if (which == 0)
-        OPH_LAUNCH(ctx, name, abs2_minmax_partial, dim3(nb), dim3(RT), 0, static_cast<const float2*>(src), n, part);
-    else
-        OPH_LAUNCH(ctx, name, minmax_partial_f, dim3(nb), dim3(RT), 0, static_cast<const float*>(src), n, part);
-    OPH_LAUNCH(ctx, "minmax_combine", minmax_combine, dim3(1), dim3(RT), 0, part, nb);
+template <int L, bool COLS>
+int launch_ssb(oph_ctx* ctx, const float2* u, float* out, int lines, int upper, float2* part, int* nb) {
+    const float2* tw = oph_twiddles(ctx, L);
+    if (!tw) return OPH_ENOMEM;
+    constexpr int B = ssb_lines<L>(COLS), NT = B * (L / 16);
+    constexpr size_t shm = (size_t)B * (fft::padded_len(L) + (COLS ? 4 : 0)) * sizeof(float2);
+    static bool attr = false;
+    if (!attr) {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&ssb_filter<L, COLS>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+        hipGetLastError();
+        attr = true;
+    }
+    *nb = std::min(RB, (lines + B - 1) / B);
+    OPH_LAUNCH(ctx, "ssb_filter", (ssb_filter<L, COLS>), dim3(*nb), dim3(NT), shm, u, out, lines, upper,
+               (float)(1.0 / (double)L), tw, part);
     return OPH_OK;
+}
+
+template <bool COLS>
+int ssb_dispatch(oph_ctx* ctx, int L, const float2* u, float* out, int lines, int upper, float2* part, int* nb) {
+    switch (L) {
+#define OPH_SSB_CASE(n) \
+    case n: return launch_ssb<n, COLS>(ctx, u, out, lines, upper, part, nb);
+        OPH_FFT_LENGTHS(OPH_SSB_CASE)
+#undef OPH_SSB_CASE
+    }
+    return oph_fail(ctx, OPH_ENOTSUP, "FFT length %d not supported (16..8192)", L);
 }
 
 }  // namespace
@@ -227,43 +309,52 @@ extern "C" int oph_encode_field(oph_ctx* ctx, const oph_c64* field, int nx, int 
         OPH_HIP_CHECK(ctx, hipMemcpyAsync(du, field, n * sizeof(float2), hipMemcpyHostToDevice, ctx->stream));
         u = du;
     }
-    // two reductions' partials (NI reads the first's result during the second)
-    float* part = static_cast<float*>(oph_scratch(ctx, SLOT_AUX1, sizeof(float) * 4 * RB));
+    // two reductions' pairs (NI reads the first's during the second)
+    float2* part = static_cast<float2*>(oph_scratch(ctx, SLOT_AUX1, sizeof(float2) * 2 * RB));
     if (!part) return OPH_ENOMEM;
-    float* part2 = part + 2 * RB;
-    const dim3 grid((unsigned)((n + 255) / 256)), blk(256);
+    float2* part2 = part + RB;
+    int nb = (int)std::min<int64_t>(RB, (n + RT - 1) / RT);
+    const dim3 grid(nb), blk(RT);
+    // passes without a reduction of their own (each workgroup first combines
+    // the pairs): eight pixels a thread, fewer while that leaves the chip idle
+    // (Burckhardt: 1024 x 512 11.6 us at two, 15.2 at eight; 4096^2 120 us at
+    // eight, 137 in 1,024 workgroups of 64)
+    const dim3 mgrid((unsigned)std::min<int64_t>(MB, std::max<int64_t>(nb, (n + 8 * RT - 1) / (8 * RT))));
+    if (method != OPH_ENC_SSB && method != OPH_ENC_P2A && method != OPH_ENC_REAL)
+        OPH_LAUNCH(ctx, "abs2_minmax_partial", abs2_minmax_partial, grid, blk, 0, u, n, part);
     switch (method) {
         case OPH_ENC_SSB: {
-            float2* w = static_cast<float2*>(oph_scratch(ctx, SLOT_WORK0, n * sizeof(float2)));
-            if (!w) return OPH_ENOMEM;
-            OPH_HIP_CHECK(ctx, hipMemcpyAsync(w, u, n * sizeof(float2), hipMemcpyDeviceToDevice, ctx->stream));
-            if ((rc = oph_fft_rows(ctx, nx, -1, w, ny, nx, 1.f))) return rc;
-            if ((rc = oph_fft_cols(ctx, ny, -1, w, nx, nx, 1.f))) return rc;
-            OPH_LAUNCH(ctx, "ssb_mask", ssb_mask, grid, blk, 0, w, nx, ny, passband);
-            if ((rc = oph_fft_rows(ctx, nx, +1, w, ny, nx, 1.f))) return rc;
-            if ((rc = oph_fft_cols(ctx, ny, +1, w, nx, nx, (float)(1.0 / (double)n)))) return rc;
-            OPH_LAUNCH(ctx, "real_part", real_part, grid, blk, 0, w, o, n);
-            if ((rc = reduce(ctx, "minmax_partial_f", 1, o, n, part))) return rc;
-            OPH_LAUNCH(ctx, "shift_scale", shift_scale, grid, blk, 0, o, n, part);
+            const int upper = passband == OPH_PASS_RIGHT || passband == OPH_PASS_BOTTOM;
+            int np = 0;
+            if (reinterpret_cast<const char*>(u) < reinterpret_cast<const char*>(o + n) &&
+                reinterpret_cast<const char*>(o) < reinterpret_cast<const char*>(u + n)) {
+                // out overlaps the field, which the filter still reads while it writes
+                float2* w = static_cast<float2*>(oph_scratch(ctx, SLOT_WORK0, n * sizeof(float2)));
+                if (!w) return OPH_ENOMEM;
+                OPH_HIP_CHECK(ctx, hipMemcpyAsync(w, u, n * sizeof(float2), hipMemcpyDeviceToDevice, ctx->stream));
+                u = w;
+            }
+            rc = passband == OPH_PASS_LEFT || passband == OPH_PASS_RIGHT
+                     ? ssb_dispatch<false>(ctx, nx, u, o, ny, upper, part, &np)
+                     : ssb_dispatch<true>(ctx, ny, u, o, nx, upper, part, &np);
+            if (rc) return rc;
+            OPH_LAUNCH(ctx, "ssb_scale", ssb_scale, mgrid, blk, 0, o, n, part, np);
             break;
         }
         case OPH_ENC_NI:
-            if ((rc = reduce(ctx, "abs2_minmax_partial", 0, u, n, part))) return rc;
-            OPH_LAUNCH(ctx, "ni_map", ni_map, grid, blk, 0, u, o, n, part);
-            if ((rc = reduce(ctx, "minmax_partial_f", 1, o, n, part2))) return rc;
-            OPH_LAUNCH(ctx, "div_max", div_max, grid, blk, 0, o, n, part2);
+            OPH_LAUNCH(ctx, "ni_map", ni_map, grid, blk, 0, u, o, n, part, nb, part2);
+            OPH_LAUNCH(ctx, "div_max", div_max, mgrid, blk, 0, o, n, part2, nb);
             break;
         case OPH_ENC_P2A:
         case OPH_ENC_REAL:
-            OPH_LAUNCH(ctx, "p2a_real_map", p2a_real_map, grid, blk, 0, u, o, n, method == OPH_ENC_P2A ? 1 : 0);
+            OPH_LAUNCH(ctx, "p2a_real_map", p2a_real_map, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, u, o, n,
+                       method == OPH_ENC_P2A ? 1 : 0);
             break;
         case OPH_ENC_BURCKHARDT:
-            if ((rc = reduce(ctx, "abs2_minmax_partial", 0, u, n, part))) return rc;
-            OPH_LAUNCH(ctx, "burckhardt_map", burckhardt_map, grid, blk, 0, u, o, nx, n, part);
+            OPH_LAUNCH(ctx, "burckhardt_map", burckhardt_map, mgrid, blk, 0, u, o, n, part, nb);
             break;
         default:
-            if ((rc = reduce(ctx, "abs2_minmax_partial", 0, u, n, part))) return rc;
-            OPH_LAUNCH(ctx, "two_phase_map", two_phase_map, grid, blk, 0, u, o, nx, n, part);
+            OPH_LAUNCH(ctx, "two_phase_map", two_phase_map, mgrid, blk, 0, u, o, n, part, nb);
             break;
     }
     if (!(flags & OPH_DEVICE_PTR))

@@ -304,6 +304,100 @@ __device__ __forceinline__ void line_tw(float2* buf, const float2* __restrict__ 
 template <int L>
 __host__ __device__ constexpr bool regs_fusable() { return n16(L) >= 2 && last_radix(L) == 1; }
 
+// Full transform with the thread's elements in registers at both ends: on
+// entry v[m] is input element t + m L/16, on return output element t + m L/16.
+// True of every length here: the last stage, of radix RL and Ns = L/RL, takes
+// butterfly j = t + p L/16 (p < 16/RL) whose inputs and outputs are both
+// elements j + r L/RL = t + (p + 16 r/RL) L/16.  So a line passes through LDS
+// only between stages (half the LDS accesses of line() with the line staged
+// in LDS at both ends, at three stages).  The caller syncs before the line is
+// written again (other threads may still read the last stage's inputs).
+//
+// w16(s, w) gives the 15 twiddles of radix-16 stage s, wl(p, w) those of the
+// last radix-RL stage's butterfly p.
+template <int L, int SIGN, typename W16, typename WL>
+__device__ __forceinline__ void line_regs_w(float2 (&v)[16], float2* buf, int t, W16&& w16, WL&& wl) {
+    constexpr int TPL = L / 16;
+    constexpr int A = n16(L);
+    constexpr int RL = last_radix(L);
+    Dft<16, SIGN>::run(v);
+    if constexpr (L > 16) {
+        float2* dst = buf + pad16(16 * t);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dst[r] = v[r];
+        __syncthreads();
+        int Ns = 16;
+        constexpr int MID = RL > 1 ? A - 1 : A - 2;
+#pragma unroll
+        for (int s = 1; s <= MID; ++s) {
+            float2 w[1][16];
+            w16(s, w[0]);
+            stage<L, 16, SIGN, TPL>(buf, w, Ns, t);
+            Ns *= 16;
+        }
+#pragma unroll
+        for (int m = 0; m < 16; ++m) v[m] = buf[lane_pad<L>(t, m)];
+        if constexpr (RL > 1) {
+            constexpr int PL = 16 / RL;
+#pragma unroll
+            for (int p = 0; p < PL; ++p) {
+                float2 u[RL], w[RL];
+                wl(p, w);
+                u[0] = v[p];
+#pragma unroll
+                for (int r = 1; r < RL; ++r)
+                    u[r] = SIGN < 0 ? cmul(v[p + r * PL], w[r]) : cmulc(v[p + r * PL], w[r]);
+                Dft<RL, SIGN>::run(u);
+#pragma unroll
+                for (int r = 0; r < RL; ++r) v[p + r * PL] = u[r];
+            }
+        } else {
+            float2 w[16];
+            w16(A - 1, w);
+#pragma unroll
+            for (int r = 1; r < 16; ++r) v[r] = SIGN < 0 ? cmul(v[r], w[r]) : cmulc(v[r], w[r]);
+            Dft<16, SIGN>::run(v);
+        }
+    }
+}
+
+// ... with every stage's twiddles in registers
+template <int L, int SIGN>
+__device__ __forceinline__ void line_regs(float2 (&v)[16], float2* buf, const Twiddles<L>& T, int t) {
+    line_regs_w<L, SIGN>(
+        v, buf, t,
+        [&](int s, float2 (&w)[16]) {
+#pragma unroll
+            for (int r = 1; r < 16; ++r) w[r] = T.w16[s - 1][0][r];
+        },
+        [&](int p, float2 (&w)[last_radix(L)]) {
+#pragma unroll
+            for (int r = 1; r < last_radix(L); ++r) w[r] = T.wl[p][r];
+        });
+}
+
+// ... with each stage's twiddles loaded from the table just before it
+template <int L, int SIGN>
+__device__ __forceinline__ void line_regs_tw(float2 (&v)[16], float2* buf, const float2* __restrict__ tw, int t) {
+    constexpr int TPL = L / 16, RL = last_radix(L), N = RL > 1 ? L / RL : 1;   // N = 16^A where RL > 1
+    line_regs_w<L, SIGN>(
+        v, buf, t,
+        [&](int s, float2 (&w)[16]) {
+            int Ns = 16, off = 0;
+            for (int i = 1; i < s; ++i) {
+                off += 15 * Ns;
+                Ns *= 16;
+            }
+#pragma unroll
+            for (int r = 1; r < 16; ++r) w[r] = tw[off + (r - 1) * Ns + (t & (Ns - 1))];
+        },
+        [&](int p, float2 (&w)[RL]) {
+            // the radix-16 tables before it hold 15 (16 + ... + 16^(A-1)) = 16^A - 16 entries
+#pragma unroll
+            for (int r = 1; r < RL; ++r) w[r] = tw[N - 16 + (r - 1) * N + t + p * TPL];
+        });
+}
+
 // Stage 0 (Ns = 1) on v (elements t + r L/16), result written to the line.
 template <int L, int SIGN>
 __device__ __forceinline__ void stage0_from_regs(float2 (&v)[16], float2* buf, int t) {

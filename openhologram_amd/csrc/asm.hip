@@ -126,7 +126,9 @@ __device__ __forceinline__ void apply_transfer(float2 (&v)[N], const float4 ax, 
         v[j] = fft::cmul(v[j], transfer<EXACT, BAND>(ax, ay[j], bz[j], c, t + (m0 + j) * (L / 16), k));
 }
 
-template <int L>
+// HALF (this and asm_rows_inv): the data columns are the middle half of the
+// row (twofold padding), so only m in [4, 12) can be nonzero or is needed.
+template <int L, bool HALF>
 __global__ __launch_bounds__(512) void asm_rows_fwd(const float2* __restrict__ in, int nx, int ny, int ox,
                                                     int oy, float2* __restrict__ work,
                                                     const float2* __restrict__ tw, TabJob tj) {
@@ -142,17 +144,23 @@ __global__ __launch_bounds__(512) void asm_rows_fwd(const float2* __restrict__ i
     const float2* src = in + (size_t)(ok ? r : 0) * nx;
     fft::Twiddles<L> T;
     T.load(tw, t);
+    float2 v[16];
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
         const int c = t + m * TPL - ox;
-        buf[fft::lane_pad<L>(t, m)] = (ok && c >= 0 && c < nx) ? src[c] : make_float2(0.f, 0.f);
+        if (HALF) {
+            v[m] = m >= 4 && m < 12 ? src[c] : make_float2(0.f, 0.f);   // (a row past the end: row 0, dropped)
+        } else {
+            const bool in_row = c >= 0 && c < nx;
+            const float2 x = src[in_row ? c : 0];
+            v[m] = in_row ? x : make_float2(0.f, 0.f);
+        }
     }
-    __syncthreads();
-    fft::line<L, -1>(buf, T, t);
+    fft::line_regs<L, -1>(v, buf, T, t);
     if (ok) {
         float2* dst = work + (size_t)(oy + r) * L;
 #pragma unroll
-        for (int m = 0; m < 16; ++m) dst[t + m * TPL] = buf[fft::lane_pad<L>(t, m)];
+        for (int m = 0; m < 16; ++m) dst[t + m * TPL] = v[m];
     }
 }
 
@@ -291,6 +299,60 @@ __global__ __launch_bounds__(1024) void asm_cols(float2* work, int npx, int ny, 
     }
 }
 
+// Columns with the elements in registers at both ends of each transform
+// (thread T: column T mod B, rows t + m L/16, t = T / B): the forward
+// transform's outputs are multiplied by the transfer and enter the inverse one
+// without a pass through LDS, and the columns go from and to global memory
+// without staging.  Range-checked buffer accesses: rows outside [oy, oy + ny)
+// read zeros and write nothing.  HALF: the data rows are the middle half
+// (twofold padding), so only m in [4, 12) is read, can be nonzero and is kept.
+// REG_TW: twiddles in registers (up to 512 threads), else read from the table
+// at each stage.
+template <int L, int B, bool EXACT, bool REG_TW, bool HALF>
+__global__ __launch_bounds__(B * (L / 16)) void asm_cols_r(float2* work, int npx, int ny, int oy,
+                                                          const float4* __restrict__ tabx,
+                                                          const float4* __restrict__ taby,
+                                                          const float2* __restrict__ taby2, AsmConst k,
+                                                          const float2* __restrict__ tw) {
+    constexpr int TPL = L / 16;
+    constexpr int PL = fft::skewed_len(L, B);
+    constexpr int M0 = HALF ? 4 : 0, M1 = HALF ? 12 : 16;
+    extern __shared__ float2 lds[];
+    const int b = threadIdx.x % B, t = threadIdx.x / B;
+    const int c = xcd_remap(blockIdx.x, gridDim.x) * B + b;   // npx is a power of two >= B
+    float2* buf = lds + b * PL;
+    const auto rs = oph_buf_rsrc(work, (unsigned)((size_t)(oy + ny) * npx * sizeof(float2)));
+    auto at = [&](int m) {
+        const int i = t + m * TPL;
+        return HALF || (i >= oy && i < oy + ny) ? (unsigned)(((size_t)i * npx + c) * sizeof(float2)) : OPH_BUF_OOB;
+    };
+    float2 v[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) v[m] = m >= M0 && m < M1 ? oph_buf_load_f2(rs, at(m)) : make_float2(0.f, 0.f);
+    fft::Twiddles<REG_TW ? L : 16> T;
+    if constexpr (REG_TW) T.load(tw, t);
+    const float4 ax = tabx[c];
+    if constexpr (REG_TW) fft::line_regs<L, -1>(v, buf, T, t);
+    else fft::line_regs_tw<L, -1>(v, buf, tw, t);
+    // (a few rows at a time: the table entries of all 16 would take 32 registers)
+    constexpr int CH = EXACT ? 2 : 4;
+#pragma unroll
+    for (int m0 = 0; m0 < 16; m0 += CH) {
+        float2 u[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) u[j] = v[m0 + j];
+        if (k.band) apply_transfer<L, EXACT, true>(u, ax, taby2, taby, c, t, m0, k);
+        else apply_transfer<L, EXACT, false>(u, ax, taby2, taby, c, t, m0, k);
+#pragma unroll
+        for (int j = 0; j < CH; ++j) v[m0 + j] = u[j];
+    }
+    __syncthreads();   // every lane has read the line
+    if constexpr (REG_TW) fft::line_regs<L, +1>(v, buf, T, t);
+    else fft::line_regs_tw<L, +1>(v, buf, tw, t);
+#pragma unroll
+    for (int m = M0; m < M1; ++m) oph_buf_store_f2(v[m], rs, at(m));
+}
+
 // 4096-point columns whose data rows are exactly the middle half,
 // [1024, 3072) (twofold padding), B columns per step, persistent.  The first
 // forward butterfly's inputs t + m 256 with m outside [4, 12) are known zeros
@@ -416,7 +478,7 @@ __global__ __launch_bounds__(B * (MID_L / 16), 4) void asm_cols_mid(
     }
 }
 
-template <int L>
+template <int L, bool HALF>
 __global__ __launch_bounds__(512) void asm_rows_inv(const float2* __restrict__ work, int nx, int ny, int ox,
                                                     int oy, float scale, float2* __restrict__ out,
                                                     const float2* __restrict__ tw) {
@@ -431,15 +493,16 @@ __global__ __launch_bounds__(512) void asm_rows_inv(const float2* __restrict__ w
     const float2* src = work + (size_t)(oy + (ok ? r : 0)) * L;
     fft::Twiddles<L> T;
     T.load(tw, t);
+    float2 v[16];
 #pragma unroll
-    for (int m = 0; m < 16; ++m) buf[fft::lane_pad<L>(t, m)] = ok ? src[t + m * TPL] : make_float2(0.f, 0.f);
-    __syncthreads();
-    fft::line<L, +1>(buf, T, t);
+    for (int m = 0; m < 16; ++m) v[m] = src[t + m * TPL];   // (a row past the end: row 0, dropped)
+    fft::line_regs<L, +1>(v, buf, T, t);
     if (ok) {
         float2* dst = out + (size_t)r * nx;
-        for (int c = t; c < nx; c += TPL) {
-            const float2 v = buf[fft::pad16(c + ox)];
-            dst[c] = make_float2(v.x * scale, v.y * scale);
+#pragma unroll
+        for (int m = HALF ? 4 : 0; m < (HALF ? 12 : 16); ++m) {
+            const int c = t + m * TPL - ox;
+            if (HALF || (c >= 0 && c < nx)) dst[c] = make_float2(v[m].x * scale, v[m].y * scale);
         }
     }
 }
@@ -680,8 +743,11 @@ int launch_rows_fwd(oph_ctx* ctx, const float2* in, int nx, int ny, int ox, int 
                    tj);
         return OPH_OK;
     }
-    OPH_LAUNCH(ctx, "asm_rows_fwd", asm_rows_fwd<LX>, dim3((ny + LPW - 1) / LPW), dim3(LPW * (LX / 16)), 0, in,
-               nx, ny, ox, oy, work, tw, tj);
+    const dim3 grid((ny + LPW - 1) / LPW), block(LPW * (LX / 16));
+    if (ox == LX / 4 && nx == LX / 2)
+        OPH_LAUNCH(ctx, "asm_rows_fwd", (asm_rows_fwd<LX, true>), grid, block, 0, in, nx, ny, ox, oy, work, tw, tj);
+    else
+        OPH_LAUNCH(ctx, "asm_rows_fwd", (asm_rows_fwd<LX, false>), grid, block, 0, in, nx, ny, ox, oy, work, tw, tj);
     return OPH_OK;
 }
 
@@ -708,8 +774,13 @@ int launch_rows_inv(oph_ctx* ctx, const float2* work, int nx, int ny, int ox, in
                    out, tw);
         return OPH_OK;
     }
-    OPH_LAUNCH(ctx, "asm_rows_inv", asm_rows_inv<LX>, dim3((ny + LPW - 1) / LPW), dim3(LPW * (LX / 16)), 0, work,
-               nx, ny, ox, oy, scale, out, tw);
+    const dim3 grid((ny + LPW - 1) / LPW), block(LPW * (LX / 16));
+    if (ox == LX / 4 && nx == LX / 2)
+        OPH_LAUNCH(ctx, "asm_rows_inv", (asm_rows_inv<LX, true>), grid, block, 0, work, nx, ny, ox, oy, scale, out,
+                   tw);
+    else
+        OPH_LAUNCH(ctx, "asm_rows_inv", (asm_rows_inv<LX, false>), grid, block, 0, work, nx, ny, ox, oy, scale, out,
+                   tw);
     return OPH_OK;
 }
 
@@ -749,7 +820,7 @@ int launch_cols_mid(oph_ctx* ctx, float2* work, int npx, const float4* tx, const
 }
 
 template <int LY, int B, bool EXACT>
-int launch_cols_b(oph_ctx* ctx, float2* work, int npx, int ny, int oy, const float4* tx, const float4* ty,
+int launch_cols_staged(oph_ctx* ctx, float2* work, int npx, int ny, int oy, const float4* tx, const float4* ty,
                   const AsmConst& k, const float2* tw) {
     const size_t shm = ((size_t)B * fft::padded_len(LY) + (asm_cols_fused<LY>() ? 256 : 0)) * sizeof(float2);
     static bool attr = false;
@@ -764,6 +835,49 @@ int launch_cols_b(oph_ctx* ctx, float2* work, int npx, int ny, int oy, const flo
     OPH_LAUNCH(ctx, "asm_cols", (asm_cols<LY, B, EXACT>), dim3((npx + B - 1) / B), dim3(B * (LY / 16)), shm,
                work, npx, ny, oy, tx, ty, ty2, k, tw);
     return OPH_OK;
+}
+
+template <int LY, int B, bool EXACT, bool REG_TW, bool HALF>
+int launch_cols_r(oph_ctx* ctx, float2* work, int npx, int ny, int oy, const float4* tx, const float4* ty,
+                  const AsmConst& k, const float2* tw) {
+    constexpr size_t shm = (size_t)B * fft::skewed_len(LY, B) * sizeof(float2);
+    static bool attr = false;
+    if (!attr) {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&asm_cols_r<LY, B, EXACT, REG_TW, HALF>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+        hipGetLastError();
+        attr = true;
+    }
+    const float2* ty2 = reinterpret_cast<const float2*>(ty + LY);
+    OPH_LAUNCH(ctx, "asm_cols", (asm_cols_r<LY, B, EXACT, REG_TW, HALF>), dim3(npx / B), dim3(B * (LY / 16)), shm,
+               work, npx, ny, oy, tx, ty, ty2, k, tw);
+    return OPH_OK;
+}
+
+// Grids up to 2048 columns: the register form (1024^2 unpadded 38.1 -> 31.0
+// us for the three passes, 2048^2 66.2 -> 58.4, 2048 x 8192 316 -> 288).  Wider
+// ones keep the staged kernel, whose 16-byte lane accesses move the longer
+// rows' pieces faster (4096 x 1024: 55 us against 57-61; 4096^2 unpadded 213
+// against 223-252).  Twiddles in registers while every workgroup is resident
+// at once anyway (1024^2: 31.0 us, from the table 31.8), else from the table,
+// which fits two workgroups to a CU (2048^2: 58.4, in registers 62.9).
+template <int LY, int B, bool EXACT>
+int launch_cols_b(oph_ctx* ctx, float2* work, int npx, int ny, int oy, const float4* tx, const float4* ty,
+                  const AsmConst& k, const float2* tw) {
+    // (the register form is built for the default number of columns only)
+    if constexpr (B != std::min(fftk::col_lines(LY), LY >= 4096 ? 2 : LY >= 2048 ? 4 : 8)) {
+        return launch_cols_staged<LY, B, EXACT>(ctx, work, npx, ny, oy, tx, ty, k, tw);
+    } else {
+        if (npx > 2048) return launch_cols_staged<LY, B, EXACT>(ctx, work, npx, ny, oy, tx, ty, k, tw);
+        const bool half = oy == LY / 4 && ny == LY / 2;
+        if constexpr (B * (LY / 16) <= 512 && !EXACT) {
+            if (npx / B <= ctx->cu_count)
+                return half ? launch_cols_r<LY, B, EXACT, true, true>(ctx, work, npx, ny, oy, tx, ty, k, tw)
+                            : launch_cols_r<LY, B, EXACT, true, false>(ctx, work, npx, ny, oy, tx, ty, k, tw);
+        }
+        return half ? launch_cols_r<LY, B, EXACT, false, true>(ctx, work, npx, ny, oy, tx, ty, k, tw)
+                    : launch_cols_r<LY, B, EXACT, false, false>(ctx, work, npx, ny, oy, tx, ty, k, tw);
+    }
 }
 
 template <int LY, bool EXACT>

@@ -110,9 +110,7 @@ __global__ __launch_bounds__(ssb_lines<L>(COLS) * (L / 16)) void ssb_filter(cons
                                                                            const float2* __restrict__ tw,
                                                                            float2* part) {
     constexpr int TPL = L / 16, B = ssb_lines<L>(COLS), NT = B * TPL;
-    // (columns: 4 more elements a line, so that the lanes of a wave, which hold
-    // neighbouring columns, fall on different banks)
-    constexpr int PL = fft::padded_len(L) + (COLS ? 4 : 0);
+    constexpr int PL = COLS ? fft::skewed_len(L, B) : fft::padded_len(L);
     extern __shared__ float2 ssb_lds[];
     const int b = COLS ? threadIdx.x % B : threadIdx.x / TPL;
     const int t = COLS ? threadIdx.x / B : threadIdx.x % TPL;
@@ -257,7 +255,7 @@ int launch_ssb(oph_ctx* ctx, const float2* u, float* out, int lines, int upper, 
     const float2* tw = oph_twiddles(ctx, L);
     if (!tw) return OPH_ENOMEM;
     constexpr int B = ssb_lines<L>(COLS), NT = B * (L / 16);
-    constexpr size_t shm = (size_t)B * (fft::padded_len(L) + (COLS ? 4 : 0)) * sizeof(float2);
+    constexpr size_t shm = (size_t)B * (COLS ? fft::skewed_len(L, B) : fft::padded_len(L)) * sizeof(float2);
     static bool attr = false;
     if (!attr) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(&ssb_filter<L, COLS>),

@@ -136,16 +136,13 @@ __global__ __launch_bounds__(512) void fft_rows_kernel(float2* data, int rows, i
     float2* src = data + (size_t)(ok ? row : 0) * stride;
     fft::Twiddles<L> T;
     T.load(tw, t);
+    float2 v[16];
 #pragma unroll
-    for (int m = 0; m < 16; ++m) buf[fft::lane_pad<L>(t, m)] = ok ? src[t + m * TPL] : make_float2(0.f, 0.f);
-    __syncthreads();
-    fft::line<L, SIGN>(buf, T, t);
+    for (int m = 0; m < 16; ++m) v[m] = src[t + m * TPL];   // (a row past the end: row 0, dropped)
+    fft::line_regs<L, SIGN>(v, buf, T, t);
     if (ok) {
 #pragma unroll
-        for (int m = 0; m < 16; ++m) {
-            const float2 v = buf[fft::lane_pad<L>(t, m)];
-            src[t + m * TPL] = make_float2(v.x * scale, v.y * scale);
-        }
+        for (int m = 0; m < 16; ++m) src[t + m * TPL] = make_float2(v[m].x * scale, v[m].y * scale);
     }
 }
 
@@ -206,73 +203,36 @@ __global__ __launch_bounds__(L / 16) void fft_rows_f(float2* data, int rows, int
     }
 }
 
-// wide: every column of the workgroup exists, the stride is even and the
-// L x stride array is below 2 GiB; then each lane moves two neighbouring
-// columns of a row (16 bytes) with range-checked buffer accesses, and its 8
-// loads are all issued before the first is used (a load loop with a bounds
-// branch completes each load before issuing the next).
+// Thread T transforms column T mod B as butterfly t = T / B, its elements in
+// registers at both ends (rows t + m L/16): a wave's 8-byte accesses cover
+// 64/B rows of B columns.  Up to 512 threads hold the twiddles in registers;
+// more (128 registers each) read them from the table at each stage.
 template <int L, int SIGN, int B>
-__global__ __launch_bounds__(1024) void fft_cols_kernel(float2* data, int ncols, int stride, float scale,
-                                                        const float2* __restrict__ tw, int wide) {
+__global__ __launch_bounds__(B * (L / 16)) void fft_cols_kernel(float2* data, int ncols, int stride, float scale,
+                                                               const float2* __restrict__ tw) {
     constexpr int TPL = L / 16;
-    constexpr int PL = fft::padded_len(L);
+    constexpr int PL = fft::skewed_len(L, B);
+    constexpr bool REG_TW = B * TPL <= 512;
     extern __shared__ float2 lds[];
-    const int nthr = TPL * B;
-    const int g = xcd_remap(blockIdx.x, gridDim.x);
-    const int c0 = g * B;
-    constexpr int PER = (L * B / 2) / (TPL * B);  // 16-byte pieces per lane
-    const bool w2 = B % 2 == 0 && wide && c0 + B <= ncols;
-    const auto rs = oph_buf_rsrc(data, (unsigned)((size_t)L * stride * sizeof(float2)));
-    if constexpr (B % 2 == 0 && L <= 4096) {
-        if (w2) {
-            float4 ld[PER];
+    const int b = threadIdx.x % B, t = threadIdx.x / B;
+    const int c = xcd_remap(blockIdx.x, gridDim.x) * B + b;
+    const bool ok = c < ncols;
+    float2* col = data + (ok ? c : 0);
+    float2 v[16];
 #pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                const int idx = threadIdx.x + j * nthr;
-                const int pr = idx % (B / 2), i = idx / (B / 2);
-                ld[j] = oph_buf_load_f4(rs, (unsigned)(((size_t)i * stride + c0 + 2 * pr) * sizeof(float2)));
-            }
-#pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                const int idx = threadIdx.x + j * nthr;
-                const int pr = idx % (B / 2), i = idx / (B / 2);
-                lds[(2 * pr) * PL + fft::pad16(i)] = make_float2(ld[j].x, ld[j].y);
-                lds[(2 * pr + 1) * PL + fft::pad16(i)] = make_float2(ld[j].z, ld[j].w);
-            }
-        }
-    }
-    if (!w2 || !(B % 2 == 0 && L <= 4096)) {
-        for (int idx = threadIdx.x; idx < L * B; idx += nthr) {
-            const int b = idx % B, i = idx / B;
-            const int c = c0 + b;
-            lds[b * PL + fft::pad16(i)] = c < ncols ? data[(size_t)i * stride + c] : make_float2(0.f, 0.f);
-        }
-    }
+    for (int m = 0; m < 16; ++m) v[m] = col[(size_t)(t + m * TPL) * stride];
     // (twiddles after the column data: their loads do not hold up the data's)
-    fft::Twiddles<L> T;
-    T.load(tw, threadIdx.x % TPL);
-    __syncthreads();
-    const int b = threadIdx.x / TPL, t = threadIdx.x % TPL;
-    fft::line<L, SIGN>(lds + b * PL, T, t);
-    if (w2) {
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int idx = threadIdx.x + j * nthr;
-            const int pr = idx % (B / 2), i = idx / (B / 2);
-            const float2 u = lds[(2 * pr) * PL + fft::pad16(i)], v = lds[(2 * pr + 1) * PL + fft::pad16(i)];
-            oph_buf_store_f4(make_float4(u.x * scale, u.y * scale, v.x * scale, v.y * scale), rs,
-                             (unsigned)(((size_t)i * stride + c0 + 2 * pr) * sizeof(float2)));
-        }
+    if constexpr (REG_TW) {
+        fft::Twiddles<L> T;
+        T.load(tw, t);
+        fft::line_regs<L, SIGN>(v, lds + b * PL, T, t);
     } else {
-        for (int idx = threadIdx.x; idx < L * B; idx += nthr) {
-            const int bb = idx % B, i = idx / B;
-            const int c = c0 + bb;
-            if (c < ncols) {
-                const float2 v = lds[bb * PL + fft::pad16(i)];
-                data[(size_t)i * stride + c] = make_float2(v.x * scale, v.y * scale);
-            }
-        }
+        fft::line_regs_tw<L, SIGN>(v, lds + b * PL, tw, t);
     }
+    if (!ok) return;
+#pragma unroll
+    for (int m = 0; m < 16; ++m)
+        col[(size_t)(t + m * TPL) * stride] = make_float2(v[m].x * scale, v[m].y * scale);
 }
 
 // 4096-point columns, persistent: workgroups of four columns (1024 threads,
@@ -381,7 +341,7 @@ int launch_rows(oph_ctx* ctx, float2* data, int rows, int stride, float scale) {
 
 template <int L, int SIGN, int B>
 int launch_cols_b(oph_ctx* ctx, float2* data, int ncols, int stride, float scale, const float2* tw) {
-    const size_t shm = (size_t)B * fft::padded_len(L) * sizeof(float2);
+    const size_t shm = (size_t)B * fft::skewed_len(L, B) * sizeof(float2);
     static bool attr = false;
     if (!attr) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(&fft_cols_kernel<L, SIGN, B>),
@@ -390,9 +350,8 @@ int launch_cols_b(oph_ctx* ctx, float2* data, int ncols, int stride, float scale
         attr = true;
     }
     const int grid = (ncols + B - 1) / B;
-    const int wide = stride % 2 == 0 && (size_t)L * stride * sizeof(float2) < (1u << 31);
     OPH_LAUNCH(ctx, "fft_cols", (fft_cols_kernel<L, SIGN, B>), dim3(grid), dim3(B * (L / 16)), shm, data,
-               ncols, stride, scale, tw, wide);
+               ncols, stride, scale, tw);
     return OPH_OK;
 }
 

@@ -304,6 +304,11 @@ __device__ __forceinline__ void line_tw(float2* buf, const float2* __restrict__ 
 template <int L>
 __host__ __device__ constexpr bool regs_fusable() { return n16(L) >= 2 && last_radix(L) == 1; }
 
+// Columns in LDS when the lanes of a wave hold B neighbouring columns (lane T:
+// column T mod B, butterfly T / B): one column's line plus 32/B elements, so
+// that B columns times 32/B consecutive elements fall on distinct banks.
+__host__ __device__ constexpr int skewed_len(int L, int B) { return padded_len(L) + (B > 1 ? 32 / B : 0); }
+
 // Full transform with the thread's elements in registers at both ends: on
 // entry v[m] is input element t + m L/16, on return output element t + m L/16.
 // True of every length here: the last stage, of radix RL and Ns = L/RL, takes

@@ -350,3 +350,19 @@ def test_wrp_mode3_matlab_vs_oracle(ctx, res, pitch, lam):
     # the phase is read by mode 3 only
     assert np.array_equal(ctx.wrp(128, 128, pitch, lam, zw, x * 0.1, y * 0.1, z, a, mode=1, phase=ph),
                           ctx.wrp(128, 128, pitch, lam, zw, x * 0.1, y * 0.1, z, a, mode=1))
+
+
+@pytest.mark.parametrize("nx,ny,pad", [(16, 16, 1), (16, 32, 2), (1024, 64, 1), (64, 512, 2), (512, 1024, 2),
+                                       (2048, 16, 1), (16, 4096, 1), (32, 4096, 2), (16, 8192, 1)])
+@pytest.mark.parametrize("pitch,band", [(8e-6, False), (8e-6, True), (0.4e-6, False)])
+def test_asm_register_columns(ctx, nx, ny, pad, pitch, band):
+    """Column pass with the elements in registers (grids up to 2048 columns): every
+    column length, data in the middle half and not, the series and the FP64
+    transfer, with and without the band limit.  Bound: four FP32 transforms of
+    at most four stages, about 1e-7 a stage, and the transfer's phase (1e-7
+    turns): 2e-6."""
+    print(f"case: asm {nx}x{ny} pad {pad} pitch {pitch} band {band}", flush=True)
+    rng = np.random.default_rng(nx + ny)
+    f = (rng.normal(size=(ny, nx)) + 1j * rng.normal(size=(ny, nx))).astype(np.complex64)
+    out = ctx.asm(f, pitch, 532e-9, 0.01, pad=pad, band_limit=band)
+    assert rel_l2(out, O.asm(f, pitch, pitch, 532e-9, 0.01, pad=pad, band_limit=band)) < 2e-6

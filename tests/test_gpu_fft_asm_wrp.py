@@ -366,3 +366,18 @@ def test_asm_register_columns(ctx, nx, ny, pad, pitch, band):
     f = (rng.normal(size=(ny, nx)) + 1j * rng.normal(size=(ny, nx))).astype(np.complex64)
     out = ctx.asm(f, pitch, 532e-9, 0.01, pad=pad, band_limit=band)
     assert rel_l2(out, O.asm(f, pitch, pitch, 532e-9, 0.01, pad=pad, band_limit=band)) < 2e-6
+
+
+@pytest.mark.parametrize("nx,ny,n", [(64, 64, 1), (256, 256, 256), (256, 192, 257), (300, 130, 1023), (512, 512, 1024),
+                                     (200, 256, 1025), (1024, 1024, 700), (2048, 2048, 1000)])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+def test_wrp_small_calls(ctx, nx, ny, n, mode):
+    """One-kernel binning (up to 1024 points and tiles; 1025 takes the three
+    passes) and tiles split into strips of rows, whole and partial tiles."""
+    print(f"case: wrp {nx}x{ny} P={n} mode {mode}", flush=True)
+    x, y, z, a, zw = scenes.wrp_points(n, seed=n)
+    x, y = x * nx / 2048, y * ny / 2048
+    ph = np.linspace(0, 6, n)
+    U = ctx.wrp(nx, ny, 8e-6, 532e-9, zw, x, y, z, a, mode=mode, phase=ph)
+    assert np.array_equal(U, ctx.wrp(nx, ny, 8e-6, 532e-9, zw, x, y, z, a, mode=mode, phase=ph))
+    assert rel_l2(U, O.wrp(nx, ny, 8e-6, 532e-9, zw, x, y, z, a, mode=mode, phase=ph)) < 1e-5

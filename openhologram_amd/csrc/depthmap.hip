@@ -32,7 +32,10 @@
 //   dm_cols   a workgroup owns 4 scene columns and a range of layers; two
 //             real columns are packed into one complex column, transformed
 //             along y (length Ny) and separated; only rows ky <= Ny/2 are
-//             stored (Hermitian symmetry of real input), with a presence flag
+//             stored (Hermitian symmetry of real input), and of these, for an
+//             encoded output, only those whose row pair the crop keeps (half:
+//             K below; 3 x 1920 x 1080 on 4096 x 2048, 256 layers: row pass
+//             3196 -> 1720 us a colour), with a presence flag
 //             per (layer, column group) -- absent groups are never written;
 //   dm_rows   a workgroup owns the row pair (ky, Ny-ky): per layer it
 //             transforms row ky along x once and obtains row Ny-ky from the
@@ -42,9 +45,10 @@
 //             Rows 0 and Ny/2 are real (transforms of real columns at the DC
 //             and Nyquist frequencies): workgroup 0 packs them into one
 //             complex row and separates the transform, so the pass is Ny/2
-//             workgroups (a multiple of the CU count) instead of Ny/2 + 1;
+//             pairs (a multiple of the CU count) instead of Ny/2 + 1;
 //   dm_final  inverse column transform, 1/(Nx Ny), the shift phase and the
 //             real part (or the complex field) in the scene window.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -63,8 +67,9 @@ struct DmArgs {
     int ngroups;
     const unsigned char* img;      // h x w, this colour
     const unsigned short* idx;     // h x w
-    float2* I;                     // [L][ngroups][Ny/2 + 1][GROUP]: each column group's
-                                   // rows contiguous (I_l(ky, x) at group x / GROUP)
+    float2* I;                     // [L][ngroups][K][GROUP]: each column group's rows
+                                   // contiguous (I_l(ky, x) at group x / GROUP)
+    int K;                         // stored rows: ky = 0 .. K - 2, then Ny/2
     unsigned char* flags;          // [L][ngroups]
     unsigned char* any;            // [L]
     unsigned* fbits;               // [L][fwpl]: the flags as bits (group g: word g/32, bit g%32)
@@ -81,6 +86,8 @@ struct DmArgs {
     float2* T;                     // [Ny][w] after the inverse row transform
     float2* spectrum;              // optional centred spectrum [Ny][Nx]
     double scale;                  // 1/(Nx Ny)
+    int n_main, nsplit;            // dm_rows_h: row pairs taken whole; workgroups per further pair
+    float2* part;                  // ... and their partial sums [pair][nsplit][2][Nx]
     double* fringe;                // h x w (double) or
     float* fringe32;               // h x w (float) or
     float2* field;                 // h x w complex
@@ -146,7 +153,7 @@ __global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int layers_pe
         pix[e] = v;
     }
     __syncthreads();
-    const size_t gstride = (size_t)(a.Ny / 2 + 1) * GROUP;
+    const size_t gstride = (size_t)a.K * GROUP;
     const size_t lstride = gstride * a.ngroups;
     for (int l = l_begin; l <= l_end; ++l) {
         if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
@@ -167,8 +174,8 @@ __global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int layers_pe
         fft::line<LY, -1>(line, Tw, t);
         // separate: A(k) = (Z(k) + conj Z(-k))/2, B(k) = (Z(k) - conj Z(-k))/(2i)
         float2* dst = a.I + (size_t)(l - 1) * lstride + (size_t)g * gstride;
-        for (int e = threadIdx.x; e < (LY / 2 + 1) * GROUP; e += NT) {
-            const int c = e % GROUP, ky = e / GROUP;
+        for (int e = threadIdx.x; e < a.K * GROUP; e += NT) {
+            const int c = e % GROUP, ky = e / GROUP < a.K - 1 ? e / GROUP : LY / 2;
             const int x = x0 + c;
             if (x >= a.w) continue;
             const float2* ln = lines + (c >> 1) * PL;
@@ -253,13 +260,13 @@ __global__ __launch_bounds__(LX / 16) void dm_rows(DmArgs a, const float2* __res
     constexpr int PL = fft::padded_len(LX);
     __shared__ float2 line[PL];
     const int t = threadIdx.x;
-    const int kya = xcd_remap(blockIdx.x, gridDim.x);  // 0 .. Ny/2 - 1
+    const int kya = xcd_remap(blockIdx.x, gridDim.x);  // 0 .. K - 2
     const bool pair0 = kya == 0;              // real rows 0 and Ny/2 packed as re/im
     const int kyb = pair0 ? a.Ny / 2 : a.Ny - kya;
     const int sya = sgnidx(kya, a.Ny) + 1;
     const int syb = sgnidx(kyb, a.Ny) + 1;
-    const size_t nyq = (size_t)(a.Ny / 2) * GROUP;  // row Ny/2 relative to row 0
-    const size_t gstride = (size_t)(a.Ny / 2 + 1) * GROUP;
+    const size_t nyq = (size_t)(a.K - 1) * GROUP;  // row Ny/2 relative to row 0
+    const size_t gstride = (size_t)a.K * GROUP;
     fft::Twiddles<LX> Tw;
     Tw.load(twx, t);
     float2 acca[16], accb[16];
@@ -391,8 +398,11 @@ __device__ __forceinline__ void lds_copy(E* dst, const E* __restrict__ src, int 
     }
 }
 
+// lo .. hi: the layers taken (lo on a chunk boundary).  part: the sums of both
+// rows are written there instead of being finished.
 template <int LX, bool PAIR0, bool FBITS>
-__device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __restrict__ tw8, float2* sm, int kya) {
+__device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __restrict__ tw8, float2* sm, int kya,
+                                            int lo, int hi, float2* part) {
     constexpr int TPL = LX / 8;
     constexpr int PL = fft::padded_len(LX);
     constexpr int CH = 16;
@@ -417,8 +427,8 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
     const int kyb = PAIR0 ? a.Ny / 2 : a.Ny - kya;
     const int sya = sgnidx(kya, a.Ny) + 1;
     const int syb = sgnidx(kyb, a.Ny) + 1;
-    const size_t nyq = (size_t)(a.Ny / 2) * GROUP;
-    const size_t gstride = (size_t)(a.Ny / 2 + 1) * GROUP;
+    const size_t nyq = (size_t)(a.K - 1) * GROUP;
+    const size_t gstride = (size_t)a.K * GROUP;
     // Thread t owns row a at kx = t + m TPL and row b at kb = -kx mod LX:
     // row b's transform at kb is conj Z(kx) of the thread's own element of
     // row a's transform Z, and the transfer depends on kx only through kx^2,
@@ -450,8 +460,8 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
     // its latency hides behind the transform.
     auto next_layer = [&](int l) -> int {
         for (;;) {
-            const int c = a.lo + (l - a.lo) / CH * CH;
-            l = l > c ? l - 1 : (c + CH <= a.hi ? min(a.hi, c + 2 * CH - 1) : 0);
+            const int c = lo + (l - lo) / CH * CH;
+            l = l > c ? l - 1 : (c + CH <= hi ? min(hi, c + 2 * CH - 1) : 0);
             if (l == 0 || present(l)) return l;
         }
     };
@@ -497,11 +507,11 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
                 nv[m] = in ? src[o] : make_float2(0.f, 0.f);
         }
     };
-    int pl = min(a.hi, a.lo + CH - 1);
+    int pl = min(hi, lo + CH - 1);
     if (!present(pl)) pl = next_layer(pl);
     if (pl) fetch(pl);
-    for (int cs = a.lo; cs <= a.hi; cs += CH) {
-        const int ce = min(a.hi, cs + CH - 1);
+    for (int cs = lo; cs <= hi; cs += CH) {
+        const int ce = min(hi, cs + CH - 1);
         bool anyc = false;
         for (int l = cs; l <= ce; ++l) anyc |= present(l);
         if (!anyc) continue;
@@ -570,6 +580,14 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
         }
     }
     __syncthreads();  // Sb entries were written by the threads owning -kx
+    if (part) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            part[t + m * TPL] = Sa[t + m * TPL];
+            part[LX + t + m * TPL] = Sb[t + m * TPL];
+        }
+        return;
+    }
     float2 acca[8], accb[8];
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
@@ -586,13 +604,46 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
 template <int LX, bool FBITS>
 __global__ __launch_bounds__(LX / 8, 2) void dm_rows_h(DmArgs a, const float2* __restrict__ tw8) {
     extern __shared__ float2 sm[];
+    if ((int)blockIdx.x >= a.n_main) {
+        // a pair beyond the last full round of workgroups: part of its layers
+        const int k = blockIdx.x - a.n_main, i = k / a.nsplit, j = k % a.nsplit;
+        const int per = ((a.hi - a.lo + 16) / 16 + a.nsplit - 1) / a.nsplit * 16;
+        const int lo = a.lo + j * per, hi = min(a.hi, lo + per - 1);
+        float2* part = a.part + (size_t)k * 2 * LX;
+        if (a.n_main + i == 0) rows_h_body<LX, true, FBITS>(a, tw8, sm, 0, lo, hi, part);
+        else rows_h_body<LX, false, FBITS>(a, tw8, sm, a.n_main + i, lo, hi, part);
+        return;
+    }
     // XCD-aware: neighbouring rows, which share the cache lines of I, run on
     // the same XCD at the same time
-    const int kya = xcd_remap(blockIdx.x, gridDim.x);  // 0 .. Ny/2 - 1
+    const int kya = xcd_remap(blockIdx.x, a.n_main);  // 0 .. n_main - 1
     if (kya == 0)
-        rows_h_body<LX, true, FBITS>(a, tw8, sm, 0);
+        rows_h_body<LX, true, FBITS>(a, tw8, sm, 0, a.lo, a.hi, nullptr);
     else
-        rows_h_body<LX, false, FBITS>(a, tw8, sm, kya);
+        rows_h_body<LX, false, FBITS>(a, tw8, sm, kya, a.lo, a.hi, nullptr);
+}
+
+// The pairs whose layers were split: their partial sums in order (the same
+// additions as a whole pair's), then as a whole pair's
+template <int LX>
+__global__ __launch_bounds__(LX / 8) void dm_rows_h_sum(DmArgs a, const float2* __restrict__ tw8) {
+    constexpr int TPL = LX / 8;
+    __shared__ float2 line[fft::padded_len(LX)];
+    const int t = threadIdx.x, kya = a.n_main + blockIdx.x, kyb = kya == 0 ? a.Ny / 2 : a.Ny - kya;
+    const float2* p = a.part + (size_t)blockIdx.x * a.nsplit * 2 * LX;
+#pragma unroll
+    for (int row = 0; row < 2; ++row) {
+        float2 acc[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) acc[m] = make_float2(0.f, 0.f);
+        for (int j = 0; j < a.nsplit; ++j)
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+                acc[m] = fft::cadd(acc[m], p[((size_t)2 * j + row) * LX + t + m * TPL]);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) acc[m] = fft::cmul(acc[m], a.rho);
+        finish_row8<LX>(a, acc, row ? kyb : kya, line, tw8, t);
+    }
 }
 
 // ---- final column pass ---------------------------------------------------------
@@ -709,7 +760,7 @@ __global__ __launch_bounds__(2 * fftm::threads(LY)) void dm_cols_m(DmArgs a, int
         pix[e] = v;
     }
     __syncthreads();
-    const size_t gstride = (size_t)(a.Ny / 2 + 1) * GROUP;
+    const size_t gstride = (size_t)a.K * GROUP;
     const size_t lstride = gstride * a.ngroups;
     for (int l = l_begin; l <= l_end; ++l) {
         if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
@@ -730,8 +781,8 @@ __global__ __launch_bounds__(2 * fftm::threads(LY)) void dm_cols_m(DmArgs a, int
         __syncthreads();
         fftm::line<LY, NT, -1>(line, twy, t);
         float2* dst = a.I + (size_t)(l - 1) * lstride + (size_t)g * gstride;
-        for (int e = threadIdx.x; e < (LY / 2 + 1) * GROUP; e += 2 * NT) {
-            const int c = e % GROUP, ky = e / GROUP;
+        for (int e = threadIdx.x; e < a.K * GROUP; e += 2 * NT) {
+            const int c = e % GROUP, ky = e / GROUP < a.K - 1 ? e / GROUP : LY / 2;
             const int x = x0 + c;
             if (x >= a.w) continue;
             const float2* ln = lines + (c >> 1) * PL;
@@ -788,13 +839,13 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
     constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
     const int t = threadIdx.x;
-    const int kya = xcd_remap(blockIdx.x, gridDim.x);  // 0 .. Ny/2 - 1
+    const int kya = xcd_remap(blockIdx.x, gridDim.x);  // 0 .. K - 2
     const bool pair0 = kya == 0;              // real rows 0 and Ny/2 packed as re/im
     const int kyb = pair0 ? a.Ny / 2 : a.Ny - kya;
     const int sya = sgnidx(kya, a.Ny) + 1;
     const int syb = sgnidx(kyb, a.Ny) + 1;
-    const size_t nyq = (size_t)(a.Ny / 2) * GROUP;
-    const size_t gstride = (size_t)(a.Ny / 2 + 1) * GROUP;
+    const size_t nyq = (size_t)(a.K - 1) * GROUP;
+    const size_t gstride = (size_t)a.K * GROUP;
     // (the per-element x factors are recomputed per layer: the two rows'
     // accumulators already take most of the registers of a 768-thread line)
     float2 acca[EPT], accb[EPT];
@@ -989,17 +1040,37 @@ int launch_dm_rows(oph_ctx* ctx, const DmArgs& a) {
             const size_t fbytes = (size_t)a.L * a.fwpl * sizeof(unsigned);
             b.fbits_lds = rows_h_lds<LX>() + fbytes <= 160 * 1024 ? 1 : 0;
             const size_t shm = rows_h_lds<LX>() + (b.fbits_lds ? fbytes : 0);
+            // A workgroup's LDS leaves one or two per CU, so a few pairs beyond
+            // the last full round would cost a whole round: their layers are
+            // split over several workgroups instead (2048 rows of which 514
+            // pairs are needed: 2 rounds and a sixteenth, not 3), as are all
+            // pairs of a grid that does not fill one round.
+            const int n = a.K - 1, slots = std::max(ctx->cu_count, 1) * (2 * shm <= 160 * 1024 ? 2 : 1);
+            const int nch = (a.hi - a.lo + 16) / 16;   // chunks of 16 layers
+            b.n_main = n / slots * slots;
+            b.nsplit = std::min(nch, 16);
+            if (b.nsplit < 2 || 2 * (n - b.n_main) > slots) b.n_main = n;
+            const int left = n - b.n_main;
+            if (left > 0) {
+                b.nsplit = (nch + (nch + b.nsplit - 1) / b.nsplit - 1) / ((nch + b.nsplit - 1) / b.nsplit);
+                b.part = static_cast<float2*>(
+                    oph_scratch(ctx, SLOT_WORK0, (size_t)left * b.nsplit * 2 * LX * sizeof(float2)));
+                if (!b.part) return OPH_ENOMEM;
+            }
+            const dim3 grid(b.n_main + left * b.nsplit);
             if (b.fbits_lds)
-                OPH_LAUNCH(ctx, "dm_rows", (dm_rows_h<LX, true>), dim3(a.Ny / 2), dim3(LX / 8), shm, b, tw8);
+                OPH_LAUNCH(ctx, "dm_rows", (dm_rows_h<LX, true>), grid, dim3(LX / 8), shm, b, tw8);
             else
-                OPH_LAUNCH(ctx, "dm_rows", (dm_rows_h<LX, false>), dim3(a.Ny / 2), dim3(LX / 8), shm, b, tw8);
+                OPH_LAUNCH(ctx, "dm_rows", (dm_rows_h<LX, false>), grid, dim3(LX / 8), shm, b, tw8);
+            if (left > 0)
+                OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_h_sum<LX>, dim3(left), dim3(LX / 8), 0, b, tw8);
             return OPH_OK;
         }
     }
     if (a.exact)
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, true>), dim3(a.Ny / 2), dim3(LX / 16), 0, a, tw);
+        OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, true>), dim3(a.K - 1), dim3(LX / 16), 0, a, tw);
     else
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, false>), dim3(a.Ny / 2), dim3(LX / 16), 0, a, tw);
+        OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, false>), dim3(a.K - 1), dim3(LX / 16), 0, a, tw);
     return OPH_OK;
 }
 
@@ -1060,9 +1131,9 @@ int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
         attr = true;
     }
     if (a.exact)
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, true>), dim3(a.Ny / 2), dim3(fftm::threads(LX)), shm, a, tw);
+        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, true>), dim3(a.K - 1), dim3(fftm::threads(LX)), shm, a, tw);
     else
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, false>), dim3(a.Ny / 2), dim3(fftm::threads(LX)), shm, a, tw);
+        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, false>), dim3(a.K - 1), dim3(fftm::threads(LX)), shm, a, tw);
     return OPH_OK;
 }
 
@@ -1184,7 +1255,11 @@ extern "C" int oph_depthmap(oph_ctx* ctx, const oph_dm_spec* s, int ncolor, cons
 
     const size_t npx = (size_t)w * h;
     const int ngroups = (w + GROUP - 1) / GROUP;
-    const size_t lstride = (size_t)(Ny / 2 + 1) * GROUP * ngroups;
+    // Encoding keeps the centred rows [Ny/4 - 1, 3 Ny/4 - 2], ky from -(Ny/4 + 1)
+    // to Ny/4 - 2: only the row pairs (ky, -ky) up to ky = Ny/4 + 1 are formed
+    // (and row Ny/2, which shares row 0's transform); a field needs all
+    const int K = fmt != OPH_DM_OUT_FIELD ? std::min(Ny / 2 + 1, Ny / 4 + 3) : Ny / 2 + 1;
+    const size_t lstride = (size_t)K * GROUP * ngroups;
     // device buffers
     unsigned char* dimg = const_cast<unsigned char*>(intensity);
     unsigned char* ddep = const_cast<unsigned char*>(depth);
@@ -1256,6 +1331,7 @@ extern "C" int oph_depthmap(oph_ctx* ctx, const oph_dm_spec* s, int ncolor, cons
         a.img = dimg + npx * c;
         a.idx = didx;
         a.I = I;
+        a.K = K;
         a.flags = dflags;
         a.any = dany;
         a.fbits = dfbits;

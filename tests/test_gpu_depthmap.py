@@ -160,3 +160,21 @@ def test_depthmap_unsupported_grid_reports(ctx):
         ctx.depthmap(100, 60, 100, 60, 8e-6, 0.09, 0.11, 8, [532e-9], img, dep)
     with pytest.raises(OphError):
         ctx.depthmap(100, 60, 720, 64, 8e-6, 0.09, 0.11, 8, [532e-9], img, dep)
+
+
+@pytest.mark.parametrize("w,h,Nx,Ny,L,layers,out", [
+    (64, 48, 128, 64, 17, None, "field"),        # every pair split, the second part one layer
+    (64, 48, 128, 64, 100, (5, 77), "fringe"),   # a layer range that starts off a multiple of 16
+    (48, 1000, 64, 2048, 40, None, "fringe"),    # pairs taken whole and a remainder that is split
+    (20, 12, 32, 16, 300, None, "fringe"),       # 19 chunks of layers over 10 parts
+    (30, 12, 64, 16, 16, None, "fringe"),        # one chunk: nothing to split
+])
+def test_depthmap_row_pairs_kept_and_split(ctx, w, h, Nx, Ny, L, layers, out):
+    """Only the row pairs that the encode crop keeps are formed, and pairs
+    beyond full rounds of workgroups are split over their layers."""
+    print(f"case: depthmap {w}x{h} grid {Nx}x{Ny} L={L} layers={layers} {out}", flush=True)
+    img, dep = scenes.depth_scene(w, h, seed=11, colors=1)
+    kw = dict(quant_mode=1) if layers is None else dict(quant_mode=1, layers=layers)
+    u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.09, 0.11, L, [532e-9], img, dep, out=out, **kw)
+    ref = _oracle_rgb(img, dep, Nx, Ny, 8e-6, [532e-9], 0.09, 0.11, L, out=out, **kw)
+    assert rel_l2(u, ref) < TOL

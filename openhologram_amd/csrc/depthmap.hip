@@ -86,7 +86,7 @@ struct DmArgs {
     float2* T;                     // [Ny][w] after the inverse row transform
     float2* spectrum;              // optional centred spectrum [Ny][Nx]
     double scale;                  // 1/(Nx Ny)
-    int n_main, nsplit;            // dm_rows_h: row pairs taken whole; workgroups per further pair
+    int n_main, nsplit;            // row pairs taken whole; workgroups per further pair
     float2* part;                  // ... and their partial sums [pair][nsplit][2][Nx]
     double* fringe;                // h x w (double) or
     float* fringe32;               // h x w (float) or
@@ -834,12 +834,21 @@ __device__ __forceinline__ void finish_row_m(const DmArgs& a, const float2 (&acc
     __syncthreads();
 }
 
+// Bound by vector instructions once enough waves are resident: one workgroup
+// a pair leaves 272 two-wave workgroups for 256 CUs at 1920 x 1080 encoded
+// (2483 us, 256 layers), the layers split into 3 parts 795 us; holding it to
+// 168 or 128 registers for more waves spills (1010 and 1456 us).
 template <int LX, bool EXACT>
 __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const float2* __restrict__ twx) {
     constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
     const int t = threadIdx.x;
-    const int kya = xcd_remap(blockIdx.x, gridDim.x);  // 0 .. K - 2
+    // part j of the pair's layers (XCD-aware: neighbouring pairs, which share
+    // the cache lines of I, run their same part on one XCD at the same time)
+    const int lin = xcd_remap(blockIdx.x, gridDim.x), npair = a.K - 1;
+    const int j = lin / npair, kya = lin - j * npair;  // kya = 0 .. K - 2
+    const int per = (a.hi - a.lo + a.nsplit) / a.nsplit;
+    const int lo = a.lo + j * per, hi = min(a.hi, lo + per - 1);
     const bool pair0 = kya == 0;              // real rows 0 and Ny/2 packed as re/im
     const int kyb = pair0 ? a.Ny / 2 : a.Ny - kya;
     const int sya = sgnidx(kya, a.Ny) + 1;
@@ -855,7 +864,7 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
     // a layer's slice of I addressed by 32-bit buffer offsets when it is
     // below 2 GiB (else plain loads with a branch per element)
     const bool bufs = lstride * sizeof(float2) < ((size_t)1 << 31);
-    for (int l = a.lo; l <= a.hi; ++l) {
+    for (int l = lo; l <= hi; ++l) {
         if (!a.any[l - 1]) continue;
         // the thread index through a zero the compiler cannot see through:
         // the transforms' LDS addresses are then formed per layer instead of
@@ -952,6 +961,18 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
         }
         __syncthreads();
     }
+    if (a.nsplit > 1) {
+        float2* part = a.part + ((size_t)kya * a.nsplit + j) * 2 * LX;
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int kx = t + m * NT;
+            if (EPT * NT == LX || kx < LX) {
+                part[kx] = acca[m];
+                part[LX + kx] = accb[m];
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < EPT; ++m) {
         acca[m] = fft::cmul(acca[m], a.rho);
@@ -959,6 +980,28 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
     }
     finish_row_m<LX>(a, acca, kya, line, twx, t);
     finish_row_m<LX>(a, accb, kyb, line, twx, t);
+}
+
+// The partial sums of a pair's layers in order, then as a whole pair's
+template <int LX>
+__global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m_sum(DmArgs a, const float2* __restrict__ twx) {
+    constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
+    extern __shared__ float2 line[];  // fftm::padded_len(LX)
+    const int t = threadIdx.x, kya = blockIdx.x >> 1, row = blockIdx.x & 1;
+    const int ky = row == 0 ? kya : kya == 0 ? a.Ny / 2 : a.Ny - kya;
+    const float2* p = a.part + ((size_t)kya * a.nsplit * 2 + row) * LX;
+    float2 acc[EPT];
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) acc[m] = make_float2(0.f, 0.f);
+    for (int j = 0; j < a.nsplit; ++j)
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const int kx = t + m * NT;
+            if (EPT * NT == LX || kx < LX) acc[m] = fft::cadd(acc[m], p[(size_t)2 * j * LX + kx]);
+        }
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) acc[m] = fft::cmul(acc[m], a.rho);
+    finish_row_m<LX>(a, acc, ky, line, twx, t);
 }
 
 template <int LY, int B>
@@ -1117,23 +1160,53 @@ int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
     }
 }
 
+// Into how many parts a pair's layers are split, with `resident` workgroups
+// of the row pass on a CU: the fewest layer times of whole rounds, a part
+// costing three layer times of its own (its set-up, its sums written and
+// read again).
+int rows_parts(oph_ctx* ctx, int pairs, int layers, int resident) {
+    const long long slots = (long long)std::max(ctx->cu_count, 1) * resident;
+    int best = 1;
+    long long cost = (pairs + slots - 1) / slots * layers;
+    for (int n = 2; n <= 16 && 4 * n <= layers; ++n) {
+        const long long c = ((long long)pairs * n + slots - 1) / slots * ((layers + n - 1) / n + 3);
+        if (c < cost) { cost = c; best = n; }
+    }
+    const int per = (layers + best - 1) / best;
+    return (layers + per - 1) / per;
+}
+
 template <int LX>
 int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
     const float2* tw = oph_twiddles_mixed(ctx, LX);
     if (!tw) return OPH_ENOMEM;
     const size_t shm = (size_t)fftm::padded_len(LX) * sizeof(float2);
-    static bool attr = false;
-    if (!attr) {
+    static int resident[2] = {0, 0};
+    if (!resident[a.exact]) {
         for (const void* k : {reinterpret_cast<const void*>(&dm_rows_m<LX, true>),
-                              reinterpret_cast<const void*>(&dm_rows_m<LX, false>)})
+                              reinterpret_cast<const void*>(&dm_rows_m<LX, false>),
+                              reinterpret_cast<const void*>(&dm_rows_m_sum<LX>)})
             hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+        int n = 0;
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>,
+                                                     fftm::threads(LX), shm);
         hipGetLastError();
-        attr = true;
+        resident[a.exact] = std::max(n, 1);
     }
+    DmArgs b = a;
+    b.nsplit = rows_parts(ctx, a.K - 1, a.hi - a.lo + 1, resident[a.exact]);
+    if (b.nsplit > 1) {
+        b.part = static_cast<float2*>(
+            oph_scratch(ctx, SLOT_WORK0, (size_t)(a.K - 1) * b.nsplit * 2 * LX * sizeof(float2)));
+        if (!b.part) return OPH_ENOMEM;
+    }
+    const dim3 grid((a.K - 1) * b.nsplit);
     if (a.exact)
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, true>), dim3(a.K - 1), dim3(fftm::threads(LX)), shm, a, tw);
+        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, true>), grid, dim3(fftm::threads(LX)), shm, b, tw);
     else
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, false>), dim3(a.K - 1), dim3(fftm::threads(LX)), shm, a, tw);
+        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, false>), grid, dim3(fftm::threads(LX)), shm, b, tw);
+    if (b.nsplit > 1)
+        OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_m_sum<LX>, dim3(2 * (a.K - 1)), dim3(fftm::threads(LX)), shm, b, tw);
     return OPH_OK;
 }
 

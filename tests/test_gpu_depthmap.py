@@ -178,3 +178,20 @@ def test_depthmap_row_pairs_kept_and_split(ctx, w, h, Nx, Ny, L, layers, out):
     u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.09, 0.11, L, [532e-9], img, dep, out=out, **kw)
     ref = _oracle_rgb(img, dep, Nx, Ny, 8e-6, [532e-9], 0.09, 0.11, L, out=out, **kw)
     assert rel_l2(u, ref) < TOL
+
+
+@pytest.mark.parametrize("w,h,Nx,Ny,L,layers,out", [
+    (720, 500, 720, 540, 37, None, "field"),     # parts of unequal length, both rows kept
+    (500, 540, 540, 1080, 16, (2, 15), "fringe"),  # a short layer range, half of the pairs
+    (720, 540, 720, 540, 3, None, "fringe"),     # too few layers to split
+])
+def test_depthmap_lens_row_pairs_split(ctx, w, h, Nx, Ny, L, layers, out):
+    """With a field lens: a pair's layers split over workgroups and summed."""
+    print(f"case: depthmap lens {w}x{h} grid {Nx}x{Ny} L={L} layers={layers} {out}", flush=True)
+    img, dep = scenes.depth_scene(w, h, seed=12, colors=1)
+    kw = dict(quant_mode=1, field_lens=1.0)
+    if layers is not None:
+        kw["layers"] = layers
+    u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.2, 0.7, L, [532e-9], img, dep, out=out, **kw)
+    ref = _oracle_rgb(img, dep, Nx, Ny, 8e-6, [532e-9], 0.2, 0.7, L, out=out, **kw)
+    assert rel_l2(u, ref) < TOL

@@ -86,7 +86,7 @@ struct DmArgs {
     float2* T;                     // [Ny][w] after the inverse row transform
     float2* spectrum;              // optional centred spectrum [Ny][Nx]
     double scale;                  // 1/(Nx Ny)
-    int n_main, nsplit;            // row pairs taken whole; workgroups per further pair
+    int n_main, nsplit, per;       // row pairs taken whole; workgroups per further pair, their layers
     float2* part;                  // ... and their partial sums [pair][nsplit][2][Nx]
     double* fringe;                // h x w (double) or
     float* fringe32;               // h x w (float) or
@@ -331,7 +331,15 @@ __global__ __launch_bounds__(LX / 16) void dm_rows(DmArgs a, const float2* __res
     finish_row<LX>(a, accb, kyb, line, twx, t);
 }
 
-// Row pass for equally spaced layers (no field lens).  The transfer of
+// Row pass of power-of-two rows of 64 to 4096.  MODE 1 and 2 (a field lens, or
+// a pitch that needs the transfer in full: 2) evaluate the transfer of every
+// layer; against one thread per 16 elements (dm_rows below 64 and at 8192:
+// 434 registers, one wave per SIMD, a line's loads waited for before its
+// transform) a frame of 512^2, 64 layers fell from 482 to 69 us and of
+// 4096 x 2048 from 1782 to 763; held to 168 or 128 registers it spills
+// (1135, 1432 us).
+//
+// MODE 0: equally spaced layers (no field lens).  The transfer of
 // layer l is H_l = exp(i 2 pi z_l Phi(kx, ky)) with one Phi for all layers,
 // so over a chunk of 16 consecutive layers starting at c,
 //   sum_j H_{c+j} G_{c+j} = H_c sum_j R^j G_{c+j},   R = exp(i 2 pi dz Phi),
@@ -344,9 +352,9 @@ __global__ __launch_bounds__(LX / 16) void dm_rows(DmArgs a, const float2* __res
 // in LDS, each element touched only by its owner thread.  The twiddle table
 // and a bitmask of the present layers are copied to LDS at the start, so
 // that inside the layer loop only the prefetched rows are global loads.
-template <int LX>
+template <int LX, int MODE>
 __host__ __device__ constexpr size_t rows_h_lds() {
-    return (fft::padded_len(LX) + 2 * (size_t)LX + fft::table_len8(LX)) * sizeof(float2) +
+    return (fft::padded_len(LX) + (MODE == 0 ? 2 * (size_t)LX : 0) + fft::table_len8(LX)) * sizeof(float2) +
            (size_t)(MAX_LAYERS / 32) * sizeof(unsigned);
 }
 
@@ -398,9 +406,9 @@ __device__ __forceinline__ void lds_copy(E* dst, const E* __restrict__ src, int 
     }
 }
 
-// lo .. hi: the layers taken (lo on a chunk boundary).  part: the sums of both
-// rows are written there instead of being finished.
-template <int LX, bool PAIR0, bool FBITS>
+// lo .. hi: the layers taken (MODE 0: in chunks from lo).  part: the sums of
+// both rows are written there instead of being finished.
+template <int LX, int MODE, bool PAIR0, bool FBITS>
 __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __restrict__ tw8, float2* sm, int kya,
                                             int lo, int hi, float2* part) {
     constexpr int TPL = LX / 8;
@@ -408,9 +416,9 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
     constexpr int CH = 16;
     constexpr int NTW = fft::table_len8(LX);
     float2* line = sm;
-    float2* Sa = sm + PL;
+    float2* Sa = sm + PL;             // MODE 0: the chunk sums of both rows
     float2* Sb = Sa + LX;
-    float2* tws = Sb + LX;
+    float2* tws = sm + PL + (MODE == 0 ? 2 * LX : 0);
     unsigned* amask = reinterpret_cast<unsigned*>(tws + NTW);
     // presence bits of every (layer, column group), when they fit in LDS:
     // then only present groups' rows of I are loaded
@@ -433,8 +441,11 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
     // row b's transform at kb is conj Z(kx) of the thread's own element of
     // row a's transform Z, and the transfer depends on kx only through kx^2,
     // which is the same at kb, so one set of per-element factors serves both.
-    float2 Ra[8], Rb[8];
-    {
+    float2 Ra[8], Rb[8];   // MODE 0
+    float2 Ta[8], Tb[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) Ta[m] = Tb[m] = make_float2(0.f, 0.f);
+    if constexpr (MODE == 0) {
         double tya = a.dcy * (double)sya * sya;
         tya -= rint(tya);
         double tyb = a.dcy * (double)syb * syb;
@@ -507,6 +518,27 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
                 nv[m] = in ? src[o] : make_float2(0.f, 0.f);
         }
     };
+    // MODE != 0: T += H_l G_l, the transfer evaluated for every layer
+    auto add_layer = [&](int l, const float2 (&va)[8], const float2 (&vb)[8]) {
+        const double cx = a.lc[3 * (l - 1)], cy = a.lc[3 * (l - 1) + 1], K = a.lc[3 * (l - 1) + 2];
+        const float Kf = (float)K;
+        double tya = cy * (double)sya * sya;
+        tya -= rint(tya);
+        double tyb = cy * (double)syb * syb;
+        tyb -= rint(tyb);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const int sx = sgnidx(t + m * TPL, LX);
+            const double sx2 = (double)(sx * sx);
+            double txd = cx * sx2;
+            txd -= rint(txd);
+            const float usx = a.ux * (float)(sx * sx);
+            const float2 ha = dm_transfer<MODE == 2>(a, (float)txd, tya, usx, sya, K, Kf, sx2);
+            Ta[m] = fft::cadd(Ta[m], fft::cmul(ha, va[m]));
+            const float2 hb = dm_transfer<MODE == 2>(a, (float)txd, tyb, usx, syb, K, Kf, sx2);
+            Tb[m] = fft::cadd(Tb[m], fft::cmul(hb, PAIR0 ? vb[m] : make_float2(va[m].x, -va[m].y)));
+        }
+    };
     int pl = min(hi, lo + CH - 1);
     if (!present(pl)) pl = next_layer(pl);
     if (pl) fetch(pl);
@@ -515,18 +547,21 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
         bool anyc = false;
         for (int l = cs; l <= ce; ++l) anyc |= present(l);
         if (!anyc) continue;
-        float2 Ta[8], Tb[8];
+        if constexpr (MODE == 0) {
 #pragma unroll
-        for (int m = 0; m < 8; ++m) Ta[m] = Tb[m] = make_float2(0.f, 0.f);
+            for (int m = 0; m < 8; ++m) Ta[m] = Tb[m] = make_float2(0.f, 0.f);
+        }
         for (int l = ce; l >= cs; --l) {
+            if constexpr (MODE == 0) {
 #pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                Ta[m] = fft::cmul(Ta[m], Ra[m]);
-                Tb[m] = fft::cmul(Tb[m], Rb[m]);
+                for (int m = 0; m < 8; ++m) {
+                    Ta[m] = fft::cmul(Ta[m], Ra[m]);
+                    Tb[m] = fft::cmul(Tb[m], Rb[m]);
+                }
             }
             if (!present(l)) continue;
             // l is the prefetched layer
-            float2 v[8];
+            float2 v[8], vb[8];   // vb: row b of PAIR0 (MODE != 0)
 #pragma unroll
             for (int m = 0; m < 8; ++m) v[m] = ((nf >> m) & 1u) ? nv[m] : make_float2(0.f, 0.f);
             pl = next_layer(l);
@@ -546,40 +581,72 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
                     const float2 gm = line[fft::pad16((LX - kx) & (LX - 1))];
                     float2 z = v[m], zc = make_float2(gm.x, -gm.y);
                     split_real_pair(z, zc);
-                    Ta[m] = fft::cadd(Ta[m], z);
-                    Tb[m] = fft::cadd(Tb[m], make_float2(zc.x, -zc.y));
+                    v[m] = z;
+                    if constexpr (MODE == 0)
+                        Tb[m] = fft::cadd(Tb[m], make_float2(zc.x, -zc.y));
+                    else
+                        vb[m] = make_float2(zc.x, -zc.y);
                 }
-            } else {
+            }
+            if constexpr (MODE == 0) {
 #pragma unroll
                 for (int m = 0; m < 8; ++m) {
                     Ta[m] = fft::cadd(Ta[m], v[m]);
-                    Tb[m] = fft::cadd(Tb[m], make_float2(v[m].x, -v[m].y));
+                    if constexpr (!PAIR0) Tb[m] = fft::cadd(Tb[m], make_float2(v[m].x, -v[m].y));
                 }
+            } else {
+                add_layer(l, v, vb);
             }
         }
+        if constexpr (MODE != 0) continue;
         // anchor: S += H_cs T
-        const double cx = a.lc[3 * (cs - 1)], cy = a.lc[3 * (cs - 1) + 1], K = a.lc[3 * (cs - 1) + 2];
-        const float Kf = (float)K;
-        double tya = cy * (double)sya * sya;
-        tya -= rint(tya);
-        double tyb = cy * (double)syb * syb;
-        tyb -= rint(tyb);
+        if constexpr (MODE == 0) {
+            const double cx = a.lc[3 * (cs - 1)], cy = a.lc[3 * (cs - 1) + 1], K = a.lc[3 * (cs - 1) + 2];
+            const float Kf = (float)K;
+            double tya = cy * (double)sya * sya;
+            tya -= rint(tya);
+            double tyb = cy * (double)syb * syb;
+            tyb -= rint(tyb);
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const int kx = t + m * TPL;
-            const int sx = sgnidx(kx, LX);
-            const double sx2 = (double)sx * sx;
-            double txd = cx * sx2;
-            txd -= rint(txd);
-            const float usx = a.ux * (float)(sx * sx);
-            const float2 ha = dm_transfer<false>(a, (float)txd, tya, usx, sya, K, Kf, sx2);
-            Sa[kx] = fft::cadd(Sa[kx], fft::cmul(ha, Ta[m]));
-            const float2 hb = dm_transfer<false>(a, (float)txd, tyb, usx, syb, K, Kf, sx2);
-            const int kb = (LX - kx) & (LX - 1);
-            Sb[kb] = fft::cadd(Sb[kb], fft::cmul(hb, Tb[m]));
+            for (int m = 0; m < 8; ++m) {
+                const int kx = t + m * TPL;
+                const int sx = sgnidx(kx, LX);
+                const double sx2 = (double)sx * sx;
+                double txd = cx * sx2;
+                txd -= rint(txd);
+                const float usx = a.ux * (float)(sx * sx);
+                const float2 ha = dm_transfer<false>(a, (float)txd, tya, usx, sya, K, Kf, sx2);
+                Sa[kx] = fft::cadd(Sa[kx], fft::cmul(ha, Ta[m]));
+                const float2 hb = dm_transfer<false>(a, (float)txd, tyb, usx, syb, K, Kf, sx2);
+                const int kb = (LX - kx) & (LX - 1);
+                Sb[kb] = fft::cadd(Sb[kb], fft::cmul(hb, Tb[m]));
+            }
         }
     }
-    __syncthreads();  // Sb entries were written by the threads owning -kx
+    __syncthreads();  // Sb entries were written by the threads owning -kx; the line is free
+    if constexpr (MODE != 0) {
+        if (part) {
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                const int kx = t + m * TPL;
+                part[kx] = Ta[m];
+                part[LX + ((LX - kx) & (LX - 1))] = Tb[m];
+            }
+            return;
+        }
+#pragma unroll
+        for (int m = 0; m < 8; ++m) line[fft::pad16((LX - t - m * TPL) & (LX - 1))] = Tb[m];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            Tb[m] = fft::cmul(line[fft::pad16(t + m * TPL)], a.rho);
+            Ta[m] = fft::cmul(Ta[m], a.rho);
+        }
+        __syncthreads();
+        finish_row8<LX>(a, Ta, kya, line, tws, t);
+        finish_row8<LX>(a, Tb, kyb, line, tws, t);
+        return;
+    }
     if (part) {
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
@@ -601,26 +668,28 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
 
 // (two waves per SIMD: 256 registers, the budget of two 2048-point
 // workgroups per CU or one 4096-point workgroup)
-template <int LX, bool FBITS>
+template <int LX, int MODE, bool FBITS>
 __global__ __launch_bounds__(LX / 8, 2) void dm_rows_h(DmArgs a, const float2* __restrict__ tw8) {
     extern __shared__ float2 sm[];
-    if ((int)blockIdx.x >= a.n_main) {
-        // a pair beyond the last full round of workgroups: part of its layers
-        const int k = blockIdx.x - a.n_main, i = k / a.nsplit, j = k % a.nsplit;
-        const int per = ((a.hi - a.lo + 16) / 16 + a.nsplit - 1) / a.nsplit * 16;
-        const int lo = a.lo + j * per, hi = min(a.hi, lo + per - 1);
-        float2* part = a.part + (size_t)k * 2 * LX;
-        if (a.n_main + i == 0) rows_h_body<LX, true, FBITS>(a, tw8, sm, 0, lo, hi, part);
-        else rows_h_body<LX, false, FBITS>(a, tw8, sm, a.n_main + i, lo, hi, part);
-        return;
-    }
     // XCD-aware: neighbouring rows, which share the cache lines of I, run on
     // the same XCD at the same time
-    const int kya = xcd_remap(blockIdx.x, a.n_main);  // 0 .. n_main - 1
+    int kya, lo = a.lo, hi = a.hi;
+    float2* part = nullptr;
+    if ((int)blockIdx.x >= a.n_main) {
+        // a pair beyond the last full round of workgroups: part j of its layers
+        const int lin = xcd_remap(blockIdx.x - a.n_main, gridDim.x - a.n_main), left = a.K - 1 - a.n_main;
+        const int j = lin / left, i = lin - j * left;
+        lo = a.lo + j * a.per;
+        hi = min(a.hi, lo + a.per - 1);
+        kya = a.n_main + i;
+        part = a.part + ((size_t)i * a.nsplit + j) * 2 * LX;
+    } else {
+        kya = xcd_remap(blockIdx.x, a.n_main);  // 0 .. n_main - 1
+    }
     if (kya == 0)
-        rows_h_body<LX, true, FBITS>(a, tw8, sm, 0, a.lo, a.hi, nullptr);
+        rows_h_body<LX, MODE, true, FBITS>(a, tw8, sm, 0, lo, hi, part);
     else
-        rows_h_body<LX, false, FBITS>(a, tw8, sm, kya, a.lo, a.hi, nullptr);
+        rows_h_body<LX, MODE, false, FBITS>(a, tw8, sm, kya, lo, hi, part);
 }
 
 // The pairs whose layers were split: their partial sums in order (the same
@@ -629,21 +698,18 @@ template <int LX>
 __global__ __launch_bounds__(LX / 8) void dm_rows_h_sum(DmArgs a, const float2* __restrict__ tw8) {
     constexpr int TPL = LX / 8;
     __shared__ float2 line[fft::padded_len(LX)];
-    const int t = threadIdx.x, kya = a.n_main + blockIdx.x, kyb = kya == 0 ? a.Ny / 2 : a.Ny - kya;
-    const float2* p = a.part + (size_t)blockIdx.x * a.nsplit * 2 * LX;
+    const int t = threadIdx.x, i = blockIdx.x >> 1, row = blockIdx.x & 1, kya = a.n_main + i;
+    const int ky = row == 0 ? kya : kya == 0 ? a.Ny / 2 : a.Ny - kya;
+    const float2* p = a.part + ((size_t)i * a.nsplit * 2 + row) * LX;
+    float2 acc[8];
 #pragma unroll
-    for (int row = 0; row < 2; ++row) {
-        float2 acc[8];
+    for (int m = 0; m < 8; ++m) acc[m] = make_float2(0.f, 0.f);
+    for (int j = 0; j < a.nsplit; ++j)
 #pragma unroll
-        for (int m = 0; m < 8; ++m) acc[m] = make_float2(0.f, 0.f);
-        for (int j = 0; j < a.nsplit; ++j)
+        for (int m = 0; m < 8; ++m) acc[m] = fft::cadd(acc[m], p[(size_t)2 * j * LX + t + m * TPL]);
 #pragma unroll
-            for (int m = 0; m < 8; ++m)
-                acc[m] = fft::cadd(acc[m], p[((size_t)2 * j + row) * LX + t + m * TPL]);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) acc[m] = fft::cmul(acc[m], a.rho);
-        finish_row8<LX>(a, acc, row ? kyb : kya, line, tw8, t);
-    }
+    for (int m = 0; m < 8; ++m) acc[m] = fft::cmul(acc[m], a.rho);
+    finish_row8<LX>(a, acc, ky, line, tw8, t);
 }
 
 // ---- final column pass ---------------------------------------------------------
@@ -836,19 +902,26 @@ __device__ __forceinline__ void finish_row_m(const DmArgs& a, const float2 (&acc
 
 // Bound by vector instructions once enough waves are resident: one workgroup
 // a pair leaves 272 two-wave workgroups for 256 CUs at 1920 x 1080 encoded
-// (2483 us, 256 layers), the layers split into 3 parts 795 us; holding it to
+// (2483 us, 256 layers), the layers split into 7 parts 795 us; holding it to
 // 168 or 128 registers for more waves spills (1010 and 1456 us).
 template <int LX, bool EXACT>
 __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const float2* __restrict__ twx) {
     constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
     const int t = threadIdx.x;
-    // part j of the pair's layers (XCD-aware: neighbouring pairs, which share
-    // the cache lines of I, run their same part on one XCD at the same time)
-    const int lin = xcd_remap(blockIdx.x, gridDim.x), npair = a.K - 1;
-    const int j = lin / npair, kya = lin - j * npair;  // kya = 0 .. K - 2
-    const int per = (a.hi - a.lo + a.nsplit) / a.nsplit;
-    const int lo = a.lo + j * per, hi = min(a.hi, lo + per - 1);
+    // XCD-aware, as dm_rows_h
+    int kya, lo = a.lo, hi = a.hi;
+    float2* part = nullptr;
+    if ((int)blockIdx.x >= a.n_main) {
+        const int lin = xcd_remap(blockIdx.x - a.n_main, gridDim.x - a.n_main), left = a.K - 1 - a.n_main;
+        const int j = lin / left, i = lin - j * left;
+        lo = a.lo + j * a.per;
+        hi = min(a.hi, lo + a.per - 1);
+        kya = a.n_main + i;
+        part = a.part + ((size_t)i * a.nsplit + j) * 2 * LX;
+    } else {
+        kya = xcd_remap(blockIdx.x, a.n_main);
+    }
     const bool pair0 = kya == 0;              // real rows 0 and Ny/2 packed as re/im
     const int kyb = pair0 ? a.Ny / 2 : a.Ny - kya;
     const int sya = sgnidx(kya, a.Ny) + 1;
@@ -961,8 +1034,7 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
         }
         __syncthreads();
     }
-    if (a.nsplit > 1) {
-        float2* part = a.part + ((size_t)kya * a.nsplit + j) * 2 * LX;
+    if (part) {
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
             const int kx = t + m * NT;
@@ -987,9 +1059,9 @@ template <int LX>
 __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m_sum(DmArgs a, const float2* __restrict__ twx) {
     constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
-    const int t = threadIdx.x, kya = blockIdx.x >> 1, row = blockIdx.x & 1;
+    const int t = threadIdx.x, i = blockIdx.x >> 1, row = blockIdx.x & 1, kya = a.n_main + i;
     const int ky = row == 0 ? kya : kya == 0 ? a.Ny / 2 : a.Ny - kya;
-    const float2* p = a.part + ((size_t)kya * a.nsplit * 2 + row) * LX;
+    const float2* p = a.part + ((size_t)i * a.nsplit * 2 + row) * LX;
     float2 acc[EPT];
 #pragma unroll
     for (int m = 0; m < EPT; ++m) acc[m] = make_float2(0.f, 0.f);
@@ -1063,58 +1135,86 @@ int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
     return OPH_OK;
 }
 
+// How the row pairs are spread over the chip, with `resident` workgroups of
+// the row pass on a CU: the first n_main pairs (whole rounds of workgroups)
+// are taken whole, the layers of each of the rest are split over nsplit
+// workgroups of `per` layers, at least four.  The cost of a choice is its
+// rounds times the layers of each; a part costs three layer times of its own
+// (its set-up, its sums written and read again).  4096 x 2048 encoded needs
+// 514 pairs: 2 rounds and a sixteenth, not 3.  (A frame of 720 x 540 and 256
+// layers, field: 2.29 -> 0.55 ms.)
+int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int resident) {
+    const int pairs = a.K - 1, layers = a.hi - a.lo + 1;
+    const int slots = std::max(ctx->cu_count, 1) * resident;
+    a.n_main = pairs;
+    a.nsplit = 1;
+    a.per = layers;
+    long long best = (long long)((pairs + slots - 1) / slots) * layers;
+    for (const int n_main : {pairs / slots * slots, 0})
+        for (int n = 2; n <= 16; ++n) {
+            const int per = (layers + n - 1) / n;
+            const int parts = (layers + per - 1) / per, left = pairs - n_main;
+            if (per < 4 || parts < 2 || left == 0) continue;
+            const long long c = (long long)(n_main / slots) * layers +
+                                ((long long)left * parts + slots - 1) / slots * (per + 3);
+            if (c < best) {
+                best = c;
+                a.n_main = n_main;
+                a.nsplit = parts;
+                a.per = per;
+            }
+        }
+    if (a.n_main < pairs) {
+        a.part = static_cast<float2*>(
+            oph_scratch(ctx, SLOT_WORK0, (size_t)(pairs - a.n_main) * a.nsplit * 2 * LX * sizeof(float2)));
+        if (!a.part) return OPH_ENOMEM;
+    }
+    return OPH_OK;
+}
+
+// Workgroups of a kernel on a CU with this much dynamic LDS, which it is
+// allowed to ask for
+template <typename F>
+int rows_resident(F kernel, int threads, size_t shm) {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    int n = 0;
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, shm);
+    hipGetLastError();
+    return std::max(n, 1);
+}
+
+template <int LX, int MODE>
+int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
+    const float2* tw8 = oph_twiddles(ctx, LX, 8);
+    if (!tw8) return OPH_ENOMEM;
+    const size_t fbytes = (size_t)a.L * a.fwpl * sizeof(unsigned);
+    const bool fbits = rows_h_lds<LX, MODE>() + fbytes <= 160 * 1024;
+    const size_t shm = rows_h_lds<LX, MODE>() + (fbits ? fbytes : 0);
+    auto* kernel = fbits ? dm_rows_h<LX, MODE, true> : dm_rows_h<LX, MODE, false>;
+    DmArgs b = a;
+    const int rc = rows_plan(ctx, b, LX, rows_resident(kernel, LX / 8, shm));
+    if (rc) return rc;
+    const int left = a.K - 1 - b.n_main;
+    OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(LX / 8), shm, b, tw8);
+    if (left > 0)
+        OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_h_sum<LX>, dim3(2 * left), dim3(LX / 8), 0, b, tw8);
+    return OPH_OK;
+}
+
 template <int LX>
 int launch_dm_rows(oph_ctx* ctx, const DmArgs& a) {
-    const float2* tw = oph_twiddles(ctx, LX);
-    if (!tw) return OPH_ENOMEM;
     if constexpr (LX >= 64 && LX <= 4096) {
-        if (a.horner) {
-            const float2* tw8 = oph_twiddles(ctx, LX, 8);
-            if (!tw8) return OPH_ENOMEM;
-            static bool attr = false;
-            if (!attr) {
-                for (const void* k : {reinterpret_cast<const void*>(&dm_rows_h<LX, true>),
-                                      reinterpret_cast<const void*>(&dm_rows_h<LX, false>)})
-                    hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-                hipGetLastError();
-                attr = true;
-            }
-            DmArgs b = a;
-            const size_t fbytes = (size_t)a.L * a.fwpl * sizeof(unsigned);
-            b.fbits_lds = rows_h_lds<LX>() + fbytes <= 160 * 1024 ? 1 : 0;
-            const size_t shm = rows_h_lds<LX>() + (b.fbits_lds ? fbytes : 0);
-            // A workgroup's LDS leaves one or two per CU, so a few pairs beyond
-            // the last full round would cost a whole round: their layers are
-            // split over several workgroups instead (2048 rows of which 514
-            // pairs are needed: 2 rounds and a sixteenth, not 3), as are all
-            // pairs of a grid that does not fill one round.
-            const int n = a.K - 1, slots = std::max(ctx->cu_count, 1) * (2 * shm <= 160 * 1024 ? 2 : 1);
-            const int nch = (a.hi - a.lo + 16) / 16;   // chunks of 16 layers
-            b.n_main = n / slots * slots;
-            b.nsplit = std::min(nch, 16);
-            if (b.nsplit < 2 || 2 * (n - b.n_main) > slots) b.n_main = n;
-            const int left = n - b.n_main;
-            if (left > 0) {
-                b.nsplit = (nch + (nch + b.nsplit - 1) / b.nsplit - 1) / ((nch + b.nsplit - 1) / b.nsplit);
-                b.part = static_cast<float2*>(
-                    oph_scratch(ctx, SLOT_WORK0, (size_t)left * b.nsplit * 2 * LX * sizeof(float2)));
-                if (!b.part) return OPH_ENOMEM;
-            }
-            const dim3 grid(b.n_main + left * b.nsplit);
-            if (b.fbits_lds)
-                OPH_LAUNCH(ctx, "dm_rows", (dm_rows_h<LX, true>), grid, dim3(LX / 8), shm, b, tw8);
-            else
-                OPH_LAUNCH(ctx, "dm_rows", (dm_rows_h<LX, false>), grid, dim3(LX / 8), shm, b, tw8);
-            if (left > 0)
-                OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_h_sum<LX>, dim3(left), dim3(LX / 8), 0, b, tw8);
-            return OPH_OK;
-        }
+        if (a.horner) return launch_dm_rows_h<LX, 0>(ctx, a);
+        return a.exact ? launch_dm_rows_h<LX, 2>(ctx, a) : launch_dm_rows_h<LX, 1>(ctx, a);
+    } else {
+        const float2* tw = oph_twiddles(ctx, LX);
+        if (!tw) return OPH_ENOMEM;
+        if (a.exact)
+            OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, true>), dim3(a.K - 1), dim3(LX / 16), 0, a, tw);
+        else
+            OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, false>), dim3(a.K - 1), dim3(LX / 16), 0, a, tw);
+        return OPH_OK;
     }
-    if (a.exact)
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, true>), dim3(a.K - 1), dim3(LX / 16), 0, a, tw);
-    else
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows<LX, false>), dim3(a.K - 1), dim3(LX / 16), 0, a, tw);
-    return OPH_OK;
 }
 
 template <int LY>
@@ -1160,53 +1260,22 @@ int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
     }
 }
 
-// Into how many parts a pair's layers are split, with `resident` workgroups
-// of the row pass on a CU: the fewest layer times of whole rounds, a part
-// costing three layer times of its own (its set-up, its sums written and
-// read again).
-int rows_parts(oph_ctx* ctx, int pairs, int layers, int resident) {
-    const long long slots = (long long)std::max(ctx->cu_count, 1) * resident;
-    int best = 1;
-    long long cost = (pairs + slots - 1) / slots * layers;
-    for (int n = 2; n <= 16 && 4 * n <= layers; ++n) {
-        const long long c = ((long long)pairs * n + slots - 1) / slots * ((layers + n - 1) / n + 3);
-        if (c < cost) { cost = c; best = n; }
-    }
-    const int per = (layers + best - 1) / best;
-    return (layers + per - 1) / per;
-}
-
 template <int LX>
 int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
     const float2* tw = oph_twiddles_mixed(ctx, LX);
     if (!tw) return OPH_ENOMEM;
     const size_t shm = (size_t)fftm::padded_len(LX) * sizeof(float2);
-    static int resident[2] = {0, 0};
-    if (!resident[a.exact]) {
-        for (const void* k : {reinterpret_cast<const void*>(&dm_rows_m<LX, true>),
-                              reinterpret_cast<const void*>(&dm_rows_m<LX, false>),
-                              reinterpret_cast<const void*>(&dm_rows_m_sum<LX>)})
-            hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-        int n = 0;
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>,
-                                                     fftm::threads(LX), shm);
-        hipGetLastError();
-        resident[a.exact] = std::max(n, 1);
-    }
+    constexpr int NT = fftm::threads(LX);
+    auto* kernel = a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>;
     DmArgs b = a;
-    b.nsplit = rows_parts(ctx, a.K - 1, a.hi - a.lo + 1, resident[a.exact]);
-    if (b.nsplit > 1) {
-        b.part = static_cast<float2*>(
-            oph_scratch(ctx, SLOT_WORK0, (size_t)(a.K - 1) * b.nsplit * 2 * LX * sizeof(float2)));
-        if (!b.part) return OPH_ENOMEM;
+    const int rc = rows_plan(ctx, b, LX, rows_resident(kernel, NT, shm));
+    if (rc) return rc;
+    const int left = a.K - 1 - b.n_main;
+    OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(NT), shm, b, tw);
+    if (left > 0) {
+        rows_resident(dm_rows_m_sum<LX>, NT, shm);
+        OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_m_sum<LX>, dim3(2 * left), dim3(NT), shm, b, tw);
     }
-    const dim3 grid((a.K - 1) * b.nsplit);
-    if (a.exact)
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, true>), grid, dim3(fftm::threads(LX)), shm, b, tw);
-    else
-        OPH_LAUNCH(ctx, "dm_rows", (dm_rows_m<LX, false>), grid, dim3(fftm::threads(LX)), shm, b, tw);
-    if (b.nsplit > 1)
-        OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_m_sum<LX>, dim3(2 * (a.K - 1)), dim3(fftm::threads(LX)), shm, b, tw);
     return OPH_OK;
 }
 

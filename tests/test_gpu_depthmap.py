@@ -195,3 +195,24 @@ def test_depthmap_lens_row_pairs_split(ctx, w, h, Nx, Ny, L, layers, out):
     u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.2, 0.7, L, [532e-9], img, dep, out=out, **kw)
     ref = _oracle_rgb(img, dep, Nx, Ny, 8e-6, [532e-9], 0.2, 0.7, L, out=out, **kw)
     assert rel_l2(u, ref) < TOL
+
+
+@pytest.mark.parametrize("w,h,Nx,Ny,L,pitch,layers,out", [
+    (40, 30, 64, 64, 33, 8e-6, None, "field"),        # the shortest row of the radix-8 pass
+    (100, 60, 256, 128, 20, 8e-6, (3, 19), "fringe"),
+    (30, 1000, 64, 2048, 40, 8e-6, None, "fringe"),   # 514 pairs
+    (1000, 24, 4096, 32, 12, 8e-6, None, "field"),    # the longest
+    (100, 60, 256, 128, 20, 1e-6, None, "fringe"),    # the transfer in full (short wavelengths' pitch)
+    (100, 60, 256, 128, 5, 1e-6, None, "field"),
+    (20, 20, 32, 32, 40, 8e-6, None, "fringe"),       # below it: the radix-16 pass
+])
+def test_depthmap_lens_power_of_two_rows(ctx, w, h, Nx, Ny, L, pitch, layers, out):
+    """With a field lens on power-of-two grids: the transfer of every layer."""
+    print(f"case: depthmap lens {w}x{h} grid {Nx}x{Ny} L={L} pitch={pitch} layers={layers} {out}", flush=True)
+    img, dep = scenes.depth_scene(w, h, seed=13, colors=1)
+    kw = dict(quant_mode=1, field_lens=1.0)
+    if layers is not None:
+        kw["layers"] = layers
+    u = ctx.depthmap(w, h, Nx, Ny, pitch, 0.2, 0.7, L, [532e-9], img, dep, out=out, **kw)
+    ref = _oracle_rgb(img, dep, Nx, Ny, pitch, [532e-9], 0.2, 0.7, L, out=out, **kw)
+    assert rel_l2(u, ref) < TOL

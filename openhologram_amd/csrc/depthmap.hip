@@ -74,7 +74,6 @@ struct DmArgs {
     unsigned char* any;            // [L]
     unsigned* fbits;               // [L][fwpl]: the flags as bits (group g: word g/32, bit g%32)
     int fwpl;                      // words per layer of fbits
-    int fbits_lds;                 // dm_rows_h stages fbits in LDS and loads present groups only
     const double* lc;              // per layer: cx, cy, K (3 doubles)
     float ux, uy;                  // lambda^2 / Sx^2, lambda^2 / Sy^2
     int exact;                     // FP64 transfer path
@@ -110,95 +109,6 @@ __global__ void dm_zero(unsigned char* p, int n) {
     if (i < n) p[i] = 0;
 }
 
-// ---- column pass ---------------------------------------------------------------
-
-template <int LY>
-__global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int layers_per_wg,
-                                                         const float2* __restrict__ twy) {
-    constexpr int TPL = LY / 16;
-    constexpr int NT = 2 * TPL;
-    constexpr int PL = fft::padded_len(LY);
-    extern __shared__ unsigned char smem[];
-    float2* lines = reinterpret_cast<float2*>(smem);                 // 2 x PL
-    unsigned* pix = reinterpret_cast<unsigned*>(lines + 2 * PL);     // h x GROUP: idx << 8 | img
-    unsigned* mask = pix + (size_t)a.h * GROUP;                      // layer bitmask
-    // XCD-aware: neighbouring column groups (whose 32-byte row segments share
-    // cache lines of I) run on the same XCD at the same time
-    const int lin = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-    const int g = lin % gridDim.x;
-    const int x0 = g * GROUP;
-    const int l_begin = a.lo + lin / gridDim.x * layers_per_wg;
-    const int l_end = min(a.hi, l_begin + layers_per_wg - 1);
-    const int nwords = (a.L + 32) / 32;
-    const int p = threadIdx.x / TPL, t = threadIdx.x % TPL;
-    float2* line = lines + p * PL;
-    fft::Twiddles<LY> Tw;
-    Tw.load(twy, t);
-    for (int i = threadIdx.x; i < nwords; i += NT) mask[i] = 0u;
-    __syncthreads();
-    for (int e = threadIdx.x; e < a.h * GROUP; e += NT) {
-        const int c = e % GROUP, r = e / GROUP;
-        const int x = x0 + c;
-        unsigned v = 0u;
-        if (x < a.w) {
-            const size_t o = (size_t)r * a.w + x;
-            const unsigned im = a.img[o];
-            const unsigned id = a.idx[o];
-            // alpha = [img > 0] (CPU.cpp:61): a zero pixel contributes nothing
-            if (im > 0u && id >= (unsigned)l_begin && id <= (unsigned)l_end) {
-                v = (id << 8) | im;
-                atomicOr(&mask[id >> 5], 1u << (id & 31));
-            }
-        }
-        pix[e] = v;
-    }
-    __syncthreads();
-    const size_t gstride = (size_t)a.K * GROUP;
-    const size_t lstride = gstride * a.ngroups;
-    for (int l = l_begin; l <= l_end; ++l) {
-        if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
-        // two real columns (x0 + 2p, x0 + 2p + 1) as one complex column
-#pragma unroll
-        for (int m = 0; m < 16; ++m) {
-            const int i = t + m * TPL;
-            const int r = i - a.oy;
-            float2 v = make_float2(0.f, 0.f);
-            if (r >= 0 && r < a.h) {
-                const unsigned wa = pix[r * GROUP + 2 * p], wb = pix[r * GROUP + 2 * p + 1];
-                if ((int)(wa >> 8) == l) v.x = (float)(wa & 255u) * (1.f / 255.f);
-                if ((int)(wb >> 8) == l) v.y = (float)(wb & 255u) * (1.f / 255.f);
-            }
-            line[fft::lane_pad<LY>(t, m)] = v;
-        }
-        __syncthreads();
-        fft::line<LY, -1>(line, Tw, t);
-        // separate: A(k) = (Z(k) + conj Z(-k))/2, B(k) = (Z(k) - conj Z(-k))/(2i)
-        float2* dst = a.I + (size_t)(l - 1) * lstride + (size_t)g * gstride;
-        for (int e = threadIdx.x; e < a.K * GROUP; e += NT) {
-            const int c = e % GROUP, ky = e / GROUP < a.K - 1 ? e / GROUP : LY / 2;
-            const int x = x0 + c;
-            if (x >= a.w) continue;
-            const float2* ln = lines + (c >> 1) * PL;
-            const float2 Z = ln[fft::pad16(ky)];
-            const float2 Zm = ln[fft::pad16((LY - ky) & (LY - 1))];
-            float2 v;
-            if ((c & 1) == 0)
-                v = make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
-            else
-                v = make_float2(0.5f * (Z.y + Zm.y), -0.5f * (Z.x - Zm.x));
-            dst[e] = v;
-        }
-        if (threadIdx.x == 0) {
-            a.flags[(size_t)(l - 1) * a.ngroups + g] = 1;
-            a.any[l - 1] = 1;
-            atomicOr(&a.fbits[(size_t)(l - 1) * a.fwpl + (g >> 5)], 1u << (g & 31));
-        }
-        __syncthreads();
-    }
-}
-
-// ---- row pass ------------------------------------------------------------------
-
 // Z = FFT(a + i b) of two real rows a, b; on entry z = Z(k), zc = conj Z(-k).
 // On exit z = A(k) = (Z(k) + conj Z(-k))/2 and zc = B(k) = (Z(k) - conj Z(-k))/(2i).
 __device__ __forceinline__ void split_real_pair(float2& z, float2& zc) {
@@ -206,6 +116,141 @@ __device__ __forceinline__ void split_real_pair(float2& z, float2& zc) {
     z = make_float2(0.5f * (z.x + zc.x), 0.5f * (z.y + zc.y));
     zc = make_float2(0.5f * dy, -0.5f * dx);
 }
+
+// ---- column pass ---------------------------------------------------------------
+
+// A pixel's amplitude, rounded by itself (not fused into the additions after it)
+__device__ __forceinline__ float pixel_value(unsigned img) {
+#pragma clang fp contract(off)
+    return (float)img * (1.f / 255.f);
+}
+
+// A thread owns 16 rows of a column pair (x0 + 2p, x0 + 2p + 1; neighbouring
+// threads take the two pairs): their pixels stay in registers over all of the
+// layers, a layer's values go straight into the transform's first radix-16
+// stage, and the result is separated from registers -- only the mirrored
+// rows that the stored ones need pass through LDS.  Bound by vector
+// instructions and LDS; 1920 x 1080 on 2048 rows, 256 layers: 690 us, against
+// 921 with pixels, input and output of the transform in LDS.
+template <int LY>
+__host__ __device__ constexpr bool cols_shared() { return LY > 4096; }   // the mirrored rows in the line itself
+template <int LY>
+__host__ __device__ constexpr int cols_mirror_stride(int K) { return cols_shared<LY>() ? 0 : (K + 31) / 32 * 32 + 16; }
+
+// HALF: only the row pairs of an encoded output's crop are stored (K = Ny/4 +
+// 3); its row Ny/2 is of no pair that is kept and stays zero.  MID: the scene's
+// rows are among the middle ten sixteenths of the grid's.
+template <int LY, bool HALF, bool MID>
+__global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int layers_per_wg,
+                                                         const float2* __restrict__ twy) {
+    constexpr int TPL = LY / 16;
+    constexpr int NT = 2 * TPL;
+    constexpr int M0 = MID ? 3 : 0, M1 = MID ? 13 : 16;
+    extern __shared__ unsigned char smem[];
+    const int p = threadIdx.x & 1, t = threadIdx.x >> 1;
+    constexpr int PL = fft::skewed_len(LY, 2);
+    constexpr bool SHARED = cols_shared<LY>();
+    float2* line = reinterpret_cast<float2*>(smem) + p * PL;
+    const int ms = cols_mirror_stride<LY>(a.K);
+    float2* mirrors = reinterpret_cast<float2*>(smem) + 2 * PL;
+    float2* mirror = SHARED ? line : mirrors + p * ms;               // Z(-k) at k = 1 .. K - 2
+    unsigned* mask = reinterpret_cast<unsigned*>(mirrors + 2 * ms);  // layer bitmask
+    // XCD-aware: neighbouring column groups (whose 32-byte row segments share
+    // cache lines of I) run on the same XCD at the same time
+    const int lin = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int g = lin % gridDim.x;
+    const int l_begin = a.lo + lin / gridDim.x * layers_per_wg;
+    const int l_end = min(a.hi, l_begin + layers_per_wg - 1);
+    const int nwords = (a.L + 32) / 32;
+    for (int i = threadIdx.x; i < nwords; i += NT) mask[i] = 0u;
+    __syncthreads();
+    unsigned pa[16], pb[16];   // idx << 16 | img; 0: no contribution
+    {
+        const int x = g * GROUP + 2 * p;
+#pragma unroll
+        for (int m = M0; m < M1; ++m) {
+            const int r = t + m * TPL - a.oy;
+            unsigned v[2] = {0u, 0u};
+            if (r >= 0 && r < a.h)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    if (x + c < a.w) {
+                        const size_t o = (size_t)r * a.w + x + c;
+                        const unsigned im = a.img[o];
+                        const unsigned id = a.idx[o];
+                        // alpha = [img > 0] (CPU.cpp:61): a zero pixel contributes nothing
+                        if (im > 0u && id >= (unsigned)l_begin && id <= (unsigned)l_end) {
+                            v[c] = (id << 16) | im;
+                            atomicOr(&mask[id >> 5], 1u << (id & 31));
+                        }
+                    }
+            pa[m] = v[0];
+            pb[m] = v[1];
+        }
+    }
+    fft::Twiddles<LY> Tw;   // (8192: too many registers with 1024 threads)
+    if constexpr (!SHARED) Tw.load(twy, t);
+    __syncthreads();
+    const size_t gstride = (size_t)a.K * GROUP;
+    const size_t lstride = gstride * a.ngroups;
+    for (int l = l_begin; l <= l_end; ++l) {
+        if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
+        // the two real columns as one complex column
+        float2 v[16];
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            if (m < M0 || m >= M1) {
+                v[m] = make_float2(0.f, 0.f);
+                continue;
+            }
+            const unsigned wa = pa[m] >> 16 == (unsigned)l ? pa[m] : 0u;
+            const unsigned wb = pb[m] >> 16 == (unsigned)l ? pb[m] : 0u;
+            v[m] = make_float2(pixel_value(wa & 255u), pixel_value(wb & 255u));
+        }
+        if constexpr (SHARED)
+            fft::line_regs_tw<LY, -1, M0, M1>(v, line, twy, t);
+        else
+            fft::line_regs<LY, -1, M0, M1>(v, line, Tw, t);
+        if constexpr (!HALF) {
+            // every element here, none computed within the branch that uses it
+            // (a product and the addition after it would then round apart)
+#pragma unroll
+            for (int m = 0; m < 16; ++m) asm volatile("" : "+v"(v[m].x), "+v"(v[m].y));
+        }
+        // the mirrored rows (the previous layer's were read before the
+        // barriers of this layer's transform; LY = 16 has none)
+        if constexpr (SHARED || LY == 16) __syncthreads();
+#pragma unroll
+        for (int m = HALF ? 11 : 7; m < 16; ++m) {
+            const int k = LY - (t + m * TPL);
+            if (k < a.K - 1) mirror[k] = v[m];
+        }
+        __syncthreads();
+        // separate: A(k) = (Z(k) + conj Z(-k))/2, B(k) = (Z(k) - conj Z(-k))/(2i)
+        float2* dst = a.I + (size_t)(l - 1) * lstride + (size_t)g * gstride + 2 * p;
+        constexpr float sc = 0.5f;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const int k = t + m * TPL;
+            if (m <= (HALF ? TPL == 1 ? 5 : 4 : 7) && k < a.K - 1) {
+                const float2 z = v[m], zm = k == 0 ? z : mirror[k];
+                *reinterpret_cast<float4*>(dst + (size_t)k * GROUP) =
+                    make_float4(sc * (z.x + zm.x), sc * (z.y - zm.y), sc * (z.y + zm.y), sc * (zm.x - z.x));
+            }
+        }
+        if (t == 0)
+            *reinterpret_cast<float4*>(dst + (size_t)(a.K - 1) * GROUP) =
+                HALF ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(v[8].x, 0.f, v[8].y, 0.f);
+        if (threadIdx.x == 0) {
+            a.flags[(size_t)(l - 1) * a.ngroups + g] = 1;
+            a.any[l - 1] = 1;
+            atomicOr(&a.fbits[(size_t)(l - 1) * a.fwpl + (g >> 5)], 1u << (g & 31));
+        }
+        if constexpr (SHARED) __syncthreads();
+    }
+}
+
+// ---- row pass ------------------------------------------------------------------
 
 template <bool EXACT>
 __device__ __forceinline__ float2 dm_transfer(const DmArgs& a, float tx, double ty, float usx, int sy,
@@ -385,7 +430,7 @@ __device__ __forceinline__ void finish_row8(const DmArgs& a, const float2 (&acc)
 }
 
 // PAIR0: workgroup 0, the real rows 0 and Ny/2 packed as re/im.  FBITS:
-// the presence bits of every (layer, group) fit in LDS (a.fbits_lds).
+// the presence bits of every (layer, group) fit in LDS.
 // Copies n elements of a table to LDS with NT threads, eight loads per
 // thread requested before any is stored (a plain loop waits for each load
 // before the next is issued).
@@ -1121,29 +1166,39 @@ template <int LY>
 int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
     const float2* tw = oph_twiddles(ctx, LY);
     if (!tw) return OPH_ENOMEM;
-    const size_t shm = 2 * fft::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 +
-                       (size_t)((a.L + 32) / 32) * 4;
-    if (shm > 160 * 1024) return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
-    static bool attr = false;
-    if (!attr) {
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&dm_cols<LY>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    const size_t words = (size_t)((a.L + 32) / 32) * 4;
+    // (the limit on the scene's height is the general lengths' too)
+    if (2 * fft::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 + words > 160 * 1024)
+        return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
+    const size_t shm = 2 * ((size_t)fft::skewed_len(LY, 2) + cols_mirror_stride<LY>(a.K)) * sizeof(float2) + words;
+    const auto launch = [&](auto* kernel) -> int {
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            160 * 1024);
         hipGetLastError();
-        attr = true;
+        OPH_LAUNCH(ctx, "dm_cols", kernel, dim3(a.ngroups, chunks), dim3(2 * (LY / 16)), shm, a, lpw, tw);
+        return OPH_OK;
+    };
+    if constexpr (LY >= 512) {
+        const bool half = a.K == LY / 4 + 3;
+        const bool mid = a.oy >= 3 * (LY / 16) && a.oy + a.h <= 13 * (LY / 16);
+        if (half) return mid ? launch(dm_cols<LY, true, true>) : launch(dm_cols<LY, true, false>);
+        return mid ? launch(dm_cols<LY, false, true>) : launch(dm_cols<LY, false, false>);
+    } else {
+        return launch(dm_cols<LY, false, false>);
     }
-    OPH_LAUNCH(ctx, "dm_cols", dm_cols<LY>, dim3(a.ngroups, chunks), dim3(2 * (LY / 16)), shm, a, lpw, tw);
-    return OPH_OK;
 }
 
 // How the row pairs are spread over the chip, with `resident` workgroups of
 // the row pass on a CU: the first n_main pairs (whole rounds of workgroups)
 // are taken whole, the layers of each of the rest are split over nsplit
-// workgroups of `per` layers, at least four.  The cost of a choice is its
+// workgroups of `per` layers, a multiple of gran.  The cost of a choice is its
 // rounds times the layers of each; a part costs three layer times of its own
 // (its set-up, its sums written and read again).  4096 x 2048 encoded needs
-// 514 pairs: 2 rounds and a sixteenth, not 3.  (A frame of 720 x 540 and 256
+// 514 pairs: 2 rounds and a sixteenth, not 3.  The chunked recurrence is split
+// between its chunks only (gran = 16), which leaves its sums as they are.
+// (A frame of 720 x 540 and 256
 // layers, field: 2.29 -> 0.55 ms.)
-int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int resident) {
+int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int gran, int resident) {
     const int pairs = a.K - 1, layers = a.hi - a.lo + 1;
     const int slots = std::max(ctx->cu_count, 1) * resident;
     a.n_main = pairs;
@@ -1152,9 +1207,9 @@ int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int resident) {
     long long best = (long long)((pairs + slots - 1) / slots) * layers;
     for (const int n_main : {pairs / slots * slots, 0})
         for (int n = 2; n <= 16; ++n) {
-            const int per = (layers + n - 1) / n;
+            const int per = ((layers + n - 1) / n + gran - 1) / gran * gran;
             const int parts = (layers + per - 1) / per, left = pairs - n_main;
-            if (per < 4 || parts < 2 || left == 0) continue;
+            if (parts < 2 || left == 0) continue;
             const long long c = (long long)(n_main / slots) * layers +
                                 ((long long)left * parts + slots - 1) / slots * (per + 3);
             if (c < best) {
@@ -1192,7 +1247,7 @@ int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
     const size_t shm = rows_h_lds<LX, MODE>() + (fbits ? fbytes : 0);
     auto* kernel = fbits ? dm_rows_h<LX, MODE, true> : dm_rows_h<LX, MODE, false>;
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, rows_resident(kernel, LX / 8, shm));
+    const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 4, rows_resident(kernel, LX / 8, shm));
     if (rc) return rc;
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(LX / 8), shm, b, tw8);
@@ -1268,7 +1323,7 @@ int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
     constexpr int NT = fftm::threads(LX);
     auto* kernel = a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>;
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, rows_resident(kernel, NT, shm));
+    const int rc = rows_plan(ctx, b, LX, 4, rows_resident(kernel, NT, shm));
     if (rc) return rc;
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(NT), shm, b, tw);

@@ -59,6 +59,19 @@ template <int SIGN>
 struct Dft<2, SIGN> {
     __device__ static void run(float2* v) { dft2<SIGN>(v[0], v[1]); }
 };
+// dft4 of v[N], v[N + 4], v[N + 8], v[N + 12], of which those outside LO .. HI - 1
+// are zeros (LO <= 4, HI >= 12: at most one of each pair two apart)
+template <int SIGN, int N, int LO, int HI>
+__device__ __forceinline__ void dft4_in(float2* v) {
+    static_assert(LO <= 4 && HI >= 12, "the middle half at least");
+    const float2 a = v[N], b = v[N + 4], c = v[N + 8], d = v[N + 12];
+    const float2 s02 = N < LO ? c : cadd(a, c), d02 = N < LO ? make_float2(-c.x, -c.y) : csub(a, c);
+    const float2 s13 = N + 12 >= HI ? b : cadd(b, d), d13 = mul_si<SIGN>(N + 12 >= HI ? b : csub(b, d));
+    v[N] = cadd(s02, s13);
+    v[N + 8] = csub(s02, s13);
+    v[N + 4] = cadd(d02, d13);
+    v[N + 12] = csub(d02, d13);
+}
 template <int SIGN>
 struct Dft<4, SIGN> {
     __device__ static void run(float2* v) { dft4<SIGN>(v[0], v[1], v[2], v[3]); }
@@ -89,10 +102,14 @@ struct Dft<8, SIGN> {
 };
 template <int SIGN>
 struct Dft<16, SIGN> {
+    // inputs below LO and from HI on are zeros, which no operation is spent on
+    template <int LO = 0, int HI = 16>
     __device__ static void run(float2* v) {
         // 4 x 4: X[k1 + 4 k2] = sum_{n2} W4^{n2 k2} W16^{n2 k1} sum_{n1} W4^{n1 k1} x[4 n1 + n2]
-#pragma unroll
-        for (int n2 = 0; n2 < 4; ++n2) dft4<SIGN>(v[n2], v[n2 + 4], v[n2 + 8], v[n2 + 12]);
+        dft4_in<SIGN, 0, LO, HI>(v);
+        dft4_in<SIGN, 1, LO, HI>(v);
+        dft4_in<SIGN, 2, LO, HI>(v);
+        dft4_in<SIGN, 3, LO, HI>(v);
         // now v[n2 + 4 k1] holds inner DFT k1 of column n2; twiddle W16^{n2 k1}
         constexpr float c1 = 0.92387953251128676f, s1 = 0.38268343236508977f, h = 0.70710678118654752f;
         const float2 w1 = make_float2(c1, SIGN * s1), w2 = make_float2(h, SIGN * h),
@@ -319,13 +336,13 @@ __host__ __device__ constexpr int skewed_len(int L, int B) { return padded_len(L
 // written again (other threads may still read the last stage's inputs).
 //
 // w16(s, w) gives the 15 twiddles of radix-16 stage s, wl(p, w) those of the
-// last radix-RL stage's butterfly p.
-template <int L, int SIGN, typename W16, typename WL>
+// last radix-RL stage's butterfly p.  Inputs v[m], m < LO or m >= HI, are zeros.
+template <int L, int SIGN, int LO, int HI, typename W16, typename WL>
 __device__ __forceinline__ void line_regs_w(float2 (&v)[16], float2* buf, int t, W16&& w16, WL&& wl) {
     constexpr int TPL = L / 16;
     constexpr int A = n16(L);
     constexpr int RL = last_radix(L);
-    Dft<16, SIGN>::run(v);
+    Dft<16, SIGN>::template run<LO, HI>(v);
     if constexpr (L > 16) {
         float2* dst = buf + pad16(16 * t);
 #pragma unroll
@@ -367,9 +384,9 @@ __device__ __forceinline__ void line_regs_w(float2 (&v)[16], float2* buf, int t,
 }
 
 // ... with every stage's twiddles in registers
-template <int L, int SIGN>
+template <int L, int SIGN, int LO = 0, int HI = 16>
 __device__ __forceinline__ void line_regs(float2 (&v)[16], float2* buf, const Twiddles<L>& T, int t) {
-    line_regs_w<L, SIGN>(
+    line_regs_w<L, SIGN, LO, HI>(
         v, buf, t,
         [&](int s, float2 (&w)[16]) {
 #pragma unroll
@@ -382,10 +399,10 @@ __device__ __forceinline__ void line_regs(float2 (&v)[16], float2* buf, const Tw
 }
 
 // ... with each stage's twiddles loaded from the table just before it
-template <int L, int SIGN>
+template <int L, int SIGN, int LO = 0, int HI = 16>
 __device__ __forceinline__ void line_regs_tw(float2 (&v)[16], float2* buf, const float2* __restrict__ tw, int t) {
     constexpr int TPL = L / 16, RL = last_radix(L), N = RL > 1 ? L / RL : 1;   // N = 16^A where RL > 1
-    line_regs_w<L, SIGN>(
+    line_regs_w<L, SIGN, LO, HI>(
         v, buf, t,
         [&](int s, float2 (&w)[16]) {
             int Ns = 16, off = 0;

@@ -216,3 +216,15 @@ def test_depthmap_lens_power_of_two_rows(ctx, w, h, Nx, Ny, L, pitch, layers, ou
     u = ctx.depthmap(w, h, Nx, Ny, pitch, 0.2, 0.7, L, [532e-9], img, dep, out=out, **kw)
     ref = _oracle_rgb(img, dep, Nx, Ny, pitch, [532e-9], 0.2, 0.7, L, out=out, **kw)
     assert rel_l2(u, ref) < TOL
+
+
+@pytest.mark.parametrize("out", ["field", "fringe"])
+@pytest.mark.parametrize("h,Ny", [(16, 16), (9, 32), (64, 64), (300, 512), (1100, 4096), (1200, 8192)])
+def test_depthmap_column_lengths(ctx, h, Ny, out):
+    """Every kind of column transform, a width that is no multiple of the
+    column group, an odd offset of the scene in its grid."""
+    print(f"case: depthmap 21x{h} grid 32x{Ny} {out}", flush=True)
+    img, dep = scenes.depth_scene(21, h, seed=14, colors=1)
+    u = ctx.depthmap(21, h, 32, Ny, 8e-6, 0.09, 0.11, 6, [532e-9], img, dep, out=out, quant_mode=1)
+    ref = _oracle_rgb(img, dep, 32, Ny, 8e-6, [532e-9], 0.09, 0.11, 6, out=out, quant_mode=1)
+    assert rel_l2(u, ref) < TOL

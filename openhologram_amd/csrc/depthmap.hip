@@ -384,6 +384,11 @@ __global__ __launch_bounds__(LX / 16) void dm_rows(DmArgs a, const float2* __res
 // 4096 x 2048 from 1782 to 763; held to 168 or 128 registers it spills
 // (1135, 1432 us).
 //
+// A scene in the middle half of the columns (HALF) loads half of the row and
+// spares the first butterfly's operations on zeros; rows of 4096 go through
+// line_r8_split4096 (together 1700 -> 1430 us at 4096 x 2048 encoded, 256
+// layers; shorter rows, of at most four waves, keep the stage order).
+//
 // MODE 0: equally spaced layers (no field lens).  The transfer of
 // layer l is H_l = exp(i 2 pi z_l Phi(kx, ky)) with one Phi for all layers,
 // so over a chunk of 16 consecutive layers starting at c,
@@ -452,14 +457,18 @@ __device__ __forceinline__ void lds_copy(E* dst, const E* __restrict__ src, int 
 }
 
 // lo .. hi: the layers taken (MODE 0: in chunks from lo).  part: the sums of
-// both rows are written there instead of being finished.
-template <int LX, int MODE, bool PAIR0, bool FBITS>
+// both rows are written there instead of being finished.  HALF: the scene's
+// columns are among the middle half of the grid's, so of a thread's eight
+// inputs the outer four are zeros.
+template <int LX, int MODE, bool PAIR0, bool FBITS, bool HALF>
 __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __restrict__ tw8, float2* sm, int kya,
                                             int lo, int hi, float2* part) {
     constexpr int TPL = LX / 8;
     constexpr int PL = fft::padded_len(LX);
     constexpr int CH = 16;
     constexpr int NTW = fft::table_len8(LX);
+    constexpr bool SPLIT = LX == 4096;
+    constexpr int M0 = HALF ? 2 : 0, M1 = HALF ? 6 : 8;
     float2* line = sm;
     float2* Sa = sm + PL;             // MODE 0: the chunk sums of both rows
     float2* Sb = Sa + LX;
@@ -482,10 +491,12 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
     const int syb = sgnidx(kyb, a.Ny) + 1;
     const size_t nyq = (size_t)(a.K - 1) * GROUP;
     const size_t gstride = (size_t)a.K * GROUP;
-    // Thread t owns row a at kx = t + m TPL and row b at kb = -kx mod LX:
+    // Thread t owns row a at kx = tk + m TPL (tk: as the transform leaves them) and row b at kb = -kx mod LX:
     // row b's transform at kb is conj Z(kx) of the thread's own element of
     // row a's transform Z, and the transfer depends on kx only through kx^2,
     // which is the same at kb, so one set of per-element factors serves both.
+    const int tk = SPLIT ? fft::split_k(t) : t;
+    const auto slot = [](int k) { return SPLIT ? (k & ~(TPL - 1)) + fft::split_slot(k & (TPL - 1)) : k; };
     float2 Ra[8], Rb[8];   // MODE 0
     float2 Ta[8], Tb[8];
 #pragma unroll
@@ -498,15 +509,14 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
         const float dKf = (float)a.dK;
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-            const int kx = t + m * TPL;
-            const int sx = sgnidx(kx, LX);
+            const int sx = sgnidx(tk + m * TPL, LX);
             const double sx2 = (double)sx * sx;
             double txd = a.dcx * sx2;
             txd -= rint(txd);
             const float usx = a.ux * (float)(sx * sx);
             Ra[m] = dm_transfer<false>(a, (float)txd, tya, usx, sya, a.dK, dKf, sx2);
             Rb[m] = dm_transfer<false>(a, (float)txd, tyb, usx, syb, a.dK, dKf, sx2);
-            Sa[kx] = Sb[(LX - kx) & (LX - 1)] = make_float2(0.f, 0.f);
+            Sa[t + m * TPL] = Sb[t + m * TPL] = make_float2(0.f, 0.f);   // at its owner's place
         }
     }
     const size_t lstride = gstride * a.ngroups;
@@ -534,7 +544,7 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
             const unsigned* fl = fb + (size_t)(l - 1) * a.fwpl;
             const auto rs = oph_buf_rsrc(a.I + (size_t)(l - 1) * lstride, (unsigned)(lstride * sizeof(float2)));
 #pragma unroll
-            for (int m = 0; m < 8; ++m) {
+            for (int m = M0; m < M1; ++m) {
                 const int x = t + m * TPL - a.ox;
                 const int gx = x >> 2;  // x / GROUP for x >= 0
                 const bool on = (x >= 0 && x < a.w) && ((fl[gx >> 5] >> (gx & 31)) & 1u);
@@ -552,7 +562,7 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
         const unsigned char* fl = a.flags + (size_t)(l - 1) * a.ngroups;
         nf = 0u;
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
+        for (int m = M0; m < M1; ++m) {
             const int x = t + m * TPL - a.ox;
             const bool in = x >= 0 && x < a.w;
             const size_t o = (size_t)(x / GROUP) * gstride + x % GROUP;
@@ -573,7 +583,7 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
         tyb -= rint(tyb);
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-            const int sx = sgnidx(t + m * TPL, LX);
+            const int sx = sgnidx(tk + m * TPL, LX);
             const double sx2 = (double)(sx * sx);
             double txd = cx * sx2;
             txd -= rint(txd);
@@ -608,21 +618,26 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
             // l is the prefetched layer
             float2 v[8], vb[8];   // vb: row b of PAIR0 (MODE != 0)
 #pragma unroll
-            for (int m = 0; m < 8; ++m) v[m] = ((nf >> m) & 1u) ? nv[m] : make_float2(0.f, 0.f);
+            for (int m = 0; m < 8; ++m)
+                v[m] = m >= M0 && m < M1 && ((nf >> m) & 1u) ? nv[m] : make_float2(0.f, 0.f);
             pl = next_layer(l);
             if (pl) fetch(pl);
-            __syncthreads();  // the previous transform's readers are done with the line
-            fft::line_r8_regs<LX, -1>(v, line, tws, t);
+            if constexpr (SPLIT) {
+                fft::line_r8_split4096<-1, HALF>(v, line, tws, t);
+            } else {
+                __syncthreads();  // the previous transform's readers are done with the line
+                fft::line_r8_regs<LX, -1, false, HALF>(v, line, tws, t);
+            }
             if constexpr (PAIR0) {
                 // A(kx) = (Z(kx) + conj Z(-kx))/2 for row 0 and, row Ny/2
                 // being real, B(-kx) = conj B(kx): exchange through the line
                 __syncthreads();
 #pragma unroll
-                for (int m = 0; m < 8; ++m) line[fft::pad16(t + m * TPL)] = v[m];
+                for (int m = 0; m < 8; ++m) line[fft::pad16(tk + m * TPL)] = v[m];
                 __syncthreads();
 #pragma unroll
                 for (int m = 0; m < 8; ++m) {
-                    const int kx = t + m * TPL;
+                    const int kx = tk + m * TPL;
                     const float2 gm = line[fft::pad16((LX - kx) & (LX - 1))];
                     float2 z = v[m], zc = make_float2(gm.x, -gm.y);
                     split_real_pair(z, zc);
@@ -654,66 +669,61 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
             tyb -= rint(tyb);
 #pragma unroll
             for (int m = 0; m < 8; ++m) {
-                const int kx = t + m * TPL;
-                const int sx = sgnidx(kx, LX);
+                const int sx = sgnidx(tk + m * TPL, LX), own = t + m * TPL;
                 const double sx2 = (double)sx * sx;
                 double txd = cx * sx2;
                 txd -= rint(txd);
                 const float usx = a.ux * (float)(sx * sx);
                 const float2 ha = dm_transfer<false>(a, (float)txd, tya, usx, sya, K, Kf, sx2);
-                Sa[kx] = fft::cadd(Sa[kx], fft::cmul(ha, Ta[m]));
+                Sa[own] = fft::cadd(Sa[own], fft::cmul(ha, Ta[m]));
                 const float2 hb = dm_transfer<false>(a, (float)txd, tyb, usx, syb, K, Kf, sx2);
-                const int kb = (LX - kx) & (LX - 1);
-                Sb[kb] = fft::cadd(Sb[kb], fft::cmul(hb, Tb[m]));
+                Sb[own] = fft::cadd(Sb[own], fft::cmul(hb, Tb[m]));
             }
         }
     }
-    __syncthreads();  // Sb entries were written by the threads owning -kx; the line is free
-    if constexpr (MODE != 0) {
-        if (part) {
-#pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                const int kx = t + m * TPL;
-                part[kx] = Ta[m];
-                part[LX + ((LX - kx) & (LX - 1))] = Tb[m];
-            }
-            return;
-        }
-#pragma unroll
-        for (int m = 0; m < 8; ++m) line[fft::pad16((LX - t - m * TPL) & (LX - 1))] = Tb[m];
+    // the rows in natural order: row a's sum at kx, row b's at -kx (MODE 0: the
+    // sums are already in LDS, at their owners' places)
+    if constexpr (MODE == 0) {
         __syncthreads();
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-            Tb[m] = fft::cmul(line[fft::pad16(t + m * TPL)], a.rho);
-            Ta[m] = fft::cmul(Ta[m], a.rho);
+            const int k = t + m * TPL;
+            Ta[m] = Sa[slot(k)];
+            Tb[m] = Sb[slot((LX - k) & (LX - 1))];
         }
-        __syncthreads();
-        finish_row8<LX>(a, Ta, kya, line, tws, t);
-        finish_row8<LX>(a, Tb, kyb, line, tws, t);
-        return;
+    } else {
+        const auto reorder = [&](float2 (&v)[8], int sg) {
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < 8; ++m) line[fft::pad16((sg * (tk + m * TPL)) & (LX - 1))] = v[m];
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < 8; ++m) v[m] = line[fft::pad16(t + m * TPL)];
+        };
+        if constexpr (SPLIT) reorder(Ta, 1);
+        reorder(Tb, -1);
     }
     if (part) {
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-            part[t + m * TPL] = Sa[t + m * TPL];
-            part[LX + t + m * TPL] = Sb[t + m * TPL];
+            part[t + m * TPL] = Ta[m];
+            part[LX + t + m * TPL] = Tb[m];
         }
         return;
     }
-    float2 acca[8], accb[8];
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
-        const int kx = t + m * TPL;
-        acca[m] = fft::cmul(Sa[kx], a.rho);
-        accb[m] = fft::cmul(Sb[kx], a.rho);
+        Ta[m] = fft::cmul(Ta[m], a.rho);
+        Tb[m] = fft::cmul(Tb[m], a.rho);
     }
-    finish_row8<LX>(a, acca, kya, line, tws, t);
-    finish_row8<LX>(a, accb, kyb, line, tws, t);
+    __syncthreads();
+    finish_row8<LX>(a, Ta, kya, line, tws, t);
+    finish_row8<LX>(a, Tb, kyb, line, tws, t);
 }
 
 // (two waves per SIMD: 256 registers, the budget of two 2048-point
 // workgroups per CU or one 4096-point workgroup)
-template <int LX, int MODE, bool FBITS>
+template <int LX, int MODE, bool FBITS, bool HALF>
 __global__ __launch_bounds__(LX / 8, 2) void dm_rows_h(DmArgs a, const float2* __restrict__ tw8) {
     extern __shared__ float2 sm[];
     // XCD-aware: neighbouring rows, which share the cache lines of I, run on
@@ -732,9 +742,9 @@ __global__ __launch_bounds__(LX / 8, 2) void dm_rows_h(DmArgs a, const float2* _
         kya = xcd_remap(blockIdx.x, a.n_main);  // 0 .. n_main - 1
     }
     if (kya == 0)
-        rows_h_body<LX, MODE, true, FBITS>(a, tw8, sm, 0, lo, hi, part);
+        rows_h_body<LX, MODE, true, FBITS, HALF>(a, tw8, sm, 0, lo, hi, part);
     else
-        rows_h_body<LX, MODE, false, FBITS>(a, tw8, sm, kya, lo, hi, part);
+        rows_h_body<LX, MODE, false, FBITS, HALF>(a, tw8, sm, kya, lo, hi, part);
 }
 
 // The pairs whose layers were split: their partial sums in order (the same
@@ -1245,7 +1255,9 @@ int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
     const size_t fbytes = (size_t)a.L * a.fwpl * sizeof(unsigned);
     const bool fbits = rows_h_lds<LX, MODE>() + fbytes <= 160 * 1024;
     const size_t shm = rows_h_lds<LX, MODE>() + (fbits ? fbytes : 0);
-    auto* kernel = fbits ? dm_rows_h<LX, MODE, true> : dm_rows_h<LX, MODE, false>;
+    auto* kernel = fbits ? dm_rows_h<LX, MODE, true, false> : dm_rows_h<LX, MODE, false, false>;
+    if constexpr (LX >= 512)
+        if (fbits && a.w <= LX / 2) kernel = dm_rows_h<LX, MODE, true, true>;   // then ox >= LX/4
     DmArgs b = a;
     const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 4, rows_resident(kernel, LX / 8, shm));
     if (rc) return rc;

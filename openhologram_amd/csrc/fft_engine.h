@@ -59,6 +59,15 @@ template <int SIGN>
 struct Dft<2, SIGN> {
     __device__ static void run(float2* v) { dft2<SIGN>(v[0], v[1]); }
 };
+// dft4 of (0, b, c, 0)
+template <int SIGN>
+__device__ __forceinline__ void dft4_mid(float2& a0, float2& a1, float2& a2, float2& a3) {
+    const float2 b = a1, c = a2, ib = mul_si<SIGN>(b);
+    a0 = cadd(c, b);
+    a2 = csub(c, b);
+    a1 = csub(ib, c);
+    a3 = make_float2(-c.x - ib.x, -c.y - ib.y);
+}
 // dft4 of v[N], v[N + 4], v[N + 8], v[N + 12], of which those outside LO .. HI - 1
 // are zeros (LO <= 4, HI >= 12: at most one of each pair two apart)
 template <int SIGN, int N, int LO, int HI>
@@ -78,11 +87,18 @@ struct Dft<4, SIGN> {
 };
 template <int SIGN>
 struct Dft<8, SIGN> {
+    // HALF: v[0], v[1], v[6], v[7] are zeros, which no operation is spent on
+    template <bool HALF = false>
     __device__ static void run(float2* v) {
         // radix 2 x 4: v[n], n = 4 n1 + n2?  use decimation: even/odd split
         constexpr float h = 0.70710678118654752f;
-        dft4<SIGN>(v[0], v[2], v[4], v[6]);
-        dft4<SIGN>(v[1], v[3], v[5], v[7]);
+        if constexpr (HALF) {
+            dft4_mid<SIGN>(v[0], v[2], v[4], v[6]);
+            dft4_mid<SIGN>(v[1], v[3], v[5], v[7]);
+        } else {
+            dft4<SIGN>(v[0], v[2], v[4], v[6]);
+            dft4<SIGN>(v[1], v[3], v[5], v[7]);
+        }
         // twiddle odd part by W8^k, k = 0..3 (W8 = exp(SIGN i 2pi/8))
         v[3] = make_float2(h * (v[3].x - SIGN * v[3].y), h * (v[3].y + SIGN * v[3].x));
         v[5] = mul_si<SIGN>(v[5]);
@@ -160,9 +176,22 @@ __host__ __device__ constexpr int padded_len(int L) { return L + L / 16; }
 // consecutive entries.  The tables of all stages of one length are
 // concatenated; stage 0 (Ns = 1) has none.
 
+// Orders a line's LDS accesses among the threads that transform it: a barrier
+// of the workgroup, or, if they are all of one wave (whose LDS accesses are
+// carried out in order), nothing but the order itself.
+template <bool WAVE>
+__device__ __forceinline__ void line_sync() {
+    if constexpr (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
 // One Stockham stage of radix R over a line in LDS (padded indexing), with the
 // stage's twiddles already in registers (w[p][r], r >= 1; unused for Ns = 1).
-template <int L, int R, int SIGN, int TPL>
+template <int L, int R, int SIGN, int TPL, bool WAVE = false>
 __device__ __forceinline__ void stage(float2* buf, const float2 (&w)[L / R / TPL][R], int Ns, int t) {
     constexpr int NB = L / R;
     constexpr int PER = NB / TPL;  // butterflies per thread (TPL divides NB)
@@ -181,7 +210,7 @@ __device__ __forceinline__ void stage(float2* buf, const float2 (&w)[L / R / TPL
             for (int r = 0; r < R; ++r) v[p][r] = buf[pad16(j + r * NB)];
         }
     }
-    __syncthreads();
+    line_sync<WAVE>();
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
         const int j = t + p * TPL;
@@ -207,7 +236,7 @@ __device__ __forceinline__ void stage(float2* buf, const float2 (&w)[L / R / TPL
             for (int r = 0; r < R; ++r) buf[pad16(base + r * Ns)] = v[p][r];
         }
     }
-    __syncthreads();
+    line_sync<WAVE>();
 }
 
 // Element i = t + m*TPL of a line, m = 0..15, padded: pad16(t) + m*(TPL + TPL/16)
@@ -546,26 +575,28 @@ __device__ __forceinline__ void line_r8(float2* buf, const float2* __restrict__ 
 // stay in v; otherwise the last stage goes through the line and v is read
 // back.  The caller syncs before the line is written again (other threads
 // may still read the last stage's inputs).
-template <int L, int SIGN>
+// WAVE: all of the line's threads are of one wave.  HALF: v[0], v[1], v[6],
+// v[7] are zeros on entry.
+template <int L, int SIGN, bool WAVE = false, bool HALF = false>
 __device__ __forceinline__ void line_r8_regs(float2 (&v)[8], float2* buf, const float2* __restrict__ tw, int t) {
     static_assert(L >= 64, "at least two radix-8 stages");
     constexpr int TPL = L / 8;
     constexpr int A = n8(L);
     constexpr int RL = last_radix8(L);
-    Dft<8, SIGN>::run(v);
+    Dft<8, SIGN>::template run<HALF>(v);
     {
         float2* dst = buf + pad16(8 * t);
 #pragma unroll
         for (int r = 0; r < 8; ++r) dst[r] = v[r];
     }
-    __syncthreads();
+    line_sync<WAVE>();
     int Ns = 8, off = 0;
     constexpr int NMID = RL == 1 ? A - 2 : A - 1;
 #pragma unroll
     for (int s = 0; s < NMID; ++s) {
         float2 w[1][8];
         load_stage_tw<L, 8, TPL>(tw, off, Ns, t, w);
-        stage<L, 8, SIGN, TPL>(buf, w, Ns, t);
+        stage<L, 8, SIGN, TPL, WAVE>(buf, w, Ns, t);
         off += 7 * Ns;
         Ns *= 8;
     }
@@ -581,10 +612,42 @@ __device__ __forceinline__ void line_r8_regs(float2 (&v)[8], float2* buf, const 
     } else {
         float2 w[L / RL / TPL][RL];
         load_stage_tw<L, RL, TPL>(tw, off, Ns, t, w);
-        stage<L, RL, SIGN, TPL>(buf, w, Ns, t);
+        stage<L, RL, SIGN, TPL, WAVE>(buf, w, Ns, t);
 #pragma unroll
         for (int m = 0; m < 8; ++m) v[m] = buf[pad16(t + m * TPL)];
     }
+}
+
+// line_r8_regs for L = 4096 (512 threads, eight waves), decimated in frequency
+// first: one radix-8 butterfly of the whole line, whose output r is the input
+// of a 512-point transform that wave r does by itself, with no barrier of the
+// workgroup in it.  Two barriers a line, against six where every stage's
+// exchange crosses the waves.  On entry v[m] is input element t + m 512, on
+// return output element split_k(t) + m 512.  tw is the radix-8 table of 4096
+// points (its last stage holds the first butterfly's twiddles, what is before
+// it the 512-point table).  The first barrier orders the line's writes after
+// the previous transform's reads.
+__device__ __forceinline__ int split_k(int t) { return 8 * (t & 63) + (t >> 6); }
+__device__ __forceinline__ int split_slot(int k) { return (k & 7) * 64 + (k >> 3); }   // inverse of split_k
+template <int SIGN, bool HALF>
+__device__ __forceinline__ void line_r8_split4096(float2 (&v)[8], float2* buf, const float2* __restrict__ tw, int t) {
+    constexpr int M = 512, PM = padded_len(M);
+    Dft<8, SIGN>::template run<HALF>(v);
+#pragma unroll
+    for (int r = 1; r < 8; ++r) {
+        const float2 w = tw[table_len8(M) + (r - 1) * M + t];
+        v[r] = SIGN < 0 ? cmul(v[r], w) : cmulc(v[r], w);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 8; ++r) buf[r * PM + pad16(t)] = v[r];
+    __syncthreads();
+    float2* sub = buf + (t >> 6) * PM;
+    const int q = t & 63;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) v[m] = sub[pad16(q + m * 64)];
+    line_sync<true>();
+    line_r8_regs<M, SIGN, true>(v, sub, tw, q);
 }
 
 // Convenience: load the twiddles and transform.

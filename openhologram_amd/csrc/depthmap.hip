@@ -125,13 +125,48 @@ __device__ __forceinline__ float pixel_value(unsigned img) {
     return (float)img * (1.f / 255.f);
 }
 
+// The pixels (idx << 16 | img) of rows t + m ST of columns x and x + 1, M0 <= m
+// < M1, and the layers they are in; 0 for a pixel that contributes nothing
+// (alpha = [img > 0], CPU.cpp:61; a layer outside lo .. hi; no pixel).  Range-
+// checked loads, all requested before the first is used.
+template <int M0, int M1, int ST, int N>
+__device__ __forceinline__ void load_pixels(const DmArgs& a, int x, int t, unsigned* mask, unsigned (&pa)[N],
+                                            unsigned (&pb)[N]) {
+    const unsigned npx = (unsigned)a.w * (unsigned)a.h;
+    const auto ri = oph_buf_rsrc(a.img, npx), rd = oph_buf_rsrc(a.idx, npx * 2u);
+    unsigned char im[2][N];
+    unsigned short id[2][N];
+#pragma unroll
+    for (int m = M0; m < M1; ++m) {
+        const int r = t + m * ST - a.oy;
+        const bool in = r >= 0 && r < a.h;
+        const unsigned o = (unsigned)r * (unsigned)a.w + (unsigned)x;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const bool ok = in && x + c < a.w;
+            im[c][m] = __builtin_amdgcn_raw_buffer_load_b8(ri, ok ? o + c : OPH_BUF_OOB, 0, 0);
+            id[c][m] = __builtin_amdgcn_raw_buffer_load_b16(rd, ok ? 2u * (o + c) : OPH_BUF_OOB, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int m = M0; m < M1; ++m)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const unsigned d = id[c][m], i = im[c][m];
+            const bool on = i > 0u && d >= (unsigned)a.lo && d <= (unsigned)a.hi;
+            if (on) atomicOr(&mask[d >> 5], 1u << (d & 31));
+            (c ? pb : pa)[m] = on ? d << 16 | i : 0u;
+        }
+}
+
 // A thread owns 16 rows of a column pair (x0 + 2p, x0 + 2p + 1; neighbouring
 // threads take the two pairs): their pixels stay in registers over all of the
 // layers, a layer's values go straight into the transform's first radix-16
 // stage, and the result is separated from registers -- only the mirrored
 // rows that the stored ones need pass through LDS.  Bound by vector
-// instructions and LDS; 1920 x 1080 on 2048 rows, 256 layers: 690 us, against
-// 921 with pixels, input and output of the transform in LDS.
+// instructions and LDS; 1920 x 1080 on 2048 rows, 256 layers: 442 us a colour,
+// against 921 with pixels, input and output of the transform in LDS and runs
+// of layers instead of every chunks-th.
 template <int LY>
 __host__ __device__ constexpr bool cols_shared() { return LY > 4096; }   // the mirrored rows in the line itself
 template <int LY>
@@ -141,7 +176,7 @@ __host__ __device__ constexpr int cols_mirror_stride(int K) { return cols_shared
 // 3); its row Ny/2 is of no pair that is kept and stays zero.  MID: the scene's
 // rows are among the middle ten sixteenths of the grid's.
 template <int LY, bool HALF, bool MID>
-__global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int layers_per_wg,
+__global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int chunks,
                                                          const float2* __restrict__ twy) {
     constexpr int TPL = LY / 16;
     constexpr int NT = 2 * TPL;
@@ -159,41 +194,18 @@ __global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int layers_pe
     // cache lines of I) run on the same XCD at the same time
     const int lin = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int g = lin % gridDim.x;
-    const int l_begin = a.lo + lin / gridDim.x * layers_per_wg;
-    const int l_end = min(a.hi, l_begin + layers_per_wg - 1);
+    const int chunk = lin / gridDim.x;   // layers lo + chunk, then every chunks-th
     const int nwords = (a.L + 32) / 32;
     for (int i = threadIdx.x; i < nwords; i += NT) mask[i] = 0u;
     __syncthreads();
     unsigned pa[16], pb[16];   // idx << 16 | img; 0: no contribution
-    {
-        const int x = g * GROUP + 2 * p;
-#pragma unroll
-        for (int m = M0; m < M1; ++m) {
-            const int r = t + m * TPL - a.oy;
-            unsigned v[2] = {0u, 0u};
-            if (r >= 0 && r < a.h)
-#pragma unroll
-                for (int c = 0; c < 2; ++c)
-                    if (x + c < a.w) {
-                        const size_t o = (size_t)r * a.w + x + c;
-                        const unsigned im = a.img[o];
-                        const unsigned id = a.idx[o];
-                        // alpha = [img > 0] (CPU.cpp:61): a zero pixel contributes nothing
-                        if (im > 0u && id >= (unsigned)l_begin && id <= (unsigned)l_end) {
-                            v[c] = (id << 16) | im;
-                            atomicOr(&mask[id >> 5], 1u << (id & 31));
-                        }
-                    }
-            pa[m] = v[0];
-            pb[m] = v[1];
-        }
-    }
+    load_pixels<M0, M1, TPL>(a, g * GROUP + 2 * p, t, mask, pa, pb);
     fft::Twiddles<LY> Tw;   // (8192: too many registers with 1024 threads)
     if constexpr (!SHARED) Tw.load(twy, t);
     __syncthreads();
     const size_t gstride = (size_t)a.K * GROUP;
     const size_t lstride = gstride * a.ngroups;
-    for (int l = l_begin; l <= l_end; ++l) {
+    for (int l = a.lo + chunk; l <= a.hi; l += chunks) {
         if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
         // the two real columns as one complex column
         float2 v[16];
@@ -846,57 +858,37 @@ bool dm_mixed_length(int n) {
 }
 
 template <int LY>
-__global__ __launch_bounds__(2 * fftm::threads(LY)) void dm_cols_m(DmArgs a, int layers_per_wg,
+__global__ __launch_bounds__(2 * fftm::threads(LY)) void dm_cols_m(DmArgs a, int chunks,
                                                                  const float2* __restrict__ twy) {
     constexpr int NT = fftm::threads(LY);
     constexpr int EPT = fftm::ept(LY);
     constexpr int PL = fftm::padded_len(LY);
     extern __shared__ unsigned char smem[];
     float2* lines = reinterpret_cast<float2*>(smem);                 // 2 x PL
-    unsigned* pix = reinterpret_cast<unsigned*>(lines + 2 * PL);     // h x GROUP: idx << 8 | img
-    unsigned* mask = pix + (size_t)a.h * GROUP;                      // layer bitmask
+    unsigned* mask = reinterpret_cast<unsigned*>(lines + 2 * PL);    // layer bitmask
     const int lin = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int g = lin % gridDim.x;
     const int x0 = g * GROUP;
-    const int l_begin = a.lo + lin / gridDim.x * layers_per_wg;
-    const int l_end = min(a.hi, l_begin + layers_per_wg - 1);
+    const int chunk = lin / gridDim.x;   // layers lo + chunk, then every chunks-th
     const int nwords = (a.L + 32) / 32;
     const int p = threadIdx.x / NT, t = threadIdx.x % NT;
     float2* line = lines + p * PL;
     for (int i = threadIdx.x; i < nwords; i += 2 * NT) mask[i] = 0u;
     __syncthreads();
-    for (int e = threadIdx.x; e < a.h * GROUP; e += 2 * NT) {
-        const int c = e % GROUP, r = e / GROUP;
-        const int x = x0 + c;
-        unsigned v = 0u;
-        if (x < a.w) {
-            const size_t o = (size_t)r * a.w + x;
-            const unsigned im = a.img[o];
-            const unsigned id = a.idx[o];
-            if (im > 0u && id >= (unsigned)l_begin && id <= (unsigned)l_end) {
-                v = (id << 8) | im;
-                atomicOr(&mask[id >> 5], 1u << (id & 31));
-            }
-        }
-        pix[e] = v;
-    }
+    unsigned pa[EPT], pb[EPT];   // (rows from LY on are beyond the scene: zeros)
+    load_pixels<0, EPT, NT>(a, x0 + 2 * p, t, mask, pa, pb);
     __syncthreads();
     const size_t gstride = (size_t)a.K * GROUP;
     const size_t lstride = gstride * a.ngroups;
-    for (int l = l_begin; l <= l_end; ++l) {
+    for (int l = a.lo + chunk; l <= a.hi; l += chunks) {
         if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
             const int i = t + m * NT;
             if (EPT * NT == LY || i < LY) {
-                const int r = i - a.oy;
-                float2 v = make_float2(0.f, 0.f);
-                if (r >= 0 && r < a.h) {
-                    const unsigned wa = pix[r * GROUP + 2 * p], wb = pix[r * GROUP + 2 * p + 1];
-                    if ((int)(wa >> 8) == l) v.x = (float)(wa & 255u) * (1.f / 255.f);
-                    if ((int)(wb >> 8) == l) v.y = (float)(wb & 255u) * (1.f / 255.f);
-                }
-                line[fft::pad16(i)] = v;
+                const unsigned wa = pa[m] >> 16 == (unsigned)l ? pa[m] : 0u;
+                const unsigned wb = pb[m] >> 16 == (unsigned)l ? pb[m] : 0u;
+                line[fft::pad16(i)] = make_float2(pixel_value(wa & 255u), pixel_value(wb & 255u));
             }
         }
         __syncthreads();
@@ -1173,11 +1165,10 @@ __global__ __launch_bounds__(B * fftm::threads(LY)) void dm_final_m(DmArgs a, co
 // ---- launchers -------------------------------------------------------------------
 
 template <int LY>
-int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
+int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks) {
     const float2* tw = oph_twiddles(ctx, LY);
     if (!tw) return OPH_ENOMEM;
     const size_t words = (size_t)((a.L + 32) / 32) * 4;
-    // (the limit on the scene's height is the general lengths' too)
     if (2 * fft::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 + words > 160 * 1024)
         return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
     const size_t shm = 2 * ((size_t)fft::skewed_len(LY, 2) + cols_mirror_stride<LY>(a.K)) * sizeof(float2) + words;
@@ -1185,7 +1176,7 @@ int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                             160 * 1024);
         hipGetLastError();
-        OPH_LAUNCH(ctx, "dm_cols", kernel, dim3(a.ngroups, chunks), dim3(2 * (LY / 16)), shm, a, lpw, tw);
+        OPH_LAUNCH(ctx, "dm_cols", kernel, dim3(a.ngroups, chunks), dim3(2 * (LY / 16)), shm, a, chunks, tw);
         return OPH_OK;
     };
     if constexpr (LY >= 512) {
@@ -1302,17 +1293,15 @@ int launch_dm_final(oph_ctx* ctx, const DmArgs& a) {
 }
 
 template <int LY>
-int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
+int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks) {
     const float2* tw = oph_twiddles_mixed(ctx, LY);
     if (!tw) return OPH_ENOMEM;
     if constexpr (2 * (size_t)fftm::padded_len(LY) * sizeof(float2) > 150 * 1024) {
         (void)chunks;
-        (void)lpw;
         return oph_fail(ctx, OPH_ENOTSUP, "grid height %d too large for the column pass", LY);
     } else {
-        const size_t shm = 2 * (size_t)fftm::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 +
-                           (size_t)((a.L + 32) / 32) * 4;
-        if (shm > 160 * 1024)
+        const size_t shm = 2 * (size_t)fftm::padded_len(LY) * sizeof(float2) + (size_t)((a.L + 32) / 32) * 4;
+        if (shm + (size_t)a.h * GROUP * 4 > 160 * 1024)   // (as the power-of-two lengths)
             return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
         static bool attr = false;
         if (!attr) {
@@ -1322,7 +1311,7 @@ int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks, int lpw) {
             attr = true;
         }
         OPH_LAUNCH(ctx, "dm_cols", dm_cols_m<LY>, dim3(a.ngroups, chunks), dim3(2 * fftm::threads(LY)), shm, a,
-                   lpw, tw);
+                   chunks, tw);
         return OPH_OK;
     }
 }
@@ -1568,14 +1557,20 @@ extern "C" int oph_depthmap(oph_ctx* ctx, const oph_dm_spec* s, int ncolor, cons
         const int nfl = (int)nfl_bytes;   // flags, any and the flag bits
         OPH_LAUNCH(ctx, "dm_zero", dm_zero, dim3((nfl + 255) / 256), dim3(256), 0, dflags, nfl);
         const int nl = hi - lo + 1;
-        int chunks = (int)((4LL * ctx->cu_count + ngroups - 1) / ngroups);
+        // column workgroups: four a CU, eight where each still has 16 layers to
+        // spread its loading of the pixels over (2048 rows, 480 column groups:
+        // 256 layers in 3 parts 466 us, in 5 442; 256 groups, 16 layers in 4
+        // parts 49 us, in 8 78).  A part takes every chunks-th layer, which
+        // evens out the layers that a column group has pixels in (in runs of
+        // 86 layers: 690 us).
+        const int groups4 = (int)((4LL * ctx->cu_count + ngroups - 1) / ngroups);
+        const int groups8 = (int)((8LL * ctx->cu_count + ngroups - 1) / ngroups);
+        int chunks = std::max(groups4, std::min(groups8, nl / 16));
         if (chunks > nl) chunks = nl;
         if (chunks < 1) chunks = 1;
-        const int lpw = (nl + chunks - 1) / chunks;
-        chunks = (nl + lpw - 1) / lpw;
         if (mixed) {
             switch (Ny) {
-#define OPH_DMC(n) case n: rc = launch_dm_cols_m<n>(ctx, a, chunks, lpw); break;
+#define OPH_DMC(n) case n: rc = launch_dm_cols_m<n>(ctx, a, chunks); break;
                 OPH_DM_MIXED_LENGTHS(OPH_DMC)
 #undef OPH_DMC
             }
@@ -1595,7 +1590,7 @@ extern "C" int oph_depthmap(oph_ctx* ctx, const oph_dm_spec* s, int ncolor, cons
             continue;
         }
         switch (Ny) {
-#define OPH_DMC(n) case n: rc = launch_dm_cols<n>(ctx, a, chunks, lpw); break;
+#define OPH_DMC(n) case n: rc = launch_dm_cols<n>(ctx, a, chunks); break;
             OPH_FFT_LENGTHS(OPH_DMC)
 #undef OPH_DMC
         }

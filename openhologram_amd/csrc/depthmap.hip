@@ -125,12 +125,12 @@ __device__ __forceinline__ float pixel_value(unsigned img) {
     return (float)img * (1.f / 255.f);
 }
 
-// The pixels (idx << 16 | img) of rows t + m ST of columns x and x + 1, M0 <= m
-// < M1, and the layers they are in; 0 for a pixel that contributes nothing
+// The pixels (idx << 16 | img) of grid rows row(m), M0 <= m < M1, of columns x
+// and x + 1, and the layers they are in; 0 for a pixel that contributes nothing
 // (alpha = [img > 0], CPU.cpp:61; a layer outside lo .. hi; no pixel).  Range-
 // checked loads, all requested before the first is used.
-template <int M0, int M1, int ST, int N>
-__device__ __forceinline__ void load_pixels(const DmArgs& a, int x, int t, unsigned* mask, unsigned (&pa)[N],
+template <int M0, int M1, int N, typename Row>
+__device__ __forceinline__ void load_pixels(const DmArgs& a, int x, Row&& row, unsigned* mask, unsigned (&pa)[N],
                                             unsigned (&pb)[N]) {
     const unsigned npx = (unsigned)a.w * (unsigned)a.h;
     const auto ri = oph_buf_rsrc(a.img, npx), rd = oph_buf_rsrc(a.idx, npx * 2u);
@@ -138,7 +138,7 @@ __device__ __forceinline__ void load_pixels(const DmArgs& a, int x, int t, unsig
     unsigned short id[2][N];
 #pragma unroll
     for (int m = M0; m < M1; ++m) {
-        const int r = t + m * ST - a.oy;
+        const int r = row(m) - a.oy;
         const bool in = r >= 0 && r < a.h;
         const unsigned o = (unsigned)r * (unsigned)a.w + (unsigned)x;
 #pragma unroll
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(2 * (LY / 16)) void dm_cols(DmArgs a, int chunks,
     for (int i = threadIdx.x; i < nwords; i += NT) mask[i] = 0u;
     __syncthreads();
     unsigned pa[16], pb[16];   // idx << 16 | img; 0: no contribution
-    load_pixels<M0, M1, TPL>(a, g * GROUP + 2 * p, t, mask, pa, pb);
+    load_pixels<M0, M1>(a, g * GROUP + 2 * p, [&](int m) { return t + m * TPL; }, mask, pa, pb);
     fft::Twiddles<LY> Tw;   // (8192: too many registers with 1024 threads)
     if constexpr (!SHARED) Tw.load(twy, t);
     __syncthreads();
@@ -840,8 +840,8 @@ __global__ __launch_bounds__(B * (LY / 16)) void dm_final(DmArgs a, const float2
 // The same three passes for grids whose sides are 2^a 3^b 5^c but not powers
 // of two (the shipped 11520 x 2160 configuration, HD scenes transformed
 // unpadded): mixed-radix line transforms (fft_mixed.h) by NT =
-// fftm::threads(N) threads per line, thread t owning elements t + m NT
-// (m < fftm::ept(N)), index arithmetic mod N (N even: the fftshifts are
+// fftm::threads(N) threads per line, in natural order thread t owning elements
+// t + m NT (m < fftm::ept(N)), index arithmetic mod N (N even: the fftshifts are
 // still the (-1)^k factors above).  No chunked recurrence: every layer's
 // transfer is evaluated (dm_transfer).
 
@@ -857,63 +857,86 @@ bool dm_mixed_length(int n) {
     }
 }
 
+// As dm_cols: pixels, a layer's values and its transform's result in registers
+// (1080 rows, 1920 columns, 256 layers: 595 -> 390 us with 12 x 10 x 9 in place
+// of 8 x 5 x 3 x 3 x 3).
+template <int LY>
+__host__ __device__ constexpr int cols_m_line() {   // lines 16 float2 apart modulo all banks
+    return (fftm::padded_len(LY) + 31) / 32 * 32 + 16;
+}
+
 template <int LY>
 __global__ __launch_bounds__(2 * fftm::threads(LY)) void dm_cols_m(DmArgs a, int chunks,
                                                                  const float2* __restrict__ twy) {
-    constexpr int NT = fftm::threads(LY);
-    constexpr int EPT = fftm::ept(LY);
-    constexpr int PL = fftm::padded_len(LY);
+    using E = fftm::Ends<LY>;
+    constexpr int NT = E::NT;
     extern __shared__ unsigned char smem[];
-    float2* lines = reinterpret_cast<float2*>(smem);                 // 2 x PL
-    unsigned* mask = reinterpret_cast<unsigned*>(lines + 2 * PL);    // layer bitmask
+    const int p = threadIdx.x & 1, t = threadIdx.x >> 1;
+    float2* line = reinterpret_cast<float2*>(smem) + p * cols_m_line<LY>();
+    const int ms = cols_mirror_stride<0>(a.K);
+    float2* mirrors = reinterpret_cast<float2*>(smem) + 2 * cols_m_line<LY>();
+    float2* mirror = mirrors + p * ms;                               // Z(-k) at k = 1 .. K - 2
+    unsigned* mask = reinterpret_cast<unsigned*>(mirrors + 2 * ms);  // layer bitmask
     const int lin = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int g = lin % gridDim.x;
-    const int x0 = g * GROUP;
     const int chunk = lin / gridDim.x;   // layers lo + chunk, then every chunks-th
     const int nwords = (a.L + 32) / 32;
-    const int p = threadIdx.x / NT, t = threadIdx.x % NT;
-    float2* line = lines + p * PL;
     for (int i = threadIdx.x; i < nwords; i += 2 * NT) mask[i] = 0u;
     __syncthreads();
-    unsigned pa[EPT], pb[EPT];   // (rows from LY on are beyond the scene: zeros)
-    load_pixels<0, EPT, NT>(a, x0 + 2 * p, t, mask, pa, pb);
+    unsigned pa[E::PER0 * E::R0], pb[E::PER0 * E::R0];
+    load_pixels<0, E::PER0 * E::R0>(
+        a, g * GROUP + 2 * p,
+        [&](int m) {
+            const int jj = t + m / E::R0 * NT;
+            return jj < E::NB0 ? jj + m % E::R0 * E::NB0 : -1;   // (-1: no row)
+        },
+        mask, pa, pb);
     __syncthreads();
     const size_t gstride = (size_t)a.K * GROUP;
     const size_t lstride = gstride * a.ngroups;
     for (int l = a.lo + chunk; l <= a.hi; l += chunks) {
         if (!((mask[l >> 5] >> (l & 31)) & 1u)) continue;
+        // the thread index through a zero the compiler cannot see through:
+        // the transforms' LDS addresses are then formed per layer instead of
+        // being hoisted out of the loop into ~100 registers
+        int zero;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+        const int tl = t + zero;
+        float2 vi[E::PER0][E::R0], v[E::PERL][E::RL];
 #pragma unroll
-        for (int m = 0; m < EPT; ++m) {
-            const int i = t + m * NT;
-            if (EPT * NT == LY || i < LY) {
-                const unsigned wa = pa[m] >> 16 == (unsigned)l ? pa[m] : 0u;
-                const unsigned wb = pb[m] >> 16 == (unsigned)l ? pb[m] : 0u;
-                line[fft::pad16(i)] = make_float2(pixel_value(wa & 255u), pixel_value(wb & 255u));
+        for (int m = 0; m < E::PER0 * E::R0; ++m) {
+            const unsigned wa = pa[m] >> 16 == (unsigned)l ? pa[m] : 0u;
+            const unsigned wb = pb[m] >> 16 == (unsigned)l ? pb[m] : 0u;
+            vi[m / E::R0][m % E::R0] = make_float2(pixel_value(wa & 255u), pixel_value(wb & 255u));
+        }
+        fftm::line_ends<LY, -1>(vi, v, line, twy, tl);
+#pragma unroll
+        for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+            for (int r = 0; r < E::RL; ++r) {
+                const int j = tl + q * NT, k = LY - (j + r * E::NBL);
+                if ((E::PERL * NT == E::NBL || j < E::NBL) && k < a.K - 1) mirror[k] = v[q][r];
             }
-        }
         __syncthreads();
-        fftm::line<LY, NT, -1>(line, twy, t);
-        float2* dst = a.I + (size_t)(l - 1) * lstride + (size_t)g * gstride;
-        for (int e = threadIdx.x; e < a.K * GROUP; e += 2 * NT) {
-            const int c = e % GROUP, ky = e / GROUP < a.K - 1 ? e / GROUP : LY / 2;
-            const int x = x0 + c;
-            if (x >= a.w) continue;
-            const float2* ln = lines + (c >> 1) * PL;
-            const float2 Z = ln[fft::pad16(ky)];
-            const float2 Zm = ln[fft::pad16(ky == 0 ? 0 : LY - ky)];
-            float2 v;
-            if ((c & 1) == 0)
-                v = make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
-            else
-                v = make_float2(0.5f * (Z.y + Zm.y), -0.5f * (Z.x - Zm.x));
-            dst[e] = v;
-        }
+        // separate: A(k) = (Z(k) + conj Z(-k))/2, B(k) = (Z(k) - conj Z(-k))/(2i)
+        float2* dst = a.I + (size_t)(l - 1) * lstride + (size_t)g * gstride + 2 * p;
+#pragma unroll
+        for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+            for (int r = 0; r < E::RL; ++r) {
+                const int j = tl + q * NT, k = j + r * E::NBL;
+                const bool nyq = k == LY / 2;
+                if ((E::PERL * NT == E::NBL || j < E::NBL) && (k < a.K - 1 || nyq)) {
+                    const float2 z = v[q][r], zm = k == 0 || nyq ? z : mirror[k];
+                    *reinterpret_cast<float4*>(dst + (size_t)(nyq ? a.K - 1 : k) * GROUP) =
+                        make_float4(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y), 0.5f * (z.y + zm.y), 0.5f * (zm.x - z.x));
+                }
+            }
         if (threadIdx.x == 0) {
             a.flags[(size_t)(l - 1) * a.ngroups + g] = 1;
             a.any[l - 1] = 1;
             atomicOr(&a.fbits[(size_t)(l - 1) * a.fwpl + (g >> 5)], 1u << (g & 31));
         }
-        __syncthreads();
     }
 }
 
@@ -947,13 +970,18 @@ __device__ __forceinline__ void finish_row_m(const DmArgs& a, const float2 (&acc
     __syncthreads();
 }
 
-// Bound by vector instructions once enough waves are resident: one workgroup
-// a pair leaves 272 two-wave workgroups for 256 CUs at 1920 x 1080 encoded
-// (2483 us, 256 layers), the layers split into 7 parts 795 us; holding it to
-// 168 or 128 registers for more waves spills (1010 and 1456 us).
+// Bound by vector instructions and the waits between a layer's stages.  1920 x
+// 1080 encoded, 256 layers (272 pairs, of which one workgroup each fills two
+// waves a CU: 2483 us): the layers split into 7 parts 795 us; the transform's
+// ends in registers, 16 x 15 x 8 in place of 16 x 8 x 5 x 3, row b from the
+// thread's own elements and the next layer's row requested before the
+// transform 640 us.  Held to 168 or 128 registers it spills (1010, 1456 us).
 template <int LX, bool EXACT>
 __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const float2* __restrict__ twx) {
-    constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
+    using E = fftm::Ends<LX>;
+    constexpr int NT = E::NT, EPT = fftm::ept(LX);
+    constexpr int N0 = E::PER0 * E::R0;
+    constexpr bool PREF = N0 <= 16;   // the next layer's values fit in registers
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
     const int t = threadIdx.x;
     // XCD-aware, as dm_rows_h
@@ -975,130 +1003,162 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
     const int syb = sgnidx(kyb, a.Ny) + 1;
     const size_t nyq = (size_t)(a.K - 1) * GROUP;
     const size_t gstride = (size_t)a.K * GROUP;
-    // (the per-element x factors are recomputed per layer: the two rows'
-    // accumulators already take most of the registers of a 768-thread line)
-    float2 acca[EPT], accb[EPT];
-#pragma unroll
-    for (int m = 0; m < EPT; ++m) acca[m] = accb[m] = make_float2(0.f, 0.f);
     const size_t lstride = gstride * a.ngroups;
-    // a layer's slice of I addressed by 32-bit buffer offsets when it is
-    // below 2 GiB (else plain loads with a branch per element)
-    const bool bufs = lstride * sizeof(float2) < ((size_t)1 << 31);
-    for (int l = lo; l <= hi; ++l) {
-        if (!a.any[l - 1]) continue;
+    // Row a's sum at the transform's outputs kx = (t + q NT) + r NBL and row b's
+    // at -kx, whose transform is conj Z(kx) and whose kx^2 is the same (as
+    // dm_rows_h)
+    float2 acca[E::PERL][E::RL], accb[E::PERL][E::RL];
+#pragma unroll
+    for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+        for (int r = 0; r < E::RL; ++r) acca[q][r] = accb[q][r] = make_float2(0.f, 0.f);
+    const auto next_layer = [&](int l) {
+        while (l <= hi && !a.any[l - 1]) ++l;
+        return l;
+    };
+    // Input element m of layer l: range-checked buffer loads, first the presence
+    // flag of its column group, then the value, whose offset is out of range (a
+    // zero, no memory access) for absent groups and columns outside the image.
+    const auto column = [&](int m, int tl) {
+        const int j = tl + m / E::R0 * NT, x = j + m % E::R0 * E::NB0 - a.ox;
+        return j < E::NB0 && x >= 0 && x < a.w ? x : -1;
+    };
+    const auto load_flags = [&](int l, int tl, unsigned char (&f)[N0]) {
+        const auto rf = oph_buf_rsrc(a.flags + (size_t)(l - 1) * a.ngroups, (unsigned)a.ngroups);
+#pragma unroll
+        for (int m = 0; m < N0; ++m) {
+            const int x = column(m, tl);
+            f[m] = __builtin_amdgcn_raw_buffer_load_b8(rf, x >= 0 ? (unsigned)(x / GROUP) : OPH_BUF_OOB, 0, 0);
+        }
+    };
+    const auto load_values = [&](int l, int tl, const unsigned char (&f)[N0], float2 (&v)[E::PER0][E::R0]) {
+        const auto ri = oph_buf_rsrc(a.I + (size_t)(l - 1) * lstride, (unsigned)(lstride * sizeof(float2)));
+#pragma unroll
+        for (int m = 0; m < N0; ++m) {
+            const int x = column(m, tl);
+            const unsigned o = x >= 0 && f[m] ? (unsigned)(((size_t)(x / GROUP) * gstride + x % GROUP +
+                                                            (size_t)kya * GROUP) * sizeof(float2))
+                                              : OPH_BUF_OOB;
+            v[m / E::R0][m % E::R0] = oph_buf_load_f2(ri, o);
+            if (pair0)   // (workgroup 0 only)
+                v[m / E::R0][m % E::R0].y = oph_buf_load_f2(ri, o == OPH_BUF_OOB ? o : o + (unsigned)(nyq * sizeof(float2))).x;
+        }
+    };
+    // The values of the next present layer are requested before this layer's
+    // transform, the flags of the one after it after them (PREF)
+    unsigned char f[N0];
+    float2 vi[E::PER0][E::R0], nv[E::PER0][E::R0];
+    int l = next_layer(lo), ln = l <= hi ? next_layer(l + 1) : hi + 1;
+    if (PREF && l <= hi) {
+        load_flags(l, t, f);
+        load_values(l, t, f, nv);
+        if (ln <= hi) load_flags(ln, t, f);
+    }
+    while (l <= hi) {
         // the thread index through a zero the compiler cannot see through:
         // the transforms' LDS addresses are then formed per layer instead of
         // being hoisted out of the loop into ~100 registers
         int zero;
         asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
         const int tl = t + zero;
-        if (bufs) {
-            // range-checked buffer loads, eight elements at a time: the
-            // presence flags of their column groups, then the values, whose
-            // offset is out of range (a zero, no memory access) for absent
-            // groups and columns outside the image -- each batch is
-            // requested before any of it is used, with no branch per element
-            const auto rf = oph_buf_rsrc(a.flags + (size_t)(l - 1) * a.ngroups, (unsigned)a.ngroups);
-            const auto ri = oph_buf_rsrc(a.I + (size_t)(l - 1) * lstride, (unsigned)(lstride * sizeof(float2)));
-            constexpr int CHB = 8;
+        if constexpr (PREF) {
 #pragma unroll
-            for (int m0 = 0; m0 < EPT; m0 += CHB) {
-                unsigned char f[CHB];
-                unsigned o[CHB];
-#pragma unroll
-                for (int j = 0; j < CHB; ++j) {
-                    const int kx = tl + (m0 + j) * NT;
-                    const int x = kx - a.ox;
-                    const bool in = m0 + j < EPT && (EPT * NT == LX || kx < LX) && x >= 0 && x < a.w;
-                    f[j] = __builtin_amdgcn_raw_buffer_load_b8(rf, in ? (unsigned)(x / GROUP) : OPH_BUF_OOB, 0, 0);
-                    o[j] = in ? (unsigned)(((size_t)(x / GROUP) * gstride + x % GROUP + (size_t)kya * GROUP) *
-                                           sizeof(float2))
-                              : OPH_BUF_OOB;
-                }
-                float2 v[CHB];
-                float vy[CHB];
-#pragma unroll
-                for (int j = 0; j < CHB; ++j) {
-                    const unsigned oj = f[j] ? o[j] : OPH_BUF_OOB;
-                    v[j] = oph_buf_load_f2(ri, oj);
-                    // the packed Nyquist row (workgroup 0 only; elsewhere an
-                    // out-of-range offset: no memory access)
-                    const unsigned oy = pair0 && oj != OPH_BUF_OOB ? oj + (unsigned)(nyq * sizeof(float2)) : OPH_BUF_OOB;
-                    vy[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ri, oy, 0, 0));
-                }
-#pragma unroll
-                for (int j = 0; j < CHB; ++j) {
-                    const int kx = tl + (m0 + j) * NT;
-                    if (m0 + j < EPT && (EPT * NT == LX || kx < LX))
-                        line[fft::pad16(kx)] = pair0 ? make_float2(v[j].x, vy[j]) : v[j];
-                }
+            for (int m = 0; m < N0; ++m) vi[m / E::R0][m % E::R0] = nv[m / E::R0][m % E::R0];
+            if (ln <= hi) {
+                load_values(ln, tl, f, nv);
+                const int l2 = next_layer(ln + 1);
+                if (l2 <= hi) load_flags(l2, tl, f);
             }
         } else {
-            const float2* src = a.I + (size_t)(l - 1) * lstride + (size_t)kya * GROUP;
-            const unsigned char* fl = a.flags + (size_t)(l - 1) * a.ngroups;
-#pragma unroll
-            for (int m = 0; m < EPT; ++m) {
-                const int kx = tl + m * NT;
-                if (EPT * NT == LX || kx < LX) {
-                    const int x = kx - a.ox;
-                    float2 v = make_float2(0.f, 0.f);
-                    if (x >= 0 && x < a.w && fl[x / GROUP]) {
-                        const size_t o = (size_t)(x / GROUP) * gstride + x % GROUP;
-                        v = src[o];
-                        if (pair0) v.y = src[nyq + o].x;
-                    }
-                    line[fft::pad16(kx)] = v;
-                }
-            }
+            load_flags(l, tl, f);
+            load_values(l, tl, f, vi);
         }
-        __syncthreads();
-        fftm::line<LX, NT, -1>(line, twx, tl);
+        __syncthreads();  // the previous transform's readers are done with the line
+        float2 v[E::PERL][E::RL];
+        fftm::line_ends<LX, -1>(vi, v, line, twx, tl);
         const double cx = a.lc[3 * (l - 1)], cy = a.lc[3 * (l - 1) + 1], K = a.lc[3 * (l - 1) + 2];
         const float Kf = (float)K;
         double tya = cy * (double)sya * sya;
         tya -= rint(tya);
         double tyb = cy * (double)syb * syb;
         tyb -= rint(tyb);
+        if (pair0) {
+            __syncthreads();
 #pragma unroll
-        for (int m = 0; m < EPT; ++m) {
-            const int kx = tl + m * NT;
-            if (EPT * NT == LX || kx < LX) {
-                const int sx = sgnidx(kx, LX);
-                const double sx2 = (double)sx * sx;
-                const float usx = a.ux * (float)(sx * sx);
-                double txd = cx * sx2;
-                txd -= rint(txd);
-                const float tx = (float)txd;
-                float2 gv = line[fft::pad16(kx)];
-                const float2 gm = line[fft::pad16(kx == 0 ? 0 : LX - kx)];
-                float2 gmc = make_float2(gm.x, -gm.y);
-                if (pair0) split_real_pair(gv, gmc);
-                const float2 ha = dm_transfer<EXACT>(a, tx, tya, usx, sya, K, Kf, sx2);
-                acca[m] = fft::cadd(acca[m], fft::cmul(ha, gv));
-                const float2 hb = dm_transfer<EXACT>(a, tx, tyb, usx, syb, K, Kf, sx2);
-                accb[m] = fft::cadd(accb[m], fft::cmul(hb, gmc));
-            }
+            for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+                for (int r = 0; r < E::RL; ++r) {
+                    const int j = tl + q * NT;
+                    if (j < E::NBL) line[fft::pad16(j + r * E::NBL)] = v[q][r];
+                }
+            __syncthreads();
         }
-        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+            for (int r = 0; r < E::RL; ++r) {
+                const int j = tl + q * NT, kx = j + r * E::NBL;
+                if (E::PERL * NT == E::NBL || j < E::NBL) {
+                    const int sx = sgnidx(kx, LX);
+                    const double sx2 = (double)sx * sx;
+                    const float usx = a.ux * (float)(sx * sx);
+                    double txd = cx * sx2;
+                    txd -= rint(txd);
+                    const float tx = (float)txd;
+                    float2 ga = v[q][r], gb = make_float2(ga.x, -ga.y);
+                    if (pair0) {
+                        const float2 gm = line[fft::pad16(kx == 0 ? 0 : LX - kx)];
+                        gb = make_float2(gm.x, -gm.y);
+                        split_real_pair(ga, gb);
+                        gb.y = -gb.y;   // row Ny/2 is real: at -kx the conjugate
+                    }
+                    const float2 ha = dm_transfer<EXACT>(a, tx, tya, usx, sya, K, Kf, sx2);
+                    acca[q][r] = fft::cadd(acca[q][r], fft::cmul(ha, ga));
+                    const float2 hb = dm_transfer<EXACT>(a, tx, tyb, usx, syb, K, Kf, sx2);
+                    accb[q][r] = fft::cadd(accb[q][r], fft::cmul(hb, gb));
+                }
+            }
+        if constexpr (PREF) {
+            l = ln;
+            ln = l <= hi ? next_layer(l + 1) : hi + 1;
+        } else {
+            l = next_layer(l + 1);
+        }
     }
     if (part) {
 #pragma unroll
-        for (int m = 0; m < EPT; ++m) {
-            const int kx = t + m * NT;
-            if (EPT * NT == LX || kx < LX) {
-                part[kx] = acca[m];
-                part[LX + kx] = accb[m];
+        for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+            for (int r = 0; r < E::RL; ++r) {
+                const int j = t + q * NT, kx = j + r * E::NBL;
+                if (j < E::NBL) {
+                    part[kx] = acca[q][r];
+                    part[LX + (kx == 0 ? 0 : LX - kx)] = accb[q][r];
+                }
             }
-        }
         return;
     }
 #pragma unroll
-    for (int m = 0; m < EPT; ++m) {
-        acca[m] = fft::cmul(acca[m], a.rho);
-        accb[m] = fft::cmul(accb[m], a.rho);
+    for (int row = 0; row < 2; ++row) {
+        // in natural order
+        float2 acc[EPT];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < E::PERL; ++q)
+#pragma unroll
+            for (int r = 0; r < E::RL; ++r) {
+                const int j = t + q * NT, kx = j + r * E::NBL;
+                if (j < E::NBL)
+                    line[fft::pad16(row == 0 || kx == 0 ? kx : LX - kx)] =
+                        fft::cmul(row == 0 ? acca[q][r] : accb[q][r], a.rho);
+            }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < EPT; ++m)
+            if (EPT * NT == LX || t + m * NT < LX) acc[m] = line[fft::pad16(t + m * NT)];
+        __syncthreads();
+        finish_row_m<LX>(a, acc, row == 0 ? kya : kyb, line, twx, t);
     }
-    finish_row_m<LX>(a, acca, kya, line, twx, t);
-    finish_row_m<LX>(a, accb, kyb, line, twx, t);
 }
 
 // The partial sums of a pair's layers in order, then as a whole pair's
@@ -1300,8 +1360,9 @@ int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks) {
         (void)chunks;
         return oph_fail(ctx, OPH_ENOTSUP, "grid height %d too large for the column pass", LY);
     } else {
-        const size_t shm = 2 * (size_t)fftm::padded_len(LY) * sizeof(float2) + (size_t)((a.L + 32) / 32) * 4;
-        if (shm + (size_t)a.h * GROUP * 4 > 160 * 1024)   // (as the power-of-two lengths)
+        const size_t words = (size_t)((a.L + 32) / 32) * 4;
+        const size_t shm = 2 * ((size_t)cols_m_line<LY>() + cols_mirror_stride<0>(a.K)) * sizeof(float2) + words;
+        if (2 * (size_t)fftm::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 + words > 160 * 1024)
             return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
         static bool attr = false;
         if (!attr) {

@@ -1,18 +1,20 @@
 // fft_mixed.h -- LDS-resident Stockham FFT for lengths N = 2^a 3^b 5^c on
 // gfx950 (the SLM grids that are not powers of two, e.g. 11520 x 2160).
 //
-// A line of N complex64 values sits in LDS in natural order (fft::pad16
-// indexing).  NT threads transform it, stage by stage over a compile-time
-// radix plan: radix 16 while 16 divides what is left, then one radix 8, 4
-// or 2 for the rest of the power of two, then the 5s and the 3s.  A stage of
-// radix R after radices of product Ns has N/R butterflies; butterfly j reads
-// j + r N/R (r < R), multiplies by exp(SIGN i 2 pi r k/(Ns R)), k = j mod Ns,
-// does the R-point DFT in registers and writes (j - k) R + k + r Ns
-// (self-sorting, output in natural order).  Each thread keeps all of its
-// butterflies' inputs in registers across the stage's barrier, so stages
-// work in place.  Twiddles come from a per-length table (oph_twiddles_mixed)
-// laid out as the power-of-two engine's: stage s >= 1 holds
-// tws[(r-1) Ns + k] = exp(-2 pi i k r/(Ns R)), stages concatenated.
+// A line of N complex64 values is transformed by NT threads, stage by stage
+// over a compile-time radix plan (plan(N): the few large radices that cost
+// least, e.g. 1920 = 16 x 15 x 8).  A stage of radix R after radices of product
+// Ns has N/R butterflies; butterfly j reads j + r N/R (r < R), multiplies by
+// exp(SIGN i 2 pi r k/(Ns R)), k = j mod Ns, does the R-point DFT in registers
+// and writes (j - k) R + k + r Ns (self-sorting, output in natural order).
+// Each thread keeps all of its butterflies' inputs in registers across the
+// stage's barrier, so stages work in place.  line() takes and leaves the line
+// in LDS (natural order, fft::pad16 indexing); line_ends() takes the first
+// stage's inputs and leaves the last stage's outputs in registers, so that
+// the line passes through LDS only between stages.  Twiddles come from a
+// per-length table (oph_twiddles_mixed) laid out as the power-of-two
+// engine's: stage s >= 1 holds tws[(r-1) Ns + k] = exp(-2 pi i k r/(Ns R)),
+// stages concatenated.
 #pragma once
 
 #include "fft_engine.h"
@@ -57,6 +59,71 @@ struct Dft<5, SIGN> {
     }
 };
 
+// N = A B with A and B coprime, without twiddles: input (B n1 + A n2) mod N is
+// element (n1, n2) of an A x B transform, whose output (k1, k2) is the k with
+// k mod A = k1 and k mod B = k2 (n k/N = n1 k/A + n2 k/B up to whole numbers).
+template <int A, int B, int SIGN>
+struct DftCoprime {
+    static constexpr int crt(int k1, int k2) {
+        int k = k1;
+        while (k % B != k2) k += A;
+        return k;
+    }
+    __device__ static void run(float2* v) {
+        float2 x[B][A], y[B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < A; ++n1) x[n2][n1] = v[(B * n1 + A * n2) % (A * B)];
+            Dft<A, SIGN>::run(x[n2]);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; ++k1) {
+#pragma unroll
+            for (int n2 = 0; n2 < B; ++n2) y[n2] = x[n2][k1];
+            Dft<B, SIGN>::run(y);
+#pragma unroll
+            for (int k2 = 0; k2 < B; ++k2) v[crt(k1, k2)] = y[k2];
+        }
+    }
+};
+template <int SIGN>
+struct Dft<6, SIGN> : DftCoprime<2, 3, SIGN> {};
+template <int SIGN>
+struct Dft<10, SIGN> : DftCoprime<2, 5, SIGN> {};
+template <int SIGN>
+struct Dft<12, SIGN> : DftCoprime<4, 3, SIGN> {};
+template <int SIGN>
+struct Dft<15, SIGN> : DftCoprime<3, 5, SIGN> {};
+
+// 9 = 3 x 3: X[k1 + 3 k2] = sum_{n2} W3^{n2 k2} W9^{n2 k1} sum_{n1} W3^{n1 k1} x[3 n1 + n2]
+template <int SIGN>
+struct Dft<9, SIGN> {
+    __device__ static void run(float2* v) {
+        constexpr float c1 = 0.76604444311897804f, s1 = 0.64278760968653933f;   // 2 pi/9
+        constexpr float c2 = 0.17364817766693035f, s2 = 0.98480775301220806f;   // 4 pi/9
+        constexpr float c4 = -0.93969262078590838f, s4 = 0.34202014332566873f;  // 8 pi/9
+        float2 x[3][3];
+#pragma unroll
+        for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < 3; ++n1) x[n2][n1] = v[3 * n1 + n2];
+            Dft<3, SIGN>::run(x[n2]);
+        }
+        x[1][1] = cmul(x[1][1], make_float2(c1, SIGN * s1));
+        x[1][2] = cmul(x[1][2], make_float2(c2, SIGN * s2));
+        x[2][1] = cmul(x[2][1], make_float2(c2, SIGN * s2));
+        x[2][2] = cmul(x[2][2], make_float2(c4, SIGN * s4));
+#pragma unroll
+        for (int k1 = 0; k1 < 3; ++k1) {
+            float2 y[3] = {x[0][k1], x[1][k1], x[2][k1]};
+            Dft<3, SIGN>::run(y);
+#pragma unroll
+            for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = y[k2];
+        }
+    }
+};
+
 }  // namespace fft
 
 namespace fftm {
@@ -66,27 +133,54 @@ struct Plan {
     int r[24];   // radices in order
 };
 
-__host__ __device__ constexpr Plan plan(int N) {
-    Plan p{0, {}};
-    int rest = N;
-    while (rest % 16 == 0) { p.r[p.n++] = 16; rest /= 16; }
-    if (rest % 8 == 0) { p.r[p.n++] = 8; rest /= 8; }
-    else if (rest % 4 == 0) { p.r[p.n++] = 4; rest /= 4; }
-    else if (rest % 2 == 0) { p.r[p.n++] = 2; rest /= 2; }
-    while (rest % 5 == 0) { p.r[p.n++] = 5; rest /= 5; }
-    while (rest % 3 == 0) { p.r[p.n++] = 3; rest /= 3; }
-    if (rest != 1) p.n = -1;
-    return p;
-}
-
-// Threads per line: the radix-16 stage's butterfly count rounded up to whole
-// waves (every stage then has at most ~6 butterflies per thread), at most
+// Threads per line: a radix-16 stage's butterfly count rounded up to whole
+// waves, at most
 // 512 (a longer line keeps more elements per thread, but 8 waves of up to
 // 256 registers each, where 12 would be held to 168).
 __host__ __device__ constexpr int threads(int N) {
     const int t = ((N + 15) / 16 + 63) / 64 * 64;
     return t < 512 ? t : 512;
 }
+// Cost of a radix-R stage of an N-point line to a thread: its butterflies'
+// instructions, twiddles and LDS accesses, and the stage's barriers.
+__host__ __device__ constexpr int stage_cost(int N, int R, bool first) {
+    const int ops = R == 16 ? 190 : R == 15 ? 220 : R == 12 ? 140 : R == 10 ? 124 : R == 9 ? 120 : R == 8 ? 76
+                  : R == 6 ? 60 : R == 5 ? 48 : R == 4 ? 24 : R == 3 ? 22 : 8;
+    const int per = (N / R + threads(N) - 1) / threads(N);
+    return per * (ops + (first ? 0 : 8 * (R - 1)) + 16 * R) + 60;
+}
+
+// The radices in falling order whose stages together cost least.
+struct Search {
+    int cost;
+    Plan best;
+};
+__host__ __device__ constexpr void search(int N, int rest, int max_radix, const Plan& path, int cost, Search& s) {
+    if (rest == 1) {
+        if (cost < s.cost) {
+            s.cost = cost;
+            s.best = path;
+        }
+        return;
+    }
+    for (int R = max_radix; R >= 2; --R) {
+        if (rest % R || (R > 6 && (R < 8 || R == 11 || R == 13 || R == 14))) continue;
+        Plan next = path;
+        next.r[next.n++] = R;
+        search(N, rest / R, R, next, cost + stage_cost(N, R, path.n == 0), s);
+    }
+}
+__host__ __device__ constexpr Plan plan(int N) {
+    int rest = N;
+    for (int f = 2; f <= 5; ++f)
+        while (f != 4 && rest > 1 && rest % f == 0) rest /= f;
+    Search s{1 << 30, {-1, {}}};
+    if (rest == 1 && N > 1) search(N, N, 16, Plan{0, {}}, 0, s);
+    return s.best;
+}
+template <int N>
+constexpr Plan PLAN = plan(N);   // (searched once per length)
+
 // Elements per thread when a thread owns t + m NT, m < ept(N).
 __host__ __device__ constexpr int ept(int N) { return (N + threads(N) - 1) / threads(N); }
 
@@ -143,9 +237,8 @@ __device__ __forceinline__ void stage(float2* buf, const float2* __restrict__ tw
 
 template <int N, int NT, int SIGN, int S, int NS, int OFF>
 __device__ __forceinline__ void line_from(float2* buf, const float2* __restrict__ tw, int t) {
-    constexpr Plan P = plan(N);
-    if constexpr (S < P.n) {
-        constexpr int R = P.r[S];
+    if constexpr (S < PLAN<N>.n) {
+        constexpr int R = PLAN<N>.r[S];
         stage<N, R, NS, NT, SIGN>(buf, tw + OFF, t);
         line_from<N, NT, SIGN, S + 1, NS * R, OFF + (NS > 1 ? (R - 1) * NS : 0)>(buf, tw, t);
     }
@@ -156,8 +249,77 @@ __device__ __forceinline__ void line_from(float2* buf, const float2* __restrict_
 // stages hold barriers).  Caller syncs before (line loaded).
 template <int N, int NT, int SIGN>
 __device__ __forceinline__ void line(float2* buf, const float2* __restrict__ tw, int t) {
-    static_assert(plan(N).n > 0, "length must be 2^a 3^b 5^c");
+    static_assert(PLAN<N>.n > 0, "length must be 2^a 3^b 5^c");
     line_from<N, NT, SIGN, 0, 1, 0>(buf, tw, t);
+}
+
+// ---- register-ended lines ----
+// The first stage's butterfly t + p NT has the inputs (t + p NT) + r NB0, the
+// last stage's the outputs (t + p NT) + r NBL: per thread PER0 x R0 and PERL x
+// RL elements, of which those of butterflies beyond NB0 (NBL) do not exist.
+template <int N>
+struct Ends {
+    static constexpr int NT = threads(N), LAST = PLAN<N>.n - 1;
+    static_assert(PLAN<N>.n >= 2, "two stages at least");
+    static constexpr int R0 = PLAN<N>.r[0], NB0 = N / R0, PER0 = (NB0 + NT - 1) / NT;
+    static constexpr int RL = PLAN<N>.r[LAST], NBL = N / RL, PERL = (NBL + NT - 1) / NT;
+};
+
+// Stages S .. n - 2, in LDS
+template <int N, int SIGN, int S, int NS, int OFF>
+__device__ __forceinline__ void mid_stages(float2* buf, const float2* __restrict__ tw, int t) {
+    if constexpr (S < Ends<N>::LAST) {
+        constexpr int R = PLAN<N>.r[S];
+        stage<N, R, NS, Ends<N>::NT, SIGN>(buf, tw + OFF, t);
+        mid_stages<N, SIGN, S + 1, NS * R, OFF + (R - 1) * NS>(buf, tw, t);
+    }
+}
+template <int N>
+constexpr int last_offset() {
+    int off = 0, ns = PLAN<N>.r[0];
+    for (int s = 1; s < PLAN<N>.n - 1; ++s) {
+        off += (PLAN<N>.r[s] - 1) * ns;
+        ns *= PLAN<N>.r[s];
+    }
+    return off;
+}
+
+// Full transform of a line from vi (first stage's inputs) to vo (last stage's
+// outputs).  The caller syncs before the line is written again (other threads
+// may still read the last stage's inputs); every thread of the workgroup calls
+// it.
+template <int N, int SIGN>
+__device__ __forceinline__ void line_ends(float2 (&vi)[Ends<N>::PER0][Ends<N>::R0],
+                                          float2 (&vo)[Ends<N>::PERL][Ends<N>::RL], float2* buf,
+                                          const float2* __restrict__ tw, int t) {
+    using E = Ends<N>;
+#pragma unroll
+    for (int p = 0; p < E::PER0; ++p) {
+        const int j = t + p * E::NT;
+        if (E::PER0 * E::NT == E::NB0 || j < E::NB0) {
+            fft::Dft<E::R0, SIGN>::run(vi[p]);
+#pragma unroll
+            for (int r = 0; r < E::R0; ++r) buf[fft::pad16(j * E::R0 + r)] = vi[p][r];
+        }
+    }
+    __syncthreads();
+    mid_stages<N, SIGN, 1, E::R0, 0>(buf, tw, t);
+    const float2* tl = tw + last_offset<N>();
+#pragma unroll
+    for (int p = 0; p < E::PERL; ++p) {
+        const int j = t + p * E::NT;
+        if (E::PERL * E::NT == E::NBL || j < E::NBL) {
+            float2 w[E::RL];
+#pragma unroll
+            for (int r = 1; r < E::RL; ++r) w[r] = tl[(r - 1) * E::NBL + j];
+#pragma unroll
+            for (int r = 0; r < E::RL; ++r) vo[p][r] = buf[fft::pad16(j + r * E::NBL)];
+            batch_ready(w);
+#pragma unroll
+            for (int r = 1; r < E::RL; ++r) vo[p][r] = SIGN < 0 ? fft::cmul(vo[p][r], w[r]) : fft::cmulc(vo[p][r], w[r]);
+            fft::Dft<E::RL, SIGN>::run(vo[p]);
+        }
+    }
 }
 
 // LDS elements of a padded line

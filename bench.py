@@ -29,15 +29,16 @@ VALU_LANE_OPS = 256 * 4 * 16 * 2.4e9      # VALU issue peak, unpacked FP32 lane-
 # SQ_INSTS_VALU ... -- python3 bench.py --workload <rs|wrp> --only --steps 2
 # --warmup 1 --no-cpu` commands recorded there); valid for the kernels as
 # built at that time: re-measure after changing them.
-PROFILED_VALU_INSTS = {"rs_accumulate": 181600256, "asm_cols": 25980928, "wrp_gather": 23896245}
+PROFILED_VALU_INSTS = {"rs_accumulate": 31413884, "asm_cols": 25980928, "wrp_gather": 23896245}
+PROFILED_RS_MFMA = 3565554                 # of rs_accumulate's, v_mfma_f32_32x32x2f32 (SQ_INSTS_MFMA)
 PROFILE_SOURCES = {"valu": "profiles/valu_counters_rs_wrp.md (rocprofv3 --pmc SQ_INSTS_VALU)",
                    "traffic": "profiles/hbm_traffic_wrp_depthmap.md (rocprofv3 --pmc FETCH_SIZE, then "
                               "WRITE_SIZE, calibrated on copy_kernel)"}
-# RS issue model: per point-pixel pair the kernel needs at least 2 FMAs for
-# the phase polynomial, 1 add (q), 2 FMAs of accumulation and sin + cos,
-# which issue at a quarter of the rate (4 slots each): 13 issue slots per
-# pair at the VALU issue peak.
-RS_SLOTS_PER_PAIR = 13
+# RS: the sum over points is a matrix product on the FP32 matrix units, each
+# instruction 4096 flops in 64 cycles of its SIMD (157 TFLOP/s); the other
+# vector instructions form its operands, 4 cycles each, and do not overlap
+# with it on a SIMD.
+MFMA_F32_TFLOPS = 256 * 4 * 64 * 2.4e9 / 1e12
 
 
 def rel_l2(a, b):
@@ -74,20 +75,19 @@ def bench_rs(ctx, args):
     ctx.profile(False)
     pairs = 1000 * spec["nx"] * spec["ny"]
     k_avg = kms / max(n, 1) / 1e3
-    lane_ops = PROFILED_VALU_INSTS["rs_accumulate"] * 64
-    peak_pairs = VALU_LANE_OPS / RS_SLOTS_PER_PAIR
+    mfma_tflops = PROFILED_RS_MFMA * 4096 / k_avg / 1e12
+    busy = PROFILED_RS_MFMA * 64 + (PROFILED_VALU_INSTS["rs_accumulate"] - PROFILED_RS_MFMA) * 4
     line = {
         "metric": METRIC, "value": args.steps / wall, "unit": "holograms/s",
         "ms_per_step": wall / args.steps * 1e3, "dtype": "f64-phase/f32-acc",
         "config": {"workload": "rs_pointcloud_1000pts_1024x1024_8um_532nm"},
         "point_pixel_per_s": pairs / (wall / args.steps),
-        # point-pixel pairs per second of rs_accumulate against the pair rate
-        # the VALU issue peak allows at RS_SLOTS_PER_PAIR slots per pair
-        "roofline": {"kernel": "rs_accumulate", "bound": "valu", "achieved": pairs / k_avg / 1e12,
-                     "peak": peak_pairs / 1e12, "unit": "Tpair/s", "frac": pairs / k_avg / peak_pairs,
-                     "traffic": None, "slots_per_pair_model": RS_SLOTS_PER_PAIR,
-                     "valu_issue_frac_counted": lane_ops / k_avg / VALU_LANE_OPS,
-                     "valu_lane_ops_per_pair_counted": lane_ops / pairs,
+        # the matrix units' rate from the counted instructions, and the share
+        # of the SIMDs' cycles that all of the kernel's vector instructions take
+        "roofline": {"kernel": "rs_accumulate", "bound": "mfma", "achieved": mfma_tflops,
+                     "peak": MFMA_F32_TFLOPS, "unit": "TFLOP/s", "frac": mfma_tflops / MFMA_F32_TFLOPS,
+                     "traffic": None, "pairs_per_s": pairs / k_avg,
+                     "valu_and_mfma_issue_frac": busy / (k_avg * 256 * 4 * 2.4e9),
                      "counted_from": PROFILE_SOURCES["valu"]},
     }
     if not args.no_cpu:
@@ -249,12 +249,12 @@ def cpu_wrp(x, y, z, a, zw, n_side, pitch, lam, dist, pad):
                       f"by point count) + one full {n_side * pad}^2 padded ASM ({t_asm:.2f} s)"}, m, ref
 
 
-DM_KERNELS = ["dm_index", "dm_zero", "dm_cols", "dm_rows", "dm_final"]
-# The depth-map row pass (`dm_rows_h<4096, true>`, one launch per colour of
+DM_KERNELS = ["dm_index", "dm_zero", "dm_cols", "dm_rows", "dm_rows_sum", "dm_final"]
+# The depth-map row pass (`dm_rows_h<4096, 0, true, true>`, one launch per colour of
 # the RGB workload): wave-level VALU instructions (SQ_INSTS_VALU) and HBM
 # bytes (FETCH_SIZE + WRITE_SIZE, calibrated as PROFILED_TRAFFIC) per launch,
 # from the `--workload depthmap --only --steps 2 --warmup 1 --no-cpu` runs.
-PROFILED_DM_ROWS = {"valu_insts": 1.022e9, "traffic": (1905.2 + 15.0) * 2**20}
+PROFILED_DM_ROWS = {"valu_insts": 4.831e8, "traffic": (962.1 + 17.0) * 2**20}
 
 
 def bench_depthmap(ctx, args):
@@ -277,10 +277,12 @@ def bench_depthmap(ctx, args):
     line = {"value": steps / wall, "unit": "holograms/s (RGB)", "ms_per_step": wall / steps * 1e3,
             "config": {"workload": "depthmap_rgb_1920x1080_grid4096x2048_256layers_8um"}, "kernels": per}
     # algorithmic HBM bytes of the layer passes (complex64 intermediates of
-    # the Hermitian half, written once by dm_cols and read once by dm_rows)
+    # the Hermitian half's rows that the crop keeps, in the column groups with
+    # a pixel in the layer, written once by dm_cols and read once by dm_rows)
     idx = 256 - dep.astype(np.int64)
     layers = int((np.bincount(idx.ravel(), minlength=257)[1:] > 0).sum())
-    inter = layers * (Ny // 2 + 1) * w * 8
+    groups = sum(len(np.unique(idx[:, x:x + 4])) for x in range(0, w, 4))
+    inter = groups * (Ny // 4 + 3) * 4 * 8
     line["layers_populated"] = layers
     if "dm_rows" in per:
         t = (per["dm_rows"]["avg_us"] + per["dm_cols"]["avg_us"]) * 1e-6
@@ -292,7 +294,7 @@ def bench_depthmap(ctx, args):
         ops = PROFILED_DM_ROWS["valu_insts"] * 64
         line["roofline"] = {"kernel": "dm_rows", "bound": "valu", "achieved": ops / tr / 1e12,
                             "peak": VALU_LANE_OPS / 1e12, "unit": "Tlane-ops/s", "frac": ops / tr / VALU_LANE_OPS,
-                            "traffic": PROFILED_DM_ROWS["traffic"], "algorithmic_bytes": inter + (Ny // 2 + 1) * w * 8,
+                            "traffic": PROFILED_DM_ROWS["traffic"], "algorithmic_bytes": inter + Ny // 2 * w * 8,
                             "hbm_frac": PROFILED_DM_ROWS["traffic"] / tr / (HBM_PEAK_GBS * 1e9),
                             "counted_from": "profiles/sq_counters_fresnel_depthmap.md (SQ_INSTS_VALU) and "
                                             "profiles/hbm_traffic_wrp_depthmap.md (FETCH_SIZE, WRITE_SIZE)"}
@@ -424,7 +426,8 @@ def bench_fresnel(ctx, args):
     return line
 
 
-CNN_KERNELS = ["conv3x3_fwd", "conv3x3_dw", "dw_reduce", "pack_weights", "relu_mask", "mse_grad", "sum_partials",
+CNN_KERNELS = ["conv3x3_fwd", "conv3x3_dw", "dw_reduce", "pack_weights", "resblock_f32",
+               "resblock_f32_bwd", "mse_grad", "sum_partials",
                "adam_step"]
 
 

@@ -29,23 +29,24 @@
 // Passes (per colour; the depth index is shared):
 //   dm_index  depth index of every pixel by a 256-entry table of the u8 depth
 //             (built on the host; the reference makes one pass per level);
-//   dm_cols   a workgroup owns 4 scene columns and a range of layers; two
+//   dm_cols   a workgroup owns 4 scene columns and every n-th layer; two
 //             real columns are packed into one complex column, transformed
 //             along y (length Ny) and separated; only rows ky <= Ny/2 are
 //             stored (Hermitian symmetry of real input), and of these, for an
 //             encoded output, only those whose row pair the crop keeps (half:
 //             K below; 3 x 1920 x 1080 on 4096 x 2048, 256 layers: row pass
-//             3196 -> 1720 us a colour), with a presence flag
+//             3196 -> 1720 us a colour by this alone), with a presence flag
 //             per (layer, column group) -- absent groups are never written;
 //   dm_rows   a workgroup owns the row pair (ky, Ny-ky): per layer it
 //             transforms row ky along x once and obtains row Ny-ky from the
 //             same transform by symmetry, multiplies both by H and
-//             accumulates over all layers in registers; then the encode crop,
-//             the inverse row transforms, and the scene columns are stored.
+//             accumulates over its layers; then the encode crop, the inverse
+//             row transforms, and the scene columns are stored.  Pairs that do
+//             not fill the chip have their layers split over workgroups, whose
+//             sums dm_rows_sum adds (rows_plan below);
 //             Rows 0 and Ny/2 are real (transforms of real columns at the DC
-//             and Nyquist frequencies): workgroup 0 packs them into one
-//             complex row and separates the transform, so the pass is Ny/2
-//             pairs (a multiple of the CU count) instead of Ny/2 + 1;
+//             and Nyquist frequencies): pair 0 packs them into one complex row
+//             and separates the transform;
 //   dm_final  inverse column transform, 1/(Nx Ny), the shift phase and the
 //             real part (or the complex field) in the scene window.
 #include <algorithm>

@@ -228,3 +228,18 @@ def test_depthmap_column_lengths(ctx, h, Ny, out):
     u = ctx.depthmap(21, h, 32, Ny, 8e-6, 0.09, 0.11, 6, [532e-9], img, dep, out=out, quant_mode=1)
     ref = _oracle_rgb(img, dep, 32, Ny, 8e-6, [532e-9], 0.09, 0.11, 6, out=out, quant_mode=1)
     assert rel_l2(u, ref) < TOL
+
+
+@pytest.mark.parametrize("out", ["field", "fringe"])
+@pytest.mark.parametrize("w,h,Nx,Ny", [
+    (3840, 30, 3840, 540), (2160, 30, 2160, 540), (1920, 30, 1920, 720), (5001, 30, 11520, 540),
+    (30, 3001, 540, 3840), (31, 2160, 540, 2160), (30, 1500, 720, 1920), (30, 1080, 540, 1080),
+])
+def test_depthmap_general_lengths(ctx, w, h, Nx, Ny, out):
+    """Every general length's plan, along the rows and along the columns."""
+    print(f"case: depthmap {w}x{h} grid {Nx}x{Ny} {out}", flush=True)
+    img, dep = scenes.depth_scene(w, h, seed=15, colors=1)
+    kw = dict(quant_mode=1, field_lens=1.0)
+    u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.2, 0.7, 5, [532e-9], img, dep, out=out, **kw)
+    ref = _oracle_rgb(img, dep, Nx, Ny, 8e-6, [532e-9], 0.2, 0.7, 5, out=out, **kw)
+    assert rel_l2(u, ref) < TOL

@@ -48,12 +48,14 @@ constexpr int MB = 8192;     // workgroups of the other passes, at most
 
 // (min, max) over the workgroup of each thread's (mn, mx); every thread of
 // the workgroup calls it and gets the result.  NT threads, a multiple of 64
-// (or fewer than 64).
+// or a power of two below it: there only the lanes that exist are exchanged
+// (a shuffle reads 0 from one that does not).
 template <int NT>
 __device__ __forceinline__ float2 block_minmax(float mn, float mx) {
+    static_assert(NT % 64 == 0 || (NT < 64 && (NT & (NT - 1)) == 0), "whole waves, or a power of two of lanes");
     __shared__ float2 w[(NT + 63) / 64];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
+    for (int o = (NT < 64 ? NT : 64) / 2; o > 0; o >>= 1) {
         mn = fminf(mn, __shfl_xor(mn, o, 64));
         mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     }

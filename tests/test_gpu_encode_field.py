@@ -89,3 +89,18 @@ def test_encode_ssb_aliased_and_not_finite(ctx):
     assert np.array_equal(d.numpy().view(np.float32).ravel()[:64 * 128], ref.ravel())
     u[3, 5] = np.nan
     assert np.isnan(ctx.encode_field(u, "ssb")).all()
+
+
+@pytest.mark.parametrize("mean", [3.0, -3.0])
+@pytest.mark.parametrize("passband", ["right", "bottom"])
+@pytest.mark.parametrize("n", [16, 32, 64])
+def test_encode_ssb_one_sided(ctx, n, passband, mean):
+    """A carrier in the passband: the filtered field lies on one side of zero,
+    so a zero that enters the minimum or the maximum shows.  Lines of 16 and 32
+    columns are workgroups of less than a wave.  Bound: the transforms' 2e-6 of
+    the mean, against a spread of at least a thirtieth of it: 6e-5 of outputs
+    that are about half of one: 1.2e-4."""
+    print(f"case: ssb one-sided {n} {passband} mean {mean}", flush=True)
+    u = (mean + 0.1 * _field(*((n, 64) if passband == "bottom" else (64, n)), n)).astype(np.complex64)
+    ref = E.ssb(u.astype(np.complex128), {"right": E.RIGHT, "bottom": E.BOTTOM}[passband])
+    assert rel_l2(ctx.encode_field(u, "ssb", passband=passband), ref) < 1.2e-4

@@ -1266,6 +1266,7 @@ int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int gran, int resident) {
     a.n_main = pairs;
     a.nsplit = 1;
     a.per = layers;
+    if (layers < 2) return OPH_OK;   // (0: an empty range)
     long long best = (long long)((pairs + slots - 1) / slots) * layers;
     for (const int n_main : {pairs / slots * slots, 0})
         for (int n = 2; n <= 16; ++n) {
@@ -1478,8 +1479,9 @@ extern "C" int oph_depthmap(oph_ctx* ctx, const oph_dm_spec* s, int ncolor, cons
     for (int c = 0; c < ncolor; ++c)
         if (!(lambdas[c] > 0)) return oph_fail(ctx, OPH_EINVAL, "wavelength %d must be positive", c);
     const int fmt = flags & OPH_DM_OUT_MASK;
-    const int lo = s->layer_lo >= 1 ? s->layer_lo : 1;
     const int hi = (s->layer_hi >= 1 && s->layer_hi <= L) ? s->layer_hi : L;
+    // (a range that begins past its end is empty: lo = hi + 1, a field of zeros)
+    const int lo = std::min(s->layer_lo >= 1 ? s->layer_lo : 1, hi + 1);
 
     // depth levels (GetDepthValues, HologramGenerator.cpp:393-401: repeated
     // addition; continued to exactly L entries) and the viewing-window

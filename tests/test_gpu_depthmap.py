@@ -243,3 +243,18 @@ def test_depthmap_general_lengths(ctx, w, h, Nx, Ny, out):
     u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.2, 0.7, 5, [532e-9], img, dep, out=out, **kw)
     ref = _oracle_rgb(img, dep, Nx, Ny, 8e-6, [532e-9], 0.2, 0.7, 5, out=out, **kw)
     assert rel_l2(u, ref) < TOL
+
+
+@pytest.mark.parametrize("out", ["field", "fringe"])
+@pytest.mark.parametrize("field_lens", [0.0, 1.0])
+@pytest.mark.parametrize("w,h,Nx,Ny", [(64, 48, 128, 64), (20, 12, 32, 16), (720, 20, 720, 540)])
+def test_depthmap_empty_layer_range(ctx, w, h, Nx, Ny, field_lens, out):
+    """A layer range that begins past its end, or past the last layer, holds no
+    layer: a hologram of zeros."""
+    L = 40
+    img, dep = scenes.depth_scene(w, h, seed=16, colors=1)
+    for layers in ((10, 5), (6, 5), (39, 2), (L + 1, 0), (L + 5, L + 9), (300, 0), (2**31 - 1, 0)):
+        print(f"case: depthmap {w}x{h} grid {Nx}x{Ny} lens {field_lens} {out} layers={layers}", flush=True)
+        u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.09, 0.11, L, [532e-9], img, dep, out=out, quant_mode=1,
+                         field_lens=field_lens, layers=layers)
+        assert np.all(u == 0)

@@ -447,7 +447,6 @@ struct GatherArgs {
     double pitch, inv_lambda;
     float r_off;     // spherical amplitude a/(r + r_off): 0.05, or 0 for mode 3
     int lo_add;      // 1 for mode 3 (window [t - w + 1, t + w)), else 0
-    int strips;      // workgroups per tile, TILE / strips rows each (a power of two)
     float2* wrp;
     int accumulate;
 };
@@ -544,9 +543,11 @@ __device__ unsigned segment_end(const unsigned* pre, int nchunks, unsigned total
 // FRESNEL: the call's window mode is 2 (Fresnel phase, unit amplitude
 // factor); the spherical modes 0 and 1 use the other instantiation, so each
 // carries only its own two evaluation paths.
-template <bool FRESNEL_MODE>
+// STRIPS: workgroups per tile, TILE / STRIPS rows each.
+template <bool FRESNEL_MODE, int STRIPS>
 __global__ __launch_bounds__(GATHER_THREADS) void wrp_gather(GatherArgs g) {
-    __shared__ unsigned long long acc[TILE * TILE];
+    constexpr int rows = TILE / STRIPS;
+    __shared__ unsigned long long acc[TILE * rows];
     __shared__ GSetup recs[REC_BATCH];
     __shared__ unsigned seg_hi;
     // an overflowed binning leaves the output untouched (the call is redone
@@ -554,9 +555,9 @@ __global__ __launch_bounds__(GATHER_THREADS) void wrp_gather(GatherArgs g) {
     if (*g.overflow) return;
     // the tile, and this workgroup's rows of it (a strip's pixels get the same
     // integer sums whichever rows share the workgroup)
-    const int tile = blockIdx.x / g.strips, rows = TILE / g.strips;
+    const int tile = blockIdx.x / STRIPS;
     const int tyi = tile / g.ntx, txi = tile % g.ntx;
-    const int X0 = txi * TILE, Y0 = tyi * TILE + (int)(blockIdx.x % g.strips) * rows;
+    const int X0 = txi * TILE, Y0 = tyi * TILE + (int)(blockIdx.x % STRIPS) * rows;
     unsigned b = g.offsets[tile], e = g.offsets[tile + 1];
     if (e > g.capacity) e = g.capacity;
     if (b > e) b = e;
@@ -852,16 +853,34 @@ int wrp_core(oph_ctx* ctx, int nx, int ny, double pitch, double lambda, double z
         g.wrp = wrp;
         g.accumulate = accumulate;
         // small planes: a tile's rows over several workgroups, until there
-        // are about four per CU (256^2, 500 points of mode 1, 16 tiles: 49 us
-        // with the binning at one, 26 at 4, 20 at 8, 16.7 at 16, 16.3 at 32;
-        // 512^2, 20,000 points: 330, 144, 113, 108, 150; 1024^2, 25,000: 132
-        // at one, 98 at 4, 103 at 8; 2048^2 is fastest at one)
-        g.strips = 1;
-        while (g.strips < 16 && 2 * g.strips * ntiles <= 4 * std::max(ctx->cu_count, 1)) g.strips *= 2;
-        if (mode == 2)
-            OPH_LAUNCH(ctx, "wrp_gather", wrp_gather<true>, dim3(ntiles * g.strips), dim3(GATHER_THREADS), 0, g);
-        else
-            OPH_LAUNCH(ctx, "wrp_gather", wrp_gather<false>, dim3(ntiles * g.strips), dim3(GATHER_THREADS), 0, g);
+        // are about four per CU (with the binning, mode 1: 256^2, 2,000 points
+        // 147 us at one, 68 at 4, 39 at 16; 512^2, 20,000: 328, 144, 107;
+        // 1024^2, 100,000: 419 at one, 299 at 4, 336 at 8; 2048^2 is fastest
+        // at one: 236, 261 at two).  Mode 3 gains least: two per CU, and one
+        // workgroup per tile where the tiles alone fill the chip (512^2,
+        // 20,000: 142 at one, 74 at 8, 78 at 16; 1024^2, 100,000: 177 at one,
+        // 181 at 2, 189 at 4).
+        const int cus = std::max(ctx->cu_count, 1);
+        const int most = mode != 3 ? 4 * cus : ntiles < cus ? 2 * cus : 0;
+        int strips = 1;
+        while (strips < 16 && 2 * strips * ntiles <= most) strips *= 2;
+        const dim3 grid((unsigned)(ntiles * strips)), block(GATHER_THREADS);
+        const bool fresnel = mode == 2;
+        switch (strips) {
+#define OPH_WRP_GATHER(n)                                                          \
+    case n:                                                                        \
+        if (fresnel)                                                               \
+            OPH_LAUNCH(ctx, "wrp_gather", (wrp_gather<true, n>), grid, block, 0, g);  \
+        else                                                                       \
+            OPH_LAUNCH(ctx, "wrp_gather", (wrp_gather<false, n>), grid, block, 0, g); \
+        break;
+            OPH_WRP_GATHER(1)
+            OPH_WRP_GATHER(2)
+            OPH_WRP_GATHER(4)
+            OPH_WRP_GATHER(8)
+            OPH_WRP_GATHER(16)
+#undef OPH_WRP_GATHER
+        }
         // the list size is only known on the device; a capacity overflow is
         // detected after the fact (the gather then writes nothing, so an
         // accumulating call is still intact) and the pass is redone with the

@@ -44,7 +44,7 @@ namespace {
 
 constexpr int RT = 256;      // threads per workgroup
 constexpr int RB = 1024;     // workgroups of a reducing pass (and partial pairs), at most
-constexpr int MB = 8192;     // workgroups of the other passes, at most
+constexpr int MB = 16384;    // workgroups of the other passes, at most
 
 // (min, max) over the workgroup of each thread's (mn, mx); every thread of
 // the workgroup calls it and gets the result.  NT threads, a multiple of 64

@@ -941,34 +941,31 @@ __global__ __launch_bounds__(2 * fftm::threads(LY)) void dm_cols_m(DmArgs a, int
     }
 }
 
+// finish_row for a row already in the line, in natural order (synced); not
+// called for rows that the crop drops, unless the spectrum is wanted.
 template <int LX>
-__device__ __forceinline__ void finish_row_m(const DmArgs& a, const float2 (&acc)[fftm::ept(LX)], int ky,
-                                             float2* line, const float2* __restrict__ tw, int t) {
-    constexpr int NT = fftm::threads(LX), EPT = fftm::ept(LX);
+__device__ __forceinline__ void finish_row_m(const DmArgs& a, int ky, float2* line, const float2* __restrict__ tw,
+                                             int t) {
+    constexpr int NT = fftm::threads(LX);
     const int yc = (ky + a.Ny / 2) % a.Ny;
     if (a.spectrum) {
-#pragma unroll
-        for (int m = 0; m < EPT; ++m) {
-            const int kx = t + m * NT;
-            if (EPT * NT == LX || kx < LX) {
-                const int xc = (kx + LX / 2) % LX;
-                const float sg = ((kx + ky) & 1) ? -1.f : 1.f;
-                a.spectrum[(size_t)yc * LX + xc] = make_float2(sg * acc[m].x, sg * acc[m].y);
-            }
+        for (int kx = t; kx < LX; kx += NT) {
+            const int xc = (kx + LX / 2) % LX;
+            const float sg = ((kx + ky) & 1) ? -1.f : 1.f;
+            const float2 v = line[fft::pad16(kx)];
+            a.spectrum[(size_t)yc * LX + xc] = make_float2(sg * v.x, sg * v.y);
         }
+        __syncthreads();
     }
-    const bool kept = !a.encode || (yc >= a.cy1 && yc <= a.cy2);
-    if (!kept) return;  // uniform over the workgroup
-#pragma unroll
-    for (int m = 0; m < EPT; ++m) {
-        const int kx = t + m * NT;
-        if (EPT * NT == LX || kx < LX) line[fft::pad16(kx)] = acc[m];
-    }
-    __syncthreads();
+    if (a.encode && !(yc >= a.cy1 && yc <= a.cy2)) return;  // uniform over the workgroup
     fftm::line<LX, NT, +1>(line, tw, t);
     float2* dst = a.T + (size_t)ky * a.w;
     for (int x = t; x < a.w; x += NT) dst[x] = line[fft::pad16(x + a.ox)];
-    __syncthreads();
+}
+template <int LX>
+__device__ __forceinline__ bool row_wanted_m(const DmArgs& a, int ky) {
+    const int yc = (ky + a.Ny / 2) % a.Ny;
+    return a.spectrum || !a.encode || (yc >= a.cy1 && yc <= a.cy2);
 }
 
 // Bound by vector instructions and the waits between a layer's stages.  1920 x
@@ -980,7 +977,7 @@ __device__ __forceinline__ void finish_row_m(const DmArgs& a, const float2 (&acc
 template <int LX, bool EXACT>
 __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const float2* __restrict__ twx) {
     using E = fftm::Ends<LX>;
-    constexpr int NT = E::NT, EPT = fftm::ept(LX);
+    constexpr int NT = E::NT;
     constexpr int N0 = E::PER0 * E::R0;
     constexpr bool PREF = N0 <= 16;   // the next layer's values fit in registers
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
@@ -1141,24 +1138,26 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const f
     }
 #pragma unroll
     for (int row = 0; row < 2; ++row) {
-        // in natural order
-        float2 acc[EPT];
+        const int ky = row == 0 ? kya : kyb;
+        if (!row_wanted_m<LX>(a, ky)) continue;
+        // into the line in natural order; no copy of the row in registers, and
+        // each row's LDS addresses formed for it alone (as in the layer loop):
+        // at 11520 the one or the other spills
+        int zero;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+        const int tl = t + zero;
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < E::PERL; ++q)
 #pragma unroll
             for (int r = 0; r < E::RL; ++r) {
-                const int j = t + q * NT, kx = j + r * E::NBL;
+                const int j = tl + q * NT, kx = j + r * E::NBL;
                 if (j < E::NBL)
                     line[fft::pad16(row == 0 || kx == 0 ? kx : LX - kx)] =
                         fft::cmul(row == 0 ? acca[q][r] : accb[q][r], a.rho);
             }
         __syncthreads();
-#pragma unroll
-        for (int m = 0; m < EPT; ++m)
-            if (EPT * NT == LX || t + m * NT < LX) acc[m] = line[fft::pad16(t + m * NT)];
-        __syncthreads();
-        finish_row_m<LX>(a, acc, row == 0 ? kya : kyb, line, twx, t);
+        finish_row_m<LX>(a, ky, line, twx, tl);
     }
 }
 
@@ -1179,9 +1178,14 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m_sum(DmArgs a, con
             const int kx = t + m * NT;
             if (EPT * NT == LX || kx < LX) acc[m] = fft::cadd(acc[m], p[(size_t)2 * j * LX + kx]);
         }
+    if (!row_wanted_m<LX>(a, ky)) return;
 #pragma unroll
-    for (int m = 0; m < EPT; ++m) acc[m] = fft::cmul(acc[m], a.rho);
-    finish_row_m<LX>(a, acc, ky, line, twx, t);
+    for (int m = 0; m < EPT; ++m) {
+        const int kx = t + m * NT;
+        if (EPT * NT == LX || kx < LX) line[fft::pad16(kx)] = fft::cmul(acc[m], a.rho);
+    }
+    __syncthreads();
+    finish_row_m<LX>(a, ky, line, twx, t);
 }
 
 template <int LY, int B>

@@ -968,6 +968,13 @@ __device__ __forceinline__ bool row_wanted_m(const DmArgs& a, int ky) {
     return a.spectrum || !a.encode || (yc >= a.cy1 && yc <= a.cy2);
 }
 
+// Workgroups of three waves (2160): at two waves per SIMD only two fit a CU,
+// at three, four.  Without the next layer's values its registers allow that
+// (152, none spilled): a field of 2160^2 and 4 layers takes 235 us, of 32 950;
+// with the values requested ahead 265 and 996 (and 248 and 1108 before either).
+template <int LX>
+__host__ __device__ constexpr bool rows_m_three() { return fftm::threads(LX) == 192; }
+
 // Bound by vector instructions and the waits between a layer's stages.  1920 x
 // 1080 encoded, 256 layers (272 pairs, of which one workgroup each fills two
 // waves a CU: 2483 us): the layers split into 7 parts 795 us; the transform's
@@ -975,11 +982,11 @@ __device__ __forceinline__ bool row_wanted_m(const DmArgs& a, int ky) {
 // thread's own elements and the next layer's row requested before the
 // transform 640 us.  Held to 168 or 128 registers it spills (1010, 1456 us).
 template <int LX, bool EXACT>
-__global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m(DmArgs a, const float2* __restrict__ twx) {
+__global__ __launch_bounds__(fftm::threads(LX), rows_m_three<LX>() ? 3 : 1) void dm_rows_m(DmArgs a, const float2* __restrict__ twx) {
     using E = fftm::Ends<LX>;
     constexpr int NT = E::NT;
     constexpr int N0 = E::PER0 * E::R0;
-    constexpr bool PREF = N0 <= 16;   // the next layer's values fit in registers
+    constexpr bool PREF = N0 <= 16 && !rows_m_three<LX>();   // the next layer's values fit in registers
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
     const int t = threadIdx.x;
     // XCD-aware, as dm_rows_h

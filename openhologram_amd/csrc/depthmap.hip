@@ -1638,9 +1638,19 @@ extern "C" int oph_depthmap(oph_ctx* ctx, const oph_dm_spec* s, int ncolor, cons
         // parts 49 us, in 8 78).  A part takes every chunks-th layer, which
         // evens out the layers that a column group has pixels in (in runs of
         // 86 layers: 690 us).
-        const int groups4 = (int)((4LL * ctx->cu_count + ngroups - 1) / ngroups);
-        const int groups8 = (int)((8LL * ctx->cu_count + ngroups - 1) / ngroups);
-        int chunks = std::max(groups4, std::min(groups8, nl / 16));
+        const auto per_cu = [&](int n) { return (int)(((long long)n * ctx->cu_count + ngroups - 1) / ngroups); };
+        int chunks = std::max(per_cu(4), std::min(per_cu(8), nl / 16));
+        // Loading the pixels costs as much as some nine layers, so beyond one
+        // per CU no part has fewer than four layers; fewer still up to two or,
+        // on general lengths (fewer rows a thread), three per CU (480 groups of
+        // 3840 rows, 4 layers in 3 parts 168 us, in one 90; 256 groups of 1024,
+        // 8 layers in 4 parts 38, in 2 31; 180 groups of 540, 8 layers in 6
+        // parts 26, in 4 20).  Below 512 rows a workgroup is less than a wave,
+        // and the number of them counts more (32 groups of 256, 64 layers in 8
+        // parts 24, in 32 16).
+        if (mixed || Ny >= 512)
+            chunks = std::min(chunks, std::max({per_cu(1), nl / 4, mixed ? std::min(3 * ctx->cu_count / ngroups, nl / 2)
+                                                                         : std::min(2 * ctx->cu_count / ngroups, nl / 3)}));
         if (chunks > nl) chunks = nl;
         if (chunks < 1) chunks = 1;
         if (mixed) {

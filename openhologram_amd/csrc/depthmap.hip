@@ -1236,6 +1236,31 @@ __global__ __launch_bounds__(B * fftm::threads(LY)) void dm_final_m(DmArgs a, co
 
 // ---- launchers -------------------------------------------------------------------
 
+// The context's entry of a kernel, which is allowed all of the LDS the first
+// time (asked of the runtime once per context, not at every launch)
+oph_ctx::KernelFit& full_lds(oph_ctx* ctx, const void* fn) {
+    for (auto& k : ctx->kernel_fit)
+        if (k.fn == fn) return k;
+    hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    hipGetLastError();
+    ctx->kernel_fit.push_back({fn, 0, 0});
+    return ctx->kernel_fit.back();
+}
+
+// Workgroups of a kernel on a CU with this much dynamic LDS
+template <typename F>
+int rows_resident(oph_ctx* ctx, F kernel, int threads, size_t shm) {
+    auto& k = full_lds(ctx, reinterpret_cast<const void*>(kernel));
+    if (k.resident == 0 || k.shm != shm) {
+        int n = 0;
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, shm);
+        hipGetLastError();
+        k.shm = shm;
+        k.resident = std::max(n, 1);
+    }
+    return k.resident;
+}
+
 template <int LY>
 int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks) {
     const float2* tw = oph_twiddles(ctx, LY);
@@ -1245,9 +1270,7 @@ int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks) {
         return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
     const size_t shm = 2 * ((size_t)fft::skewed_len(LY, 2) + cols_mirror_stride<LY>(a.K)) * sizeof(float2) + words;
     const auto launch = [&](auto* kernel) -> int {
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            160 * 1024);
-        hipGetLastError();
+        full_lds(ctx, reinterpret_cast<const void*>(kernel));
         OPH_LAUNCH(ctx, "dm_cols", kernel, dim3(a.ngroups, chunks), dim3(2 * (LY / 16)), shm, a, chunks, tw);
         return OPH_OK;
     };
@@ -1301,17 +1324,6 @@ int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int gran, int resident) {
     return OPH_OK;
 }
 
-// Workgroups of a kernel on a CU with this much dynamic LDS, which it is
-// allowed to ask for
-template <typename F>
-int rows_resident(F kernel, int threads, size_t shm) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    int n = 0;
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, shm);
-    hipGetLastError();
-    return std::max(n, 1);
-}
-
 template <int LX, int MODE>
 int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
     const float2* tw8 = oph_twiddles(ctx, LX, 8);
@@ -1323,7 +1335,7 @@ int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
     if constexpr (LX >= 512)
         if (fbits && a.w <= LX / 2) kernel = dm_rows_h<LX, MODE, true, true>;   // then ox >= LX/4
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 4, rows_resident(kernel, LX / 8, shm));
+    const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 4, rows_resident(ctx, kernel, LX / 8, shm));
     if (rc) return rc;
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(LX / 8), shm, b, tw8);
@@ -1377,13 +1389,7 @@ int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks) {
         const size_t shm = 2 * ((size_t)cols_m_line<LY>() + cols_mirror_stride<0>(a.K)) * sizeof(float2) + words;
         if (2 * (size_t)fftm::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 + words > 160 * 1024)
             return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
-        static bool attr = false;
-        if (!attr) {
-            hipFuncSetAttribute(reinterpret_cast<const void*>(&dm_cols_m<LY>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            hipGetLastError();
-            attr = true;
-        }
+        full_lds(ctx, reinterpret_cast<const void*>(&dm_cols_m<LY>));
         OPH_LAUNCH(ctx, "dm_cols", dm_cols_m<LY>, dim3(a.ngroups, chunks), dim3(2 * fftm::threads(LY)), shm, a,
                    chunks, tw);
         return OPH_OK;
@@ -1398,12 +1404,12 @@ int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
     constexpr int NT = fftm::threads(LX);
     auto* kernel = a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>;
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, 4, rows_resident(kernel, NT, shm));
+    const int rc = rows_plan(ctx, b, LX, 4, rows_resident(ctx, kernel, NT, shm));
     if (rc) return rc;
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(NT), shm, b, tw);
     if (left > 0) {
-        rows_resident(dm_rows_m_sum<LX>, NT, shm);
+        full_lds(ctx, reinterpret_cast<const void*>(&dm_rows_m_sum<LX>));
         OPH_LAUNCH(ctx, "dm_rows_sum", dm_rows_m_sum<LX>, dim3(2 * left), dim3(NT), shm, b, tw);
     }
     return OPH_OK;

@@ -55,6 +55,14 @@ struct oph_ctx {
     int twm_len[16] = {};  // ... and their lengths
     unsigned* wrp_flag = nullptr;          // device word set by an async WRP call whose lists overflowed
     std::vector<double> host_scratch;      // per-call host tables uploaded to the device
+    // kernels already allowed all of the LDS, and the workgroups of theirs that
+    // fit a CU with shm bytes of it (0: not asked yet)
+    struct KernelFit {
+        const void* fn;
+        size_t shm;
+        int resident;
+    };
+    std::vector<KernelFit> kernel_fit;
 };
 
 // Records an error message on the context and returns code.

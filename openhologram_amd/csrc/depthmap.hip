@@ -87,7 +87,8 @@ struct DmArgs {
     float2* spectrum;              // optional centred spectrum [Ny][Nx]
     double scale;                  // 1/(Nx Ny)
     int n_main, nsplit, per;       // row pairs taken whole; workgroups per further pair, their layers
-    float2* part;                  // ... and their partial sums [pair][nsplit][2][Nx]
+    int nsums;                     // ... and their partial sums:
+    float2* part;                  // [pair][nsums][2][Nx]
     double* fringe;                // h x w (double) or
     float* fringe32;               // h x w (float) or
     float2* field;                 // h x w complex
@@ -470,10 +471,11 @@ __device__ __forceinline__ void lds_copy(E* dst, const E* __restrict__ src, int 
 }
 
 // lo .. hi: the layers taken (MODE 0: in chunks from lo).  part: the sums of
-// both rows are written there instead of being finished.  HALF: the scene's
+// both rows are written there instead of being finished; CHUNKS (MODE 0): of
+// each chunk, one after the other.  HALF: the scene's
 // columns are among the middle half of the grid's, so of a thread's eight
 // inputs the outer four are zeros.
-template <int LX, int MODE, bool PAIR0, bool FBITS, bool HALF>
+template <int LX, int MODE, bool PAIR0, bool FBITS, bool HALF, bool CHUNKS>
 __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __restrict__ tw8, float2* sm, int kya,
                                             int lo, int hi, float2* part) {
     constexpr int TPL = LX / 8;
@@ -483,7 +485,7 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
     constexpr bool SPLIT = LX == 4096;
     constexpr int M0 = HALF ? 2 : 0, M1 = HALF ? 6 : 8;
     float2* line = sm;
-    float2* Sa = sm + PL;             // MODE 0: the chunk sums of both rows
+    float2* Sa = sm + PL;             // MODE 0, not CHUNKS: the chunk sums of both rows
     float2* Sb = Sa + LX;
     float2* tws = sm + PL + (MODE == 0 ? 2 * LX : 0);
     unsigned* amask = reinterpret_cast<unsigned*>(tws + NTW);
@@ -529,7 +531,7 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
             const float usx = a.ux * (float)(sx * sx);
             Ra[m] = dm_transfer<false>(a, (float)txd, tya, usx, sya, a.dK, dKf, sx2);
             Rb[m] = dm_transfer<false>(a, (float)txd, tyb, usx, syb, a.dK, dKf, sx2);
-            Sa[t + m * TPL] = Sb[t + m * TPL] = make_float2(0.f, 0.f);   // at its owner's place
+            if constexpr (!CHUNKS) Sa[t + m * TPL] = Sb[t + m * TPL] = make_float2(0.f, 0.f);   // at its owner's place
         }
     }
     const size_t lstride = gstride * a.ngroups;
@@ -614,7 +616,14 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
         const int ce = min(hi, cs + CH - 1);
         bool anyc = false;
         for (int l = cs; l <= ce; ++l) anyc |= present(l);
-        if (!anyc) continue;
+        float2* sums = part + (size_t)((cs - lo) / CH) * 2 * LX;   // CHUNKS: this chunk's
+        if (!anyc) {
+            if constexpr (CHUNKS) {
+#pragma unroll
+                for (int m = 0; m < 16; ++m) sums[t + m * TPL] = make_float2(0.f, 0.f);
+            }
+            continue;
+        }
         if constexpr (MODE == 0) {
 #pragma unroll
             for (int m = 0; m < 8; ++m) Ta[m] = Tb[m] = make_float2(0.f, 0.f);
@@ -688,12 +697,19 @@ __device__ __forceinline__ void rows_h_body(const DmArgs& a, const float2* __res
                 txd -= rint(txd);
                 const float usx = a.ux * (float)(sx * sx);
                 const float2 ha = dm_transfer<false>(a, (float)txd, tya, usx, sya, K, Kf, sx2);
-                Sa[own] = fft::cadd(Sa[own], fft::cmul(ha, Ta[m]));
                 const float2 hb = dm_transfer<false>(a, (float)txd, tyb, usx, syb, K, Kf, sx2);
-                Sb[own] = fft::cadd(Sb[own], fft::cmul(hb, Tb[m]));
+                if constexpr (CHUNKS) {   // in natural order: row a at kx, row b at -kx
+                    const int kx = tk + m * TPL;
+                    sums[kx] = fft::cmul(ha, Ta[m]);
+                    sums[LX + ((LX - kx) & (LX - 1))] = fft::cmul(hb, Tb[m]);
+                } else {
+                    Sa[own] = fft::cadd(Sa[own], fft::cmul(ha, Ta[m]));
+                    Sb[own] = fft::cadd(Sb[own], fft::cmul(hb, Tb[m]));
+                }
             }
         }
     }
+    if constexpr (CHUNKS) return;
     // the rows in natural order: row a's sum at kx, row b's at -kx (MODE 0: the
     // sums are already in LDS, at their owners' places)
     if constexpr (MODE == 0) {
@@ -750,29 +766,39 @@ __global__ __launch_bounds__(LX / 8, 2) void dm_rows_h(DmArgs a, const float2* _
         lo = a.lo + j * a.per;
         hi = min(a.hi, lo + a.per - 1);
         kya = a.n_main + i;
-        part = a.part + ((size_t)i * a.nsplit + j) * 2 * LX;
+        part = a.part + ((size_t)i * a.nsums + (MODE == 0 ? j * (a.per / 16) : j)) * 2 * LX;
     } else {
         kya = xcd_remap(blockIdx.x, a.n_main);  // 0 .. n_main - 1
     }
+    if constexpr (MODE == 0) {
+        if (part) {
+            if (kya == 0)
+                rows_h_body<LX, MODE, true, FBITS, HALF, true>(a, tw8, sm, 0, lo, hi, part);
+            else
+                rows_h_body<LX, MODE, false, FBITS, HALF, true>(a, tw8, sm, kya, lo, hi, part);
+            return;
+        }
+    }
     if (kya == 0)
-        rows_h_body<LX, MODE, true, FBITS, HALF>(a, tw8, sm, 0, lo, hi, part);
+        rows_h_body<LX, MODE, true, FBITS, HALF, false>(a, tw8, sm, 0, lo, hi, part);
     else
-        rows_h_body<LX, MODE, false, FBITS, HALF>(a, tw8, sm, kya, lo, hi, part);
+        rows_h_body<LX, MODE, false, FBITS, HALF, false>(a, tw8, sm, kya, lo, hi, part);
 }
 
-// The pairs whose layers were split: their partial sums in order (the same
-// additions as a whole pair's), then as a whole pair's
+// The pairs whose layers were split: their partial sums in order (with the
+// chunked recurrence one per chunk, and these are the additions of a whole
+// pair), then as a whole pair's
 template <int LX>
 __global__ __launch_bounds__(LX / 8) void dm_rows_h_sum(DmArgs a, const float2* __restrict__ tw8) {
     constexpr int TPL = LX / 8;
     __shared__ float2 line[fft::padded_len(LX)];
     const int t = threadIdx.x, i = blockIdx.x >> 1, row = blockIdx.x & 1, kya = a.n_main + i;
     const int ky = row == 0 ? kya : kya == 0 ? a.Ny / 2 : a.Ny - kya;
-    const float2* p = a.part + ((size_t)i * a.nsplit * 2 + row) * LX;
+    const float2* p = a.part + ((size_t)i * a.nsums * 2 + row) * LX;
     float2 acc[8];
 #pragma unroll
     for (int m = 0; m < 8; ++m) acc[m] = make_float2(0.f, 0.f);
-    for (int j = 0; j < a.nsplit; ++j)
+    for (int j = 0; j < a.nsums; ++j)
 #pragma unroll
         for (int m = 0; m < 8; ++m) acc[m] = fft::cadd(acc[m], p[(size_t)2 * j * LX + t + m * TPL]);
 #pragma unroll
@@ -998,7 +1024,7 @@ __global__ __launch_bounds__(fftm::threads(LX), rows_m_three<LX>() ? 3 : 1) void
         lo = a.lo + j * a.per;
         hi = min(a.hi, lo + a.per - 1);
         kya = a.n_main + i;
-        part = a.part + ((size_t)i * a.nsplit + j) * 2 * LX;
+        part = a.part + ((size_t)i * a.nsums + j) * 2 * LX;
     } else {
         kya = xcd_remap(blockIdx.x, a.n_main);
     }
@@ -1175,11 +1201,11 @@ __global__ __launch_bounds__(fftm::threads(LX)) void dm_rows_m_sum(DmArgs a, con
     extern __shared__ float2 line[];  // fftm::padded_len(LX)
     const int t = threadIdx.x, i = blockIdx.x >> 1, row = blockIdx.x & 1, kya = a.n_main + i;
     const int ky = row == 0 ? kya : kya == 0 ? a.Ny / 2 : a.Ny - kya;
-    const float2* p = a.part + ((size_t)i * a.nsplit * 2 + row) * LX;
+    const float2* p = a.part + ((size_t)i * a.nsums * 2 + row) * LX;
     float2 acc[EPT];
 #pragma unroll
     for (int m = 0; m < EPT; ++m) acc[m] = make_float2(0.f, 0.f);
-    for (int j = 0; j < a.nsplit; ++j)
+    for (int j = 0; j < a.nsums; ++j)
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
             const int kx = t + m * NT;
@@ -1287,38 +1313,46 @@ int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks) {
 // How the row pairs are spread over the chip, with `resident` workgroups of
 // the row pass on a CU: the first n_main pairs (whole rounds of workgroups)
 // are taken whole, the layers of each of the rest are split over nsplit
-// workgroups of `per` layers, a multiple of gran.  The cost of a choice is its
-// rounds times the layers of each; a part costs three layer times of its own
-// (its set-up, its sums written and read again).  4096 x 2048 encoded needs
-// 514 pairs: 2 rounds and a sixteenth, not 3.  The chunked recurrence is split
-// between its chunks only (gran = 16), which leaves its sums as they are.
-// (A frame of 720 x 540 and 256
-// layers, field: 2.29 -> 0.55 ms.)
-int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int gran, int resident) {
+// workgroups of `per` layers.  The cost of a choice is its rounds times the
+// layers of each; a part costs three layer times of its own (its set-up, its
+// sums written and read again).  4096 x 2048 encoded needs 514 pairs: 2 rounds
+// and a sixteenth, not 3.  (A frame of 720 x 540 and 256 layers, field: 2.29 ->
+// 0.55 ms.)
+//
+// per is a multiple of 4.  For the chunked recurrence (chunk = 16 > 0) it is
+// one of chunk, and each chunk's sums are stored, to be added chunk by chunk as
+// a whole pair's are: a split pair has the bits of a whole one, whatever the
+// size of the chip (the learned correction's BF16 network turns a last bit of
+// its field into 1e-3).  Sums that would take over four times the memory of the
+// layers' rows I are not formed.
+int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int chunk, int resident) {
     const int pairs = a.K - 1, layers = a.hi - a.lo + 1;
-    const int slots = std::max(ctx->cu_count, 1) * resident;
+    const int slots = std::max(ctx->cu_count, 1) * resident, gran = chunk ? chunk : 4;
     a.n_main = pairs;
-    a.nsplit = 1;
+    a.nsplit = a.nsums = 1;
     a.per = layers;
     if (layers < 2) return OPH_OK;   // (0: an empty range)
+    const long long most = 4LL * a.L * a.ngroups * a.K * GROUP;
     long long best = (long long)((pairs + slots - 1) / slots) * layers;
     for (const int n_main : {pairs / slots * slots, 0})
         for (int n = 2; n <= 16; ++n) {
             const int per = ((layers + n - 1) / n + gran - 1) / gran * gran;
             const int parts = (layers + per - 1) / per, left = pairs - n_main;
-            if (parts < 2 || left == 0) continue;
+            const int sums = chunk ? (layers + chunk - 1) / chunk : parts;
+            if (parts < 2 || left == 0 || (long long)left * sums * 2 * LX > most) continue;
             const long long c = (long long)(n_main / slots) * layers +
-                                ((long long)left * parts + slots - 1) / slots * (per + 3);
+                                ((long long)left * parts + slots - 1) / slots * (per + 3 + (chunk ? per / chunk : 0));
             if (c < best) {
                 best = c;
                 a.n_main = n_main;
                 a.nsplit = parts;
+                a.nsums = sums;
                 a.per = per;
             }
         }
     if (a.n_main < pairs) {
         a.part = static_cast<float2*>(
-            oph_scratch(ctx, SLOT_WORK0, (size_t)(pairs - a.n_main) * a.nsplit * 2 * LX * sizeof(float2)));
+            oph_scratch(ctx, SLOT_WORK0, (size_t)(pairs - a.n_main) * a.nsums * 2 * LX * sizeof(float2)));
         if (!a.part) return OPH_ENOMEM;
     }
     return OPH_OK;
@@ -1335,7 +1369,7 @@ int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
     if constexpr (LX >= 512)
         if (fbits && a.w <= LX / 2) kernel = dm_rows_h<LX, MODE, true, true>;   // then ox >= LX/4
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 4, rows_resident(ctx, kernel, LX / 8, shm));
+    const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 0, rows_resident(ctx, kernel, LX / 8, shm));
     if (rc) return rc;
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(LX / 8), shm, b, tw8);
@@ -1404,7 +1438,7 @@ int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
     constexpr int NT = fftm::threads(LX);
     auto* kernel = a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>;
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, 4, rows_resident(ctx, kernel, NT, shm));
+    const int rc = rows_plan(ctx, b, LX, 0, rows_resident(ctx, kernel, NT, shm));
     if (rc) return rc;
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(NT), shm, b, tw);

@@ -258,3 +258,20 @@ def test_depthmap_empty_layer_range(ctx, w, h, Nx, Ny, field_lens, out):
         u = ctx.depthmap(w, h, Nx, Ny, 8e-6, 0.09, 0.11, L, [532e-9], img, dep, out=out, quant_mode=1,
                          field_lens=field_lens, layers=layers)
         assert np.all(u == 0)
+
+
+@pytest.mark.parametrize("w,h,n", [(200, 180, 512), (300, 260, 1024), (60, 50, 128)])
+def test_depthmap_split_pairs_keep_their_bits(ctx, w, h, n):
+    """Equally spaced layers are summed in chunks of 16, one after the other,
+    however the row pairs' layers are spread over workgroups: 64 layers give
+    the same bits as the first 64 of 256 or 1024, the others empty (steps of a
+    power of two, so that the layers' distances are equal)."""
+    img, dep = scenes.depth_scene(w, h, seed=17, colors=1)
+    dep = np.maximum(dep, 192)   # layer 256 - depth: 1 .. 64
+    near, step = 0.09375, 2.0 ** -13
+    ref = None
+    for L in (64, 256, 1024):
+        print(f"case: depthmap {w}x{h} grid {n}x{n} L={L}", flush=True)
+        u = ctx.depthmap(w, h, n, n, 8e-6, near, near + (L - 1) * step, L, [532e-9], img, dep, out="field")
+        ref = u if ref is None else ref
+        assert np.array_equal(u, ref)

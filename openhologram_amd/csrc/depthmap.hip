@@ -1325,13 +1325,13 @@ int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks) {
 // size of the chip (the learned correction's BF16 network turns a last bit of
 // its field into 1e-3).  Sums that would take over four times the memory of the
 // layers' rows I are not formed.
-int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int chunk, int resident) {
+void rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int chunk, int resident) {
     const int pairs = a.K - 1, layers = a.hi - a.lo + 1;
     const int slots = std::max(ctx->cu_count, 1) * resident, gran = chunk ? chunk : 4;
     a.n_main = pairs;
     a.nsplit = a.nsums = 1;
     a.per = layers;
-    if (layers < 2) return OPH_OK;   // (0: an empty range)
+    if (layers < 2) return;   // (0: an empty range)
     const long long most = 4LL * a.L * a.ngroups * a.K * GROUP;
     long long best = (long long)((pairs + slots - 1) / slots) * layers;
     for (const int n_main : {pairs / slots * slots, 0})
@@ -1353,9 +1353,12 @@ int rows_plan(oph_ctx* ctx, DmArgs& a, int LX, int chunk, int resident) {
     if (a.n_main < pairs) {
         a.part = static_cast<float2*>(
             oph_scratch(ctx, SLOT_WORK0, (size_t)(pairs - a.n_main) * a.nsums * 2 * LX * sizeof(float2)));
-        if (!a.part) return OPH_ENOMEM;
+        if (!a.part) {   // no room for them: every pair whole
+            a.n_main = pairs;
+            a.nsplit = a.nsums = 1;
+            a.per = layers;
+        }
     }
-    return OPH_OK;
 }
 
 template <int LX, int MODE>
@@ -1369,8 +1372,7 @@ int launch_dm_rows_h(oph_ctx* ctx, const DmArgs& a) {
     if constexpr (LX >= 512)
         if (fbits && a.w <= LX / 2) kernel = dm_rows_h<LX, MODE, true, true>;   // then ox >= LX/4
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, MODE == 0 ? 16 : 0, rows_resident(ctx, kernel, LX / 8, shm));
-    if (rc) return rc;
+    rows_plan(ctx, b, LX, MODE == 0 ? 16 : 0, rows_resident(ctx, kernel, LX / 8, shm));
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(LX / 8), shm, b, tw8);
     if (left > 0)
@@ -1438,8 +1440,7 @@ int launch_dm_rows_m(oph_ctx* ctx, const DmArgs& a) {
     constexpr int NT = fftm::threads(LX);
     auto* kernel = a.exact ? dm_rows_m<LX, true> : dm_rows_m<LX, false>;
     DmArgs b = a;
-    const int rc = rows_plan(ctx, b, LX, 0, rows_resident(ctx, kernel, NT, shm));
-    if (rc) return rc;
+    rows_plan(ctx, b, LX, 0, rows_resident(ctx, kernel, NT, shm));
     const int left = a.K - 1 - b.n_main;
     OPH_LAUNCH(ctx, "dm_rows", kernel, dim3(b.n_main + left * b.nsplit), dim3(NT), shm, b, tw);
     if (left > 0) {

@@ -236,7 +236,7 @@ int oph_pc_huygens(oph_ctx* ctx, int nx, int ny, double pitch, double lambda, do
  *   X_j = (j - nx/2) pitch, Y_i = (i - ny/2) pitch (row index i is y).
  * The field is evaluated as the separable complex contraction (pixels x
  * points)(points x pixels).  Method OPH_FRESNEL_VALU keeps the chirp factors in
- * FP32 (phases reduced in FP64, FP32 sums of 256 points added in FP64); the
+ * FP32 (phases reduced in FP64, FP32 sums of 64 points added in FP64); the
  * MFMA methods round them to BF16 or FP16 (optionally split hi + lo) and
  * accumulate in FP32.
  * When the points lie on few depth planes (at most 4096 distinct z, >= 256

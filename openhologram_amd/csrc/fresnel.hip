@@ -90,16 +90,23 @@ __global__ void fresnel_prep(const double* x, const double* y, const double* z, 
 //
 // The complex product takes three real ones (sums of A.x B.x, A.y B.y and
 // (A.x + A.y)(B.x + B.y)): a quarter fewer matrix instructions; the sums'
-// rounding grows by 1.4, the error against FP64 from 4.1e-7 to 4.2e-7.
+// rounding grows by 1.4, which the short batches make up for.
+//
+// Error against FP64 in the 2-norm: 2.4e-7 from some 300 points on, at any
+// distance from 20 mm to 2 m (batches of 128: 3.1e-7, of 256: 4.2e-7, of 32:
+// 1.9e-7); 2.2e-7 at 100 points, 1.3e-7 to 1.5e-7 at one, the rounding of two
+// factors of a phase, a sin and a cos each.  A sum per pixel on the vector
+// unit had 4.3e-7 at 0.1 m, 1.5e-6 at 20 mm and 3.0e-7 to 3.2e-7 beyond 0.3 m
+// (there 2.0e-7 at 100 points, 1.0e-7 at one, which two factors cannot reach).
 //
 // Bound by the matrix cores (96 cycles per point and 32 x 32 pixels) and, as
 // vector and matrix instructions do not overlap on a SIMD here, by the
-// generation in turn with them: 1280 x 720 with 20,000 points 1.08 ms (1.30
-// with four products, of which the generation is 0.16; interleaving the two
-// instruction by instruction changed nothing).  A sum per pixel on the vector
-// unit, with its sin and cos, took 4.95 ms.
+// generation in turn with them: 1280 x 720 with 20,000 points 1.14 ms (1.08
+// with batches of 256, 1.10 of 128, 1.20 of 32; 1.30 with four products and
+// batches of 256, of which the generation is 0.16; interleaving the two
+// instruction by instruction changed nothing).  A sum per pixel took 4.95 ms.
 
-constexpr int F32_PTS = 16, F32_BATCH = 256;
+constexpr int F32_PTS = 16, F32_BATCH = 64;
 constexpr int F32_R = 64, F32_C = 128;
 
 struct F32Args {

@@ -141,3 +141,20 @@ def test_fresnel_f32_contraction_edges(ctx, nx, ny, n):
     err = rel_l2(U, O.fresnel(nx, ny, 8e-6, 532e-9, x, y, z, a, ph))
     print("rel-L2", err)
     assert err < 2e-6
+
+
+@pytest.mark.parametrize("z0", [0.1, 0.3, 0.5, 1.0, 2.0])
+def test_fresnel_f32_error_at_any_distance(ctx, z0):
+    """The single-precision method's error against FP64 does not depend on the
+    distance.  Bound: a sum per pixel (one rounded phase and 1,000 products in
+    batches of 256) has 3.2e-7 beyond 0.3 m, and the contraction, which rounds
+    two phases, may not have more."""
+    print(f"case: fresnel f32 z {z0}", flush=True)
+    g = scenes.SplitMix64(1000)
+    n = 1000
+    x, y, z = g.uniform(n, -5e-3, 5e-3), g.uniform(n, -5e-3, 5e-3), g.uniform(n, z0, 1.02 * z0)
+    a, ph = g.uniform(n), g.uniform(n, 0.0, 2 * np.pi)
+    U = ctx.fresnel(300, 200, 8e-6, 532e-9, x, y, z, a, ph, method="valu")
+    err = rel_l2(U, O.fresnel(300, 200, 8e-6, 532e-9, x, y, z, a, ph))
+    print("rel-L2", err)
+    assert err < 3.2e-7

@@ -109,6 +109,14 @@ __global__ void fresnel_prep(const double* x, const double* y, const double* z, 
 constexpr int F32_PTS = 16, F32_BATCH = 64;
 constexpr int F32_R = 64, F32_C = 128;
 
+// An amplitude so large that products of its factors may overflow where the
+// point's own value does not (or infinite, or NaN: inf - inf in the three sums
+// would be NaN where the point adds +-inf).  Such points are left out of the
+// contraction and added per pixel.
+__device__ __forceinline__ bool f32_huge(float a) {
+    return (__builtin_bit_cast(unsigned, a) & 0x7FFFFFFFu) > 0x7149F2CAu;   // 1e30
+}
+
 struct F32Args {
     const FrPoint* pts;
     int64_t npad, chunk;   // multiples of KC
@@ -124,7 +132,10 @@ struct F32Lds {
 
 __global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
     __shared__ F32Lds lds[2];
+    __shared__ int any_huge;
     const int lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) any_huge = 0;
+    __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row0 = blockIdx.y * F32_R, col0 = blockIdx.x * F32_C;
     const double Y = (row0 + lane - a.ny / 2) * a.p;
@@ -152,6 +163,10 @@ __global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
 #pragma unroll
         for (int k = 0; k < PW; ++k) {
             const int pt = wave * PW + k;
+            if (f32_huge(q[k].a)) {   // (the same for the whole wave)
+                any_huge = 1;
+                q[k].a = 0.f;
+            }
             const double dy = Y - q[k].y, d0 = X0 - q[k].x, d1 = X1 - q[k].x;
             const float ty = (float)frac_turns(fma(q[k].c, dy * dy, (double)q[k].f0));
             const float t0 = (float)frac_turns(q[k].c * (d0 * d0)), t1 = (float)frac_turns(q[k].c * (d1 * d1));
@@ -207,6 +222,23 @@ __global__ __launch_bounds__(256, 2) void fresnel_f32(F32Args a) {
             }
         }
     }
+    __syncthreads();
+    if (any_huge)
+        for (int i = 0; i < nch * F32_PTS; ++i) {
+            const FrPoint h = a.pts[pb + i];
+            if (!f32_huge(h.a)) continue;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const double dx = (col0 + wc + 32 * b + (lane & 31) - a.nx / 2) * a.p - h.x;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const double dy = (row0 + wr + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3) - a.ny / 2) * a.p - h.y;
+                    const float t = (float)frac_turns(fma(h.c, fma(dx, dx, dy * dy), (double)h.f0));
+                    sre[b][v] += (double)(h.a * cos_turns(t));
+                    sim[b][v] += (double)(h.a * sin_turns(t));
+                }
+            }
+        }
     // register v of a lane: row 8 (v/4) + 4 (lane/32) + v%4, column lane%32
     float2* dst = a.out + (size_t)blockIdx.z * a.nx * a.ny;
 #pragma unroll

@@ -158,3 +158,24 @@ def test_fresnel_f32_error_at_any_distance(ctx, z0):
     err = rel_l2(U, O.fresnel(300, 200, 8e-6, 532e-9, x, y, z, a, ph))
     print("rel-L2", err)
     assert err < 3.2e-7
+
+
+@pytest.mark.parametrize("amp", [np.inf, -np.inf, 3e38])
+@pytest.mark.parametrize("n,at", [(1, 0), (100, 37), (3000, 2999)])
+def test_fresnel_f32_huge_amplitudes(ctx, n, at, amp):
+    """A point of infinite amplitude adds +-inf to both parts of every pixel
+    (whatever the other points add), one near the largest float its finite
+    value: no NaN from the contraction's intermediate sums.  Signs are compared
+    where the cosine or sine is above 1e-3 (phases agree to 1e-6)."""
+    print(f"case: fresnel f32 amplitude {amp} at {at} of {n}", flush=True)
+    x, y, p, z, a, ph = scenes.fresnel_points(n, planes=5, seed=n, half=0.6e-3)
+    a = a.copy()
+    a[at] = amp
+    U = ctx.fresnel(150, 70, 8e-6, 532e-9, x, y, z, a, ph, method="valu")
+    one = O.fresnel(150, 70, 8e-6, 532e-9, x[at:at + 1], y[at:at + 1], z[at:at + 1], np.ones(1), ph[at:at + 1])
+    if np.isinf(amp):
+        for got, unit in ((U.real, one.real), (U.imag, one.imag)):
+            ok = np.abs(unit) > 1e-3
+            assert np.all(np.isinf(got[ok])) and np.all(np.sign(got[ok]) == np.sign(unit[ok] * amp))
+    else:
+        assert rel_l2(U / np.float32(amp), one) < 2e-6

@@ -207,39 +207,50 @@ __device__ __forceinline__ void rs_tile_direct(const RsArgs& a, RsStage& S) {
 // distance at 8 um for most points).  The factors' phases are polynomials of
 // the pixel offset j = -15.5 .. 15.5, FP32 with the linear coefficient,
 // reduced modulo 2 in FP64 (2 j is odd, so j 2 is a whole turn), split so
-// that its high part times j is exact.
+// that its high part times j is exact, and so is that plus the high part of
+// the centre phase: one rounding for each factor's phase.
 //
 // A wave owns a block.  It takes 64 points at a time: each lane forms one
 // point's record for the block in FP64, then the wave contracts them in
 // pairs (lanes 0-31 the factors of the even point, 32-63 of the odd one).
-// Points out of the expansion's range (RsRange) take the FP64 phase per
-// pixel; a tile with more than 1/8 such points runs rs_tile_direct.
+// Points out of the expansion's range (rs_terms) take the FP64 phase per
+// pixel; a tile with more than 1/8 such points, by the sample, runs
+// rs_tile_direct.  512^2 with 2000 points at 100 mm, a share of them at 3 mm:
+// none 91 us, 6% 115, 9% 128, 11% 193 (half of the tiles direct), 13% 233,
+// half 309, where the direct form for every tile took 455 to 660.
 //
 // The complex product takes three real ones instead of four, which costs the
-// sums a factor 1.4 in rounding; they are formed over 64 points at a time and
-// added per batch, which more than makes up for it (1000 points at 1024^2:
-// 3.6e-7 from FP64, 7.1e-7 with one sum per pixel of 1000 products).
+// sums a factor 1.4 in rounding; they are formed over RS_BATCH points at a
+// time and added per batch, which more than makes up for it.  Error against
+// FP64 in the 2-norm at 1000 points: 2.2e-7 at 0.1 m, 2.0e-7 beyond 0.3 m
+// (batches of 64: 3.5e-7 and 3.1e-7); one sum per pixel of 1000 products 6.6e-7
+// and 5.8e-7.  At 100 points 2.1e-7 and 1.9e-7 (per pixel 3.9e-7 and 2.0e-7),
+// at one 1.4e-7 and 1.3e-7 (2.3e-7 and 0.9e-7: the two factors' rounding is
+// what is left, beyond 0.3 m more than that of one phase per pixel).
 // Bound by matrix and vector instructions in turn (they do not overlap on a
-// SIMD here).  1024^2 with 1000 points at 100 mm: 161 us, of which 20 us are
-// the factors; 4096 x 2160 with 1453 points at 0.462 um: 1.71 ms.  A sin and
+// SIMD here).  1024^2 with 1000 points at 100 mm: 174 us (162 in batches of
+// 64); 4096 x 2160 with 1453 points at 0.462 um: 1.85 ms (1.72).  A sin and
 // cos per pixel and point took 457 us and 4.40 ms.  Records in the order of
 // their terms are worth 8% (a pair takes the larger count of its two).
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int RS_TERMS = 5;
+constexpr int RS_TERMS = 5, RS_BATCH = 16;
 
 struct RsRec {
     float4 x, y;   // high and low linear, quadratic, cubic coefficient along x and y
     float4 c;      // phase at the block centre, amplitude, quartic coefficients
     float4 m;      // 2 dx, 2 dy, delta, eta
+    float c_lo;    // the centre phase's low part (the high part is a multiple of 2^-20)
+    float pad[3];
 };
 
 // Terms the contraction needs for one point and block (0: out of range).
 // ax, ay: largest A and B over the block; hm: largest half extent.  The
-// thresholds keep the first dropped term, (delta A' B')^k / k! of root mean
-// square 1/(2 k + 1) over the block, and the dropped phase terms (fourth
-// order in q, fifth in the offset) below 3e-7 rad.
+// thresholds keep the first dropped term, (delta A' B')^k / k!, whose root mean
+// square over the block's 32 x 32 offsets is d^k / k! (32/31)^(2 k) / (2 k + 1),
+// and the dropped phase terms (fourth order in q, fifth in the offset) below
+// 3e-7 rad.
 __device__ __forceinline__ int rs_terms(float r0, float yr, float c2, float ax, float ay, float dm, float hm,
                                         float inv_l, bool huygens) {
     const float u = (ax + ay) * yr * yr;
@@ -248,7 +259,7 @@ __device__ __forceinline__ int rs_terms(float r0, float yr, float c2, float ax, 
     const float e5 = 8.f * c3 * dm * (hm * hm) * (hm * hm) * hm;
     if (!(e4 + e5 <= 5e-8f) || (huygens && !(u <= 1.5e-3f))) return 0;
     const float d = 12.5663706f * c2 * ax * ay;
-    return d <= 6e-7f ? 1 : d <= 2e-3f ? 2 : d <= 2.5e-2f ? 3 : d <= 9e-2f ? 4 : d <= 0.2f ? 5 : 0;
+    return d <= 6e-7f ? 1 : d <= 1.5e-3f ? 2 : d <= 2.1e-2f ? 3 : d <= 8e-2f ? 4 : d <= 0.18f ? 5 : 0;
 }
 
 template <bool HUYGENS>
@@ -294,7 +305,9 @@ __device__ __forceinline__ void rs_block_mfma(const RsArgs& a, RsRec* rec, int c
                 float qx, qy;
                 q.x = axis(dx, a.px, dxf, pxf, qx);
                 q.y = axis(dy, spy, dyf, pyf, qy);
-                q.c = make_float4((float)(t0 - rint(t0)), am, qx, qy);
+                const double tf = t0 - rint(t0), th = rint(tf * 1048576.0) * (1.0 / 1048576.0);
+                q.c = make_float4((float)th, am, qx, qy);
+                q.c_lo = (float)(tf - th);
                 q.m = make_float4(2.f * dxf, 2.f * dyf, -12.5663706f * c2, 0.75f * y2);
                 terms = rs_terms((float)rr, yrf, c2, hx * fmaf(2.f, fabsf(dxf), hx), hy * fmaf(2.f, fabsf(dyf), hy),
                                  fmaxf(fabsf(dxf), fabsf(dyf)), hm, inv_l, HUYGENS);
@@ -318,15 +331,21 @@ __device__ __forceinline__ void rs_block_mfma(const RsArgs& a, RsRec* rec, int c
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         const int cnt = first[RS_TERMS + 1];
         // a complex product from three real ones: sums of fr er, fi ei and
-        // (fr + fi)(er + ei), over these 64 points
+        // (fr + fi)(er + ei), over RS_BATCH points
         f32x16 s1 = (f32x16)0.f, s2 = (f32x16)0.f, s3 = (f32x16)0.f;
+        auto add_batch = [&]() {
+            re += s1 - s2;
+            im += s3 - (s1 + s2);
+            s1 = s2 = s3 = (f32x16)0.f;
+        };
         for (int p = 0; p < cnt; p += 2) {
+            if (p > 0 && p % RS_BATCH == 0) add_batch();
             const RsRec q = rec[p + (lane >> 5)];
-            float mx = j * q.x.x, my = j * q.y.x;
+            float mx = j * q.x.x, my = fmaf(j, q.y.x, q.c.x);   // exact, both
             mx -= rintf(mx);
             my -= rintf(my);
             const float tx = fmaf(fmaf(fmaf(fmaf(q.c.z, j, q.x.w), j, q.x.z), j, q.x.y), j, mx);
-            const float ty = fmaf(fmaf(fmaf(fmaf(q.c.w, j, q.y.w), j, q.y.z), j, q.y.y), j, my + q.c.x);
+            const float ty = fmaf(fmaf(fmaf(fmaf(q.c.w, j, q.y.w), j, q.y.z), j, q.y.y), j, q.c_lo) + my;
             float er = cos_turns(tx), ei = sin_turns(tx);
             float fr = q.c.y * cos_turns(ty), fi = q.c.y * sin_turns(ty);
             if (HUYGENS) {
@@ -366,10 +385,9 @@ __device__ __forceinline__ void rs_block_mfma(const RsArgs& a, RsRec* rec, int c
                 }
             }
         }
+        add_batch();
         // points out of range: FP64 phase per pixel (register v of a lane is
         // row 8 (v/4) + 4 (lane/32) + v%4, column lane%32)
-        re += s1 - s2;
-        im += s3 - (s1 + s2);
         uint64_t far = __ballot(terms == 0 && base + lane < p_end);
         while (far) {
             const int k = __ffsll((long long)far) - 1;

@@ -311,6 +311,10 @@ __device__ __forceinline__ void rs_block_mfma(const RsArgs& a, RsRec* rec, int c
                 q.m = make_float4(2.f * dxf, 2.f * dyf, -12.5663706f * c2, 0.75f * y2);
                 terms = rs_terms((float)rr, yrf, c2, hx * fmaf(2.f, fabsf(dxf), hx), hy * fmaf(2.f, fabsf(dyf), hy),
                                  fmaxf(fabsf(dxf), fabsf(dyf)), hm, inv_l, HUYGENS);
+                // (an amplitude so large that the sums' products may overflow
+                // where the point's value does not, infinite or NaN: inf - inf
+                // would be NaN where the point adds +-inf)
+                if (!(fabsf(am) <= 1e30f)) terms = 0;
                 if (terms == 0) q = {};   // summed per pixel below
             }
             // records in order of their number of terms, so that the two points

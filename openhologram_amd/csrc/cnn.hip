@@ -92,7 +92,6 @@ struct ConvArgsT {
     const TO* res;        // residual added after the bias (or null), [..][COUT]
     TO* out;              // [B][H][W][COUT]
     int B, H, W;
-    int relu;
 };
 
 // Tiled forward convolution.  A workgroup of 4 waves owns an 8-row x 32-
@@ -230,9 +229,7 @@ __global__ __launch_bounds__(64 * CT_WAVES) void conv3x3_fwd(ConvArgsT<TI, TO> a
             TO o[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float v = acc[h][4 * q + i] + bias[i];
-                if (a.relu) v = fmaxf(v, 0.f);
-                o[i] = (TO)(v + rv[h][q][i]);
+                o[i] = (TO)(acc[h][4 * q + i] + bias[i] + rv[h][q][i]);
             }
             TO* dst = a.out + (img + (size_t)y * a.W + x) * COUT + ch0;
             if constexpr (NV == 4) {
@@ -1518,8 +1515,8 @@ __global__ __launch_bounds__(256, 2) void tail_fwd(TailArgs a) {
 
 template <int CIN, int COUT, typename TI = float, typename TO = float>
 int conv_fwd(oph_ctx* ctx, const TI* in, const bf16x8* wf, const float* bias,
-             const typename std::remove_reference<TO>::type* res, TO* out, int B, int H, int W, int relu) {
-    ConvArgsT<TI, TO> a{in, wf, bias, res, out, B, H, W, relu};
+             const typename std::remove_reference<TO>::type* res, TO* out, int B, int H, int W) {
+    ConvArgsT<TI, TO> a{in, wf, bias, res, out, B, H, W};
     const dim3 grid((unsigned)((W + CT_W - 1) / CT_W), (unsigned)((H + CT_H - 1) / CT_H), (unsigned)B);
     if (B > 65535 || grid.y > 65535) return oph_fail(ctx, OPH_EINVAL, "convolution batch or height too large");
     OPH_LAUNCH(ctx, "conv3x3_fwd", (conv3x3_fwd<CIN, COUT, TI, TO>), grid, dim3(64 * CT_WAVES), 0, a);
@@ -1572,7 +1569,7 @@ int resblock_f32_run(oph_ctx* ctx, const Rb32Args& a, float* gw2 = nullptr, floa
 // dX = conv(dY, flipped/transposed W): input channels COUT, output CIN
 template <int CIN, int COUT>
 int conv_dx(oph_ctx* ctx, const float* dy, const bf16x8* wfrag, float* dx, int B, int H, int W) {
-    return conv_fwd<COUT, CIN>(ctx, dy, wfrag, nullptr, nullptr, dx, B, H, W, 0);
+    return conv_fwd<COUT, CIN>(ctx, dy, wfrag, nullptr, nullptr, dx, B, H, W);
 }
 
 constexpr int ksteps(int cin) { return (9 * cin + 15) / 16; }
@@ -1675,13 +1672,13 @@ int forward(oph_ctx* ctx, oph_cnn* net, const float* x, int B, int H, int W, Act
     const bf16x8* WF = net->wf;
     int rc;
     if (net->wf_rev != net->params_rev && (rc = pack(ctx, net, false))) return rc;
-    if ((rc = conv_fwd<2, 32>(ctx, x, WF + F.head(), P + L.head_b(), nullptr, A.h[0], B, H, W, 0))) return rc;
+    if ((rc = conv_fwd<2, 32>(ctx, x, WF + F.head(), P + L.head_b(), nullptr, A.h[0], B, H, W))) return rc;
     for (int b = 0; b < net->blocks; ++b) {
         if ((rc = resblock_f32_run(ctx, {A.h[b], nullptr, keep ? A.a[b + 1] : nullptr, A.h[b + 1], nullptr, nullptr,
                                          WF + F.conv1(b), WF + F.conv2(b), P + L.b1(b), P + L.b2(b), B, H, W})))
             return rc;
     }
-    return conv_fwd<32, 2>(ctx, A.h[net->blocks], WF + F.tail(), P + L.tail_b(), x, A.y, B, H, W, 0);
+    return conv_fwd<32, 2>(ctx, A.h[net->blocks], WF + F.tail(), P + L.tail_b(), x, A.y, B, H, W);
 }
 
 // Inference forward with BF16 activations between layers: head conv, the
@@ -1697,7 +1694,7 @@ int forward_bf16(oph_ctx* ctx, oph_cnn* net, const float* x, float* y, int B, in
     auto h = [&](int b) { return reinterpret_cast<__bf16*>(A.h[b]); };
     // with blocks, the first one computes the head on its staged tiles
     if (net->blocks == 0 &&
-        (rc = conv_fwd<2, 32, float, __bf16>(ctx, x, WF + F.head(), P + L.head_b(), nullptr, h(0), B, H, W, 0)))
+        (rc = conv_fwd<2, 32, float, __bf16>(ctx, x, WF + F.head(), P + L.head_b(), nullptr, h(0), B, H, W)))
         return rc;
     // persistent: two workgroups per CU (LDS-bound), each walking tiles
     const int64_t ntiles = (int64_t)((W + RB_TW - 1) / RB_TW) * ((H + RB_TH - 1) / RB_TH) * B;

@@ -401,7 +401,8 @@ __global__ __launch_bounds__(LX / 16) void dm_rows(DmArgs a, const float2* __res
 // A scene in the middle half of the columns (HALF) loads half of the row and
 // spares the first butterfly's operations on zeros; rows of 4096 go through
 // line_r8_split4096 (together 1700 -> 1430 us at 4096 x 2048 encoded, 256
-// layers; shorter rows, of at most four waves, keep the stage order).
+// layers; shorter rows keep the stage order and with it the bits of the learned
+// pipeline's fields, and were not timed split).
 //
 // MODE 0: equally spaced layers (no field lens).  The transfer of
 // layer l is H_l = exp(i 2 pi z_l Phi(kx, ky)) with one Phi for all layers,
@@ -1287,14 +1288,21 @@ int rows_resident(oph_ctx* ctx, F kernel, int threads, size_t shm) {
     return k.resident;
 }
 
+// The scenes that the column pass takes: its lines and four columns of pixels
+// within the LDS.  The pixels are in registers, so the kernels need less; the
+// limit is the call's and stays.
+size_t cols_limit(int line, const DmArgs& a, size_t words) {
+    return 2 * (size_t)line * sizeof(float2) + (size_t)a.h * GROUP * 4 + words;
+}
+
 template <int LY>
 int launch_dm_cols(oph_ctx* ctx, const DmArgs& a, int chunks) {
     const float2* tw = oph_twiddles(ctx, LY);
     if (!tw) return OPH_ENOMEM;
     const size_t words = (size_t)((a.L + 32) / 32) * 4;
-    if (2 * fft::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 + words > 160 * 1024)
-        return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
     const size_t shm = 2 * ((size_t)fft::skewed_len(LY, 2) + cols_mirror_stride<LY>(a.K)) * sizeof(float2) + words;
+    if (std::max(shm, cols_limit(fft::padded_len(LY), a, words)) > 160 * 1024)
+        return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
     const auto launch = [&](auto* kernel) -> int {
         full_lds(ctx, reinterpret_cast<const void*>(kernel));
         OPH_LAUNCH(ctx, "dm_cols", kernel, dim3(a.ngroups, chunks), dim3(2 * (LY / 16)), shm, a, chunks, tw);
@@ -1423,7 +1431,7 @@ int launch_dm_cols_m(oph_ctx* ctx, const DmArgs& a, int chunks) {
     } else {
         const size_t words = (size_t)((a.L + 32) / 32) * 4;
         const size_t shm = 2 * ((size_t)cols_m_line<LY>() + cols_mirror_stride<0>(a.K)) * sizeof(float2) + words;
-        if (2 * (size_t)fftm::padded_len(LY) * sizeof(float2) + (size_t)a.h * GROUP * 4 + words > 160 * 1024)
+        if (std::max(shm, cols_limit(fftm::padded_len(LY), a, words)) > 160 * 1024)
             return oph_fail(ctx, OPH_ENOTSUP, "scene height %d too large for the column pass", a.h);
         full_lds(ctx, reinterpret_cast<const void*>(&dm_cols_m<LY>));
         OPH_LAUNCH(ctx, "dm_cols", dm_cols_m<LY>, dim3(a.ngroups, chunks), dim3(2 * fftm::threads(LY)), shm, a,

@@ -29,8 +29,8 @@ VALU_LANE_OPS = 256 * 4 * 16 * 2.4e9      # VALU issue peak, unpacked FP32 lane-
 # SQ_INSTS_VALU ... -- python3 bench.py --workload <rs|wrp> --only --steps 2
 # --warmup 1 --no-cpu` commands recorded there); valid for the kernels as
 # built at that time: re-measure after changing them.
-PROFILED_VALU_INSTS = {"rs_accumulate": 31413884, "asm_cols": 25980928, "wrp_gather": 23896245}
-PROFILED_RS_MFMA = 3565554                 # of rs_accumulate's, v_mfma_f32_32x32x2f32 (SQ_INSTS_MFMA)
+PROFILED_VALU_INSTS = {"rs_accumulate": 37112514, "asm_cols": 25980928, "wrp_gather": 23896248}
+PROFILED_RS_MFMA = 3702279                 # of rs_accumulate's, v_mfma_f32_32x32x2f32 (SQ_INSTS_MFMA)
 PROFILE_SOURCES = {"valu": "profiles/valu_counters_rs_wrp.md (rocprofv3 --pmc SQ_INSTS_VALU)",
                    "traffic": "profiles/hbm_traffic_wrp_depthmap.md (rocprofv3 --pmc FETCH_SIZE, then "
                               "WRITE_SIZE, calibrated on copy_kernel)"}
@@ -254,7 +254,7 @@ DM_KERNELS = ["dm_index", "dm_zero", "dm_cols", "dm_rows", "dm_rows_sum", "dm_fi
 # the RGB workload): wave-level VALU instructions (SQ_INSTS_VALU) and HBM
 # bytes (FETCH_SIZE + WRITE_SIZE, calibrated as PROFILED_TRAFFIC) per launch,
 # from the `--workload depthmap --only --steps 2 --warmup 1 --no-cpu` runs.
-PROFILED_DM_ROWS = {"valu_insts": 4.831e8, "traffic": (962.1 + 17.0) * 2**20}
+PROFILED_DM_ROWS = {"valu_insts": 4.830e8, "traffic": (962.1 + 17.0) * 2**20}
 
 
 def bench_depthmap(ctx, args):

@@ -281,7 +281,7 @@ typedef struct oph_dm_spec {
     int default_q;         /* DEFAULT_DEPTH_QUANTIZATION (256) */
     double field_lens;     /* focal length of the field lens; <= 0: none */
     double rho_re, rho_im; /* the random-phase factor (1, 0 when RANDOM_PHASE = 0) */
-    int layer_lo, layer_hi;/* rendered layers, 1-based inclusive; 0 = all */
+    int layer_lo, layer_hi;/* rendered layers, 1-based inclusive; 0 = all; none in the range: zeros */
 } oph_dm_spec;
 
 /* output of oph_depthmap (one of; ORed into flags) */

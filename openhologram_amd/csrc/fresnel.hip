@@ -101,8 +101,9 @@ __global__ void fresnel_prep(const double* x, const double* y, const double* z, 
 //
 // Bound by the matrix cores (96 cycles per point and 32 x 32 pixels) and, as
 // vector and matrix instructions do not overlap on a SIMD here, by the
-// generation in turn with them: 1280 x 720 with 20,000 points 1.14 ms (1.08
-// with batches of 256, 1.10 of 128, 1.20 of 32; 1.30 with four products and
+// generation in turn with them: 1280 x 720 with 20,000 points 1.16 ms (before
+// the test for huge amplitudes 1.14, with batches of 256 1.08, of 128 1.10, of
+// 32 1.20; 1.30 with four products and
 // batches of 256, of which the generation is 0.16; interleaving the two
 // instruction by instruction changed nothing).  A sum per pixel took 4.95 ms.
 

@@ -216,8 +216,8 @@ __device__ __forceinline__ void rs_tile_direct(const RsArgs& a, RsStage& S) {
 // Points out of the expansion's range (rs_terms) take the FP64 phase per
 // pixel; a tile with more than 1/8 such points, by the sample, runs
 // rs_tile_direct.  512^2 with 2000 points at 100 mm, a share of them at 3 mm:
-// none 91 us, 6% 115, 9% 128, 11% 193 (half of the tiles direct), 13% 233,
-// half 309, where the direct form for every tile took 455 to 660.
+// none 92 us, 6% 115, 9% 127, 11% 189, 13% 231, half 307, all 400, where the
+// direct form for every tile took 455 to 867.
 //
 // The complex product takes three real ones instead of four, which costs the
 // sums a factor 1.4 in rounding; they are formed over RS_BATCH points at a
